@@ -123,7 +123,7 @@ __global__ void k_af_products(Dims d, const double* __restrict__ J, const double
 }
 
 // k_af_rhs for stages 0 and 1, K-marching: a workgroup owns a 64 x 4 (I x J) column of cells
-// over RK_KC consecutive K planes and keeps the last three planes of the stage inputs (one-cell
+// over kc consecutive K planes and keeps the last three planes of the stage inputs (one-cell
 // halo) in LDS, so the twelve edge neighbours of the cross terms come from LDS and every input
 // value is fetched from HBM once per column.  The metric products come from the per-stage
 // arrays of k_af_products (equal, bit for bit, to the products k_af_rhs forms); those at K+-1
@@ -131,7 +131,7 @@ __global__ void k_af_products(Dims d, const double* __restrict__ J, const double
 // TH selects ITER_T (RLES/iter_t.f90:49-55): re is PE, the stage-1 source is
 // 2 PE J^-1/dt T - 3 PE ADV + PE ADV_NM1 + DIFT + DD (A.nl = ADV, A.nl1 = ADV_NM1,
 // A.dif = DIFT) and BCT's wall fold adds 2 AW T_WALL (bct.f90:16-19).
-constexpr int RK_KC = 16;
+constexpr int RK_RES = 768;  // workgroups resident at a time (three per CU)
 
 // With DR set (stages 0 and 1 of the FP32 correction form, qform on) the kernel stores, as FP32
 // in SU's memory, the residual of the stage's line system at the stage input instead of Q:
@@ -140,7 +140,7 @@ constexpr int RK_KC = 16;
 // values BCU gives them before the sweep.  The line sweep then solves for the stage's change
 // delta = x - x_in in FP32 and adds it to the FP64 field.
 template <int S, bool TH, int NCV = 3, bool DR = false>
-__global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, AFArgs A,
+__global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
                                                    const double* const* __restrict__ P,
                                                    const double* __restrict__ ap0, double re,
                                                    const double* const* __restrict__ fa,
@@ -152,8 +152,8 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, AFArgs A,
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * RK_KC;
-  const int k1 = min(k0 + RK_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int q0 = (ty + 1) * SF_W + tx + 1;
   const long sj = d.sj, sk = d.sk;
@@ -854,16 +854,17 @@ int fvm_k_iter_u(FvmCtx* c) {
       const int qf = (s < 2 && chunked && c->af_scan[s]) ? 1 : 0;
       const double* const* fas = (const double* const*)c->dfa[s];
       const int dz = c->dd2_zero ? 1 : 0;
-      const dim3 gk((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + RK_KC - 1) / RK_KC);
+      const int kc = march_planes(d, RK_RES);
+      const dim3 gk = march_grid(d, kc);
       if (s == 0) {
         ProfScope pk(c, "k_af_rhs_i");
         auto kern = (qf && f32) ? k_af_rhs_km<0, false, 3, true> : k_af_rhs_km<0, false, 3, false>;
-        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, A, (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, fn_alias);
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, fn_alias);
       }
       if (s == 1) {
         ProfScope pk(c, "k_af_rhs_j");
         auto kern = (qf && f32) ? k_af_rhs_km<1, false, 3, true> : k_af_rhs_km<1, false, 3, false>;
-        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, A, (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0);
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0);
       }
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0, c->prm.re, fas, qf, dz);
       HIP_CHECK(hipGetLastError());
@@ -953,12 +954,13 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
       const int qf = scan ? 1 : 0;
       const double* const* fas = (const double* const*)c->dfa[s];
       const int dz = c->dd2_zero ? 1 : 0;
-      const dim3 gk((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + RK_KC - 1) / RK_KC);
+      const int kc = march_planes(d, RK_RES);
+      const dim3 gk = march_grid(d, kc);
       if (s == 0)
-        hipLaunchKernelGGL((k_af_rhs_km<0, false, 1>), gk, kBlk, 0, st, d, A,
+        hipLaunchKernelGGL((k_af_rhs_km<0, false, 1>), gk, kBlk, 0, st, d, kc, A,
                            (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, 0);
       if (s == 1)
-        hipLaunchKernelGGL((k_af_rhs_km<1, false, 1>), gk, kBlk, 0, st, d, A,
+        hipLaunchKernelGGL((k_af_rhs_km<1, false, 1>), gk, kBlk, 0, st, d, kc, A,
                            (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0);
       if (s == 2)
         hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm,
@@ -1090,13 +1092,14 @@ int fvm_k_iter_t(FvmCtx* c) {
   }
   A.ufar = c->tfar;
   const dim3 gi((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, d.nk - 1);
-  const dim3 gk((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + RK_KC - 1) / RK_KC);
+  const int kc = march_planes(d, RK_RES);
+      const dim3 gk = march_grid(d, kc);
   for (int s = 0; s < 3; ++s) {
     {
       ProfScope ps(c, "t_rhs");
       const double* const* fas = (const double* const*)c->dfa[s];
-      if (s == 0) hipLaunchKernelGGL((k_af_rhs_km<0, true>), gk, kBlk, 0, st, d, A, (const double* const*)c->dafp[0], c->ap0t, c->pe, fas, 1, 0);
-      if (s == 1) hipLaunchKernelGGL((k_af_rhs_km<1, true>), gk, kBlk, 0, st, d, A, (const double* const*)c->dafp[1], c->ap0t, c->pe, fas, 1, 0);
+      if (s == 0) hipLaunchKernelGGL((k_af_rhs_km<0, true>), gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0t, c->pe, fas, 1, 0);
+      if (s == 1) hipLaunchKernelGGL((k_af_rhs_km<1, true>), gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0t, c->pe, fas, 1, 0);
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0t, c->pe, fas, 0, c->dd2_zero ? 1 : 0);
       HIP_CHECK(hipGetLastError());
     }

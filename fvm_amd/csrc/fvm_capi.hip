@@ -333,7 +333,7 @@ static int create_impl(const fvm_params* prm, const double* xg, const double* yg
   long nblk = (long)((prm->ni - 1 + 63) / 64) * ((prm->nj - 1 + 3) / 4) * (prm->nk - 1);
   // AF chunk iteration: one partial pair per workgroup, chunks of 8 lines
   long nafw = 3L * ((std::max(prm->ni, prm->nj) + 7) / 8 + 1) * std::max(prm->nj, prm->nk) + 8;
-  c->nred = (int)std::max(std::max(nblk * 2, 2 * nafw), 4096L);
+  c->nred = (int)std::max(std::max(nblk * 3, 2 * nafw), 4096L);
   r |= dalloc(c, &c->red, c->nred);
   c->ncflpart = (int)nblk;
   r |= dalloc(c, &c->cflpart, nblk);

@@ -146,6 +146,31 @@ struct FvmCtx {
   std::vector<void*> allocs;
 };
 
+// K planes per workgroup of a K-marching stencil kernel, and its launch grid (64 x 4 (I x J) tiles
+// by groups of kc planes).  A workgroup's time is the latency of its kc + 2 planes (two halo
+// planes), one after the other, and `resident` workgroups run at a time (256 CUs times what
+// registers and LDS leave room for on a CU), so the launch takes about
+// ceil(workgroups / resident) (kc + 2) plane times; the kc <= 16 with the smallest product is
+// taken, the largest where several tie (fewer halo planes).  Small grids thus march a plane or
+// two in many workgroups, large ones 16: at 32 x 64 x 16 cells 16 planes leave 16 workgroups on
+// 256 CUs (Germano terms 68 us, strain 54, stage-1 right-hand side 59; one plane each: 17, 17,
+// 10 us); at 192 x 256 x 64 one plane costs 334, 137, 206 us against 186, 126, 167 with 16
+// (events around the launches).  32 planes are 20-40 % slower there.
+inline int march_planes(const Dims& d, int resident) {
+  const long tiles = (long)((d.ni - 1 + 63) / 64) * ((d.nj - 1 + 3) / 4);
+  long best = 0;
+  int kb = 1;
+  for (int kc = 1; kc <= 16; ++kc) {
+    const long wgs = tiles * ((d.nk - 1 + kc - 1) / kc);
+    const long cost = (wgs + resident - 1) / resident * (kc + 2);
+    if (kc == 1 || cost <= best) { best = cost; kb = kc; }
+  }
+  return kb;
+}
+inline dim3 march_grid(const Dims& d, int kc) {
+  return dim3((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + kc - 1) / kc);
+}
+
 // Kernel timing: wraps one launch in a pair of events when profiling is on.
 // arguments of the AF stage kernels
 struct AFArgs {

@@ -91,18 +91,18 @@ __global__ void k_nl(Dims d, const double* __restrict__ ju0, const double* __res
 // DIF(IN,OUT) for the three components (RLES/dif.f90:13-23): the orthogonal part
 // sum D_f (phi_nb - phi_P) plus the cross-derivative terms DIF_DIAGONAL
 // (RLES/dif_diagonal.f90:13-32, jqAB = J^-1 Q_AB), in the reference's order.  A workgroup owns a
-// 64 x 4 (I x J) column of cells over DF_KC consecutive planes and marches up K with the last
+// 64 x 4 (I x J) column of cells over kc consecutive planes and marches up K with the last
 // three planes of u_n, v_n, w_n (one-cell halo) in LDS, so the seven-point and twelve-edge
 // stencils are read from HBM once per column; J^-1 Q13, J^-1 Q23 and D_T of the planes K+-1
 // ride along in registers.
-constexpr int DF_KC = 4;
+constexpr int DF_RES = 1024;  // workgroups of k_dif_km resident at a time (four per CU)
 
 // With WNL set the same pass also forms NL(IN, NLOUT) of k_nl (RLES/nl.f90:23-31, its operation
 // order) from the staged planes and the face fluxes of ju (ju2 of the planes K+-1 in registers):
 // the whole step runs NL and DIF in one pass over u_n, v_n, w_n (DIF does not depend on NL or on
 // the SGS term added to NL in between).
 template <int NC, bool WNL = false>
-__global__ void __launch_bounds__(256) k_dif_km(Dims d, const double* __restrict__ pdI,
+__global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
                                                 const double* __restrict__ pdJ,
                                                 const double* __restrict__ pdK,
                                                 const double* __restrict__ jq12,
@@ -117,8 +117,8 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, const double* __restrict
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * DF_KC;
-  const int k1 = min(k0 + DF_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int q0 = (ty + 1) * SF_W + tx + 1;
   const long sj = d.sj;
@@ -208,13 +208,14 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, const double* __restrict
 // With CORR set, followed on the same cell by U = U + sign DTIME S / J^-1 (RLES/main.f90:108-111;
 // 90-92 with sign -1), S kept for the next step's predictor, and, when cflpart is given, the
 // local CFL number of the corrected velocity (CALCCOEF, k_cfl's formula) reduced to one maximum
-// per workgroup.  A workgroup owns a 64 x 4 (I x J) column of cells over PS_KC
+// per workgroup.  A workgroup owns a 64 x 4 (I x J) column of cells over kc
 // consecutive planes and marches up K; the products (J zeta_s p) of the planes K+-1 ride along
 // in registers, so only the I and J neighbours are fetched per cell.
-constexpr int PS_KC = 16;
+constexpr int PS_RES = 768;  // workgroups resident at a time (three per CU)
 
 template <int CORR, bool XZ0>
-__global__ void __launch_bounds__(256) k_psource_km(Dims d, const double* const* __restrict__ m,
+__global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc,
+                                                    const double* const* __restrict__ m,
                                                     const double* __restrict__ djac,
                                                     const double* __restrict__ p, double sign,
                                                     double dtime, double* s0, double* s1,
@@ -225,8 +226,8 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, const double* const*
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * PS_KC;
-  const int k1 = min(k0 + PS_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const long sj = d.sj;
   const GPW out[3] = {gpw(s0), gpw(s1), gpw(s2)};
@@ -768,13 +769,14 @@ int fvm_k_nl(FvmCtx* c) {
 int fvm_k_dif(FvmCtx* c) {
   ProfScope ps(c, "dif");
   const Dims d = c->d;
-  const dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + DF_KC - 1) / DF_KC);
+  const int kc = march_planes(d, DF_RES);
+  const dim3 g = march_grid(d, kc);
   const CompSet cs = {{c->un, c->vn, c->wn, c->tn}, {c->dif[0], c->dif[1], c->dif[2], c->dift}};
   if (c->thermal)  // DIF(T_N, DIFT), RLES/main.f90:75
-    hipLaunchKernelGGL(k_dif_km<4>, g, kBlk, 0, c->stream, c->d, c->pdI, c->pdJ, c->pdK,
+    hipLaunchKernelGGL(k_dif_km<4>, g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
                        c->jq12, c->jq13, c->jq23, cs);
   else
-    hipLaunchKernelGGL(k_dif_km<3>, g, kBlk, 0, c->stream, c->d, c->pdI, c->pdJ, c->pdK,
+    hipLaunchKernelGGL(k_dif_km<3>, g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
                        c->jq12, c->jq13, c->jq23, cs);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
@@ -787,14 +789,15 @@ int fvm_k_nl_dif(FvmCtx* c) {
   if (c->thermal) std::swap(c->adv, c->adv1);
   ProfScope ps(c, "nl_dif");
   const Dims d = c->d;
-  const dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + DF_KC - 1) / DF_KC);
+  const int kc = march_planes(d, DF_RES);
+  const dim3 g = march_grid(d, kc);
   const CompSet cs = {{c->un, c->vn, c->wn, c->tn}, {c->dif[0], c->dif[1], c->dif[2], c->dift}};
   const CompSet nlo = {{nullptr, nullptr, nullptr, nullptr}, {c->nl[0], c->nl[1], c->nl[2], c->adv}};
   if (c->thermal)
-    hipLaunchKernelGGL((k_dif_km<4, true>), g, kBlk, 0, c->stream, c->d, c->pdI, c->pdJ, c->pdK,
+    hipLaunchKernelGGL((k_dif_km<4, true>), g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
                        c->jq12, c->jq13, c->jq23, cs, c->ju[0], c->ju[1], c->ju[2], nlo);
   else
-    hipLaunchKernelGGL((k_dif_km<3, true>), g, kBlk, 0, c->stream, c->d, c->pdI, c->pdJ, c->pdK,
+    hipLaunchKernelGGL((k_dif_km<3, true>), g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
                        c->jq12, c->jq13, c->jq23, cs, c->ju[0], c->ju[1], c->ju[2], nlo);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
@@ -804,13 +807,14 @@ int fvm_k_p_source(FvmCtx* c) {
   double** m = c->dm;
   ProfScope ps(c, "p_source");
   const Dims d = c->d;
-  const dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + PS_KC - 1) / PS_KC);
+  const int kc = march_planes(d, PS_RES);
+  const dim3 g = march_grid(d, kc);
   if (c->xz_zero)
-    hipLaunchKernelGGL((k_psource_km<0, true>), g, kBlk, 0, c->stream, c->d,
+    hipLaunchKernelGGL((k_psource_km<0, true>), g, kBlk, 0, c->stream, c->d, kc,
                        (const double* const*)m, c->djac, c->p, 0.0, 0.0, c->s[0], c->s[1],
                        c->s[2], nullptr, nullptr, nullptr, nullptr);
   else
-    hipLaunchKernelGGL((k_psource_km<0, false>), g, kBlk, 0, c->stream, c->d,
+    hipLaunchKernelGGL((k_psource_km<0, false>), g, kBlk, 0, c->stream, c->d, kc,
                        (const double* const*)m, c->djac, c->p, 0.0, 0.0, c->s[0], c->s[1],
                        c->s[2], nullptr, nullptr, nullptr, nullptr);
   HIP_CHECK(hipGetLastError());
@@ -895,11 +899,12 @@ int fvm_k_nl_one(FvmCtx* c, const double* in, double* out) {
 int fvm_k_dif_one(FvmCtx* c, const double* in, double* out) {
   ProfScope ps(c, "dif");
   const Dims d = c->d;
-  const dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + DF_KC - 1) / DF_KC);
+  const int kc = march_planes(d, DF_RES);
+  const dim3 g = march_grid(d, kc);
   CompSet cs{};
   cs.in[0] = in;
   cs.out[0] = out;
-  hipLaunchKernelGGL(k_dif_km<1>, g, kBlk, 0, c->stream, c->d, c->pdI, c->pdJ, c->pdK, c->jq12,
+  hipLaunchKernelGGL(k_dif_km<1>, g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK, c->jq12,
                      c->jq13, c->jq23, cs);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
@@ -1069,16 +1074,16 @@ int fvm_wall2d_setup(FvmCtx* c, const double* xg, const double* yg) {
 int fvm_k_psource_correct(FvmCtx* c, double sign, bool with_cfl) {
   ProfScope ps(c, "psource_correct");
   const Dims d = c->d;
-  const dim3 gt = interior_grid(d);
-  const dim3 g(gt.x, gt.y, (d.nk - 1 + PS_KC - 1) / PS_KC);  // CFL maxima: one per workgroup
+  const int kc = march_planes(d, PS_RES);
+  const dim3 g = march_grid(d, kc);  // CFL maxima: one per workgroup
   if (with_cfl && (long)g.x * g.y * g.z > c->ncflpart) return FVM_ERR_SIZE;
   if (with_cfl) c->ncflused = (int)(g.x * g.y * g.z);
   if (c->xz_zero)
-    hipLaunchKernelGGL((k_psource_km<1, true>), g, kBlk, 0, c->stream, c->d,
+    hipLaunchKernelGGL((k_psource_km<1, true>), g, kBlk, 0, c->stream, c->d, kc,
                        (const double* const*)c->dm, c->djac, c->p, sign, c->prm.dtime, c->s[0],
                        c->s[1], c->s[2], c->u, c->v, c->w, with_cfl ? c->cflpart : nullptr);
   else
-    hipLaunchKernelGGL((k_psource_km<1, false>), g, kBlk, 0, c->stream, c->d,
+    hipLaunchKernelGGL((k_psource_km<1, false>), g, kBlk, 0, c->stream, c->d, kc,
                        (const double* const*)c->dm, c->djac, c->p, sign, c->prm.dtime, c->s[0],
                        c->s[1], c->s[2], c->u, c->v, c->w, with_cfl ? c->cflpart : nullptr);
   HIP_CHECK(hipGetLastError());

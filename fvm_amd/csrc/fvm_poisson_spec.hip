@@ -30,12 +30,12 @@ const dim3 kBlk(64, 4, 1);
 // residual r = sum A_nb p_nb + (rhs - DD(p)) - AP p of every interior cell (iter_p.f90:50-53
 // with SU = rhs - DD, DD the twelve cross terms of p weighted by J^-1 Q12, Q13, Q23), written to
 // the compact interior array R (I fastest), plus per-workgroup sums of |r| and |AP p|.
-// K-marching: a workgroup owns a 64 x 4 (I x J) column over RS_KC planes and
+// K-marching: a workgroup owns a 64 x 4 (I x J) column over kc planes and
 // keeps three consecutive p planes (one-cell halo) in an LDS ring, so every p value is read from
 // memory once per column instead of once per plane that needs it; the own-column values of the
 // planes below and above (J^-1 Q13, J^-1 Q23 at K +- 1, D_T at K - 1) ride along in registers.
 // One pair of partial sums per workgroup.
-constexpr int RS_KC = 16;
+constexpr int RS_RES = 768;  // workgroups resident at a time (three per CU)
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __restrict__ p,
@@ -613,8 +613,8 @@ int fvm_k_iter_p_sep(FvmCtx* c, bool mixed, double* resip, int* niter) {
     return FVM_ERR_ARG;
   }
   const Dims d = c->d;
-  const int kc = RS_KC;
-  dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + kc - 1) / kc);
+  const int kc = march_planes(d, RS_RES);
+  const dim3 g = march_grid(d, kc);
   long nb = (long)g.x * g.y * g.z;
   int outer = 0;
   double res = INFINITY, res_prev = INFINITY;

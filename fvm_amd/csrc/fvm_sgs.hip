@@ -92,14 +92,14 @@ __global__ void k_strain_iplanes(Dims d, const double* const* __restrict__ m,
 }
 
 // Strain on the interior cells fused with the (1,2,1)^3/64 test filter of u, v, w
-// (test_filter.f90:13-30).  A workgroup owns a 64 x 4 (I x J) column of cells over SF_KC
+// (test_filter.f90:13-30).  A workgroup owns a 64 x 4 (I x J) column of cells over kc
 // consecutive K planes and marches up K with the last three planes of u, v, w (one-cell halo)
 // in LDS, so every velocity value is fetched from HBM once per column.  The filter sums its 27
 // terms in the reference's order: K-1 plane, K plane, K+1 plane; rows J-1, J, J+1; columns
 // I-1, I, I+1.
 // With NF = 4 the temperature rides along: its gradient dT/dx_i = 0.5 (xi_i dT/dxi +
 // eta_i dT/deta + zeta_i dT/dzeta) (stress_tensor_dy.f90:78-94) and its test filter T^.
-constexpr int SF_KC = 16;
+constexpr int SF_RES = 768;  // workgroups resident at a time (three per CU)
 
 struct SfOut {
   const double* in[4];  // u, v, w, T
@@ -108,7 +108,8 @@ struct SfOut {
 };
 
 template <int NF, bool XZ0>
-__global__ void __launch_bounds__(256) k_strain_filter(Dims d, const double* const* __restrict__ m,
+__global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc,
+                                                       const double* const* __restrict__ m,
                                                        SfOut io, double* const* __restrict__ L,
                                                        double* mag) {
   const uint3 bb = xcd_block();
@@ -116,8 +117,8 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, const double* con
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * SF_KC;
-  const int k1 = min(k0 + SF_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int q0 = (ty + 1) * SF_W + tx + 1;
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
@@ -179,7 +180,7 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, const double* con
 
 // Germano/Lilly contractions LM and MM per interior cell (stress_tensor_dy.f90:236-483).
 // The twelve test-filtered products (u_i u_j and |S| S_ij) are never stored: a workgroup owns a
-// 64 x 4 (I x J) column of cells over LM_KC consecutive K planes, stages each plane of the ten
+// 64 x 4 (I x J) column of cells over kc consecutive K planes, stages each plane of the ten
 // factor fields (with a one-cell halo) in LDS (|S| formed from the six S_ij as it is staged, so
 // only nine fields are read), forms the in-plane (1,2,1)x(1,2,1) sums of the
 // products once per plane and combines three consecutive planes with (1,2,1) weights.  The sum
@@ -189,8 +190,8 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, const double* con
 // test-filtered velocity stencil, Delta^2) are issued before plane k's in-plane sums are formed,
 // so they arrive while the LDS work runs; the three-plane combination is carried as two running
 // sums, X = P(k-1) + 2 P(k) for the cell finished next and Y = P(k) for the one after.
-constexpr int LM_KC = 16;
-constexpr int SD_KC = 16;  // planes per workgroup of the K-marching SGS divergences
+constexpr int LM_RES = 512;  // workgroups resident at a time (two per CU by their registers)
+constexpr int SD_RES = 768;  // the same for the K-marching SGS divergences (three per CU)
 constexpr int LM_W = 66, LM_H = 6;  // tile with halo
 constexpr int LM_NQ = (LM_W * LM_H + 255) / 256;  // tile cells staged per thread
 
@@ -374,7 +375,7 @@ __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __re
 // filtered products are never stored; each plane of u, v, w, T, |S|, dT/dx_i is staged in LDS
 // (one-cell halo), its in-plane (1,2,1)x(1,2,1) sums are formed once, and three consecutive
 // planes are combined with (1,2,1) weights.
-__global__ void __launch_bounds__(256) k_lm_t(Dims d, const double* const* __restrict__ m,
+__global__ void __launch_bounds__(256) k_lm_t(Dims d, int kc, const double* const* __restrict__ m,
                                               const double* __restrict__ U,
                                               const double* __restrict__ V,
                                               const double* __restrict__ W,
@@ -395,8 +396,8 @@ __global__ void __launch_bounds__(256) k_lm_t(Dims d, const double* const* __res
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * LM_KC;
-  const int k1 = min(k0 + LM_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   // in-plane sums of uT vT wT |S|dT/dx |S|dT/dy |S|dT/dz for planes k-1, k, k+1
   double Pa[6], Pb[6], Pc[6];
@@ -464,7 +465,7 @@ __global__ void __launch_bounds__(256) k_lm_t(Dims d, const double* const* __res
 // divergence of the subgrid heat flux -2 kappa dT/dx_i (stress_tensor_dy.f90:719-736), added to
 // ADV with the inverse Jacobian (RLES/main.f90:67-68).  K-marching like k_sgs_div with the three
 // products (2 kappa) dT/dx_i.
-__global__ void __launch_bounds__(256) k_sgs_t_div(Dims d, const double* const* __restrict__ m,
+__global__ void __launch_bounds__(256) k_sgs_t_div(Dims d, int kc, const double* const* __restrict__ m,
                                                    const double* __restrict__ kappa,
                                                    const double* __restrict__ DX,
                                                    const double* __restrict__ DY,
@@ -476,8 +477,8 @@ __global__ void __launch_bounds__(256) k_sgs_t_div(Dims d, const double* const* 
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * SD_KC;
-  const int k1 = min(k0 + SD_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int e0 = (ty + 1) * SF_W + tx + 1;
   double Pm[3] = {0.0, 0.0, 0.0};  // own-column products of plane k-1
@@ -586,13 +587,13 @@ __global__ void k_nut(Dims d, const double* __restrict__ cavg, const double* __r
 
 // divergence of the SGS stress -2 nu_t S_ij (stress_tensor_dy.f90:541-583), added to NL
 // with the inverse Jacobian (RLES/main.f90:61-66).  A workgroup owns a 64 x 4 (I x J) column
-// of cells over SD_KC consecutive K planes and marches up K: the six products
+// of cells over kc consecutive K planes and marches up K: the six products
 // P_q = (2 nu_t) S_q of each plane are formed once, with a one-cell halo, in one of two LDS
 // slots (the I and J differences of plane k and the own-column value of plane k+1), and the
 // own-column products of plane k-1 are kept in registers.  Differences, products and sums are
 // the reference's, in its order.
 template <bool XZ0>
-__global__ void __launch_bounds__(256) k_sgs_div(Dims d, const double* const* __restrict__ m,
+__global__ void __launch_bounds__(256) k_sgs_div(Dims d, int kc, const double* const* __restrict__ m,
                                                  const double* __restrict__ filt2,
                                                  const double* __restrict__ cavg,
                                                  const double* const* __restrict__ L,
@@ -604,8 +605,8 @@ __global__ void __launch_bounds__(256) k_sgs_div(Dims d, const double* const* __
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
-  const int k0 = 1 + bb.z * SD_KC;
-  const int k1 = min(k0 + SD_KC - 1, d.nk - 1);
+  const int k0 = 1 + bb.z * kc;
+  const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int e0 = (ty + 1) * SF_W + tx + 1;
   const GP S0 = gp(L[0]), S1 = gp(L[1]), S2 = gp(L[2]);
@@ -698,9 +699,10 @@ int fvm_k_nut_out(FvmCtx* c) {
 int fvm_k_sgs_out(FvmCtx* c) {
   if (!c->sgs_stale) return FVM_OK;
   const Dims d = c->d;
-  const dim3 gs((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + SD_KC - 1) / SD_KC);
+  const int kc = march_planes(d, SD_RES);
+  const dim3 gs = march_grid(d, kc);
   auto kern = c->xz_zero ? k_sgs_div<true> : k_sgs_div<false>;
-  hipLaunchKernelGGL(kern, gs, kBlk, 0, c->stream, d, (const double* const*)c->dm, c->filt2,
+  hipLaunchKernelGGL(kern, gs, kBlk, 0, c->stream, d, kc, (const double* const*)c->dm, c->filt2,
                      c->scal + 0, (const double* const*)c->dlss, c->djac, c->nl[0], c->nl[1],
                      c->nl[2], c->sgs[0], c->sgs[1], c->sgs[2], 2);
   HIP_CHECK(hipGetLastError());
@@ -716,12 +718,13 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
   const bool th = c->thermal;
   {
     ProfScope pk(c, "k_strain_filter");
-    const dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + SF_KC - 1) / SF_KC);
+    const int kc = march_planes(d, SF_RES);
+    const dim3 g = march_grid(d, kc);
     const SfOut io = {{c->u, c->v, c->w, c->t}, {c->uh[0], c->uh[1], c->uh[2], c->that},
                       {c->dtd[0], c->dtd[1], c->dtd[2]}};
     auto kern = th ? k_strain_filter<4, false>
                    : (c->xz_zero ? k_strain_filter<3, true> : k_strain_filter<3, false>);
-    hipLaunchKernelGGL(kern, g, kBlk, 0, st, d, (const double* const*)m, io,
+    hipLaunchKernelGGL(kern, g, kBlk, 0, st, d, kc, (const double* const*)m, io,
                        (double* const*)c->dlss, c->mag);
     const long nb = 2L * (d.nj - 1) * (d.nk - 1);
     hipLaunchKernelGGL(k_strain_iplanes, grid1(nb, 256), dim3(256), 0, st, d,
@@ -741,8 +744,8 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
   if (r) return r;
   {
     ProfScope pk(c, "k_lm");
-    const int kc = LM_KC;
-    const dim3 gl((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + kc - 1) / kc);
+    const int kc = march_planes(d, LM_RES);
+    const dim3 gl = march_grid(d, kc);
     auto kern = c->xz_zero ? k_lm<true> : k_lm<false>;
     hipLaunchKernelGGL(kern, gl, kBlk, 0, st, d, (const double* const*)m, c->u, c->v, c->w,
                        c->uh[0], c->uh[1], c->uh[2], (const double* const*)c->dlss, c->filt2,
@@ -760,9 +763,10 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
   c->nut_stale = !sgs_out;
   {
     ProfScope pk(c, "k_sgs_div");
-    const dim3 gs((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + SD_KC - 1) / SD_KC);
+    const int kc = march_planes(d, SD_RES);
+  const dim3 gs = march_grid(d, kc);
     auto kern = c->xz_zero ? k_sgs_div<true> : k_sgs_div<false>;
-    hipLaunchKernelGGL(kern, gs, kBlk, 0, st, d, (const double* const*)m, c->filt2, c->scal + 0,
+    hipLaunchKernelGGL(kern, gs, kBlk, 0, st, d, kc, (const double* const*)m, c->filt2, c->scal + 0,
                        (const double* const*)c->dlss, c->djac, c->nl[0], c->nl[1], c->nl[2],
                        c->sgs[0], c->sgs[1], c->sgs[2],
                        (nl_update ? 1 : 0) | (sgs_out ? 2 : 0));
@@ -771,16 +775,18 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
   }
   if (th) {  // the temperature's dynamic model (stress_tensor_dy.f90:589-738), main.f90:67-68
     ProfScope pk(c, "sgs_t");
-    const dim3 gl((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + LM_KC - 1) / LM_KC);
-    hipLaunchKernelGGL(k_lm_t, gl, kBlk, 0, st, d, (const double* const*)m, c->u, c->v, c->w,
+    const int kl = march_planes(d, LM_RES);
+    const dim3 gl = march_grid(d, kl);
+    hipLaunchKernelGGL(k_lm_t, gl, kBlk, 0, st, d, kl, (const double* const*)m, c->u, c->v, c->w,
                        c->t, c->uh[0], c->uh[1], c->uh[2], c->that, c->mag, c->dtd[0],
                        c->dtd[1], c->dtd[2], c->magh, c->filt2, c->su[0], c->su[1]);
     hipLaunchKernelGGL(k_lm_reduce, dim3(nb), dim3(256), 0, st, d, c->su[0], c->su[1], c->red);
     hipLaunchKernelGGL(k_lm_final, dim3(1), dim3(256), 0, st, c->red, nb, c->scal + 1);
     hipLaunchKernelGGL(k_nut, grid1(d.n, 256), dim3(256), 0, st, d, c->scal + 1, c->filt2,
                        c->mag, c->kappa);
-    const dim3 gs((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, (d.nk - 1 + SD_KC - 1) / SD_KC);
-    hipLaunchKernelGGL(k_sgs_t_div, gs, kBlk, 0, st, d, (const double* const*)m, c->kappa,
+    const int kc = march_planes(d, SD_RES);
+  const dim3 gs = march_grid(d, kc);
+    hipLaunchKernelGGL(k_sgs_t_div, gs, kBlk, 0, st, d, kc, (const double* const*)m, c->kappa,
                        c->dtd[0], c->dtd[1], c->dtd[2], c->djac, c->adv, c->sgst);
     HIP_CHECK(hipGetLastError());
   }
