@@ -586,7 +586,8 @@ __global__ void __launch_bounds__(192) k_af_thomas_k_reg(Dims d, AFArgs A,
   constexpr int KB = 8, NB = NMAX / KB;
   static_assert(NMAX % KB == 0, "row blocks");
   double xs[NMAX];
-  double x = f[c0];  // K ghost of the stage input
+  // the K ghosts of the stage input are the periodic partners, rows n and 1
+  double x = f[c0 + (long)n * d.sk], xn = f[c0 + d.sk];
   double bs[KB], ba[KB], bd[KB];
 #pragma unroll
   for (int r = 0; r < KB; ++r) {
@@ -616,7 +617,6 @@ __global__ void __launch_bounds__(192) k_af_thomas_k_reg(Dims d, AFArgs A,
       for (int r = 0; r < KB; ++r) { bs[r] = ns[r]; ba[r] = na[r]; bd[r] = nd[r]; }
     }
   }
-  double xn = f[c0 + (long)(n + 1) * d.sk];
   double bt[KB];
 #pragma unroll
   for (int r = 0; r < KB; ++r) bt[r] = tb[c0 + (long)min(NMAX - r, n) * d.sk];
@@ -750,13 +750,13 @@ __global__ void __launch_bounds__(192) k_af_thomas_k(Dims d, AFArgs A,
   const double* su = A.su[comp];
   const int n = d.nk - 1;
   const long c0 = cidx(d, i, j, 0);
-  double x = f[c0];  // K ghost of the stage input
+  // the K ghosts of the stage input are the periodic partners, rows n and 1
+  double x = f[c0 + (long)n * d.sk], xn = f[c0 + d.sk];
   for (int k = 1; k <= n; ++k) {
     const long c = c0 + (long)k * d.sk;
     x = (su[c] - ta[c] * x) / td[c];
     f[c] = x;
   }
-  double xn = f[c0 + (long)(n + 1) * d.sk];
   for (int k = n; k >= 1; --k) {
     const long c = c0 + (long)k * d.sk;
     x = f[c] - tb[c] * xn;
@@ -825,7 +825,10 @@ static int chunk_stage(FvmCtx* c, AFArgs& A, int* iters) {
   return FVM_OK;
 }
 
-int fvm_k_iter_u(FvmCtx* c) {
+// With last_ghosts unset the ghosts of the third stage's input are not set where nothing reads
+// them (the K-line solve takes its end values from the periodic partners): the caller sets every
+// ghost of u, v, w next.
+int fvm_k_iter_u(FvmCtx* c, bool last_ghosts) {
   const Dims d = c->d;
   hipStream_t st = c->stream;
   const int fn_alias = c->u_is_un ? 1 : 0;
@@ -869,11 +872,14 @@ int fvm_k_iter_u(FvmCtx* c) {
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0, c->prm.re, fas, qf, dz);
       HIP_CHECK(hipGetLastError());
     }
-    // boundary ghosts of the stage input (BCU, iter_u.f90:83,160,237)
-    int r = fvm_k_bcu_ghosts(c, fld, 3);
+    // boundary ghosts of the stage input (BCU, iter_u.f90:83,160,237); the change form's first
+    // pass sets them itself
+    const bool klines = s == 2 && chunked && c->tk_a && c->af_zero_a[2] && c->af_zero_b[2];
+    const bool scan = s < 2 && chunked && c->af_scan[s];
+    int r = (scan && f32) || (klines && !last_ghosts) ? FVM_OK : fvm_k_bcu_ghosts(c, fld, 3);
     if (r) return r;
     ProfScope ps(c, s == 0 ? "af_sweep_i" : (s == 1 ? "af_sweep_j" : "af_sweep_k"));
-    if (s == 2 && chunked && c->tk_a && c->af_zero_a[2] && c->af_zero_b[2]) {
+    if (klines) {
       // independent K-lines: the exact sweep in one pass
       ProfScope pk(c, "k_af_thomas_k");
       const dim3 g((d.ni - 1 + 63) / 64, d.nj - 1, 1);
@@ -885,7 +891,7 @@ int fvm_k_iter_u(FvmCtx* c) {
                            c->tk_b);
       HIP_CHECK(hipGetLastError());
       c->af_iters[s] = 1;
-    } else if (s < 2 && chunked && c->af_scan[s]) {
+    } else if (scan) {
       int it = 0;
       r = fvm_af_scan_stage(c, s, A, &it, false, f32);
       if (r) return r;
@@ -1103,7 +1109,8 @@ int fvm_k_iter_t(FvmCtx* c) {
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0t, c->pe, fas, 0, c->dd2_zero ? 1 : 0);
       HIP_CHECK(hipGetLastError());
     }
-    int r = fvm_k_bct_ghosts(c, c->t);  // iter_t.f90:84,150,226
+    // iter_t.f90:84,150,226; nothing reads the third stage's ghosts before the final BCT
+    int r = s < 2 ? fvm_k_bct_ghosts(c, c->t) : FVM_OK;
     if (r) return r;
     ProfScope ps(c, "t_sweep");
     if (s < 2) {

@@ -184,12 +184,12 @@ __global__ void k_to_float(long n, const double* __restrict__ a, float* b) {
     b[t] = (float)a[t];
 }
 
-// boundary lines of the first pass: the stage input at the last line of every chunk
-// (bnd[((comp nb + b-1) nchunk + ca) n + p-1])
-// (T = float: the change form, whose stage input is the zero change)
-template <int S, typename T>
-__global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, T* bnd) {
-  const ScanGeo g = scan_geo(d, S);
+// boundary lines of the FP64 I stage's first pass: the stage input at the last line of every
+// chunk (bnd[((comp nb + b-1) nchunk + ca) n + p-1]).  That stage writes its iterate over the
+// field, so a chunk cannot read its neighbour's line there; the J stage, whose iterate is a work
+// array, and the change form, whose stage input is the zero change, take it in the first pass.
+__global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, double* bnd) {
+  const ScanGeo g = scan_geo(d, 0);
   const long tot = (long)A.nc * g.nb * nchunk * g.n;
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot;
        t += (long)gridDim.x * blockDim.x) {
@@ -200,8 +200,7 @@ __global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, T* bnd) {
     const int b = 1 + (int)(r % g.nb);
     const int comp = (int)(r / g.nb);
     const int a = min((ca + 1) * SC_C, g.na);
-    bnd[t] = std::is_same<T, float>::value ? (T)0
-                                           : (T)A.f[comp][g.ns_p * p + g.ns_a * a + g.ns_b * b];
+    bnd[t] = A.f[comp][g.ns_p * p + g.ns_a * a + g.ns_b * b];
   }
 }
 
@@ -241,8 +240,8 @@ __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o,
 // order (the component is the fastest index of w, so the three wavefronts sharing the line
 // factors run side by side on one XCD).  Lane l owns rows l*R+1 .. l*R+R.  The loads of line
 // a+1 are issued before line a is solved.  Writes the iterate (line-major), the chunk's last line
-// to bnd_out, and per wavefront the largest change of that line between passes and the largest
-// |x| (part[2w], part[2w+1]).
+// to bnd_out, and, in passes after the first (EARLY), per wavefront the largest change of that
+// line between passes and the largest |x| (part[2w], part[2w+1]).
 //
 // Early stop (passes after the first, early != 0): a pass only changes a chunk through its
 // incoming line a0-1, and a change d of line a moves line a+1 by at most rho d, with
@@ -256,7 +255,9 @@ __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o,
 // T = float: the FP32 correction form.  q holds the FP32 residual of the line systems at the stage
 // input (k_af_rhs_km with DR), the factors are FP32 copies, the iterate is the change of the
 // stage (zero at the line ends and on the ghost line before the first chunk) and the arithmetic
-// is FP32; the FP64 field is updated with the converged change afterwards.
+// is FP32; the FP64 field is updated with the converged change afterwards.  The stage's field is
+// then neither read nor written, so the workgroups past the first G of the first pass set its
+// BCU ghosts (bc_ghost), which the right-hand sides of the next stage read: one launch less.
 template <int S, int R, bool EARLY, typename T>
 __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __restrict__ beta,
                                                   const T* __restrict__ invd,
@@ -265,11 +266,16 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
                                                   const double* const* qt, double* const* xot,
                                                   const T* __restrict__ bnd_in,
                                                   T* bnd_out, int nchunk, double* part,
-                                                  double tol, double* sinkd) {
+                                                  double tol, double* sinkd, long G) {
   constexpr bool DELTA = std::is_same<T, float>::value;
   const ScanGeo g = scan_geo(d, S);
-  const long G = gridDim.x;
   const long lin = blockIdx.x;
+  if (DELTA && !EARLY && lin >= G) {  // uniform over the workgroup
+    const long cnt = bc_ghost_count(d), step = ((long)gridDim.x - G) * 64;
+    for (long t = (lin - G) * 64 + threadIdx.x; t < A.nc * cnt; t += step)
+      bc_ghost(d, A.f[t / cnt], A.ufar + (t / cnt) * (long)(d.nj + 1) * (d.nk + 1), 0.0, t % cnt);
+    return;
+  }
   const long w = (lin % 8) * (G / 8) + lin / 8;  // XCD-aware: neighbouring items share an XCD
   const int l = threadIdx.x;
   const gptr<T> sink = glb(reinterpret_cast<T*>(sinkd));
@@ -293,8 +299,10 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
       const int p = p0 + r;
       T v = (T)0;
       if (p <= g.n) {
-        if (ca == 0)
-          v = DELTA ? (T)0 : (T)fc[g.ns_p * p + g.ns_a * (a0 - 1) + g.ns_b * b];
+        if (DELTA && (ca == 0 || !EARLY))
+          v = (T)0;
+        else if (ca == 0 || (S == 1 && !EARLY))
+          v = (T)fc[g.ns_p * p + g.ns_a * (a0 - 1) + g.ns_b * b];
         else
           v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
       }
@@ -414,12 +422,15 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
       if (p <= g.n) {
         const long o = (((long)comp * g.nb + (b - 1)) * nchunk + ca) * g.n + (p - 1);
         const T x = xp[r];
-        dmax = fmax(dmax, (double)fabs(x - bnd_in[o]));
-        xmax = fmax(xmax, (double)fabs(x));
+        if (EARLY) {
+          dmax = fmax(dmax, (double)fabs(x - bnd_in[o]));
+          xmax = fmax(xmax, (double)fabs(x));
+        }
         bnd_out[o] = x;
       }
     }
   }
+  if (!EARLY) return;
   // wavefront max
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -487,9 +498,10 @@ int scan_stage(FvmCtx* c, const AFArgs& A, int* iters, bool temp) {
       for (int k = 0; k < nc; ++k) qn.p[k] = A.su[k];
       hipLaunchKernelGGL(k_scan_q1v<T>, dim3((d.ni - 1 + 31) / 32, (d.nj - 1 + 31) / 32, nc * (d.nk - 1)),
                          dim3(256), 0, st, d, qn, dq);
+    } else if (!DELTA) {
+      hipLaunchKernelGGL(k_scan_seed, grid1((long)nc * g.nb * nchunk * g.n, 256), dim3(256), 0,
+                         st, d, A, nchunk, c->bnd[0]);
     }
-    hipLaunchKernelGGL((k_scan_seed<S, T>), grid1((long)nc * g.nb * nchunk * g.n, 256), dim3(256),
-                       0, st, d, A, nchunk, bnd[0]);
     HIP_CHECK(hipGetLastError());
   }
   // the FP32 change is resolved to its own precision
@@ -506,17 +518,19 @@ int scan_stage(FvmCtx* c, const AFArgs& A, int* iters, bool temp) {
     {
       ProfScope pk(c, S == 0 ? "k_scan_pass_i" : "k_scan_pass_j");
       auto kern = it > 0 ? k_scan_pass<S, R, true, T> : k_scan_pass<S, R, false, T>;
-      hipLaunchKernelGGL(kern, dim3((unsigned)G), dim3(64), 0, st, d, A, lf[0], lf[1], lf[2],
-                         lf[3], (const double* const*)dq, dxo, bnd[slot], bnd[slot ^ 1],
-                         nchunk, c->red, tol, c->sink);
+      // the change form's first pass also sets the field's BCU ghosts: four per lane
+      const long ng = DELTA && it == 0 ? (nc * bc_ghost_count(d) + 255) / 256 : 0;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(G + ng)), dim3(64), 0, st, d, A, lf[0], lf[1],
+                         lf[2], lf[3], (const double* const*)dq, dxo, bnd[slot], bnd[slot ^ 1],
+                         nchunk, c->red, tol, c->sink, G);
     }
-    // the first pass never suffices on its own: its maxima are not read
-    const Mailbox mb = it > 0 ? fvm_mail(c) : Mailbox{nullptr, nullptr, 0};
-    hipLaunchKernelGGL(k_scan_max, dim3(1), dim3(256), 0, st, c->red, G, c->scal + 20, mb);
     HIP_CHECK(hipGetLastError());
     slot ^= 1;
     ++it;
-    if (it < 2) continue;
+    if (it < 2) continue;  // the first pass never suffices on its own: it forms no maxima
+    const Mailbox mb = fvm_mail(c);
+    hipLaunchKernelGGL(k_scan_max, dim3(1), dim3(256), 0, st, c->red, G, c->scal + 20, mb);
+    HIP_CHECK(hipGetLastError());
     const int rf = fvm_mail_wait(c, mb, 2, c->hscal + 20);
     if (rf) return rf;
     const double dm = c->hscal[20], xm = c->hscal[21];

@@ -712,7 +712,7 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
     CK(fvm_k_sgs(c, false));  // SGS_x,y,z formed on first read (fvm_get_field)
   }
   CK(fvm_k_p_source(c));                          // :78
-  CK(fvm_k_iter_u(c));                            // :82-88
+  CK(fvm_k_iter_u(c, false));                     // :82-88 (BCU follows the correction)
   CK(fvm_k_correct_bcu_contra(c));                // :90-101 (correction, BCU, CONTRA_VEL)
   double res = 0.0;
   int it = 0;

@@ -233,6 +233,51 @@ static __global__ void k_ghost_fill_multi(Dims d, PtrSet8 set) {
   }
 }
 
+// BCU / BCT ghost t of the ghost surface of one array, the periodic MPI_X images included.  Every
+// ghost is a function of one interior cell: with (js, ks) the periodic partner of (j, k) (the cell
+// itself when j, k are interior), the wall ghost is -a(1, js, ks) + 2 wall, the far-field ghost
+// -a(NI-1, js, ks) + 2 U_F(js, ks) and any other ghost a(i, js, ks) -- exactly the values the
+// reference's BCU (wall and far-field ghosts of the interior rows) followed by MPI_X leaves.
+__host__ __device__ inline long bc_ghost_count(const Dims& d) {
+  return 2L * (d.nj - 1) * (d.nk - 1) + (long)(d.ni + 1) * 2 * (d.nk - 1) +
+         (long)(d.ni + 1) * (d.nj + 1) * 2;
+}
+
+__device__ inline void bc_ghost(const Dims& d, double* ap, const double* ufp, double wall, long t) {
+  const gptr<double> a = glb(ap);
+  const long nI = 2L * (d.nj - 1) * (d.nk - 1);          // I ghost planes, interior j, k
+  const long nJ = (long)(d.ni + 1) * 2 * (d.nk - 1);      // J ghost rows, interior k; then K planes
+  int i, j, k;
+  if (t < nI) {
+    const long q = t % (nI / 2);
+    i = t < nI / 2 ? 0 : d.ni;
+    j = 1 + (int)(q % (d.nj - 1));
+    k = 1 + (int)(q / (d.nj - 1));
+  } else if (t < nI + nJ) {
+    const long q = t - nI;
+    i = (int)(q % (d.ni + 1));
+    const long r = q / (d.ni + 1);
+    j = (r % 2) == 0 ? 0 : d.nj;
+    k = 1 + (int)(r / 2);
+  } else {
+    const long q = t - nI - nJ;
+    i = (int)(q % (d.ni + 1));
+    const long r = q / (d.ni + 1);
+    j = (int)(r % (d.nj + 1));
+    k = (r / (d.nj + 1)) == 0 ? 0 : d.nk;
+  }
+  const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
+  const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
+  double v;
+  if (i == 0)
+    v = -a[cidx(d, 1, js, ks)] + 2.0 * wall;
+  else if (i == d.ni)
+    v = -a[cidx(d, d.ni - 1, js, ks)] + 2.0 * gp(ufp)[js + (long)(d.nj + 1) * ks];
+  else
+    v = a[cidx(d, i, js, ks)];
+  a[cidx(d, i, j, k)] = v;
+}
+
 // Scaled-L1 residual sum|r| / sum|AP p| of ITER_P (iter_p.f90:45-59).  When both sums are
 // zero (p = 0 and a zero right-hand side) the reference's quotient is 0/0 = NaN, for which its
 // test 'RESIP .GT. RESIMAX' is false, so its sweep loop ends: that state is converged, and 0 is

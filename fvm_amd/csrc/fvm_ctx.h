@@ -246,7 +246,7 @@ int fvm_wall2d_setup(FvmCtx* c, const double* xg, const double* yg);
 int fvm_k_sgs(FvmCtx* c, bool sgs_out = true, bool nl_update = true);
 int fvm_k_sgs_out(FvmCtx* c);
 int fvm_k_nut_out(FvmCtx* c);
-int fvm_k_iter_u(FvmCtx* c);
+int fvm_k_iter_u(FvmCtx* c, bool last_ghosts = true);
 int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter);
 int fvm_k_div_norm(FvmCtx* c, double* out);
 int fvm_k_bcp(FvmCtx* c);

@@ -383,49 +383,13 @@ __global__ void k_copy_multi(long n, PtrSet8 dst, PtrSet8 src) {
     dst.p[blockIdx.y][n - 1] = src.p[blockIdx.y][n - 1];
 }
 
-// BCU / BCT ghosts and the periodic MPI_X copy in one pass over the ghost surface.  Every ghost
-// is a function of one interior cell: with (js, ks) the periodic partner of (j, k) (the cell
-// itself when j, k are interior), the wall ghost is -a(1, js, ks) + 2 wall, the far-field ghost
-// -a(NI-1, js, ks) + 2 U_F(js, ks) and any other ghost a(i, js, ks) -- exactly the values the
-// reference's BCU (wall and far-field ghosts of the interior rows) followed by MPI_X leaves.
+// BCU / BCT ghosts and the periodic MPI_X copy in one pass over the ghost surface (bc_ghost)
 __global__ void k_bc_ghosts(Dims d, PtrSet8 set, const double* __restrict__ ufar, double wall) {
-  double* __restrict__ a = set.p[blockIdx.y];
-  const double* __restrict__ uf = ufar + blockIdx.y * (long)(d.nj + 1) * (d.nk + 1);
-  const long nI = 2L * (d.nj - 1) * (d.nk - 1);          // I ghost planes, interior j, k
-  const long nJ = (long)(d.ni + 1) * 2 * (d.nk - 1);      // J ghost rows, interior k
-  const long nK = (long)(d.ni + 1) * (d.nj + 1) * 2;      // K ghost planes
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < nI + nJ + nK;
-       t += (long)gridDim.x * blockDim.x) {
-    int i, j, k;
-    if (t < nI) {
-      const long q = t % (nI / 2);
-      i = t < nI / 2 ? 0 : d.ni;
-      j = 1 + (int)(q % (d.nj - 1));
-      k = 1 + (int)(q / (d.nj - 1));
-    } else if (t < nI + nJ) {
-      const long q = t - nI;
-      i = (int)(q % (d.ni + 1));
-      const long r = q / (d.ni + 1);
-      j = (r % 2) == 0 ? 0 : d.nj;
-      k = 1 + (int)(r / 2);
-    } else {
-      const long q = t - nI - nJ;
-      i = (int)(q % (d.ni + 1));
-      const long r = q / (d.ni + 1);
-      j = (int)(r % (d.nj + 1));
-      k = (r / (d.nj + 1)) == 0 ? 0 : d.nk;
-    }
-    const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
-    const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
-    double v;
-    if (i == 0)
-      v = -a[cidx(d, 1, js, ks)] + 2.0 * wall;
-    else if (i == d.ni)
-      v = -a[cidx(d, d.ni - 1, js, ks)] + 2.0 * uf[js + (long)(d.nj + 1) * ks];
-    else
-      v = a[cidx(d, i, js, ks)];
-    a[cidx(d, i, j, k)] = v;
-  }
+  const long cnt = bc_ghost_count(d);
+  const double* uf = ufar + blockIdx.y * (long)(d.nj + 1) * (d.nk + 1);
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < cnt;
+       t += (long)gridDim.x * blockDim.x)
+    bc_ghost(d, set.p[blockIdx.y], uf, wall, t);
 }
 
 // U = U + sign DTIME S / J^-1 (RLES/main.f90:90-92 with sign -1, 109-111 with +1)
@@ -841,12 +805,6 @@ int fvm_k_step_copy(FvmCtx* c) {
   HIP_CHECK(hipGetLastError());
   c->u_is_un = true;
   return FVM_OK;
-}
-
-// cells of the ghost surface enumerated by k_bc_ghosts
-inline long bc_ghost_count(const Dims& d) {
-  return 2L * (d.nj - 1) * (d.nk - 1) + (long)(d.ni + 1) * 2 * (d.nk - 1) +
-         (long)(d.ni + 1) * (d.nj + 1) * 2;
 }
 
 // far-field values of T for BCT from T_N (bct.f90:28-37)
