@@ -705,8 +705,7 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
   fvm_step_info st{};
   int r;
 #define CK(x) do { r = (x); if (r && r != FVM_ERR_NOCONV) return r; } while (0)
-  CK(fvm_begin_step(c));                          // main.f90:42-45
-  CK(fvm_k_contra_vel(c));                        // :48
+  CK(fvm_k_step_begin(c));                        // main.f90:42-48
   CK(fvm_k_nl_dif(c));                            // :51-57 and DIF :72-75 in one pass
   if (c->prm.use_les) {                           // :59-69
     CK(fvm_k_sgs(c, false));  // SGS_x,y,z formed on first read (fvm_get_field)
@@ -718,10 +717,8 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
   int it = 0;
   int rp = fvm_k_iter_p(c, &res, &it);            // :103-105 (BCP included)
   if (rp && rp != FVM_ERR_NOCONV) return rp;
-  CK(fvm_k_psource_correct(c, +1.0, true));       // :108-111 (P_SOURCE, projection; CFL maxima)
-  if (!c->two_d) CK(fvm_k_pref(c, nullptr));     // :125-135 (none in 2D)
-  double* f[3] = {c->u, c->v, c->w};
-  CK(fvm_k_bcu_ghosts(c, f, 3));                  // :138-142
+  CK(fvm_k_project(c));                           // :108-111, 138-142 (P_SOURCE, projection,
+                                                  // BCU; CFL maxima, pressure reference)
   if (c->thermal) CK(fvm_k_iter_t(c));            // :145-147 (ITER_T, BCT)
   if (c->two_d) {
     const Mailbox mb = fvm_mail(c);               // the 2D CALCCOEF publishes scal[0..16]
@@ -729,7 +726,8 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
     r = fvm_mail_wait(c, mb, 17, c->hscal);
   } else {
     const Mailbox mb = fvm_mail(c);               // the force kernel publishes scal[0..16]
-    CK(fvm_k_calccoef(c, nullptr, true, &mb));    // :150
+    CK(fvm_k_calccoef(c, nullptr, true, &mb, nullptr, 0, true));  // :132-135 (p minus the
+                                                  // reference), 150
     CK(fvm_k_post_accum(c));                      // calccoef.f90:286-307 (time averages)
     r = fvm_mail_wait(c, mb, 17, c->hscal);
   }

@@ -30,13 +30,16 @@ __host__ __device__ inline long cidx(const Dims& d, int i, int j, int k) {
 // (x fastest) order, over the 8 XCDs, each with its own L2.  This bijection of the flat block id
 // hands XCD x one contiguous run of tiles in flat order (J rows, then K planes), so the J+-1 and
 // K+-1 neighbours a tile reads were mostly fetched into the same L2 by the tiles next to it.
-__device__ inline uint3 xcd_block() {
-  const unsigned gx = gridDim.x, gy = gridDim.y;
-  const unsigned nb = gx * gy * gridDim.z;
-  const unsigned b = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+// b: flat id of nb = gx gy gz tiles.
+__device__ inline uint3 xcd_tile(unsigned b, unsigned gx, unsigned gy, unsigned gz) {
+  const unsigned nb = gx * gy * gz;
   const unsigned x = b & 7u, slot = b >> 3, q = nb >> 3, r = nb & 7u;
   const unsigned w = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + slot;
   return make_uint3(w % gx, (w / gx) % gy, w / (gx * gy));
+}
+__device__ inline uint3 xcd_block() {
+  const unsigned gx = gridDim.x, gy = gridDim.y;
+  return xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx, gy, gridDim.z);
 }
 
 // Device arrays read through pointers that come from tables in device memory (the metric, strain
@@ -243,11 +246,10 @@ __host__ __device__ inline long bc_ghost_count(const Dims& d) {
          (long)(d.ni + 1) * (d.nj + 1) * 2;
 }
 
-__device__ inline void bc_ghost(const Dims& d, double* ap, const double* ufp, double wall, long t) {
-  const gptr<double> a = glb(ap);
+// ghost t of the surface: its indices (i, j, k) and the periodic partner (js, ks) of (j, k)
+__device__ inline void ghost_cell(const Dims& d, long t, int& i, int& j, int& k, int& js, int& ks) {
   const long nI = 2L * (d.nj - 1) * (d.nk - 1);          // I ghost planes, interior j, k
   const long nJ = (long)(d.ni + 1) * 2 * (d.nk - 1);      // J ghost rows, interior k; then K planes
-  int i, j, k;
   if (t < nI) {
     const long q = t % (nI / 2);
     i = t < nI / 2 ? 0 : d.ni;
@@ -266,8 +268,14 @@ __device__ inline void bc_ghost(const Dims& d, double* ap, const double* ufp, do
     j = (int)(r % (d.nj + 1));
     k = (r / (d.nj + 1)) == 0 ? 0 : d.nk;
   }
-  const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
-  const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
+  js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
+  ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
+}
+
+__device__ inline void bc_ghost(const Dims& d, double* ap, const double* ufp, double wall, long t) {
+  const gptr<double> a = glb(ap);
+  int i, j, k, js, ks;
+  ghost_cell(d, t, i, j, k, js, ks);
   double v;
   if (i == 0)
     v = -a[cidx(d, 1, js, ks)] + 2.0 * wall;
@@ -276,6 +284,44 @@ __device__ inline void bc_ghost(const Dims& d, double* ap, const double* ufp, do
   else
     v = a[cidx(d, i, js, ks)];
   a[cidx(d, i, j, k)] = v;
+}
+
+// The same ghosts written by the cell they are functions of, in the kernel that forms the cell, so
+// that no ghost pass follows it.  periodic_images: v of cell (i, j, k), interior j and k, to its
+// J and K ghost images (the periodic copy of MPI_X); bc_images: the same for an interior cell of
+// a velocity or temperature array together with the wall and far-field ghosts of its row (i = 1,
+// NI-1).  The branches on j and k are uniform over a wavefront along I.
+__device__ inline void periodic_images(const Dims& d, double* ap, int i, int j, int k, double v) {
+  const bool j1 = j == 1, jn = j == d.nj - 1, k1 = k == 1, kn = k == d.nk - 1;
+  if (!(j1 || jn || k1 || kn)) return;
+  const GPW a = gpw(ap);
+  if (j1) a[cidx(d, i, d.nj, k)] = v;
+  if (jn) a[cidx(d, i, 0, k)] = v;
+  if (k1) {
+    a[cidx(d, i, j, d.nk)] = v;
+    if (j1) a[cidx(d, i, d.nj, d.nk)] = v;
+    if (jn) a[cidx(d, i, 0, d.nk)] = v;
+  }
+  if (kn) {
+    a[cidx(d, i, j, 0)] = v;
+    if (j1) a[cidx(d, i, d.nj, 0)] = v;
+    if (jn) a[cidx(d, i, 0, 0)] = v;
+  }
+}
+
+__device__ inline void bc_images(const Dims& d, double* ap, const double* ufp, double wall, int i,
+                                 int j, int k, double v) {
+  periodic_images(d, ap, i, j, k, v);
+  if (i == 1) {
+    const double g = -v + 2.0 * wall;
+    gpw(ap)[cidx(d, 0, j, k)] = g;
+    periodic_images(d, ap, 0, j, k, g);
+  }
+  if (i == d.ni - 1) {
+    const double g = -v + 2.0 * gp(ufp)[j + (long)(d.nj + 1) * k];
+    gpw(ap)[cidx(d, d.ni, j, k)] = g;
+    periodic_images(d, ap, d.ni, j, k, g);
+  }
 }
 
 // Scaled-L1 residual sum|r| / sum|AP p| of ITER_P (iter_p.f90:45-59).  When both sums are

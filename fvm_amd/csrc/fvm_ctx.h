@@ -231,13 +231,15 @@ int fvm_k_bcu_ghosts_one(FvmCtx* c, double* f, int comp);
 int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const double* nl,
                      const double* nl1, const double* dif, const double* s);
 double* fvm_field(FvmCtx* c, int f);
-int fvm_k_psource_correct(FvmCtx* c, double sign, bool with_cfl);
+int fvm_k_project(FvmCtx* c);
+int fvm_k_step_begin(FvmCtx* c);
 int fvm_k_correct_bcu_contra(FvmCtx* c);
 int fvm_k_pref(FvmCtx* c, double* pref_host);
 // CALCCOEF; part (cap doubles) holds the CFL and force partial sums, nullptr: the context's own
 // reduction buffer.  fvm_calccoef_scratch: the doubles of part one call needs.
 int fvm_k_calccoef(FvmCtx* c, double* out8, bool cfl_ready = false,
-                   const Mailbox* mb = nullptr, double* part = nullptr, long cap = 0);
+                   const Mailbox* mb = nullptr, double* part = nullptr, long cap = 0,
+                   bool shift = false);
 int fvm_k_calccoef2d(FvmCtx* c, double* out8, bool cfl_ready = false,
                      const Mailbox* mb = nullptr, double* part = nullptr, long cap = 0);
 long fvm_calccoef_scratch(const FvmCtx* c, bool cfl_ready);

@@ -205,24 +205,48 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
 }
 
 // P_SOURCE(IN): S = -0.5 sum_dir [(J xi_s p)_+ - (J xi_s p)_-] (RLES/p_source.f90:14-42).
-// With CORR set, followed on the same cell by U = U + sign DTIME S / J^-1 (RLES/main.f90:108-111;
-// 90-92 with sign -1), S kept for the next step's predictor, and, when cflpart is given, the
-// local CFL number of the corrected velocity (CALCCOEF, k_cfl's formula) reduced to one maximum
-// per workgroup.  A workgroup owns a 64 x 4 (I x J) column of cells over kc
+// With CORR set, the projection of the step: followed on the same cell by U = U + DTIME S / J^-1
+// (RLES/main.f90:108-111), S kept for the next step's predictor, the velocity's BCU ghosts
+// (:137-142) written by the cells they are functions of, and the local CFL number of the
+// corrected velocity (CALCCOEF, k_cfl's formula) reduced to one maximum per workgroup; one more
+// workgroup forms the pressure reference into pref, when given.  A workgroup owns a 64 x 4 (I x J) column of cells over kc
 // consecutive planes and marches up K; the products (J zeta_s p) of the planes K+-1 ride along
 // in registers, so only the I and J neighbours are fetched per cell.
 constexpr int PS_RES = 768;  // workgroups resident at a time (three per CU)
 
+// span mean of p at (IE, NJ/4, K) by one workgroup of 256 threads: the span values are fetched
+// all at once, then summed in K order by one lane (RLES/main.f90:125-131, the reference's order)
+__device__ inline void pref_mean(const Dims& d, const double* __restrict__ p, double* out, int t,
+                                 double* sh) {
+  double s = 0.0;
+  for (int k0 = 1; k0 <= d.nk - 1; k0 += 256) {
+    const int k = k0 + t;
+    if (k <= d.nk - 1) sh[t] = p[cidx(d, d.ni, d.nj / 4, k)];
+    __syncthreads();
+    if (t == 0) {
+      const int cnt = min(256, d.nk - k0);
+      for (int q = 0; q < cnt; ++q) s = s + sh[q];
+    }
+    __syncthreads();
+  }
+  if (t == 0) out[0] = s / (double)(d.nk - 1);
+}
+
 template <int CORR, bool XZ0>
-__global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc,
+__global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
                                                     const double* const* __restrict__ m,
                                                     const double* __restrict__ djac,
-                                                    const double* __restrict__ p, double sign,
-                                                    double dtime, double* s0, double* s1,
-                                                    double* s2, double* u, double* v, double* w,
-                                                    double* cflpart) {
+                                                    const double* __restrict__ p, double dtime,
+                                                    double* s0, double* s1, double* s2, double* u,
+                                                    double* v, double* w,
+                                                    const double* __restrict__ ufar,
+                                                    double* cflpart, double* pref) {
   __shared__ double sh[256];
-  const uint3 bb = xcd_block();
+  if (CORR && blockIdx.x == tg.x * tg.y * tg.z) {  // one workgroup past the tiles
+    pref_mean(d, p, pref, threadIdx.y * 64 + threadIdx.x, sh);
+    return;
+  }
+  const uint3 bb = xcd_tile(blockIdx.x, tg.x, tg.y, tg.z);
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
   const int j = 1 + bb.y * 4 + ty;
@@ -266,11 +290,16 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc,
       for (int q = 0; q < 3; ++q) {
         out[q][c] = sv[q];
         if (CORR) {
-          nv[q] = sign < 0 ? fv[q] - dtime * sv[q] / J : fv[q] + dtime * sv[q] / J;
+          nv[q] = fv[q] + dtime * sv[q] / J;
           f[q][c] = nv[q];
         }
       }
-      if (CORR && cflpart) {
+      if (CORR) {
+        const long nf = (long)(d.nj + 1) * (d.nk + 1);
+        bc_images(d, u, ufar, 0.0, i, j, k, nv[0]);
+        bc_images(d, v, ufar + nf, 0.0, i, j, k, nv[1]);
+        bc_images(d, w, ufar + 2 * nf, 0.0, i, j, k, nv[2]);
+
         const double U = nv[0], V = nv[1], W = nv[2];
         const double ca = fabs(gp(m[0])[c] * U + gp(m[3])[c] * V + mget<XZ0>(m, 6, c) * W);
         const double cb = fabs(gp(m[1])[c] * U + gp(m[4])[c] * V + mget<XZ0>(m, 7, c) * W);
@@ -279,57 +308,74 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc,
       }
     }
   }
-  if (!(CORR && cflpart)) return;  // uniform over the workgroup
+  if (!CORR) return;
   sh[tid] = cmax;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if (tid < s) sh[tid] = fmax(sh[tid], sh[tid + s]);
     __syncthreads();
   }
-  if (tid == 0) cflpart[blockIdx.x + gridDim.x * (blockIdx.y + (long)gridDim.y * blockIdx.z)] = sh[0];
+  if (tid == 0) cflpart[blockIdx.x] = sh[0];
 }
 
-// predictor correction U = U - DTIME S / J^-1 fused with CONTRA_VEL on the interior cells
-// (RLES/main.f90:90-92, contra_vel.f90:13-23); the I ghost planes follow after BCU
+// J^-1 x contravariant velocity of cell c from the velocity (U, V, W) there (contra_vel.f90:13-23)
 template <bool XZ0>
-__global__ void k_correct_contra(Dims d, const double* const* __restrict__ m,
-                                 const double* __restrict__ djac, double dtime,
-                                 const double* __restrict__ s0, const double* __restrict__ s1,
-                                 const double* __restrict__ s2, double* u, double* v, double* w,
-                                 double* ju0, double* ju1, double* ju2) {
-  INTERIOR_IJK(d);
-  const double J = djac[c];
-  const double U = u[c] - dtime * s0[c] / J;
-  const double V = v[c] - dtime * s1[c] / J;
-  const double W = w[c] - dtime * s2[c] / J;
-  u[c] = U; v[c] = V; w[c] = W;
+__device__ inline void contra_cell(const double* const* __restrict__ m, long c, double J, double U,
+                                   double V, double W, double (&ju)[3]) {
   const double u1 = gp(m[0])[c] * U + gp(m[3])[c] * V + mget<XZ0>(m, 6, c) * W;
   const double u2 = gp(m[1])[c] * U + gp(m[4])[c] * V + mget<XZ0>(m, 7, c) * W;
   const double u3 = gp(m[2])[c] * U + gp(m[5])[c] * V + gp(m[8])[c] * W;
-  ju0[c] = J * u1;
-  ju1[c] = J * u2;
-  ju2[c] = J * u3;
+  ju[0] = J * u1;
+  ju[1] = J * u2;
+  ju[2] = J * u3;
 }
 
-// CONTRA_VEL on the I ghost planes i = 0 and i = NI only
-__global__ void k_contra_iplanes(Dims d, const double* const* __restrict__ m,
-                                 const double* __restrict__ djac, const double* __restrict__ u,
-                                 const double* __restrict__ v, const double* __restrict__ w,
-                                 double* ju0, double* ju1, double* ju2) {
-  const long nf = (long)(d.nj - 1) * (d.nk - 1);
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < 2 * nf;
-       t += (long)gridDim.x * blockDim.x) {
-    const int i = t < nf ? 0 : d.ni;
-    const long r = t % nf;
-    const int j = 1 + (int)(r % (d.nj - 1)), k = 1 + (int)(r / (d.nj - 1));
-    const long c = cidx(d, i, j, k);
-    const double U = u[c], V = v[c], W = w[c], J = djac[c];
-    const double u1 = gp(m[0])[c] * U + gp(m[3])[c] * V + gp(m[6])[c] * W;
-    const double u2 = gp(m[1])[c] * U + gp(m[4])[c] * V + gp(m[7])[c] * W;
-    const double u3 = gp(m[2])[c] * U + gp(m[5])[c] * V + gp(m[8])[c] * W;
-    ju0[c] = J * u1;
-    ju1[c] = J * u2;
-    ju2[c] = J * u3;
+// three arrays by value
+struct Vec3P {
+  double* p[3];
+};
+
+// Predictor correction U = U - DTIME S / J^-1, BCU and CONTRA_VEL (RLES/main.f90:90-101,
+// contra_vel.f90:13-23) in one pass: a cell writes its velocity, the BCU ghosts that are
+// functions of it, its JU, the JU of the wall / far-field ghost of its row and their periodic
+// images.  As four launches (interior, BCU ghosts, JU on the I planes, JU's periodic copy) the
+// surface kernels took 6.7 + 13.7 + 5.5 us on 192 x 256 x 64 cells for strided columns of
+// 8 bytes per cache line.
+template <bool XZ0>
+__global__ void k_correct_contra(Dims d, const double* const* __restrict__ m,
+                                 const double* __restrict__ djac, double dtime, Vec3P s, Vec3P f,
+                                 Vec3P ju, const double* __restrict__ ufar) {
+  INTERIOR_IJK(d);
+  const double J = djac[c];
+  const long nf = (long)(d.nj + 1) * (d.nk + 1);
+  double n[3], a[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) n[q] = gp(f.p[q])[c] - dtime * gp(s.p[q])[c] / J;
+  contra_cell<XZ0>(m, c, J, n[0], n[1], n[2], a);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    gpw(f.p[q])[c] = n[q];
+    bc_images(d, f.p[q], ufar + q * nf, 0.0, i, j, k, n[q]);
+    gpw(ju.p[q])[c] = a[q];
+    periodic_images(d, ju.p[q], i, j, k, a[q]);
+  }
+  if (i == 1 || i == d.ni - 1) {  // the row's ghosts, as bc_images forms them
+    for (int side = 0; side < 2; ++side) {
+      if (i != (side == 0 ? 1 : d.ni - 1)) continue;
+      const int ig = side == 0 ? 0 : d.ni;
+      const long cg = cidx(d, ig, j, k);
+      double g[3], b[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        g[q] = side == 0 ? -n[q] + 2.0 * 0.0
+                         : -n[q] + 2.0 * ufar[q * nf + j + (long)(d.nj + 1) * k];
+      contra_cell<XZ0>(m, cg, djac[cg], g[0], g[1], g[2], b);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        gpw(ju.p[q])[cg] = b[q];
+        periodic_images(d, ju.p[q], ig, j, k, b[q]);
+      }
+    }
   }
 }
 
@@ -343,6 +389,23 @@ struct FarSet {
   double uin[3];
 };
 
+__device__ inline double ufar_value(const Dims& d, const double* const* __restrict__ m,
+                                    const double* __restrict__ theta, const double* bp, double uin,
+                                    double dtime, double pi, int j, int k) {
+  const GP b = gp(bp);
+  const long c = cidx(d, d.ni, j, k), mm = c - 1;
+  const double th = theta[c];
+  if (th >= 0.5 * pi && th <= 1.5 * pi) return uin;
+  const GP xix = gp(m[0]), etx = gp(m[1]), ztx = gp(m[2]);
+  const long sj = d.sj, sk = d.sk;
+  const double t1 = 0.5 * (xix[c] + xix[mm]) * (b[c] - b[mm]);
+  const double t2 =
+      0.5 * (etx[c] + etx[mm]) * 0.25 * (b[c + sj] + b[mm + sj] - b[c - sj] - b[mm - sj]);
+  const double t3 =
+      0.5 * (ztx[c] + ztx[mm]) * 0.25 * (b[c + sk] + b[mm + sk] - b[c - sk] - b[mm - sk]);
+  return 0.5 * (b[c] + b[mm]) - dtime * 1.0 * (t1 + t2 + t3);
+}
+
 __global__ void k_ufar(Dims d, const double* const* __restrict__ m, const double* __restrict__ theta,
                        FarSet fs, int nc, double dtime, double pi, double* ufar) {
   const long nf = (long)(d.nj + 1) * (d.nk + 1);
@@ -351,22 +414,60 @@ __global__ void k_ufar(Dims d, const double* const* __restrict__ m, const double
     int comp = (int)(t / nf);
     long r = t - comp * nf;
     int j = (int)(r % (d.nj + 1)), k = (int)(r / (d.nj + 1));
-    if (j < 1 || j > d.nj - 1 || k < 1 || k > d.nk - 1) { ufar[t] = 0.0; continue; }
-    const GP b = gp(fs.b[comp]);
-    const double uin = fs.uin[comp];
-    long c = cidx(d, d.ni, j, k), mm = c - 1;
-    double th = theta[c], uf;
-    if (th >= 0.5 * pi && th <= 1.5 * pi) {
-      uf = uin;
-    } else {
-      const double *xix = m[0], *etx = m[1], *ztx = m[2];
-      const long sj = d.sj, sk = d.sk;
-      double t1 = 0.5 * (xix[c] + xix[mm]) * (b[c] - b[mm]);
-      double t2 = 0.5 * (etx[c] + etx[mm]) * 0.25 * (b[c + sj] + b[mm + sj] - b[c - sj] - b[mm - sj]);
-      double t3 = 0.5 * (ztx[c] + ztx[mm]) * 0.25 * (b[c + sk] + b[mm + sk] - b[c - sk] - b[mm - sk]);
-      uf = 0.5 * (b[c] + b[mm]) - dtime * 1.0 * (t1 + t2 + t3);
-    }
-    ufar[t] = uf;
+    const bool in = j >= 1 && j <= d.nj - 1 && k >= 1 && k <= d.nk - 1;
+    ufar[t] = in ? ufar_value(d, m, theta, fs.b[comp], fs.uin[comp], dtime, pi, j, k) : 0.0;
+  }
+}
+
+// The start of a step in one pass over every cell (RLES/main.f90:41-48): U_N = U, ..., T_N = T,
+// CONTRA_VEL (JU on i = 0..NI of the interior rows; a J or K ghost forms the JU of its periodic
+// partner) and the far-field values of BCU and BCT, from u, v, w, T, which nothing writes here.
+// U, V, W are read once for the copy and for JU: 4 launches and 25.7 + 69.8 + 5.5 us on
+// 192 x 256 x 64 cells became one.
+struct StepStart {
+  const double* f[4];  // u, v, w, T
+  double* fn[4];       // U_N, V_N, W_N, T_N
+  double* ju[3];
+  double* ufar;        // three components
+  double* tfar;        // of T, or nullptr without the passive temperature
+};
+
+template <bool XZ0>
+__global__ void __launch_bounds__(256) k_step_begin(Dims d, const double* const* __restrict__ m,
+                                                    const double* __restrict__ djac,
+                                                    const double* __restrict__ theta, StepStart a,
+                                                    double dtime, double pi) {
+  const uint3 bb = xcd_block();
+  const int i = bb.x * 64 + threadIdx.x;
+  const int j = bb.y * 4 + threadIdx.y;
+  const int k = bb.z;
+  if (i > d.ni || j > d.nj) return;
+  const long c = cidx(d, i, j, k);
+  const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
+  const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
+  const bool in = js == j && ks == k;
+  const long cs = cidx(d, i, js, ks);
+  double q[3], o[3];
+#pragma unroll
+  for (int f = 0; f < 3; ++f) {
+    q[f] = gp(a.f[f])[cs];
+    o[f] = in ? q[f] : gp(a.f[f])[c];
+  }
+  double b[3];
+  contra_cell<XZ0>(m, cs, djac[cs], q[0], q[1], q[2], b);
+#pragma unroll
+  for (int f = 0; f < 3; ++f) {
+    gpw(a.fn[f])[c] = o[f];
+    gpw(a.ju[f])[c] = b[f];
+  }
+  if (a.tfar) gpw(a.fn[3])[c] = gp(a.f[3])[c];
+  if (i == d.ni) {
+    const long nf = (long)(d.nj + 1) * (d.nk + 1), t = j + (long)(d.nj + 1) * k;
+#pragma unroll
+    for (int f = 0; f < 3; ++f)
+      a.ufar[f * nf + t] =
+          in ? ufar_value(d, m, theta, a.f[f], f == 0 ? 1.0 : 0.0, dtime, pi, j, k) : 0.0;
+    if (a.tfar) a.tfar[t] = in ? ufar_value(d, m, theta, a.f[3], 0.0, dtime, pi, j, k) : 0.0;
   }
 }
 
@@ -428,25 +529,10 @@ __global__ void k_add_sgs(Dims d, const double* __restrict__ djac, double* nl,
   nl[c] = nl[c] + sgs[c] * djac[c];
 }
 
-// span mean of p at (IE, NJ/4, K), summed in the reference's order by one lane
-// (RLES/main.f90:125-131)
+// span mean of p at (IE, NJ/4, K) (RLES/main.f90:125-131)
 __global__ void k_pref(Dims d, const double* __restrict__ p, double* out) {
-  // the span values are fetched by the whole workgroup at once, then summed in K order by one
-  // lane (the reference's order)
   __shared__ double sh[256];
-  const int t = threadIdx.x;
-  double s = 0.0;
-  for (int k0 = 1; k0 <= d.nk - 1; k0 += 256) {
-    const int k = k0 + t;
-    if (k <= d.nk - 1) sh[t] = p[cidx(d, d.ni, d.nj / 4, k)];
-    __syncthreads();
-    if (t == 0) {
-      const int cnt = min(256, d.nk - k0);
-      for (int q = 0; q < cnt; ++q) s = s + sh[q];
-    }
-    __syncthreads();
-  }
-  if (t == 0) out[0] = s / (double)(d.nk - 1);
+  pref_mean(d, p, out, threadIdx.x, sh);
 }
 
 __global__ void k_sub_pref(Dims d, double* p, const double* __restrict__ pref) {
@@ -459,19 +545,6 @@ __global__ void k_sub_pref(Dims d, double* p, const double* __restrict__ pref) {
 // ---------------------------------------------------------------------------------------
 // CALCCOEF (RLES/calccoef.f90:11-201)
 // ---------------------------------------------------------------------------------------
-__device__ inline double block_reduce_sum(double v, double* sh) {
-  const int t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (t < s) sh[t] = sh[t] + sh[t + s];
-    __syncthreads();
-  }
-  double r = sh[0];
-  __syncthreads();
-  return r;
-}
-
 __device__ inline double block_reduce_max(double v, double* sh) {
   const int t = threadIdx.x;
   sh[t] = v;
@@ -509,18 +582,65 @@ __global__ void k_cfl(Dims d, const double* const* __restrict__ m, const double*
   if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
+// Tree sums of N values per lane over a workgroup of 256, the N trees in step (one barrier per
+// level for all of them, each in the order of a tree of its own); r[q] on every lane
+template <int N>
+__device__ inline void block_reduce_sums(double (&r)[N], double (*sh)[256]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < N; ++q) sh[q][t] = r[q];
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) {
+#pragma unroll
+      for (int q = 0; q < N; ++q) sh[q][t] = sh[q][t] + sh[q][t + s];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < N; ++q) r[q] = sh[q][0];
+  __syncthreads();
+}
+
 // surface-force partial sums over the wall triangles (calccoef.f90:76-183): one element per
 // lane, a fixed-order tree per block; part[5 b + q] for pressure drag / lift, viscous drag /
 // lift and the wall heat flux sum (T - T_WALL)/D_N AREA of the Nusselt number (calccoef.f90:117-119,
-// 155-157; zero without the temperature, T = nullptr)
+// 155-157; zero without the temperature, T = nullptr).  One workgroup more forms the span mean of
+// the base pressure into part[5 nfb]: the 8-cell averages at the first wall node line
+// (calccoef.f90:39-74), one lane per K, added in K order by one lane.  pref, when given, is the
+// pressure reference that p has not been shifted by yet.
 __global__ void k_forces_part(Dims d, const double* __restrict__ wall, const double* __restrict__ p,
                               const double* __restrict__ u, const double* __restrict__ v,
                               const double* __restrict__ w, const double* __restrict__ T,
-                              double re, double* part) {
-  __shared__ double sh[256];
+                              double re, double* part, int nfb, const double* __restrict__ pref) {
+  __shared__ double sh[5][256];
+  const int tid = threadIdx.x;
+  const bool shift = pref != nullptr;
+  const double rf = shift ? pref[0] / 1.0 : 0.0;
+  if ((int)blockIdx.x == nfb) {
+    double s = 0.0;
+    const long sj = d.sj, sk = d.sk;
+    auto P = [&](long c) { return shift ? p[c] - rf : p[c]; };
+    for (int k0 = 1; k0 <= d.nk - 1; k0 += 256) {
+      const int k = k0 + tid;
+      if (k <= d.nk - 1) {
+        const long c = cidx(d, 1, 1, k);
+        sh[0][tid] = 0.125 * (P(c) + P(c - sj) + P(c - 1) + P(c - 1 - sj) + P(c + sk) +
+                              P(c - sj + sk) + P(c - 1 + sk) + P(c - 1 - sj + sk));
+      }
+      __syncthreads();
+      if (tid == 0) {
+        const int cnt = min(256, d.nk - k0);
+        for (int q = 0; q < cnt; ++q) s = s + sh[0][q];
+      }
+      __syncthreads();
+    }
+    if (tid == 0) part[5 * nfb] = s;
+    return;
+  }
   const long nw = (long)(d.nj - 1) * (d.nk - 1);
-  double pd = 0.0, ply = 0.0, td = 0.0, tly = 0.0, snu = 0.0;
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  double f[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // pressure drag, lift, viscous drag, lift, heat flux
+  const long t = blockIdx.x * 256L + tid;
   if (t < 2 * nw) {
     int tri = (int)(t / nw);
     long r = t - tri * nw;
@@ -529,79 +649,54 @@ __global__ void k_forces_part(Dims d, const double* __restrict__ wall, const dou
     const double* o = wall + 6 * t;
     double A = o[0], B = o[1], C = o[2], dum = o[3], dn = o[4], ar = o[5];
     double U = u[c], V = v[c], W = w[c];
+    const double pc = shift ? p[c] - rf : p[c];
     double t1 = V * C / dum - W * B / dum, t2 = U * C / dum - W * A / dum,
            t3 = U * B / dum - V * A / dum;
     double dudn = sqrt(t1 * t1 + t2 * t2 + t3 * t3);
     dudn = dudn / dn;
     double um = sqrt(U * U + V * V + W * W);
-    pd = -2.0 * p[c] * ar * A / dum;
-    ply = -2.0 * p[c] * ar * B / dum;
-    td = (2.0 / re) * dudn * ar * U / um;
-    tly = (2.0 / re) * dudn * ar * V / um;
+    f[0] = -2.0 * pc * ar * A / dum;
+    f[1] = -2.0 * pc * ar * B / dum;
+    f[2] = (2.0 / re) * dudn * ar * U / um;
+    f[3] = (2.0 / re) * dudn * ar * V / um;
     if (T) {
       const double dtdn = (T[c] - 1.0) / dn;  // T_WALL = 1
-      snu = dtdn * ar;
+      f[4] = dtdn * ar;
     }
   }
-  pd = block_reduce_sum(pd, sh);
-  ply = block_reduce_sum(ply, sh);
-  td = block_reduce_sum(td, sh);
-  tly = block_reduce_sum(tly, sh);
-  snu = block_reduce_sum(snu, sh);
-  if (threadIdx.x == 0) {
-    part[5 * blockIdx.x] = pd; part[5 * blockIdx.x + 1] = ply;
-    part[5 * blockIdx.x + 2] = td; part[5 * blockIdx.x + 3] = tly;
-    part[5 * blockIdx.x + 4] = snu;
+  block_reduce_sums<5>(f, sh);
+  if (tid == 0) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) part[5 * blockIdx.x + q] = f[q];
   }
 }
 
 // force coefficients, base pressure, CFL maximum and Nusselt number NU = -sum / SUM_AREA
-// (calccoef.f90:11-184), one block; out[0..7] as fvm_step_info, out[8] = NU
-__global__ void k_forces_final(Dims d, const double* __restrict__ p,
-                               const double* __restrict__ fpart, int nfb, double ref_a,
-                               double sum_area, const double* __restrict__ cflpart, int ncfl,
-                               double* out, Mailbox mb) {
-  __shared__ double sh[256];
+// (calccoef.f90:11-184) by one workgroup of 256; out[0..7] as fvm_step_info, out[8] = NU
+__device__ inline void forces_final(const Dims& d, const double* __restrict__ fpart, int nfb,
+                                    double ref_a, double sum_area,
+                                    const double* __restrict__ cflpart, int ncfl, double* out,
+                                    const Mailbox& mb) {
+  __shared__ double sh[6][256];
+  const int tid = threadIdx.x;
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int b = threadIdx.x; b < nfb; b += blockDim.x)
+  for (int b = tid; b < nfb; b += 256)
     for (int q = 0; q < 5; ++q) acc[q] = acc[q] + fpart[5 * b + q];
-  const double pd = block_reduce_sum(acc[0], sh);
-  const double ply = block_reduce_sum(acc[1], sh);
-  const double td = block_reduce_sum(acc[2], sh);
-  const double tly = block_reduce_sum(acc[3], sh);
-  const double snu = block_reduce_sum(acc[4], sh);
   double cm[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // eight loads in flight per lane
-  int q = threadIdx.x;
-  for (; q + 7 * (int)blockDim.x < ncfl; q += 8 * blockDim.x) {
+  int q = tid;
+  for (; q + 7 * 256 < ncfl; q += 8 * 256) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) cm[u] = fmax(cm[u], cflpart[q + u * blockDim.x]);
+    for (int u = 0; u < 8; ++u) cm[u] = fmax(cm[u], cflpart[q + u * 256]);
   }
-  for (; q < ncfl; q += blockDim.x) cm[0] = fmax(cm[0], cflpart[q]);
+  for (; q < ncfl; q += 256) cm[0] = fmax(cm[0], cflpart[q]);
   double cmax = cm[0];
 #pragma unroll
   for (int u = 1; u < 8; ++u) cmax = fmax(cmax, cm[u]);
-  cmax = block_reduce_max(cmax, sh);
-  // base pressure: 8-cell average at the first wall node line, span mean (calccoef.f90:39-74);
-  // the node averages are formed by one lane per K, the span sum in K order by lane 0
-  double dumb = 0.0;
-  const long sj = d.sj, sk = d.sk;
-  for (int k0 = 1; k0 <= d.nk - 1; k0 += blockDim.x) {
-    const int k = k0 + (int)threadIdx.x;
-    if (k <= d.nk - 1) {
-      const long c = cidx(d, 1, 1, k);
-      sh[threadIdx.x] = 0.125 * (p[c] + p[c - sj] + p[c - 1] + p[c - 1 - sj] + p[c + sk] +
-                                 p[c - sj + sk] + p[c - 1 + sk] + p[c - 1 - sj + sk]);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int cnt = min((int)blockDim.x, d.nk - k0);
-      for (int q = 0; q < cnt; ++q) dumb = dumb + sh[q];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    dumb = dumb / (double)(d.nk - 1);
-    double cdp = pd / ref_a, clp = ply / ref_a, cdv = td / ref_a, clv = tly / ref_a;
+  cmax = block_reduce_max(cmax, sh[5]);
+  block_reduce_sums<5>(acc, sh);
+  if (tid == 0) {
+    const double dumb = fpart[5 * nfb] / (double)(d.nk - 1);
+    double cdp = acc[0] / ref_a, clp = acc[1] / ref_a, cdv = acc[2] / ref_a, clv = acc[3] / ref_a;
     out[0] = cmax;
     out[1] = 2.0 * (0.0 - dumb);
     out[2] = cdp + cdv;
@@ -610,7 +705,7 @@ __global__ void k_forces_final(Dims d, const double* __restrict__ p,
     out[5] = cdv;
     out[6] = clp;
     out[7] = clv;
-    out[8] = sum_area > 0.0 ? -snu / sum_area : 0.0;
+    out[8] = sum_area > 0.0 ? -acc[4] / sum_area : 0.0;
     if (mb.dst) {  // scal[0..16]: out is scal + 8; the rest was written by earlier kernels
       const double* sc = out - 8;
       double v[17];
@@ -618,6 +713,31 @@ __global__ void k_forces_final(Dims d, const double* __restrict__ p,
       publish(mb, v, 17);
     }
   }
+}
+
+__global__ void __launch_bounds__(256) k_forces_final(Dims d, const double* __restrict__ fpart,
+                                                      int nfb, double ref_a, double sum_area,
+                                                      const double* __restrict__ cflpart,
+                                                      int ncfl, double* out, Mailbox mb) {
+  forces_final(d, fpart, nfb, ref_a, sum_area, cflpart, ncfl, out, mb);
+}
+
+// The end of a step: p minus the pressure reference on every cell (RLES/main.f90:132-135) and, by
+// the first workgroup, the force coefficients, published to the host while the others shift p.
+__global__ void __launch_bounds__(256) k_step_end(Dims d, double* p,
+                                                  const double* __restrict__ pref,
+                                                  const double* __restrict__ fpart, int nfb,
+                                                  double ref_a, double sum_area,
+                                                  const double* __restrict__ cflpart, int ncfl,
+                                                  double* out, Mailbox mb) {
+  if (blockIdx.x == 0) {
+    forces_final(d, fpart, nfb, ref_a, sum_area, cflpart, ncfl, out, mb);
+    return;
+  }
+  const double r = pref[0] / 1.0;
+  for (long q = (blockIdx.x - 1) * 256L + threadIdx.x; q < d.n;
+       q += (long)(gridDim.x - 1) * 256)
+    p[q] = p[q] - r;
 }
 
 // CALCCOEF of the 2D solver (cylinder/cylinder_v3.0.3_AF_original 4step_face_nl/
@@ -773,14 +893,11 @@ int fvm_k_p_source(FvmCtx* c) {
   const Dims d = c->d;
   const int kc = march_planes(d, PS_RES);
   const dim3 g = march_grid(d, kc);
-  if (c->xz_zero)
-    hipLaunchKernelGGL((k_psource_km<0, true>), g, kBlk, 0, c->stream, c->d, kc,
-                       (const double* const*)m, c->djac, c->p, 0.0, 0.0, c->s[0], c->s[1],
-                       c->s[2], nullptr, nullptr, nullptr, nullptr);
-  else
-    hipLaunchKernelGGL((k_psource_km<0, false>), g, kBlk, 0, c->stream, c->d, kc,
-                       (const double* const*)m, c->djac, c->p, 0.0, 0.0, c->s[0], c->s[1],
-                       c->s[2], nullptr, nullptr, nullptr, nullptr);
+  auto kern = c->xz_zero ? k_psource_km<0, true> : k_psource_km<0, false>;
+  hipLaunchKernelGGL(kern, dim3(g.x * g.y * g.z), kBlk, 0, c->stream, c->d, kc,
+                     make_uint3(g.x, g.y, g.z), (const double* const*)m, c->djac, c->p, 0.0,
+                     c->s[0], c->s[1], c->s[2], nullptr, nullptr, nullptr, nullptr, nullptr,
+                     nullptr);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -922,11 +1039,12 @@ long fvm_calccoef_scratch(const FvmCtx* c, bool cfl_ready) {
   const long ncfl = cfl_ready ? 0 : 512;
   if (c->two_d) return ncfl;
   const long nw2 = 2L * (c->d.nj - 1) * (c->d.nk - 1);
-  return ncfl + 5L * ((nw2 + 255) / 256);
+  return ncfl + 5L * ((nw2 + 255) / 256) + 1;
 }
 
+// shift: also p minus the pressure reference in scal[2], which the forces are formed with
 int fvm_k_calccoef(FvmCtx* c, double* out8, bool cfl_ready, const Mailbox* mb, double* part,
-                   long cap) {
+                   long cap, bool shift) {
   double** m = c->dm;
   ProfScope ps(c, "calccoef");
   if (!part) { part = c->red; cap = c->nred; }
@@ -939,11 +1057,18 @@ int fvm_k_calccoef(FvmCtx* c, double* out8, bool cfl_ready, const Mailbox* mb, d
                        c->u, c->v, c->w, c->prm.dtime, part);
   const long nw2 = 2L * (c->d.nj - 1) * (c->d.nk - 1);
   const int nfb = (int)((nw2 + 255) / 256);
-  hipLaunchKernelGGL(k_forces_part, dim3(nfb), dim3(256), 0, c->stream, c->d, c->wall, c->p,
-                     c->u, c->v, c->w, c->thermal ? c->t : nullptr, c->prm.re, part + off);
-  hipLaunchKernelGGL(k_forces_final, dim3(1), dim3(256), 0, c->stream, c->d, c->p, part + off,
-                     nfb, c->prm.ref_a, c->thermal ? c->sum_area : 0.0, cfl, ncfl, c->scal + 8,
-                     mb ? *mb : Mailbox{nullptr, nullptr, 0});
+  const Mailbox box = mb ? *mb : Mailbox{nullptr, nullptr, 0};
+  const double area = c->thermal ? c->sum_area : 0.0;
+  hipLaunchKernelGGL(k_forces_part, dim3(nfb + 1), dim3(256), 0, c->stream, c->d, c->wall, c->p,
+                     c->u, c->v, c->w, c->thermal ? c->t : nullptr, c->prm.re, part + off, nfb,
+                     shift ? c->scal + 2 : nullptr);
+  if (shift)  // p's shift by the reference runs beside the final reduction
+    hipLaunchKernelGGL(k_step_end, dim3(1 + grid1(c->d.n, 256).x), dim3(256), 0, c->stream, c->d,
+                       c->p, c->scal + 2, part + off, nfb, c->prm.ref_a, area, cfl, ncfl,
+                       c->scal + 8, box);
+  else
+    hipLaunchKernelGGL(k_forces_final, dim3(1), dim3(256), 0, c->stream, c->d, part + off, nfb,
+                       c->prm.ref_a, area, cfl, ncfl, c->scal + 8, box);
   HIP_CHECK(hipGetLastError());
   if (out8) {
     HIP_CHECK(hipMemcpyAsync(out8, c->scal + 8, 8 * sizeof(double), hipMemcpyDeviceToHost,
@@ -1026,24 +1151,22 @@ int fvm_wall2d_setup(FvmCtx* c, const double* xg, const double* yg) {
   return FVM_OK;
 }
 
-// with_cfl: also leave the per-workgroup CFL maxima of the projected velocity in c->cflpart for the
-// CALCCOEF that ends the step (the pressure reference and BCU that come between change neither
-// the interior velocity nor the metrics)
-int fvm_k_psource_correct(FvmCtx* c, double sign, bool with_cfl) {
+// P_SOURCE, projection, BCU ghosts of u, v, w, the CFL maxima of the projected velocity in
+// c->cflpart for the CALCCOEF that ends the step (what comes between changes neither the interior
+// velocity nor the metrics) and, in 3D, the pressure reference in scal[2]
+int fvm_k_project(FvmCtx* c) {
   ProfScope ps(c, "psource_correct");
   const Dims d = c->d;
   const int kc = march_planes(d, PS_RES);
   const dim3 g = march_grid(d, kc);  // CFL maxima: one per workgroup
-  if (with_cfl && (long)g.x * g.y * g.z > c->ncflpart) return FVM_ERR_SIZE;
-  if (with_cfl) c->ncflused = (int)(g.x * g.y * g.z);
-  if (c->xz_zero)
-    hipLaunchKernelGGL((k_psource_km<1, true>), g, kBlk, 0, c->stream, c->d, kc,
-                       (const double* const*)c->dm, c->djac, c->p, sign, c->prm.dtime, c->s[0],
-                       c->s[1], c->s[2], c->u, c->v, c->w, with_cfl ? c->cflpart : nullptr);
-  else
-    hipLaunchKernelGGL((k_psource_km<1, false>), g, kBlk, 0, c->stream, c->d, kc,
-                       (const double* const*)c->dm, c->djac, c->p, sign, c->prm.dtime, c->s[0],
-                       c->s[1], c->s[2], c->u, c->v, c->w, with_cfl ? c->cflpart : nullptr);
+  const long nb = (long)g.x * g.y * g.z;
+  if (nb > c->ncflpart) return FVM_ERR_SIZE;
+  c->ncflused = (int)nb;
+  auto kern = c->xz_zero ? k_psource_km<1, true> : k_psource_km<1, false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)nb + (c->two_d ? 0 : 1)), kBlk, 0, c->stream, c->d, kc,
+                     make_uint3(g.x, g.y, g.z), (const double* const*)c->dm, c->djac, c->p,
+                     c->prm.dtime, c->s[0], c->s[1], c->s[2], c->u, c->v, c->w, c->ufar,
+                     c->cflpart, c->scal + 2);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -1051,25 +1174,28 @@ int fvm_k_psource_correct(FvmCtx* c, double sign, bool with_cfl) {
 // U = U - DTIME S / J^-1, BCU on u, v, w, CONTRA_VEL (RLES/main.f90:90-101)
 int fvm_k_correct_bcu_contra(FvmCtx* c) {
   const Dims d = c->d;
-  {
-    ProfScope ps(c, "correct_contra");
-    if (c->xz_zero)
-      hipLaunchKernelGGL(k_correct_contra<true>, interior_grid(d), kBlk, 0, c->stream, d,
-                         (const double* const*)c->dm, c->djac, c->prm.dtime, c->s[0], c->s[1],
-                         c->s[2], c->u, c->v, c->w, c->ju[0], c->ju[1], c->ju[2]);
-    else
-      hipLaunchKernelGGL(k_correct_contra<false>, interior_grid(d), kBlk, 0, c->stream, d,
-                         (const double* const*)c->dm, c->djac, c->prm.dtime, c->s[0], c->s[1],
-                         c->s[2], c->u, c->v, c->w, c->ju[0], c->ju[1], c->ju[2]);
-    HIP_CHECK(hipGetLastError());
-  }
-  double* f[3] = {c->u, c->v, c->w};
-  int r = fvm_k_bcu_ghosts(c, f, 3);
-  if (r) return r;
-  const long nf = (long)(d.nj - 1) * (d.nk - 1);
-  hipLaunchKernelGGL(k_contra_iplanes, grid1(2 * nf, 256), dim3(256), 0, c->stream, d,
-                     (const double* const*)c->dm, c->djac, c->u, c->v, c->w, c->ju[0], c->ju[1],
-                     c->ju[2]);
+  ProfScope ps(c, "correct_contra");
+  const Vec3P s = {{c->s[0], c->s[1], c->s[2]}}, f = {{c->u, c->v, c->w}},
+              ju = {{c->ju[0], c->ju[1], c->ju[2]}};
+  auto kern = c->xz_zero ? k_correct_contra<true> : k_correct_contra<false>;
+  hipLaunchKernelGGL(kern, interior_grid(d), kBlk, 0, c->stream, d, (const double* const*)c->dm,
+                     c->djac, c->prm.dtime, s, f, ju, c->ufar);
   HIP_CHECK(hipGetLastError());
-  return fvm_ghost_fill_n(c, c->ju, 3);
+  return FVM_OK;
+}
+
+// fvm_begin_step and CONTRA_VEL of the step (k_step_begin)
+int fvm_k_step_begin(FvmCtx* c) {
+  const Dims d = c->d;
+  ProfScope ps(c, "step_begin");
+  const StepStart a = {{c->u, c->v, c->w, c->t}, {c->un, c->vn, c->wn, c->tn},
+                       {c->ju[0], c->ju[1], c->ju[2]}, c->ufar, c->thermal ? c->tfar : nullptr};
+  const dim3 g((d.ni + 1 + 63) / 64, (d.nj + 1 + 3) / 4, d.nk + 1);
+  auto kern = c->xz_zero ? k_step_begin<true> : k_step_begin<false>;
+  hipLaunchKernelGGL(kern, g, kBlk, 0, c->stream, d, (const double* const*)c->dm, c->djac,
+                     c->theta, a, c->prm.dtime, c->pi);
+  HIP_CHECK(hipGetLastError());
+  c->u_is_un = true;
+  c->ufar_stale = false;
+  return FVM_OK;
 }

@@ -196,17 +196,25 @@ __global__ void k_p_res_final(const double* __restrict__ part, long nb, double* 
   if (t == 0) { out[0] = s0[0]; out[1] = s1[0]; out[2] = scaled_residual(s0[0], s1[0]); }
 }
 
-// BCP ghosts: wall p(0) = p(1), outflow cubic extrapolation (bcp.f90:22-32); the periodic
-// ghosts follow (fvm_ghost_fill)
+// BCP ghosts, wall p(0) = p(1) and outflow cubic extrapolation (bcp.f90:22-32), and the periodic
+// copy of MPI_X in one pass over the ghost surface: every ghost is a function of the interior
+// cells of one radial line, that of its periodic partner (js, ks)
 template <typename T>
 __global__ void k_bcp(Dims d, T* p) {
-  const long nf = (long)(d.nj - 1) * (d.nk - 1);
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < nf;
+  const long cnt = bc_ghost_count(d);
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < cnt;
        t += (long)gridDim.x * blockDim.x) {
-    int j = 1 + (int)(t % (d.nj - 1)), k = 1 + (int)(t / (d.nj - 1));
-    long c0 = cidx(d, 0, j, k), cn = cidx(d, d.ni, j, k);
-    p[c0] = p[c0 + 1];
-    p[cn] = (T)3.0 * p[cn - 1] - (T)3.0 * p[cn - 2] + p[cn - 3];
+    int i, j, k, js, ks;
+    ghost_cell(d, t, i, j, k, js, ks);
+    const long c = cidx(d, i, js, ks);
+    T v;
+    if (i == 0)
+      v = p[c + 1];
+    else if (i == d.ni)
+      v = (T)3.0 * p[c - 1] - (T)3.0 * p[c - 2] + p[c - 3];
+    else
+      v = p[c];
+    p[cidx(d, i, j, k)] = v;
   }
 }
 
@@ -285,17 +293,15 @@ __global__ void k_p_add(Dims d, double* p, const float* __restrict__ e) {
 }  // namespace
 
 int fvm_k_bcp(FvmCtx* c) {
-  long nf = (long)(c->d.nj - 1) * (c->d.nk - 1);
-  hipLaunchKernelGGL(k_bcp<double>, grid1(nf, 256), dim3(256), 0, c->stream, c->d, c->p);
+  hipLaunchKernelGGL(k_bcp<double>, grid1(bc_ghost_count(c->d), 256), dim3(256), 0, c->stream,
+                     c->d, c->p);
   HIP_CHECK(hipGetLastError());
-  return fvm_ghost_fill(c, c->p);
+  return FVM_OK;
 }
 
 static int bcp32(FvmCtx* c, float* e) {
-  const Dims d = c->d;
-  long nf = (long)(d.nj - 1) * (d.nk - 1);
-  hipLaunchKernelGGL(k_bcp<float>, grid1(nf, 256), dim3(256), 0, c->stream, d, e);
-  hipLaunchKernelGGL(k_ghost_fill_t<float>, grid1(ghost_count(d), 256), dim3(256), 0, c->stream, d, e);
+  hipLaunchKernelGGL(k_bcp<float>, grid1(bc_ghost_count(c->d), 256), dim3(256), 0, c->stream,
+                     c->d, e);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -434,8 +440,7 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
       }
     }
   }
-  r = fvm_k_bcp(c);
-  if (r) return r;
+  // the last residual's BCP ghosts belong to the final p
   *resip = res;
   *niter = sweeps;
   c->last.nouter = outer;

@@ -663,8 +663,7 @@ int fvm_k_iter_p_sep(FvmCtx* c, bool mixed, double* resip, int* niter) {
     if (r) return r;
     ++outer;
   }
-  int r = fvm_k_bcp(c);
-  if (r) return r;
+  // the last residual's BCP ghosts belong to the final p
   *resip = res;
   *niter = outer;
   c->last.nouter = outer;

@@ -22,10 +22,11 @@ struct Diff3 {
   double i, j, k;
 };
 
+// The cell (i, j, k) = c writes its values' J and K ghost images as well.
 template <bool XZ0>
-__device__ inline void strain_store(const double* const* __restrict__ m, long c, bool onesided,
-                                    Diff3 u, Diff3 v, Diff3 w, double* const* __restrict__ L,
-                                    double* mag) {
+__device__ inline void strain_store(const Dims& d, const double* const* __restrict__ m, int i,
+                                    int j, int k, long c, bool onesided, Diff3 u, Diff3 v,
+                                    Diff3 w, double* const* __restrict__ L, double* mag) {
   const double xix = m[0][c], etx = m[1][c], ztx = m[2][c];
   const double xiy = m[3][c], ety = m[4][c], zty = m[5][c];
   const double xiz = XZ0 ? 0.0 : m[6][c], etz = XZ0 ? 0.0 : m[7][c], ztz = m[8][c];
@@ -58,36 +59,53 @@ __device__ inline void strain_store(const double* const* __restrict__ m, long c,
   L[0][c] = l11; L[1][c] = l12; L[2][c] = l13; L[3][c] = l22; L[4][c] = l23; L[5][c] = l33;
   double s = l11 * l11 + l12 * l12 + l13 * l13 + l12 * l12 + l22 * l22 + l23 * l23 +
              l13 * l13 + l23 * l23 + l33 * l33;
-  mag[c] = sqrt(2.0 * s);
+  const double mg = sqrt(2.0 * s);
+  mag[c] = mg;
+  const double lv[6] = {l11, l12, l13, l22, l23, l33};
+#pragma unroll
+  for (int q = 0; q < 6; ++q) periodic_images(d, L[q], i, j, k, lv[q]);
+  periodic_images(d, mag, i, j, k, mg);
 }
 
-// Strain on the I ghost planes i = 0 and i = NI (one-sided radial difference), interior j, k.
-__global__ void k_strain_iplanes(Dims d, const double* const* __restrict__ m,
-                                 const double* __restrict__ U, const double* __restrict__ V,
-                                 const double* __restrict__ W, double* const* __restrict__ L,
-                                 double* mag, const double* __restrict__ T, double* dtx,
-                                 double* dty, double* dtz) {
+struct SfOut {
+  const double* in[4];  // u, v, w, T
+  double* hat[4];       // u^, v^, w^, T^
+  double* dt[3];        // dT/dx, dT/dy, dT/dz
+  const double* ufar;   // far-field values of u, v, w (BCU of the filtered velocity)
+  const double* tfar;   // and of T (BCT)
+};
+
+// Strain on the I ghost planes i = 0 and i = NI (one-sided radial difference), interior j, k:
+// cell t of the two planes, with its periodic images
+template <int NF>
+__device__ inline void strain_iplane(const Dims& d, const double* const* __restrict__ m,
+                                     const SfOut& io, double* const* __restrict__ L, double* mag,
+                                     long t) {
   const long nl = (long)(d.nj - 1) * (d.nk - 1);
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (t >= 2 * nl) return;
   const bool lo = t < nl;
   const long r = lo ? t : t - nl;
-  const int j = 1 + (int)(r % (d.nj - 1)), k = 1 + (int)(r / (d.nj - 1));
-  const long c = cidx(d, lo ? 0 : d.ni, j, k);
+  const int i = lo ? 0 : d.ni, j = 1 + (int)(r % (d.nj - 1)), k = 1 + (int)(r / (d.nj - 1));
+  const long c = cidx(d, i, j, k);
   const long sj = d.sj, sk = d.sk;
-  auto diff = [&](const double* F) {
+  auto diff = [&](const double* Fp) {
+    const GP F = gp(Fp);
     Diff3 q;
     q.i = lo ? (F[c + 1] - F[c]) : (F[c] - F[c - 1]);
     q.j = F[c + sj] - F[c - sj];
     q.k = F[c + sk] - F[c - sk];
     return q;
   };
-  strain_store<false>(m, c, true, diff(U), diff(V), diff(W), L, mag);
-  if (T) {  // one-sided temperature gradient (stress_tensor_dy.f90:138-146, 188-196)
-    const Diff3 g = diff(T);
-    dtx[c] = 0.5 * (2.0 * gp(m[0])[c] * g.i + gp(m[1])[c] * g.j + gp(m[2])[c] * g.k);
-    dty[c] = 0.5 * (2.0 * gp(m[3])[c] * g.i + gp(m[4])[c] * g.j + gp(m[5])[c] * g.k);
-    dtz[c] = 0.5 * (2.0 * gp(m[6])[c] * g.i + gp(m[7])[c] * g.j + gp(m[8])[c] * g.k);
+  strain_store<false>(d, m, i, j, k, c, true, diff(io.in[0]), diff(io.in[1]), diff(io.in[2]), L,
+                      mag);
+  if (NF == 4) {  // one-sided temperature gradient (stress_tensor_dy.f90:138-146, 188-196)
+    const Diff3 g = diff(io.in[3]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const double v = 0.5 * (2.0 * gp(m[3 * q])[c] * g.i + gp(m[3 * q + 1])[c] * g.j +
+                              gp(m[3 * q + 2])[c] * g.k);
+      gpw(io.dt[q])[c] = v;
+      periodic_images(d, io.dt[q], i, j, k, v);
+    }
   }
 }
 
@@ -99,20 +117,24 @@ __global__ void k_strain_iplanes(Dims d, const double* const* __restrict__ m,
 // I-1, I, I+1.
 // With NF = 4 the temperature rides along: its gradient dT/dx_i = 0.5 (xi_i dT/dxi +
 // eta_i dT/deta + zeta_i dT/dzeta) (stress_tensor_dy.f90:78-94) and its test filter T^.
+// A cell writes the ghosts that are functions of it (the periodic images of S_ij, |S| and dT/dx_i,
+// the BCU / BCT ghosts of the filtered fields), and the workgroups past the tiles form the I ghost
+// planes' strain, so one launch leaves every array of the pass complete: the three surface
+// launches it replaces took 20 + 9 + 7 us on 192 x 256 x 64 cells.
 constexpr int SF_RES = 768;  // workgroups resident at a time (three per CU)
 
-struct SfOut {
-  const double* in[4];  // u, v, w, T
-  double* hat[4];       // u^, v^, w^, T^
-  double* dt[3];        // dT/dx, dT/dy, dT/dz
-};
-
 template <int NF, bool XZ0>
-__global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc,
+__global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc, uint3 tg,
                                                        const double* const* __restrict__ m,
                                                        SfOut io, double* const* __restrict__ L,
                                                        double* mag) {
-  const uint3 bb = xcd_block();
+  const unsigned nb = tg.x * tg.y * tg.z;
+  if (blockIdx.x >= nb) {
+    const long t = (long)(blockIdx.x - nb) * 256 + threadIdx.y * 64 + threadIdx.x;
+    if (t < 2L * (d.nj - 1) * (d.nk - 1)) strain_iplane<NF>(d, m, io, L, mag, t);
+    return;
+  }
+  const uint3 bb = xcd_tile(blockIdx.x, tg.x, tg.y, tg.z);
   __shared__ double sh[NF][3][SF_P];  // [field][plane slot][tile cell]
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i = 1 + bb.x * 64 + tx;
@@ -144,17 +166,20 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc,
       g[f].j = sh[f][s0][q0 + SF_W] - sh[f][s0][q0 - SF_W];
       g[f].k = sh[f][sp][q0] - sh[f][sm][q0];
     }
-    strain_store<XZ0>(m, c, false, g[0], g[1], g[2], L, mag);
+    strain_store<XZ0>(d, m, i, j, k, c, false, g[0], g[1], g[2], L, mag);
     if (NF == 4) {
       const double ti = sh[3][s0][q0 + 1] - sh[3][s0][q0 - 1];
       const double tj = sh[3][s0][q0 + SF_W] - sh[3][s0][q0 - SF_W];
       const double tk = sh[3][sp][q0] - sh[3][sm][q0];
-      double t = gp(m[0])[c] * ti + gp(m[1])[c] * tj + gp(m[2])[c] * tk;
-      io.dt[0][c] = 0.5 * t;
-      t = gp(m[3])[c] * ti + gp(m[4])[c] * tj + gp(m[5])[c] * tk;
-      io.dt[1][c] = 0.5 * t;
-      t = mget<XZ0>(m, 6, c) * ti + mget<XZ0>(m, 7, c) * tj + gp(m[8])[c] * tk;
-      io.dt[2][c] = 0.5 * t;
+      const double t[3] = {
+          gp(m[0])[c] * ti + gp(m[1])[c] * tj + gp(m[2])[c] * tk,
+          gp(m[3])[c] * ti + gp(m[4])[c] * tj + gp(m[5])[c] * tk,
+          mget<XZ0>(m, 6, c) * ti + mget<XZ0>(m, 7, c) * tj + gp(m[8])[c] * tk};
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        gpw(io.dt[q])[c] = 0.5 * t[q];
+        periodic_images(d, io.dt[q], i, j, k, 0.5 * t[q]);
+      }
     }
     const int pl[3] = {sm, s0, sp};
 #pragma unroll
@@ -173,7 +198,12 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc,
             t = first ? term : t + term;
             first = false;
           }
-      io.hat[f][c] = t / 64.0;
+      const double h = t / 64.0;
+      gpw(io.hat[f])[c] = h;
+      if (f < 3)
+        bc_images(d, io.hat[f], io.ufar + f * (long)(d.nj + 1) * (d.nk + 1), 0.0, i, j, k, h);
+      else  // BCT(T_HAT, T_N), T_WALL = 1 (stress_tensor_dy.f90:233)
+        bc_images(d, io.hat[f], io.tfar, 1.0, i, j, k, h);
     }
   }
 }
@@ -721,27 +751,16 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
     const int kc = march_planes(d, SF_RES);
     const dim3 g = march_grid(d, kc);
     const SfOut io = {{c->u, c->v, c->w, c->t}, {c->uh[0], c->uh[1], c->uh[2], c->that},
-                      {c->dtd[0], c->dtd[1], c->dtd[2]}};
+                      {c->dtd[0], c->dtd[1], c->dtd[2]}, c->ufar, c->tfar};
     auto kern = th ? k_strain_filter<4, false>
                    : (c->xz_zero ? k_strain_filter<3, true> : k_strain_filter<3, false>);
-    hipLaunchKernelGGL(kern, g, kBlk, 0, st, d, kc, (const double* const*)m, io,
+    const unsigned nb = g.x * g.y * g.z;
+    const long ni = 2L * (d.nj - 1) * (d.nk - 1);  // cells of the two I ghost planes
+    hipLaunchKernelGGL(kern, dim3(nb + (unsigned)((ni + 255) / 256)), kBlk, 0, st, d, kc,
+                       make_uint3(g.x, g.y, g.z), (const double* const*)m, io,
                        (double* const*)c->dlss, c->mag);
-    const long nb = 2L * (d.nj - 1) * (d.nk - 1);
-    hipLaunchKernelGGL(k_strain_iplanes, grid1(nb, 256), dim3(256), 0, st, d,
-                       (const double* const*)m, c->u, c->v, c->w, (double* const*)c->dlss,
-                       c->mag, th ? c->t : nullptr, c->dtd[0], c->dtd[1], c->dtd[2]);
     HIP_CHECK(hipGetLastError());
   }
-  double* gl[10] = {c->lss[0], c->lss[1], c->lss[2], c->lss[3], c->lss[4], c->lss[5], c->mag,
-                    c->dtd[0], c->dtd[1], c->dtd[2]};
-  int r = fvm_ghost_fill_n(c, gl, th ? 10 : 7);
-  if (r) return r;
-  if (th) {  // BCT(T_HAT, T_N) (stress_tensor_dy.f90:233)
-    r = fvm_k_bct_ghosts(c, c->that);
-    if (r) return r;
-  }
-  r = fvm_k_bcu_ghosts(c, c->uh, 3);
-  if (r) return r;
   {
     ProfScope pk(c, "k_lm");
     const int kc = march_planes(d, LM_RES);
