@@ -3,7 +3,8 @@
 //
 // Step (Main.f90:48-118): U_N copy, CONTRA_VEL + NL + DIF + P_SOURCE + the stage-1 right-hand
 // side of ITER_U/ITER_V (one fused stencil pass), the stage-1 BCU and I-line sweep, the
-// stage-2 right-hand side, BCU and J-line sweep, the predictor correction with BCU, the
+// stage-2 right-hand side with its J-line-major copy, the J-line sweep, its transposition back
+// with the predictor correction and BCU, the
 // Poisson right-hand side, ITER_P as FP64 defect correction with the separable inverse (fixed
 // pass count, converged cases skip), BCP, P_SOURCE + projection + BCU + CFL, CALCCOEF.
 #include <math.h>
@@ -56,6 +57,7 @@ __global__ void __launch_bounds__(512) k2_explicit(const Case2D* __restrict__ ta
   const auto P = glb(cs.f[F_P]);
   const auto UN = glb(cs.f[F_UN]);
   const auto VN = glb(cs.f[F_VN]);
+  if (i == 1 && j == 1) glb(cs.stat)[ST_AFCH] = 0.0;  // booked by the sweeps' last passes
   // U_N = U over the whole plane: every interior thread copies its cell and the ghosts next to
   // it (corners from the corner cells)
   {
@@ -203,7 +205,7 @@ __device__ inline void bcu_ghosts_wave(P F, int ni, int nj, int sj, B uwall, B u
 // ST_AFCH.  The operands of line L + 1 are loaded while line L is solved.
 // DIR 0: I lines (rows along I, lines J = 1..NJ-1, lagged coupling AS = AN(J-1));
 // DIR 1: J lines (rows along J, lines I = 1..NI-1, lagged coupling AW); the line ends take the
-// ghost values (BCU, applied by k2_sweep_seed) as Dirichlet data.
+// ghost values (BCU of the stage input) as Dirichlet data.
 // ---------------------------------------------------------------------------------------------
 template <int R, typename T>
 struct LineOps {
@@ -273,12 +275,14 @@ __device__ inline void sweep_load(LineOps<R, T>& o, gptr<const T> F, gptr<const 
 }
 
 // T = double: the sweep of the stage on the field itself (DIR 1 on the J-line-major copies: the
-// iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_tr_in and returned by
-// k2_tr_out).  T = float: the change form.  The sweep solves T_L d_L = r_L + AS d_(L-1) for the
+// iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_rhs2 and returned by
+// k2_correct).  T = float: the change form.  The sweep solves T_L d_L = r_L + AS d_(L-1) for the
 // change d = x - x0 of the stage input x0, with r the FP64 residual of x0 (k2_explicit,
-// k2_rhs2; the J-line stage's J-line-major copy by k2_tr_in32), zero ghosts and a zero ghost
-// line; the iterate is H_DU / H_DV (J-line-major for DIR 1).  The I-line stage's last pass adds
-// the change to the FP64 field, the J-line stage's k2_tr_out32 does.
+// k2_rhs2), zero ghosts and a zero ghost line; the iterate is H_DU / H_DV (J-line-major for
+// DIR 1).  The I-line stage's last pass adds the change to the FP64 field, the J-line stage's
+// k2_correct does.  First pass: the line before a chunk is the stage input's (no change in the
+// change form; the field in the FP64 J stage, whose iterate is a copy; k2_sweep_seed's boundary
+// lines in the FP64 I stage, which overwrites the field).
 template <int R, int DIR, bool EARLY, typename T>
 __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double tol, int final) {
   constexpr bool DELTA = std::is_same<T, float>::value;
@@ -326,9 +330,14 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
     // the line before the chunk: the ghost line 0 (no change in the change form), or the
     // preceding chunk's last line
     T v = (T)0;
-    if (r < n) {
-      if (ca > 0) v = (T)bnd[bin + (long)(ca - 1) * n + r];
-      else if (!DELTA) v = F[rs * (r + 1)];
+    if (r < n && (EARLY || !DELTA)) {
+      if (ca == 0) {
+        if (!DELTA) v = F[rs * (r + 1)];
+      } else if (!EARLY && DIR == 1) {
+        v = (T)glb(cs.f[comp ? F_V : F_U])[(a0 - 1) + (long)sj * (r + 1)];
+      } else {
+        v = (T)bnd[bin + (long)(ca - 1) * n + r];
+      }
     }
     prev[q] = v;
   }
@@ -422,14 +431,17 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
   for (int q = 0; q < R; ++q) {
     const int r = r0 + q;
     if (r < n) {
-      const double old = bnd[bin + (long)ca * n + r];
-      const double x = stopped ? old : (double)prev[q];  // a stopped chunk's last line keeps its value
-      dm = fmax(dm, fabs(x - old));
-      xm = fmax(xm, fabs(x));
+      double x = prev[q];
+      if (EARLY) {
+        const double old = bnd[bin + (long)ca * n + r];
+        if (stopped) x = old;  // a stopped chunk's last line keeps its value
+        dm = fmax(dm, fabs(x - old));
+        xm = fmax(xm, fabs(x));
+      }
       bnd[bout + (long)ca * n + r] = x;
     }
   }
-  if (final) {
+  if (EARLY && final) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       dm = fmax(dm, __shfl_xor(dm, o, 64));
@@ -443,138 +455,9 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
   }
 }
 
-// J-line-major copies for the J-line sweep: the right-hand sides and the stage input (ghosts
-// included, after BCU) of both components, 32 x 32 tiles through LDS; block table (case, tile).
-__global__ void __launch_bounds__(256) k2_tr_in(const Case2D* __restrict__ tab,
-                                                const int* __restrict__ bcase,
-                                                const int* __restrict__ btile) {
-  __shared__ double tile[4][32][33];
-  const Case2D& cs = tab[bcase[blockIdx.x]];
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int tx = (ni + 1 + 31) / 32, t = btile[blockIdx.x];
-  const int i0 = (t % tx) * 32, j0 = (t / tx) * 32;
-  const gptr<double> src[4] = {glb(cs.f[F_SU1]), glb(cs.f[F_SV1]), glb(cs.f[F_U]), glb(cs.f[F_V])};
-  const gptr<double> dst[4] = {glb(cs.f[F_TQU]), glb(cs.f[F_TQV]), glb(cs.f[F_TXU]), glb(cs.f[F_TXV])};
-  const int l = threadIdx.x;
-  for (int r = 0; r < 4; ++r) {
-    const int li = l % 32, lj = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a) tile[a][lj][li] = src[a][i + (long)sj * j];
-    }
-  }
-  __syncthreads();
-  for (int r = 0; r < 4; ++r) {
-    const int lj = l % 32, li = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a) dst[a][j + (long)(nj + 1) * i] = tile[a][lj][li];
-    }
-  }
-}
-
-// The J-line sweep's result back into the field interior.
-__global__ void __launch_bounds__(256) k2_tr_out(const Case2D* __restrict__ tab,
-                                                 const int* __restrict__ bcase,
-                                                 const int* __restrict__ btile) {
-  __shared__ double tile[2][32][33];
-  const Case2D& cs = tab[bcase[blockIdx.x]];
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int tx = (ni + 1 + 31) / 32, t = btile[blockIdx.x];
-  const int i0 = (t % tx) * 32, j0 = (t / tx) * 32;
-  const gptr<double> src[2] = {glb(cs.f[F_TXU]), glb(cs.f[F_TXV])};
-  const gptr<double> dst[2] = {glb(cs.f[F_U]), glb(cs.f[F_V])};
-  const int l = threadIdx.x;
-  for (int r = 0; r < 4; ++r) {
-    const int lj = l % 32, li = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) tile[a][lj][li] = src[a][j + (long)(nj + 1) * i];
-    }
-  }
-  __syncthreads();
-  for (int r = 0; r < 4; ++r) {
-    const int li = l % 32, lj = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i >= 1 && i <= ni - 1 && j >= 1 && j <= nj - 1) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) dst[a][i + (long)sj * j] = tile[a][lj][li];
-    }
-  }
-}
-
-// The change form's J-line-major copy of the stage-2 residual (FP32), as k2_tr_in.
-__global__ void __launch_bounds__(256) k2_tr_in32(const Case2D* __restrict__ tab,
-                                                  const int* __restrict__ bcase,
-                                                  const int* __restrict__ btile) {
-  __shared__ float tile[2][32][33];
-  const Case2D& cs = tab[bcase[blockIdx.x]];
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int tx = (ni + 1 + 31) / 32, t = btile[blockIdx.x];
-  const int i0 = (t % tx) * 32, j0 = (t / tx) * 32;
-  const gptr<float> src[2] = {glb(cs.h[H_RU]), glb(cs.h[H_RV])};
-  const gptr<float> dst[2] = {glb(cs.h[H_TRU]), glb(cs.h[H_TRV])};
-  const int l = threadIdx.x;
-  for (int r = 0; r < 4; ++r) {
-    const int li = l % 32, lj = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) tile[a][lj][li] = src[a][i + (long)sj * j];
-    }
-  }
-  __syncthreads();
-  for (int r = 0; r < 4; ++r) {
-    const int lj = l % 32, li = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) dst[a][tidx32(nj, i, j)] = tile[a][lj][li];
-    }
-  }
-}
-
-// The change form's J-line sweep result: the J-line-major change added to the field interior.
-__global__ void __launch_bounds__(256) k2_tr_out32(const Case2D* __restrict__ tab,
-                                                   const int* __restrict__ bcase,
-                                                   const int* __restrict__ btile) {
-  __shared__ float tile[2][32][33];
-  const Case2D& cs = tab[bcase[blockIdx.x]];
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int tx = (ni + 1 + 31) / 32, t = btile[blockIdx.x];
-  const int i0 = (t % tx) * 32, j0 = (t / tx) * 32;
-  const gptr<float> src[2] = {glb(cs.h[H_DU]), glb(cs.h[H_DV])};
-  const gptr<double> dst[2] = {glb(cs.f[F_U]), glb(cs.f[F_V])};
-  const int l = threadIdx.x;
-  for (int r = 0; r < 4; ++r) {
-    const int lj = l % 32, li = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i <= ni && j <= nj) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) tile[a][lj][li] = src[a][tidx32(nj, i, j)];
-    }
-  }
-  __syncthreads();
-  for (int r = 0; r < 4; ++r) {
-    const int li = l % 32, lj = l / 32 + 8 * r;
-    const int i = i0 + li, j = j0 + lj;
-    if (i >= 1 && i <= ni - 1 && j >= 1 && j <= nj - 1) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const long c = i + (long)sj * j;
-        dst[a][c] = dst[a][c] + (double)tile[a][lj][li];
-      }
-    }
-  }
-}
-
-// The first pass's chunk boundary lines (the stage input's last line of every chunk) and BCU's
-// ghosts of the stage input (by each (case, component)'s chunk-0 wavefront; the ghosts and the
-// interior lines copied here do not overlap); block table as the passes'.
-template <int DIR, bool DELTA>
+// The FP64 I stage's first chunk boundary lines (the stage input's last line of every chunk) and
+// BCU's ghosts of the stage input (by each (case, component)'s chunk-0 wavefront; the ghosts and
+// the interior lines copied here do not overlap); block table as the passes'.
 __global__ void __launch_bounds__(64) k2_sweep_seed(const Case2D* __restrict__ tab,
                                                     const int* __restrict__ bcase,
                                                     const int* __restrict__ btile) {
@@ -587,24 +470,28 @@ __global__ void __launch_bounds__(64) k2_sweep_seed(const Case2D* __restrict__ t
   if (ca == 0)
     bcu_ghosts_wave(F, cs.ni, cs.nj, cs.sj, glb(cs.b[comp ? B_VWALL : B_UWALL]),
                     glb(cs.b[comp ? B_VFAR : B_UFAR]));
-  const int n = DIR == 0 ? cs.ni - 1 : cs.nj - 1;
-  const int nl = DIR == 0 ? cs.nj - 1 : cs.ni - 1;
-  const long rs = DIR == 0 ? 1 : cs.sj, ls = DIR == 0 ? cs.sj : 1;
-  const int nch = sw_nchunk(nl);
+  const int n = cs.ni - 1, nl = cs.nj - 1, nch = sw_nchunk(nl);
   const int a1 = min((ca + 1) * SW_C, nl);
   const auto dst = glb(cs.swb) + ((long)comp * nch + ca) * n;  // slot 0
-  // the change form starts from no change
-  for (int r = threadIdx.x; r < n; r += 64) dst[r] = DELTA ? 0.0 : F[ls * a1 + rs * (r + 1)];
-  if (DIR == 0 && comp == 0 && ca == 0 && threadIdx.x == 0) cs.stat[ST_AFCH] = 0.0;
+  for (int r = threadIdx.x; r < n; r += 64) dst[r] = F[(long)cs.sj * a1 + r + 1];
 }
 
 // One pass over the chunks of every case (block table: case, 2 chunk + component; entries with
-// case -1 pad the table to whole XCD rounds).
+// case -1 pad the table to whole XCD rounds).  The change form's I-line stage leaves the field
+// alone in its first pass: 2 ncase workgroups past the table's nblk then set BCU's ghosts of the
+// stage input, which the stage-2 right-hand side reads.
 template <int DIR, bool EARLY, typename T>
 __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ tab,
                                                     const int* __restrict__ bcase,
                                                     const int* __restrict__ btile, int slot,
-                                                    double tol, int final) {
+                                                    double tol, int final, int nblk) {
+  if (std::is_same<T, float>::value && DIR == 0 && !EARLY && (int)blockIdx.x >= nblk) {
+    const int w = (int)blockIdx.x - nblk, comp = w & 1;
+    const Case2D& cg = tab[w >> 1];
+    bcu_ghosts_wave(glb(cg.f[comp ? F_V : F_U]), cg.ni, cg.nj, cg.sj,
+                    glb(cg.b[comp ? B_VWALL : B_UWALL]), glb(cg.b[comp ? B_VFAR : B_UFAR]));
+    return;
+  }
   const int cc = bcase[blockIdx.x];
   if (cc < 0) return;
   const Case2D& cs = tab[cc];
@@ -624,56 +511,95 @@ __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ t
 }
 
 // Stage-2 right-hand side SU = 2 Re DJAC / dt U + DD(U) with the stage-2 cross weights
-// (iter_u.f90:84-98) and BCU's folds with the stage-2 AW(1), AE(NI-1) (bcu.f90:15, 34).  AF32:
-// instead of SU, the FP64 residual of the stage input against the stage-2 line operator, in FP32.
+// (iter_u.f90:84-98) and BCU's folds with the stage-2 AW(1), AE(NI-1) (bcu.f90:15, 34), written
+// J-line-major for the J-line sweep: a workgroup forms a 32 x 32 (I x J) tile of interior cells
+// and transposes it through LDS.  FP64: the stage input goes along, with the BCU ghosts that the
+// sweep reads (line 0, the line ends J = 0, NJ).  AF32: instead of SU, the FP64 residual of the
+// stage input against the stage-2 line operator, in FP32.  As a stencil pass into a natural plane
+// and a transposition of it (and a pass of BCU and boundary lines before) the three launches took
+// 73 + 23 + 15 us a step on the 96-case ensemble (3.4 M cells, AF32).
 template <bool AF32>
-__global__ void __launch_bounds__(512) k2_rhs2(const Case2D* __restrict__ tab,
+__global__ void __launch_bounds__(256) k2_rhs2(const Case2D* __restrict__ tab,
                                                const int* __restrict__ bcase,
                                                const int* __restrict__ btile) {
-  const TileIdx t = tile_index(bcase, btile, tab);
-  if (t.c < 0) return;
-  const Case2D& cs = tab[t.c];
+  using T = typename std::conditional<AF32, float, double>::type;
+  constexpr int NT = AF32 ? 2 : 4;  // right-hand sides u, v; FP64: and the stage input
+  __shared__ T tile[NT][32][33];
+  const int cc = bcase[blockIdx.x];
+  if (cc < 0) return;
+  const Case2D& cs = tab[cc];
   const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int i = t.i, j = t.j;
-  if (i > ni - 1 || j > nj - 1) return;
-  const long c = (long)i + (long)sj * j;
+  const int tx = (ni - 1 + 31) / 32, t = btile[blockIdx.x];
+  const int i0 = 1 + (t % tx) * 32, j0 = 1 + (t / tx) * 32;
+  const int l = threadIdx.x;
   const auto U = glb(cs.f[F_U]);
   const auto V = glb(cs.f[F_V]);
-  // the change form leaves out the 2 Re DJAC / dt U term: it cancels against the diagonal
-  const double ap0 = AF32 ? 0.0 : glb(cs.f[G_AP0])[c];
-  double ru = ap0 * U[c] + cross2(glb(cs.f[G_JXE2]), U, c, sj);
-  double rv = ap0 * V[c] + cross2(glb(cs.f[G_JXE2]), V, c, sj);
-  if (i == 1) {  // (change form: 2 AW(1) (U_F - U))
-    ru = ru + 2.0 * glb(cs.b[B_AW2W])[j] * (AF32 ? glb(cs.b[B_UWALL])[j] - U[c] : glb(cs.b[B_UWALL])[j]);
-    rv = rv + 2.0 * glb(cs.b[B_AW2W])[j] * (AF32 ? glb(cs.b[B_VWALL])[j] - V[c] : glb(cs.b[B_VWALL])[j]);
+#pragma unroll 1
+  for (int r = 0; r < 4; ++r) {
+    const int li = l % 32, lj = l / 32 + 8 * r;
+    const int i = i0 + li, j = j0 + lj;
+    if (i > ni - 1 || j > nj - 1) continue;
+    const long c = (long)i + (long)sj * j;
+    // the change form leaves out the 2 Re DJAC / dt U term: it cancels against the diagonal
+    const double ap0 = AF32 ? 0.0 : glb(cs.f[G_AP0])[c];
+    double ru = ap0 * U[c] + cross2(glb(cs.f[G_JXE2]), U, c, sj);
+    double rv = ap0 * V[c] + cross2(glb(cs.f[G_JXE2]), V, c, sj);
+    if (i == 1) {  // (change form: 2 AW(1) (U_F - U))
+      ru = ru + 2.0 * glb(cs.b[B_AW2W])[j] * (AF32 ? glb(cs.b[B_UWALL])[j] - U[c] : glb(cs.b[B_UWALL])[j]);
+      rv = rv + 2.0 * glb(cs.b[B_AW2W])[j] * (AF32 ? glb(cs.b[B_VWALL])[j] - V[c] : glb(cs.b[B_VWALL])[j]);
+    }
+    if (i == ni - 1) {
+      ru = ru + 2.0 * glb(cs.b[B_AE2F])[j] * (AF32 ? glb(cs.b[B_UFAR])[j] - U[c] : glb(cs.b[B_UFAR])[j]);
+      rv = rv + 2.0 * glb(cs.b[B_AE2F])[j] * (AF32 ? glb(cs.b[B_VFAR])[j] - V[c] : glb(cs.b[B_VFAR])[j]);
+    }
+    const double ae = glb(cs.f[G_AE2])[c];
+    if (AF32) {
+      // the residual r = SU + AW x0(I-1) + AE x0(I+1) + AS x0(J-1) + AN x0(J+1) - AP x0 of the
+      // stage input x0 = U as differences (AP = 2 Re DJAC / dt + AE + AW + AN + AS + the folds
+      // above; folded AW(1) = AE(NI-1) = 0, AW(I) = AE(I-1), AS(J) = AN(J-1) below J = 1); the
+      // line ends' ghosts J = 0, NJ are BCU's periodic images J = NJ-1, 1, as the sweep sees them
+      const double aw = i == 1 ? 0.0 : glb(cs.f[G_AE2])[c - 1];
+      const double an = glb(cs.f[G_GC2])[c];
+      const double as = j == 1 ? glb(cs.f[G_GA2])[c] : glb(cs.f[G_GC2])[c - sj];
+      const long cs0 = j == 1 ? (long)i + (long)sj * (nj - 1) : c - sj;
+      const long cn0 = j == nj - 1 ? (long)i + sj : c + sj;
+      const double eu = ru + ae * (U[c + 1] - U[c]) + aw * (U[c - 1] - U[c]) +
+                        as * (U[cs0] - U[c]) + an * (U[cn0] - U[c]);
+      const double ev = rv + ae * (V[c + 1] - V[c]) + aw * (V[c - 1] - V[c]) +
+                        as * (V[cs0] - V[c]) + an * (V[cn0] - V[c]);
+      tile[0][lj][li] = (T)eu;
+      tile[1][lj][li] = (T)ev;
+    } else {
+      // the old next line's coupling AE U(I+1) (the far-field fold leaves AE(NI-1) = 0)
+      tile[0][lj][li] = (T)(ru + ae * U[c + 1]);
+      tile[1][lj][li] = (T)(rv + ae * V[c + 1]);
+      tile[NT - 2][lj][li] = (T)U[c];
+      tile[NT - 1][lj][li] = (T)V[c];
+    }
   }
-  if (i == ni - 1) {
-    ru = ru + 2.0 * glb(cs.b[B_AE2F])[j] * (AF32 ? glb(cs.b[B_UFAR])[j] - U[c] : glb(cs.b[B_UFAR])[j]);
-    rv = rv + 2.0 * glb(cs.b[B_AE2F])[j] * (AF32 ? glb(cs.b[B_VFAR])[j] - V[c] : glb(cs.b[B_VFAR])[j]);
-  }
-  const double ae = glb(cs.f[G_AE2])[c];
-  if (AF32) {
-    // the residual r = SU + AW x0(I-1) + AE x0(I+1) + AS x0(J-1) + AN x0(J+1) - AP x0 of the
-    // stage input x0 = U as differences (AP = 2 Re DJAC / dt + AE + AW + AN + AS + the folds
-    // above; folded AW(1) = AE(NI-1) = 0, AW(I) = AE(I-1), AS(J) = AN(J-1) below J = 1); the
-    // line ends' ghosts J = 0, NJ are BCU's periodic images J = NJ-1, 1, as the sweep sees them
-    const double aw = i == 1 ? 0.0 : glb(cs.f[G_AE2])[c - 1];
-    const double an = glb(cs.f[G_GC2])[c];
-    const double as = j == 1 ? glb(cs.f[G_GA2])[c] : glb(cs.f[G_GC2])[c - sj];
-    const long cs0 = j == 1 ? (long)i + (long)sj * (nj - 1) : c - sj;
-    const long cn0 = j == nj - 1 ? (long)i + sj : c + sj;
-    const double eu = ru + ae * (U[c + 1] - U[c]) + aw * (U[c - 1] - U[c]) +
-                      as * (U[cs0] - U[c]) + an * (U[cn0] - U[c]);
-    const double ev = rv + ae * (V[c + 1] - V[c]) + aw * (V[c - 1] - V[c]) +
-                      as * (V[cs0] - V[c]) + an * (V[cn0] - V[c]);
-    glb(cs.h[H_RU])[c] = (float)eu;
-    glb(cs.h[H_RV])[c] = (float)ev;
-  } else {
-    // the old next line's coupling AE U(I+1) (the far-field fold leaves AE(NI-1) = 0)
-    ru = ru + ae * U[c + 1];
-    rv = rv + ae * V[c + 1];
-    glb(cs.f[F_SU1])[c] = ru;
-    glb(cs.f[F_SV1])[c] = rv;
+  __syncthreads();
+  T* const* f0;
+  if constexpr (AF32) f0 = cs.h;
+  else f0 = cs.f;
+  const gptr<T> dst[2] = {glb(f0[AF32 ? (int)H_TRU : (int)F_TQU]),
+                          glb(f0[AF32 ? (int)H_TRV : (int)F_TQV])};
+  for (int r = 0; r < 4; ++r) {
+    const int lj = l % 32, li = l / 32 + 8 * r;
+    const int i = i0 + li, j = j0 + lj;
+    if (i > ni - 1 || j > nj - 1) continue;
+    const long o = AF32 ? tidx32(nj, i, j) : j + (long)(nj + 1) * i;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      dst[a][o] = tile[a][lj][li];
+      if (!AF32) {  // the stage input and its BCU ghosts
+        const auto X = glb(cs.f[a ? F_TXV : F_TXU]);
+        const double x = tile[NT - 2 + a][lj][li];
+        X[o] = x;
+        if (i == 1) X[j] = -x + 2.0 * glb(cs.b[a ? B_VWALL : B_UWALL])[j];
+        if (j == nj - 1) X[o - (nj - 1)] = x;  // J = 0
+        if (j == 1) X[o + (nj - 1)] = x;       // J = NJ
+      }
+    }
   }
 }
 
@@ -700,27 +626,71 @@ __device__ inline void own_ghosts(P F, const Case2D& cs, int i, int j, long c, d
   }
 }
 
-// Predictor correction U = U - S_U DTIME / DJAC (Main.f90:80-84) and the BCU ghosts
-// (Main.f90:86-87).
-__global__ void __launch_bounds__(512) k2_correct(const Case2D* __restrict__ tab,
+// The J-line sweep's result transposed back (32 x 32 tiles through LDS; AF32: the J-line-major
+// change added to the field), the predictor correction U = U - S_U DTIME / DJAC (Main.f90:80-84)
+// and the BCU ghosts (Main.f90:86-87) in one pass: as two, 42 + 42 us a step on the 96-case
+// ensemble (AF32), U and V written and read once more.
+template <bool AF32>
+__global__ void __launch_bounds__(256) k2_correct(const Case2D* __restrict__ tab,
                                                   const int* __restrict__ bcase,
                                                   const int* __restrict__ btile) {
-  const TileIdx t = tile_index(bcase, btile, tab);
-  if (t.c < 0) return;
-  const Case2D& cs = tab[t.c];
+  using T = typename std::conditional<AF32, float, double>::type;
+  __shared__ T tile[2][32][33];
+  const int cc = bcase[blockIdx.x];
+  if (cc < 0) return;
+  const Case2D& cs = tab[cc];
   const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int i = t.i, j = t.j;
-  if (i > ni - 1 || j > nj - 1) return;
-  const long c = (long)i + (long)sj * j;
-  const double dj = glb(cs.f[G_DJAC])[c];
+  const int tx = (ni - 1 + 31) / 32, t = btile[blockIdx.x];
+  const int i0 = 1 + (t % tx) * 32, j0 = 1 + (t / tx) * 32;
+  const int l = threadIdx.x;
+  T* const* f0;
+  if constexpr (AF32) f0 = cs.h;
+  else f0 = cs.f;
+  const gptr<T> src[2] = {glb(f0[AF32 ? (int)H_DU : (int)F_TXU]),
+                          glb(f0[AF32 ? (int)H_DV : (int)F_TXV])};
   const auto U = glb(cs.f[F_U]);
   const auto V = glb(cs.f[F_V]);
-  const double u = U[c] - glb(cs.f[F_SU])[c] * cs.dt / dj;
-  const double v = V[c] - glb(cs.f[F_SV])[c] * cs.dt / dj;
-  U[c] = u;
-  V[c] = v;
-  own_ghosts(U, cs, i, j, c, u, glb(cs.b[B_UWALL]), glb(cs.b[B_UFAR]));
-  own_ghosts(V, cs, i, j, c, v, glb(cs.b[B_VWALL]), glb(cs.b[B_VFAR]));
+  const auto S = glb(cs.f[F_SU]);
+  const auto W = glb(cs.f[F_SV]);
+  const auto DJ = glb(cs.f[G_DJAC]);
+  // the natural operands of the thread's four cells, in flight while the tile is transposed
+  double u0[4], v0[4], su[4], sv[4], dj[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = min(i0 + l % 32, ni - 1), j = min(j0 + l / 32 + 8 * r, nj - 1);
+    const long c = (long)i + (long)sj * j;
+    u0[r] = AF32 ? U[c] : 0.0;
+    v0[r] = AF32 ? V[c] : 0.0;
+    su[r] = S[c];
+    sv[r] = W[c];
+    dj[r] = DJ[c];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int lj = l % 32, li = l / 32 + 8 * r;
+    const int i = i0 + li, j = j0 + lj;
+    if (i <= ni - 1 && j <= nj - 1) {
+      const long o = AF32 ? tidx32(nj, i, j) : j + (long)(nj + 1) * i;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) tile[a][lj][li] = src[a][o];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int li = l % 32, lj = l / 32 + 8 * r;
+    const int i = i0 + li, j = j0 + lj;
+    if (i > ni - 1 || j > nj - 1) continue;
+    const long c = (long)i + (long)sj * j;
+    const double us = AF32 ? u0[r] + (double)tile[0][lj][li] : (double)tile[0][lj][li];
+    const double vs = AF32 ? v0[r] + (double)tile[1][lj][li] : (double)tile[1][lj][li];
+    const double u = us - su[r] * cs.dt / dj[r];
+    const double v = vs - sv[r] * cs.dt / dj[r];
+    U[c] = u;
+    V[c] = v;
+    own_ghosts(U, cs, i, j, c, u, glb(cs.b[B_UWALL]), glb(cs.b[B_UFAR]));
+    own_ghosts(V, cs, i, j, c, v, glb(cs.b[B_VWALL]), glb(cs.b[B_VFAR]));
+  }
 }
 
 // CONTRA_VEL of the corrected velocity and the source of ITER_P (iter_p.f90:29-32):
