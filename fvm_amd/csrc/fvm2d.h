@@ -87,7 +87,7 @@ struct Case2D {
   void* S;             // half spectrum (n1 mj complex)
   void* R32;
   void* S32;
-  double* part;        // per-block partial sums of this case (residual pairs, CFL maxima)
+  double* part;        // per-tile partials of this case: ntile residual pairs, ntile CFL maxima
   double* stat;        // per-case scalars (see ST_*)
   int ntile;           // stencil tiles of this case (partials per pass)
   double* swb;         // AF sweep chunk boundary lines [pass slot][component][chunk][row]

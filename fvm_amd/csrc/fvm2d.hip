@@ -44,7 +44,7 @@ __device__ __forceinline__ void cx_st(gptr<T> p, long o, Cx<T> v) {
 template <bool AF32>
 __global__ void __launch_bounds__(512) k2_explicit(const Case2D* __restrict__ tab,
                                                    const int* __restrict__ bcase,
-                                                   const int* __restrict__ btile) {
+                                                   const int* __restrict__ btile, long* ctr) {
   const TileIdx t = tile_index(bcase, btile, tab);
   if (t.c < 0) return;
   const Case2D& cs = tab[t.c];
@@ -57,7 +57,13 @@ __global__ void __launch_bounds__(512) k2_explicit(const Case2D* __restrict__ ta
   const auto P = glb(cs.f[F_P]);
   const auto UN = glb(cs.f[F_UN]);
   const auto VN = glb(cs.f[F_VN]);
-  if (i == 1 && j == 1) glb(cs.stat)[ST_AFCH] = 0.0;  // booked by the sweeps' last passes
+  if (i == 1 && j == 1) {  // the case's flags of the step, and the batch's step counter
+    const auto st = glb(cs.stat);
+    st[ST_AFCH] = 0.0;  // booked by the sweeps' last passes
+    st[ST_DONE] = 0.0;
+    st[ST_NAN] = 0.0;
+    if (t.c == 0) *ctr = *ctr + 1;
+  }
   // U_N = U over the whole plane: every interior thread copies its cell and the ghosts next to
   // it (corners from the corner cells)
   {
@@ -693,53 +699,14 @@ __global__ void __launch_bounds__(256) k2_correct(const Case2D* __restrict__ tab
   }
 }
 
-// CONTRA_VEL of the corrected velocity and the source of ITER_P (iter_p.f90:29-32):
-// RHS = 1 / DTIME (UE - UW + VN - VS)
-__global__ void __launch_bounds__(512) k2_prhs(const Case2D* __restrict__ tab,
-                                               const int* __restrict__ bcase,
-                                               const int* __restrict__ btile) {
-  const TileIdx t = tile_index(bcase, btile, tab);
-  if (t.c < 0) return;
-  const Case2D& cs = tab[t.c];
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const int i = t.i, j = t.j;
-  if (i > ni - 1 || j > nj - 1) return;
-  const long c = (long)i + (long)sj * j;
-  const auto U = glb(cs.f[F_U]);
-  const auto V = glb(cs.f[F_V]);
-  const GeomG g = geom2(cs);
-  const double j1 = ju1(g, U, V, c), j2 = ju2(g, U, V, c);
-  const double ue = 0.5 * (j1 + ju1(g, U, V, c + 1));
-  const double uw = i == 1 ? 0.0 : 0.5 * (j1 + ju1(g, U, V, c - 1));
-  const double vn = 0.5 * (j2 + ju2(g, U, V, c + sj));
-  const double vs = 0.5 * (j2 + ju2(g, U, V, c - sj));
-  glb(cs.f[F_RHS])[c] = 1.0 / cs.dt * (ue - uw + vn - vs);
-}
-
-// BCP (bcp.f90:12-43) of p: wall Neumann p(0) = p(1), outflow cubic extrapolation
-// p(NI) = 3 p(NI-1) - 3 p(NI-2) + p(NI-3), branch cut.  One workgroup per case; skipped for a
-// converged case unless force.
-__global__ void __launch_bounds__(256) k2_bcp(const Case2D* __restrict__ tab, int force) {
-  const Case2D& cs = tab[blockIdx.x];
-  if (!force && C2_DONE(cs)) return;
-  const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  const auto P = glb(cs.f[F_P]);
-  for (int j = 1 + threadIdx.x; j <= nj - 1; j += blockDim.x) {
-    const long c = (long)sj * j;
-    P[c] = P[c + 1];
-    P[c + ni] = 3.0 * P[c + ni - 1] - 3.0 * P[c + ni - 2] + P[c + ni - 3];
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i <= ni; i += blockDim.x) {
-    P[i] = P[i + (long)sj * (nj - 1)];
-    P[i + (long)sj * nj] = P[i + sj];
-  }
-}
-
 // Residual of ITER_P's operator (iter_p.f90:12-51 with BCP's folds AP(1) -= AW(1), AW(1) = 0,
 // AE(NI-1) = 0): r = AE p_E + AW p_W + AN p_N + AS p_S + SU - AP p, SU = RHS - DD(p), into the
-// compact array R [(i-1) + (NI-1)(j-1)], with the block's sums of |r| and |AP p|.
-template <typename T>
+// compact array R [(i-1) + (NI-1)(j-1)], with the block's sums of |r| and |AP p|.  BCP's ghosts of
+// p (bcp.f90:12-43) are formed where they are read (prow).  FIRST: the step's first residual also
+// forms its source from CONTRA_VEL of the corrected velocity, RHS = 1 / DTIME (UE - UW + VN - VS)
+// (iter_p.f90:29-32), and keeps it for the later ones.  Source, BCP and residual as three
+// launches took 65 + 6 + 35 us on the 96-case ensemble.
+template <typename T, bool FIRST>
 __global__ void __launch_bounds__(512) k2_residual(const Case2D* __restrict__ tab,
                                                    const int* __restrict__ bcase,
                                                    const int* __restrict__ btile) {
@@ -747,26 +714,49 @@ __global__ void __launch_bounds__(512) k2_residual(const Case2D* __restrict__ ta
   const TileIdx t = tile_index(bcase, btile, tab);
   if (t.c < 0) return;
   const Case2D& cs = tab[t.c];
-  if (C2_DONE(cs)) return;  // uniform over the workgroup
+  if (!FIRST && C2_DONE(cs)) return;  // uniform over the workgroup
   const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
   const int i = t.i, j = t.j;
   double ra = 0.0, rb = 0.0;
   if (i <= ni - 1 && j <= nj - 1) {
     const long c = (long)i + (long)sj * j;
     const auto P = glb(cs.f[F_P]);
+    const PRow p0 = prow(P, (long)sj * j, i, ni);
+    const PRow pn = prow(P, (long)sj * (j == nj - 1 ? 1 : j + 1), i, ni);
+    const PRow ps = prow(P, (long)sj * (j == 1 ? nj - 1 : j - 1), i, ni);
+    double rhs;
+    if (FIRST) {
+      const auto U = glb(cs.f[F_U]);
+      const auto V = glb(cs.f[F_V]);
+      const GeomG g = geom2(cs);
+      const double j1 = ju1(g, U, V, c), j2 = ju2(g, U, V, c);
+      const double ue = 0.5 * (j1 + ju1(g, U, V, c + 1));
+      const double uw = i == 1 ? 0.0 : 0.5 * (j1 + ju1(g, U, V, c - 1));
+      const double vn = 0.5 * (j2 + ju2(g, U, V, c + sj));
+      const double vs = 0.5 * (j2 + ju2(g, U, V, c - sj));
+      rhs = 1.0 / cs.dt * (ue - uw + vn - vs);
+    } else {
+      rhs = glb(cs.f[F_RHS])[c];
+    }
     const auto de = glb(cs.f[G_DE]);
     const auto dn = glb(cs.f[G_DN]);
+    const auto jq = glb(cs.f[G_JQ12]);
     const double dE = de[c], dW = de[c - 1], dN = dn[c], dS = dn[c - sj];
     double ap = -dE - dW - dN - dS;
     double ae = -dE, aw = -dW;
     const double an = -dN, as = -dS;
     if (i == 1) { ap = ap - aw; aw = 0.0; }
     if (i == ni - 1) ae = 0.0;
-    const double su = glb(cs.f[F_RHS])[c] - cross2(glb(cs.f[G_JQ12]), P, c, sj);
-    const double r = ae * P[c + 1] + aw * P[c - 1] + an * P[c + sj] + as * P[c - sj] + su -
-                     ap * P[c];
+    // cross2 of p (DIF_DIAGONAL)
+    double x = jq[c + 1] * (pn.e - ps.e);
+    x = x - jq[c - 1] * (pn.w - ps.w);
+    x = x + jq[c + sj] * (pn.e - pn.w);
+    x = x - jq[c - sj] * (ps.e - ps.w);
+    const double su = rhs - 0.25 * x;
+    const double r = ae * p0.e + aw * p0.w + an * pn.c + as * ps.c + su - ap * p0.c;
     ra = fabs(r);
-    rb = fabs(ap * P[c]);
+    rb = fabs(ap * p0.c);
+    if (FIRST) glb(cs.f[F_RHS])[c] = rhs;
     glb((T*)(sizeof(T) == 8 ? cs.R : cs.R32))[(i - 1) + (long)(ni - 1) * (j - 1)] = (T)r;
   }
   ra = wg_sum(ra, sh);
@@ -777,31 +767,32 @@ __global__ void __launch_bounds__(512) k2_residual(const Case2D* __restrict__ ta
   }
 }
 
-// Per case: RESIP = sum|r| / sum|AP p| from the tile sums (fixed order); pass q >= 1 ends the
-// case's correction when RESIP <= RESIMAX (the reference tests after a sweep,
-// iter_p.f90:36-51) or when q is the last pass; q = 0 only records the starting residual.
-__global__ void __launch_bounds__(256) k2_res_final(const Case2D* __restrict__ tab, int q,
-                                                    int last) {
-  __shared__ double sh[256];
-  const Case2D& cs = tab[blockIdx.x];
-  if (C2_DONE(cs)) return;
+// RESIP = sum|r| / sum|AP p| of a case from the tile sums of its residual after pass q (a fixed
+// order), by one workgroup of 256: the correction ends when RESIP <= RESIMAX after a pass (the
+// reference tests after a sweep, iter_p.f90:36-51), when q is the last pass or when RESIP is not a
+// number; q = 0 only records the starting residual.  Every workgroup that asks computes the same;
+// the one with record set books it in the case's scalars.
+__device__ inline bool res_done(const Case2D& cs, int q, int last, bool record, double* sh) {
   double a = 0.0, b = 0.0;
-  for (int k = threadIdx.x; k < cs.ntile; k += blockDim.x) {
+  for (int k = threadIdx.x; k < cs.ntile; k += 256) {
     a = a + cs.part[2 * k];
     b = b + cs.part[2 * k + 1];
   }
   a = wg_sum(a, sh);
   b = wg_sum(b, sh);
-  if (threadIdx.x != 0) return;
   const double res = scaled_residual(a, b);
-  double* st = cs.stat;
-  st[ST_S0] = a;
-  st[ST_S1] = b;
-  st[ST_RESIP] = res;
-  st[ST_NPASS] = (double)q;
-  if (q == 0) st[ST_RES0] = res;
-  if (!(res == res)) st[ST_NAN] = 1.0;
-  if (q >= 1 && (res <= cs.resimax || q >= last || !(res == res))) st[ST_DONE] = 1.0;
+  const bool done = q >= 1 && (res <= cs.resimax || q >= last || !(res == res));
+  if (record && threadIdx.x == 0) {
+    double* st = cs.stat;
+    st[ST_S0] = a;
+    st[ST_S1] = b;
+    st[ST_RESIP] = res;
+    st[ST_NPASS] = (double)q;
+    if (q == 0) st[ST_RES0] = res;
+    if (!(res == res)) st[ST_NAN] = 1.0;
+    if (done) st[ST_DONE] = 1.0;
+  }
+  return done;
 }
 
 __global__ void k2_begin_p(const Case2D* __restrict__ tab) {
@@ -814,14 +805,22 @@ __global__ void k2_begin_p(const Case2D* __restrict__ tab) {
 
 // Forward real J transform of the residual (two radial rows per complex sequence) into the
 // half spectrum S[i + n1 m], one workgroup per (case, tile of 2 ncol rows); see
-// fvm_poisson_spec.hip for the 3D form.
+// fvm_poisson_spec.hip for the 3D form.  q >= 0: the pass after the residual of pass q, which every
+// workgroup of the case first tests (res_done, LDS of at least 256 doubles; the one of tile 0
+// books the result, and a workgroup that sees the booked flag already stops as it would by its
+// own test); q < 0: no test.
 template <typename T>
 __global__ void __launch_bounds__(256) k2_fft_fwd(const Case2D* __restrict__ tab,
                                                   const int* __restrict__ bcase,
-                                                  const int* __restrict__ btile, int ncol) {
+                                                  const int* __restrict__ btile, int ncol, int q,
+                                                  int last) {
   extern __shared__ __align__(16) unsigned char smem[];
   const Case2D& cs = tab[bcase[blockIdx.x]];
-  if (C2_DONE(cs)) return;
+  __shared__ int skip;
+  if (threadIdx.x == 0) skip = C2_DONE(cs);
+  __syncthreads();
+  if (skip) return;
+  if (q >= 0 && res_done(cs, q, last, btile[blockIdx.x] == 0, (double*)smem)) return;
   const int N = cs.pj.n, MJ = cs.mj, n1 = cs.ni - 1;
   const auto R = glb((const T*)(sizeof(T) == 8 ? cs.R : cs.R32));
   const auto S = glb((T*)(sizeof(T) == 8 ? cs.S : cs.S32));          // complex, interleaved
@@ -855,15 +854,11 @@ __global__ void __launch_bounds__(256) k2_fft_fwd(const Case2D* __restrict__ tab
   }
 }
 
-// Radial mode lines of the half spectrum, one wavefront per (case, mode) from the block table.
+// Radial mode line of the half spectrum by one wavefront, R rows per lane.
 template <typename T, int R>
-__global__ void __launch_bounds__(64) k2_modes(const Case2D* __restrict__ tab,
-                                               const int* __restrict__ bcase,
-                                               const int* __restrict__ btile) {
-  const Case2D& cs = tab[bcase[blockIdx.x]];
-  if (C2_DONE(cs)) return;
+__device__ inline void mode_line(const Case2D& cs, int mode) {
   const int n = cs.ni - 1;
-  const long base = (long)n * btile[blockIdx.x];
+  const long base = (long)n * mode;
   const auto Z = glb((T*)(sizeof(T) == 8 ? cs.S : cs.S32));  // complex, interleaved
   const auto dW = glb((const double*)cs.pdw);
   const auto invd = glb((const double*)cs.invd);
@@ -932,6 +927,28 @@ __global__ void __launch_bounds__(64) k2_modes(const Case2D* __restrict__ tab,
   }
 }
 
+// The mode lines of every case, one wavefront per (case, mode) from the block table, each with its
+// case's own rows per lane: RMAX = 4 lines of at most 256 rows, RMAX = 8 the longer ones (whose
+// registers would halve the wavefronts in flight of the rest).
+template <typename T, int RMAX>
+__global__ void __launch_bounds__(64) k2_modes(const Case2D* __restrict__ tab,
+                                               const int* __restrict__ bcase,
+                                               const int* __restrict__ btile) {
+  const Case2D& cs = tab[bcase[blockIdx.x]];
+  if (C2_DONE(cs)) return;
+  const int mode = btile[blockIdx.x];
+  if constexpr (RMAX == 8) {
+    mode_line<T, 8>(cs, mode);
+  } else {
+    switch ((cs.ni - 1 + 63) >> 6) {
+      case 1: mode_line<T, 1>(cs, mode); break;
+      case 2: mode_line<T, 2>(cs, mode); break;
+      case 3: mode_line<T, 3>(cs, mode); break;
+      default: mode_line<T, 4>(cs, mode); break;
+    }
+  }
+}
+
 // Inverse J transform of the corrected spectrum, added to p (scale 1 / (NJ-1)).
 template <typename T>
 __global__ void __launch_bounds__(256) k2_fft_inv_add(const Case2D* __restrict__ tab,
@@ -978,7 +995,8 @@ __global__ void __launch_bounds__(256) k2_fft_inv_add(const Case2D* __restrict__
 }
 
 // P_SOURCE(p^{n+1}), the projection U = U + S_U DTIME / DJAC (Main.f90:93-103), BCU's ghosts
-// and the block maxima of the local CFL number (calccoef.f90:9-17)
+// and the block maxima of the local CFL number (calccoef.f90:9-17).  BCP's ghosts of p
+// (bcp.f90:12-43) are formed where they are read (prow) and written by the cell next to them.
 __global__ void __launch_bounds__(512) k2_project(const Case2D* __restrict__ tab,
                                                   const int* __restrict__ bcase,
                                                   const int* __restrict__ btile) {
@@ -993,8 +1011,11 @@ __global__ void __launch_bounds__(512) k2_project(const Case2D* __restrict__ tab
     const long c = (long)i + (long)sj * j;
     const GeomG g = geom2(cs);
     const auto P = glb(cs.f[F_P]);
-    const double su = psrc(g.dj, g.xix, g.etx, P, c, sj);
-    const double sv = psrc(g.dj, g.xiy, g.ety, P, c, sj);
+    const PRow p = prow(P, (long)sj * j, i, ni);
+    const double pn = P[i + (long)sj * (j == nj - 1 ? 1 : j + 1)];
+    const double ps = P[i + (long)sj * (j == 1 ? nj - 1 : j - 1)];
+    const double su = psrc_v(g.dj, g.xix, g.etx, p.e, p.w, pn, ps, c, sj);
+    const double sv = psrc_v(g.dj, g.xiy, g.ety, p.e, p.w, pn, ps, c, sj);
     const auto U = glb(cs.f[F_U]);
     const auto V = glb(cs.f[F_V]);
     const double dj = g.dj[c];
@@ -1006,26 +1027,40 @@ __global__ void __launch_bounds__(512) k2_project(const Case2D* __restrict__ tab
     glb(cs.f[F_SV])[c] = sv;
     own_ghosts(U, cs, i, j, c, u, glb(cs.b[B_UWALL]), glb(cs.b[B_UFAR]));
     own_ghosts(V, cs, i, j, c, v, glb(cs.b[B_VWALL]), glb(cs.b[B_VFAR]));
+    if (i == 1) P[c - 1] = p.w;
+    if (i == ni - 1) P[c + 1] = p.e;
+    if (j == 1 || j == nj - 1) {  // J = NJ <- 1, J = 0 <- NJ-1
+      const long q = c + (j == 1 ? (long)sj * (nj - 1) : -(long)sj * (nj - 1));
+      P[q] = p.c;
+      if (i == 1) P[q - 1] = p.w;
+      if (i == ni - 1) P[q + 1] = p.e;
+    }
     cfl = cs.dt * (fabs(g.xix[c] * u + g.xiy[c] * v) + fabs(g.etx[c] * u + g.ety[c] * v));
   }
   cfl = wg_max(cfl, sh);
-  if (threadIdx.x == 0 && threadIdx.y == 0) cs.part[2 * t.tile] = cfl;
+  // behind the residual's tile sums, which CALCCOEF may still test
+  if (threadIdx.x == 0 && threadIdx.y == 0) cs.part[2 * cs.ntile + t.tile] = cfl;
 }
 
 // CALCCOEF (calccoef.f90:9-119): CFL maximum, C_pb from the corner average PG(1,1) (the far-field
 // PG(NI,NJ/2) is not assigned by CALCCOEF: zero), and the pressure and friction drag and lift
 // summed over the wall cells in J order, each sum carried by one lane; one workgroup per case.
-// The step's scalars go to stat and to the history ring at slot *ctr.
+// A case that has not ended its pressure correction earlier books the residual of the last pass.
+// The step's scalars go to stat and to the history ring at slot *ctr - 1 (the counter moves at the
+// step's start).
 __global__ void __launch_bounds__(256) k2_calccoef(const Case2D* __restrict__ tab, int ncase,
                                                    const long* __restrict__ ctr, int hcap,
-                                                   double* __restrict__ hist) {
+                                                   double* __restrict__ hist, int npass) {
   __shared__ double sh[256];
   __shared__ double tm[4][256];
   const Case2D& cs = tab[blockIdx.x];
   const int nj = cs.nj, sj = cs.sj;
   const int t = threadIdx.x;
+  const bool open = !C2_DONE(cs);
+  __syncthreads();  // the flag is read before lane 0 may set it
+  if (open) (void)res_done(cs, npass, npass, true, sh);
   double cm = 0.0;
-  for (int k = t; k < cs.ntile; k += blockDim.x) cm = fmax(cm, cs.part[2 * k]);
+  for (int k = t; k < cs.ntile; k += blockDim.x) cm = fmax(cm, cs.part[2 * cs.ntile + k]);
   cm = wg_max(cm, sh);
   const double* P = cs.f[F_P];
   const double* U = cs.f[F_U];
@@ -1041,16 +1076,21 @@ __global__ void __launch_bounds__(256) k2_calccoef(const Case2D* __restrict__ ta
       const double dudn = (U[c] * s2 - V[c] * c2 - 0.0) / dn1;  // VEL_ROT = 0
       tm[0][t] = 2.0 * P[c] * area * ct;
       tm[1][t] = 2.0 * P[c] * area * st;
-      tm[2][t] = (2.0 / cs.re) * dudn * area * st;
+      tm[2][t] = -((2.0 / cs.re) * dudn * area * st);  // added: the others are subtracted
       tm[3][t] = (2.0 / cs.re) * dudn * area * ct;
     }
     __syncthreads();
-    if (t < 4) {
+    if (t < 4) {  // 16 LDS reads in flight ahead of the serial chain of subtractions
       const int m = min(256, nj - j0);
-      if (t == 2)
-        for (int q = 0; q < m; ++q) acc = acc + tm[2][q];
-      else
-        for (int q = 0; q < m; ++q) acc = acc - tm[t][q];
+      int q = 0;
+      for (; q + 16 <= m; q += 16) {
+        double x[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] = tm[t][q + e];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc = acc - x[e];
+      }
+      for (; q < m; ++q) acc = acc - tm[t][q];
     }
     __syncthreads();
   }
@@ -1069,7 +1109,7 @@ __global__ void __launch_bounds__(256) k2_calccoef(const Case2D* __restrict__ ta
   st[ST_CDV] = td;
   st[ST_CLP] = pl;
   st[ST_CLV] = tl;
-  double* h = hist + ((long)(*ctr % hcap) * ncase + blockIdx.x) * 8;
+  double* h = hist + ((long)((*ctr - 1) % hcap) * ncase + blockIdx.x) * 8;
   h[0] = st[ST_CD];
   h[1] = st[ST_CL];
   h[2] = st[ST_CDP];
@@ -1078,10 +1118,6 @@ __global__ void __launch_bounds__(256) k2_calccoef(const Case2D* __restrict__ ta
   h[5] = st[ST_CLV];
   h[6] = st[ST_RESIP];
   h[7] = st[ST_CFL];
-}
-
-__global__ void k2_tick(long* ctr) {
-  if (threadIdx.x == 0) *ctr = *ctr + 1;
 }
 
 }  // namespace

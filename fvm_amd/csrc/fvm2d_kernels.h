@@ -123,3 +123,29 @@ __device__ inline double psrc(W __restrict__ dj, W __restrict__ mxi, W __restric
   t = t - dj[c - sj] * met[c - sj] * P[c - sj];
   return -0.5 * t;
 }
+
+// p on the row of the plane that starts at P[o] around I = i: west, centre and east values, with
+// BCP's ghosts formed in place: p(0) = p(1), p(NI) = 3 p(NI-1) - 3 p(NI-2) + p(NI-3)
+// (bcp.f90:12-30).  The branch-cut rows J = 0, NJ are rows NJ-1, 1 (bcp.f90:32-43).
+struct PRow {
+  double w, c, e;
+};
+template <class Q>
+__device__ inline PRow prow(Q P, long o, int i, int ni) {
+  PRow r;
+  r.c = P[o + i];
+  r.w = P[o + (i == 1 ? i : i - 1)];
+  const double x = P[o + (i == ni - 1 ? i - 2 : i + 1)];
+  r.e = i == ni - 1 ? 3.0 * r.c - 3.0 * r.w + x : x;
+  return r;
+}
+// psrc with the four neighbour values of p given
+template <class W>
+__device__ inline double psrc_v(W dj, W mxi, W met, double pe, double pw, double pn, double ps,
+                                long c, int sj) {
+  double t = dj[c + 1] * mxi[c + 1] * pe;
+  t = t - dj[c - 1] * mxi[c - 1] * pw;
+  t = t + dj[c + sj] * met[c + sj] * pn;
+  t = t - dj[c - sj] * met[c - sj] * ps;
+  return -0.5 * t;
+}
