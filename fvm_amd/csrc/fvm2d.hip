@@ -18,6 +18,7 @@
 #include "../../include/fvm_capi.h"
 #include "fvm2d_host.h"
 #include "fvm2d_kernels.h"
+#include "fvm_hostio.h"
 #include "fvm_wave.h"
 
 namespace {

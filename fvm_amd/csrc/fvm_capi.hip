@@ -293,6 +293,7 @@ static int create_impl(const fvm_params* prm, const double* xg, const double* yg
   c->d.sk = (long)(prm->ni + 1) * (prm->nj + 1);
   c->d.n = c->d.sk * (prm->nk + 1);
   c->pi = 4.0 * atan(1.0);
+  c->io.field = c->d.n * sizeof(double);
   int dev_count = 0;
   if (hipGetDeviceCount(&dev_count) != hipSuccess || dev_count < 1) {
     fprintf(stderr, "fvm_amd: no HIP device\n");
@@ -400,6 +401,7 @@ int fvm_destroy(fvm_ctx* c) {
   if (!c) return FVM_ERR_ARG;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   fvm_sep_destroy(c);
+  c->io.release();
   for (auto& e : c->ev_pending) {
     (void)hipEventDestroy(e.second.first);
     (void)hipEventDestroy(e.second.second);
@@ -448,14 +450,13 @@ int fvm_set_field(fvm_ctx* c, int field, const double* host) {
       for (long q = 0; q < c->d.sk; ++q) slab[k * c->d.sk + q] = host[q] * sc;
     host = slab.data();
   }
-  HIP_CHECK(hipMemcpyAsync(dptr, host, c->d.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  if (field >= FVM_NLX && field <= FVM_NLZ)
-    HIP_CHECK(hipMemcpyAsync(c->nl1[field - FVM_NLX], host, c->d.n * sizeof(double),
-                             hipMemcpyHostToDevice, c->stream));
-  if (field == FVM_ADV)
-    HIP_CHECK(hipMemcpyAsync(c->adv1, host, c->d.n * sizeof(double), hipMemcpyHostToDevice,
+  HIP_CHECK(c->io.up(dptr, host, c->d.n * sizeof(double), c->stream));
+  // the convective history starts from the same values
+  double* hist = field >= FVM_NLX && field <= FVM_NLZ ? c->nl1[field - FVM_NLX]
+                                                       : (field == FVM_ADV ? c->adv1 : nullptr);
+  if (hist)
+    HIP_CHECK(hipMemcpyAsync(hist, dptr, c->d.n * sizeof(double), hipMemcpyDeviceToDevice,
                              c->stream));
-  HIP_CHECK(hipStreamSynchronize(c->stream));
   return FVM_OK;
 }
 
@@ -473,8 +474,7 @@ int fvm_get_field(fvm_ctx* c, int field, double* host) {
   }
   if (c->two_d) dptr += c->d.sk;  // the slab's interior plane K = 1
   const long cnt = c->two_d ? c->d.sk : c->d.n;
-  HIP_CHECK(hipMemcpyAsync(host, dptr, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_CHECK(hipStreamSynchronize(c->stream));
+  HIP_CHECK(c->io.down(host, dptr, cnt * sizeof(double), c->stream));
   if (c->two_d && span_scaled(field))
     for (long q = 0; q < cnt; ++q) host[q] /= LZ2D;
   return FVM_OK;

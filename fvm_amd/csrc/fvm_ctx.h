@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "fvm_common.h"
+#include "fvm_hostio.h"
 #include "../../include/fvm_capi.h"
 
 struct ProfAcc {
@@ -144,6 +145,7 @@ struct FvmCtx {
   std::vector<std::pair<std::string, std::pair<hipEvent_t, hipEvent_t>>> ev_pending;
   size_t ev_next = 0;
   std::vector<void*> allocs;
+  HostIo io;                 // pinned slots of fvm_set_field / fvm_get_field
 };
 
 // K planes per workgroup of a K-marching stencil kernel, and its launch grid (64 x 4 (I x J) tiles
