@@ -139,12 +139,13 @@ constexpr int RK_RES = 768;  // workgroups resident at a time (three per CU)
 // folds and couplings; the branch-cut ghosts enter as the periodic images of the interior, the
 // values BCU gives them before the sweep.  The line sweep then solves for the stage's change
 // delta = x - x_in in FP32 and adds it to the FP64 field.
-template <int S, bool TH, int NCV = 3, bool DR = false>
+template <int S, bool TH, int NCV = 3, bool DR = false, int G = kGeoAny>
 __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
                                                    const double* const* __restrict__ P,
                                                    const double* __restrict__ ap0, double re,
                                                    const double* const* __restrict__ fa,
-                                                   int qform, int fn_alias) {
+                                                   int qform, int fn_alias,
+                                                   double dtime, PlaneGeo geo) {
   constexpr double kTWall = 1.0;  // T_WALL (comdat_param.f90:40)
   constexpr int NC = TH ? 1 : NCV;  // components: T, or u, v, w (NCV = 1: one of them)
   const uint3 bb = xcd_block();
@@ -166,6 +167,7 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
   // while the current plane's cells are formed) in stage 1; stage 0's cells hold many more
   // operands, and there the registers are worth more than the overlap
   constexpr bool PF = S == 1;
+  constexpr bool PL = G == kGeoPlane;
   constexpr int NQ = (SF_P + 255) / 256;
   double tv[NQ][NC], nzx = 0.0, nze = 0.0, nat = 0.0;
   auto load = [&](int kp) {
@@ -178,11 +180,23 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
 #pragma unroll
       for (int comp = 0; comp < NC; ++comp) tv[h][comp] = gp(A.f[comp])[c];
     }
+    if (PL) return;
     const long cp = cidx(d, act ? i : 1, act ? j : 1, kp);
     nzx = PZX[cp];
     nze = PZE[cp];
     nat = (S < 2 && qform) ? fT[cp] : 0.0;
   };
+  // plane form: of the tile's cells at the plane of the cells formed, with X, E the stage's xi_s,
+  // eta_s: (J X) E, (J E) X, J X^2, J E^2; and the lanes with zeta_x, zeta_y terms
+  __shared__ double sc[4][PL ? SF_P : 1];
+  TileDer td;
+  ColDer cd{};
+  CellGeo ce;
+  if (PL) {
+    td.load(d, geo, bb, tid);
+    cd.load(d, geo, act ? i : 1, act ? j : 1);
+  }
+  const bool ed = geo_edge(d, i), ed1 = geo_edge(d, i, 1);
   if (PF) load(k0 - 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
     const int slot = (kp - (k0 - 1)) % 3;
@@ -210,12 +224,20 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
       zx[0] = zx[1]; zx[1] = zx[2];
       ze[0] = ze[1]; ze[1] = ze[2];
       at[0] = at[1]; at[1] = at[2];
-      if (act) {
+      if (act && !PL) {
         const long cp = cidx(d, i, j, kp);
         zx[2] = PZX[cp];
         ze[2] = PZE[cp];
         at[2] = (S < 2 && qform) ? fT[cp] : 0.0;
       }
+    }
+    if constexpr (PL) {
+      if (kp >= k0 + 1)
+        td.each(d, geo, kp - 1, [&](int q, const CellGeo& e, long) {
+          const double X = S == 0 ? e.xix : e.xiy, E = S == 0 ? e.etx : e.ety;
+          sc[0][q] = e.j * X * E; sc[1][q] = e.j * E * X;
+          sc[2][q] = e.j * (X * X); sc[3][q] = e.j * (E * E);
+        });
     }
     __syncthreads();
     if (PF && kp + 1 <= k1 + 1) load(kp + 1);
@@ -224,13 +246,31 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
     const int k = kp - 1;
     const int pl[3] = {(slot + 1) % 3, (slot + 2) % 3, slot};
     const long c = cidx(d, i, j, k);
-    const double pe_xe = PXE[c + 1], pw_xe = PXE[c - 1];
-    const double pe_xz = PXZ[c + 1], pw_xz = PXZ[c - 1];
-    const double pn_ex = PEX[c + sj], ps_ex = PEX[c - sj];
-    const double pn_ez = PEZ[c + sj], ps_ez = PEZ[c - sj];
-    const double pt_zx = zx[2], pb_zx = zx[0];
-    const double pt_ze = ze[2], pb_ze = ze[0];
-    const double a0 = ap0[c];
+    double pe_xe, pw_xe, pe_xz = 0.0, pw_xz = 0.0, pn_ex, ps_ex, pn_ez = 0.0, ps_ez = 0.0;
+    double pt_zx = zx[2], pb_zx = zx[0], pt_ze = ze[2], pb_ze = ze[0], a0;
+    double at1 = at[1], at0 = at[0];
+    if constexpr (PL) {
+      pe_xe = sc[0][q0 + 1]; pw_xe = sc[0][q0 - 1];
+      pn_ex = sc[1][q0 + SF_W]; ps_ex = sc[1][q0 - SF_W];
+      // AP0 = 2 Re J^-1 / dt as k_set_ap0 forms it
+      ce.form(cd, geo.z(k));
+      a0 = 2.0 * re * ce.j / dtime;
+      if (ed1) {
+        pe_xz = PXZ[c + 1]; pw_xz = PXZ[c - 1];
+        if (ed) {
+          pn_ez = PEZ[c + sj]; ps_ez = PEZ[c - sj];
+          pt_zx = PZX[c + sk]; pb_zx = PZX[c - sk];
+          pt_ze = PZE[c + sk]; pb_ze = PZE[c - sk];
+          at1 = fT[c]; at0 = fT[c - sk];
+        }
+      }
+    } else {
+      pe_xe = PXE[c + 1]; pw_xe = PXE[c - 1];
+      pe_xz = PXZ[c + 1]; pw_xz = PXZ[c - 1];
+      pn_ex = PEX[c + sj]; ps_ex = PEX[c - sj];
+      pn_ez = PEZ[c + sj]; ps_ez = PEZ[c - sj];
+      a0 = ap0[c];
+    }
     // every global input of the cell is loaded before the first SU store: the stores could alias
     // the inputs as far as the compiler knows, and loads after them would wait for them
     double vnl[NC], vnl1[NC], vdif[NC], vs[NC], vfn[NC], vuf[NC];
@@ -250,13 +290,24 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
     double qE = 0.0, qW = 0.0, qN = 0.0, rN = 0.0, rS = 0.0;
     const long nf = (long)(d.nj + 1) * (d.nk + 1);
     if (DR) {
-      rN = fN[c];
-      rS = fN[c - sj];
+      if constexpr (PL) {
+        rN = 0.5 * (sc[3][q0] + sc[3][q0 + SF_W]);
+        rS = 0.5 * (sc[3][q0 - SF_W] + sc[3][q0]);
+      } else {
+        rN = fN[c];
+        rS = fN[c - sj];
+      }
     }
     if (qform) {
-      qE = fE[c];
-      qW = fE[c - 1];
-      if (S == 0) qN = fN[c];
+      if constexpr (PL) {
+        qE = 0.5 * (sc[2][q0] + sc[2][q0 + 1]);
+        qW = 0.5 * (sc[2][q0 - 1] + sc[2][q0]);
+        if (S == 0) qN = 0.5 * (sc[3][q0] + sc[3][q0 + SF_W]);
+      } else {
+        qE = fE[c];
+        qW = fE[c - 1];
+        if (S == 0) qN = fN[c];
+      }
       if (i == d.ni - 1) {
 #pragma unroll
         for (int comp = 0; comp < NC; ++comp)
@@ -268,16 +319,20 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
 #define F(dk, dj, di) sh[comp][pl[(dk) + 1]][q0 + (dj) * SF_W + (di)]
       double r = pe_xe * (F(0, 1, 1) - F(0, -1, 1));
       r = r - pw_xe * (F(0, 1, -1) - F(0, -1, -1));
-      r = r + pe_xz * (F(1, 0, 1) - F(-1, 0, 1));
-      r = r - pw_xz * (F(1, 0, -1) - F(-1, 0, -1));
+      if (!PL || ed1) {
+        r = r + pe_xz * (F(1, 0, 1) - F(-1, 0, 1));
+        r = r - pw_xz * (F(1, 0, -1) - F(-1, 0, -1));
+      }
       r = r + pn_ex * (F(0, 1, 1) - F(0, 1, -1));
       r = r - ps_ex * (F(0, -1, 1) - F(0, -1, -1));
-      r = r + pn_ez * (F(1, 1, 0) - F(-1, 1, 0));
-      r = r - ps_ez * (F(1, -1, 0) - F(-1, -1, 0));
-      r = r + pt_zx * (F(1, 0, 1) - F(1, 0, -1));
-      r = r - pb_zx * (F(-1, 0, 1) - F(-1, 0, -1));
-      r = r + pt_ze * (F(1, 1, 0) - F(1, -1, 0));
-      r = r - pb_ze * (F(-1, 1, 0) - F(-1, -1, 0));
+      if (!PL || ed) {
+        r = r + pn_ez * (F(1, 1, 0) - F(-1, 1, 0));
+        r = r - ps_ez * (F(1, -1, 0) - F(-1, -1, 0));
+        r = r + pt_zx * (F(1, 0, 1) - F(1, 0, -1));
+        r = r - pb_zx * (F(-1, 0, 1) - F(-1, 0, -1));
+        r = r + pt_ze * (F(1, 1, 0) - F(1, -1, 0));
+        r = r - pb_ze * (F(-1, 1, 0) - F(-1, -1, 0));
+      }
       const double dd = 0.25 * r;
       double su;
       if (S == 0 && TH) {
@@ -305,15 +360,17 @@ __global__ void __launch_bounds__(256) k_af_rhs_km(Dims d, int kc, AFArgs A,
           ae = 0.0;
         }
         su = S == 0 ? su + qN * F(0, 1, 0) : su + ae * F(0, 0, 1);
-        su = su + at[1] * F(1, 0, 0);
-        su = su + at[0] * F(-1, 0, 0);
+        if (!PL || ed) {
+          su = su + at1 * F(1, 0, 0);
+          su = su + at0 * F(-1, 0, 0);
+        }
       }
       if (DR) {
         // the periodic images of the branch-cut ghosts j = 0 and j = NJ
         const GP fc = gp(A.f[comp]);
         const double xjm = j == 1 ? fc[cidx(d, i, d.nj - 1, k)] : F(0, -1, 0);
         const double xjp = j == d.nj - 1 ? fc[cidx(d, i, 1, k)] : F(0, 1, 0);
-        double fe = qE, fw = qW, ap = a0 + fe + fw + rN + rS + at[1] + at[0];
+        double fe = qE, fw = qW, ap = a0 + fe + fw + rN + rS + at1 + at0;
         if (i == 1) { ap = ap + fw; fw = 0.0; }
         if (i == d.ni - 1) { ap = ap + fe; fe = 0.0; }
         double r;
@@ -861,13 +918,19 @@ int fvm_k_iter_u(FvmCtx* c, bool last_ghosts) {
       const dim3 gk = march_grid(d, kc);
       if (s == 0) {
         ProfScope pk(c, "k_af_rhs_i");
-        auto kern = (qf && f32) ? k_af_rhs_km<0, false, 3, true> : k_af_rhs_km<0, false, 3, false>;
-        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, fn_alias);
+        auto kern = qf && c->plane ? (f32 ? k_af_rhs_km<0, false, 3, true, kGeoPlane>
+                                        : k_af_rhs_km<0, false, 3, false, kGeoPlane>)
+                                   : (qf && f32 ? k_af_rhs_km<0, false, 3, true>
+                                                : k_af_rhs_km<0, false, 3, false>);
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, fn_alias, c->prm.dtime, c->geo);
       }
       if (s == 1) {
         ProfScope pk(c, "k_af_rhs_j");
-        auto kern = (qf && f32) ? k_af_rhs_km<1, false, 3, true> : k_af_rhs_km<1, false, 3, false>;
-        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0);
+        auto kern = qf && c->plane ? (f32 ? k_af_rhs_km<1, false, 3, true, kGeoPlane>
+                                        : k_af_rhs_km<1, false, 3, false, kGeoPlane>)
+                                   : (qf && f32 ? k_af_rhs_km<1, false, 3, true>
+                                                : k_af_rhs_km<1, false, 3, false>);
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0, c->prm.dtime, c->geo);
       }
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0, c->prm.re, fas, qf, dz);
       HIP_CHECK(hipGetLastError());
@@ -964,10 +1027,10 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
       const dim3 gk = march_grid(d, kc);
       if (s == 0)
         hipLaunchKernelGGL((k_af_rhs_km<0, false, 1>), gk, kBlk, 0, st, d, kc, A,
-                           (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, 0);
+                           (const double* const*)c->dafp[0], c->ap0, c->prm.re, fas, qf, 0, c->prm.dtime, c->geo);
       if (s == 1)
         hipLaunchKernelGGL((k_af_rhs_km<1, false, 1>), gk, kBlk, 0, st, d, kc, A,
-                           (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0);
+                           (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0, c->prm.dtime, c->geo);
       if (s == 2)
         hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm,
                            c->djac, c->ap0, c->prm.re, fas, qf, dz);
@@ -1007,27 +1070,32 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
   return FVM_OK;
 }
 
+// Metric products of the stage 0 and 1 cross terms (geometry only).
+int fvm_af_products(FvmCtx* c) {
+  const Dims d = c->d;
+  hipStream_t st = c->stream;
+  for (int s = 0; s < 2; ++s) {
+    for (int q = 0; q < 6; ++q) {
+      HIP_CHECK(hipMalloc((void**)&c->afp[s][q], d.n * sizeof(double)));
+      c->allocs.push_back(c->afp[s][q]);
+    }
+    HIP_CHECK(hipMalloc((void**)&c->dafp[s], 6 * sizeof(double*)));
+    c->allocs.push_back(c->dafp[s]);
+    HIP_CHECK(hipMemcpy(c->dafp[s], c->afp[s], 6 * sizeof(double*), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_af_products, grid1(d.n, 256), dim3(256), 0, st, d, c->djac,
+                       c->m[3 * s], c->m[3 * s + 1], c->m[3 * s + 2],
+                       (double* const*)c->dafp[s]);
+    HIP_CHECK(hipGetLastError());
+  }
+  return FVM_OK;
+}
+
 // Which stage couplings vanish identically, and the K-line Thomas factors when that stage's
 // lines are independent.  Called after the geometry set-up and after every change of dt.
 int fvm_af_setup(FvmCtx* c) {
   const Dims d = c->d;
   hipStream_t st = c->stream;
   const int nb = 256;
-  if (!c->afp[0][0]) {  // metric products of the stage 0 and 1 cross terms (geometry only)
-    for (int s = 0; s < 2; ++s) {
-      for (int q = 0; q < 6; ++q) {
-        HIP_CHECK(hipMalloc((void**)&c->afp[s][q], d.n * sizeof(double)));
-        c->allocs.push_back(c->afp[s][q]);
-      }
-      HIP_CHECK(hipMalloc((void**)&c->dafp[s], 6 * sizeof(double*)));
-      c->allocs.push_back(c->dafp[s]);
-      HIP_CHECK(hipMemcpy(c->dafp[s], c->afp[s], 6 * sizeof(double*), hipMemcpyHostToDevice));
-      hipLaunchKernelGGL(k_af_products, grid1(d.n, 256), dim3(256), 0, st, d, c->djac,
-                         c->m[3 * s], c->m[3 * s + 1], c->m[3 * s + 2],
-                         (double* const*)c->dafp[s]);
-      HIP_CHECK(hipGetLastError());
-    }
-  }
   std::vector<double> h(3 * nb);
   for (int s = 0; s < 3; ++s) {
     if (s == 0) hipLaunchKernelGGL(k_af_couplings<0>, dim3(nb), dim3(256), 0, st, d, (const double* const*)c->dfa[0], c->ap0, c->red);
@@ -1104,8 +1172,14 @@ int fvm_k_iter_t(FvmCtx* c) {
     {
       ProfScope ps(c, "t_rhs");
       const double* const* fas = (const double* const*)c->dfa[s];
-      if (s == 0) hipLaunchKernelGGL((k_af_rhs_km<0, true>), gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0t, c->pe, fas, 1, 0);
-      if (s == 1) hipLaunchKernelGGL((k_af_rhs_km<1, true>), gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0t, c->pe, fas, 1, 0);
+      if (s == 0) {
+        auto kern = c->plane ? k_af_rhs_km<0, true, 3, false, kGeoPlane> : k_af_rhs_km<0, true>;
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[0], c->ap0t, c->pe, fas, 1, 0, c->prm.dtime, c->geo);
+      }
+      if (s == 1) {
+        auto kern = c->plane ? k_af_rhs_km<1, true, 3, false, kGeoPlane> : k_af_rhs_km<1, true>;
+        hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0t, c->pe, fas, 1, 0, c->prm.dtime, c->geo);
+      }
       if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0t, c->pe, fas, 0, c->dd2_zero ? 1 : 0);
       HIP_CHECK(hipGetLastError());
     }

@@ -389,6 +389,10 @@ static int create_impl(const fvm_params* prm, const double* xg, const double* yg
   }
   r = fvm_geom_setup(c);
   if (r) { fvm_destroy(c); return r; }
+  r = fvm_af_products(c);
+  if (r) { fvm_destroy(c); return r; }
+  r = fvm_plane_setup(c);
+  if (r) { fvm_destroy(c); return r; }
   r = fvm_af_setup(c);
   if (r) { fvm_destroy(c); return r; }
   r = fvm_sep_setup(c);
@@ -441,6 +445,7 @@ int fvm_set_field(fvm_ctx* c, int field, const double* host) {
   rs = fvm_k_nut_out(c);
   if (rs) return rs;
   if (field >= FVM_XIX && field <= FVM_ZTZ) c->xz_zero = false;  // re-derived only at set-up
+  if (field >= FVM_DJAC && field <= FVM_ZTZ) c->plane = false;
   if (field == FVM_UN || field == FVM_VN || field == FVM_WN) c->ufar_stale = true;
   std::vector<double> slab;
   if (c->two_d) {  // one (NI+1)(NJ+1) plane, repeated on the slab's three K planes

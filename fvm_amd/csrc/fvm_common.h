@@ -64,19 +64,164 @@ using gptr = __attribute__((address_space(1))) T*;
 template <typename T>
 __device__ __forceinline__ gptr<T> glb(T* p) { return (gptr<T>)p; }
 
-// Metric a of the table (grouped per Cartesian component: xi_s, eta_s, zeta_s for s = x, y, z)
-// at cell c.  With XZ0 the entries xi_z (a = 6) and eta_z (a = 7), which are exactly zero on
-// every cell of a grid extruded along z (FvmCtx::xz_zero), are the constant 0.0 and are not
-// loaded; a is a compile-time constant at every call, so the choice folds away.  The products
-// and sums keep the reference's order, so results are unchanged.
-template <bool XZ0>
+// What a kernel may take for granted of the geometry:
+// kGeoXz0    xi_z and eta_z are exactly zero on every cell (a grid extruded along z,
+//            FvmCtx::xz_zero) and are not loaded;
+// kGeoPlane  x and y repeat one plane of nodes bit for bit and z is a function of K alone
+//            (PlaneGeo): J^-1 and the metrics of a cell are formed again, bit for bit, from the
+//            four cross-section derivatives of its column, which a thread holds in registers for
+//            the whole column it marches up, and z_zeta of its K plane.  zeta_x, zeta_y and the
+//            coefficients with one of them as a factor are exactly zero but on the columns next
+//            to the I boundaries (geo_edge: rounding residues there), whose lanes load them.
+// The step is bound by its passes over HBM, and of the arrays a general kernel streams five to ten
+// are geometry that repeats plane by plane.  Times of the kernels with the stored arrays and in the
+// plane form, us on 192 x 256 x 64 and on 384 x 512 x 128 cells:
+//   strain and test filter  149 -> 138  1153 -> 1028    predictor's p gradient   76 -> 43  614 -> 283
+//   SGS model coefficient   181 -> 157  1232 -> 1088    corrector with CFL      135 -> 88  989 -> 687
+//   SGS stress divergence   111 -> 75    979 -> 612     Poisson residual         52 -> 48  438 -> 304
+//   convection, diffusion   131 -> 129   981 -> 892     predictor correction    100 -> 86  880 -> 619
+//   AF right-hand side, I   167 -> 125  1298 -> 936     the same, J             100 -> 78  796 -> 526
+// The convection/diffusion pass and the Poisson residual, which need J^-1 Q_ij of four neighbours
+// for few arrays of their own, read the stored arrays on plane kz[k], of which the
+// caches hold the few that differ; forming them anew took 150 and 46 us, 897 and 298 us.
+constexpr int kGeoAny = 0, kGeoXz0 = 1, kGeoPlane = 2;
+// metric a of the table (grouped per Cartesian component: xi_s, eta_s, zeta_s for s = x, y, z) at
+// cell c; a is a compile-time constant at every call, so the choice folds away.  The products and
+// sums of the callers keep the reference's order, so results are unchanged.
+template <int G>
 __device__ inline double mget(const double* const* __restrict__ m, int a, long c) {
-  return (XZ0 && (a == 6 || a == 7)) ? 0.0 : gp(m[a])[c];
+  return G >= kGeoXz0 && (a == 6 || a == 7) ? 0.0 : gp(m[a])[c];
+}
+// the nine metrics of a cell
+struct Met {
+  double v[9];
+};
+template <int G>
+__device__ inline Met load_met(const double* const* __restrict__ m, long c) {
+  Met q;
+#pragma unroll
+  for (int a = 0; a < 9; ++a) q.v[a] = mget<G>(m, a, c);
+  return q;
+}
+
+// Geometry of a kGeoPlane grid.
+struct PlaneGeo {
+  const double* d2;  // x_xi, y_xi, x_eta, y_eta of the columns: four arrays of NI+1 x NJ+1
+  const double* zz;  // z_zeta of the K planes: of the columns i = 1..NI-1, of i = 0, of i = NI
+  const int* kz;     // the first plane with the same three z_zeta, and so the same coefficients
+  // Scalar loads: without the address space the compiler, which cannot see that a kernel's stores
+  // leave the tables alone, takes vector loads and waits for every load before them.
+  __device__ inline double z(int t) const {
+    return ((const __attribute__((address_space(4))) double*)zz)[t];
+  }
+  __device__ inline int plane(int k) const {
+    return ((const __attribute__((address_space(4))) int*)kz)[k];
+  }
+};
+// lanes whose zeta_x, zeta_y terms may be nonzero; w = 1: or those of a neighbour along I
+__device__ inline bool geo_edge(const Dims& d, int i, int w = 0) {
+  return i <= 1 + w || i >= d.ni - 1 - w;
+}
+// a[c] on the lanes with e, else 0.  Every lane loads (the others the first element): where a cell
+// has only two or three such terms the wait in a branch costs more than the loads.
+__device__ inline double edge_load(GP a, long c, bool e) {
+  const double v = a[e ? c : 0];
+  return e ? v : 0.0;
+}
+struct ColDer {
+  double xx, yx, xe, ye;
+  __device__ inline void load(const Dims& d, const PlaneGeo& g, int i, int j) {
+    const long c = i + d.sj * j;
+    xx = gp(g.d2)[c]; yx = gp(g.d2)[c + d.sk];
+    xe = gp(g.d2)[c + 2 * d.sk]; ye = gp(g.d2)[c + 3 * d.sk];
+  }
+};
+// z_zeta of plane k at the columns of index i
+__device__ inline double col_zz(const Dims& d, const PlaneGeo& g, int i, int k) {
+  const int np = d.nk + 1;
+  const double z = g.z(k), z0 = g.z(np + k), z1 = g.z(2 * np + k);
+  return i == 0 ? z0 : (i == d.ni ? z1 : z);
+}
+// J^-1 and the metrics of a cell without zeta_x, zeta_y, in the operations of the set-up
+// (metric.f90:412-497) less the terms that are exactly zero.  The quotients by J^-1 share its
+// reciprocal: a y corrected by one step of its remainder is the correctly rounded a / J^-1
+// (P. Markstein, IBM J. Res. Dev. 34, 1990); the set-up compares it with the divided metrics of
+// every cell.  About 40 FP64 operations instead of 48 bytes loaded.
+struct CellGeo {
+  double j, xix, xiy, etx, ety, ztz;
+  __device__ inline void form(const ColDer& q, double zz) {
+    const double a = q.ye * zz, b = q.xe * zz;
+    j = q.xx * a - q.yx * b;
+    const double y = 1.0 / j;
+    auto quo = [&](double n) {
+      const double t = n * y;
+      return __builtin_fma(__builtin_fma(-t, j, n), y, t);
+    };
+    xix = quo(a);
+    xiy = quo(-b);
+    etx = quo(-(q.yx * zz));
+    ety = quo(zz * q.xx);
+    ztz = quo(q.xx * q.ye - q.xe * q.yx);
+  }
+  __device__ inline Met met(double ztx, double zty) const {
+    return Met{{xix, etx, ztx, xiy, ety, zty, 0.0, 0.0, ztz}};
+  }
+  __device__ inline double jq11() const { return j * (xix * xix + xiy * xiy); }
+  __device__ inline double jq12() const { return j * (xix * etx + xiy * ety); }
+  __device__ inline double jq22() const { return j * (etx * etx + ety * ety); }
+  __device__ inline double jq33() const { return j * (ztz * ztz); }
+};
+// the metrics of cell (i, j, k)
+__device__ inline Met plane_met(const Dims& d, const double* const* __restrict__ m,
+                                const CellGeo& q, int i, int j, int k) {
+  const bool e = geo_edge(d, i);
+  const long c = cidx(d, i, j, k);
+  return q.met(edge_load(gp(m[2]), c, e), edge_load(gp(m[5]), c, e));
 }
 
 // A 64 x 4 (I x J) tile of the K-marching stencil kernels with its one-cell halo, as staged in
 // LDS: SF_W x SF_H cells, row-major.
 constexpr int SF_W = 66, SF_H = 6, SF_P = SF_W * SF_H;
+constexpr int SF_NQ = (SF_P + 255) / 256;  // tile cells of a thread
+
+// The columns of a thread's tile cells in the plane form: each() forms their geometry at plane k,
+// f(tile cell, geometry, its cell index).  A neighbour's coefficients then come from LDS as the
+// tile's fields do; forming the halo cells anew costs a workgroup 1.55 cells per cell.
+struct TileDer {
+  ColDer c[SF_NQ];
+  int gi[SF_NQ], gj[SF_NQ], q0;
+  __device__ inline void load(const Dims& d, const PlaneGeo& g, uint3 bb, int tid) {
+    q0 = tid;
+#pragma unroll
+    for (int h = 0; h < SF_NQ; ++h) {
+      const int q = min(tid + 256 * h, SF_P - 1);
+      gi[h] = min((int)bb.x * 64 + q % SF_W, d.ni);
+      gj[h] = min((int)bb.y * 4 + q / SF_W, d.nj);
+      c[h].load(d, g, gi[h], gj[h]);
+    }
+  }
+  template <typename F>
+  __device__ inline void each(const Dims& d, const PlaneGeo& g, int k, F f) const {
+#pragma unroll
+    for (int h = 0; h < SF_NQ; ++h) {
+      const int q = q0 + 256 * h;
+      if (q >= SF_P) continue;
+      CellGeo e;
+      e.form(c[h], col_zz(d, g, gi[h], k));
+      f(q, e, cidx(d, gi[h], gj[h], k));
+    }
+  }
+};
+
+// A cell's face coefficients D_e, D_w, D_n, D_s and J^-1 Q12 of its four neighbours
+struct ColStencil {
+  double de, dw, dn, ds, e12, w12, n12, s12;
+  __device__ inline void load(const double* __restrict__ pdI, const double* __restrict__ pdJ,
+                              const double* __restrict__ jq12, long sj, long c) {
+    de = pdI[c]; dw = pdI[c - 1]; dn = pdJ[c]; ds = pdJ[c - sj];
+    e12 = jq12[c + 1]; w12 = jq12[c - 1]; n12 = jq12[c + sj]; s12 = jq12[c - sj];
+  }
+};
 
 // Maximum line length handled by one 64-lane wavefront (8 rows per lane).
 #define FVM_MAX_LINE 512

@@ -72,6 +72,8 @@ struct FvmCtx {
   bool af_zero_a[3] = {}, af_zero_b[3] = {};
   double af_b_ratio[3] = {};
   bool xz_zero = false;       // xi_z = eta_z = 0 on every cell (metric kernels skip them)
+  bool plane = false;         // and kGeoPlane's conditions hold
+  PlaneGeo geo{};
   bool dd2_zero = false;      // xi_z = eta_z = 0 around every cell: stage-3 cross terms vanish  // max over cells of (|b couplings|) / (2 Re J^-1/dt)
   // Thomas factors A, D, B of the K-line stage when its lines are independent
   double *tk_a = nullptr, *tk_d = nullptr, *tk_b = nullptr;
@@ -200,6 +202,8 @@ int fvm_fetch(FvmCtx* c, const double* src, int n, double* dst);
 Mailbox fvm_mail(FvmCtx* c);  // a fresh sequence number for a kernel that publishes itself
 int fvm_mail_wait(FvmCtx* c, const Mailbox& mb, int n, double* dst);
 int fvm_geom_setup(FvmCtx* c);
+int fvm_af_products(FvmCtx* c);
+int fvm_plane_setup(FvmCtx* c);
 int fvm_k_set_dtime(FvmCtx* c, double dtime);
 int fvm_af_setup(FvmCtx* c);
 int fvm_af_scan_setup(FvmCtx* c);

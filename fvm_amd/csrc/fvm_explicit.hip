@@ -27,7 +27,7 @@ const dim3 kBlk(64, 4, 1);
 
 // Contravariant velocity times J^-1 on i = 0..NI, interior j,k (RLES/contra_vel.f90:13-23);
 // the face volume fluxes are 0.5 (JU(c) + JU(c+1)) (contra_vel.f90:37-53).
-template <bool XZ0>
+template <int G>
 __global__ void k_contra(Dims d, const double* const* __restrict__ m, const double* __restrict__ djac,
                          const double* __restrict__ u, const double* __restrict__ v,
                          const double* __restrict__ w, double* ju0, double* ju1, double* ju2) {
@@ -38,8 +38,8 @@ __global__ void k_contra(Dims d, const double* const* __restrict__ m, const doub
   if (i > d.ni || j > d.nj - 1) return;
   const long c = cidx(d, i, j, k);
   double U = u[c], V = v[c], W = w[c], J = djac[c];
-  double u1 = gp(m[0])[c] * U + gp(m[3])[c] * V + mget<XZ0>(m, 6, c) * W;
-  double u2 = gp(m[1])[c] * U + gp(m[4])[c] * V + mget<XZ0>(m, 7, c) * W;
+  double u1 = gp(m[0])[c] * U + gp(m[3])[c] * V + mget<G>(m, 6, c) * W;
+  double u2 = gp(m[1])[c] * U + gp(m[4])[c] * V + mget<G>(m, 7, c) * W;
   double u3 = gp(m[2])[c] * U + gp(m[5])[c] * V + gp(m[8])[c] * W;
   ju0[c] = J * u1;
   ju1[c] = J * u2;
@@ -101,7 +101,7 @@ constexpr int DF_RES = 1024;  // workgroups of k_dif_km resident at a time (four
 // order) from the staged planes and the face fluxes of ju (ju2 of the planes K+-1 in registers):
 // the whole step runs NL and DIF in one pass over u_n, v_n, w_n (DIF does not depend on NL or on
 // the SGS term added to NL in between).
-template <int NC, bool WNL = false>
+template <int NC, bool WNL = false, int G = kGeoAny>
 __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
                                                 const double* __restrict__ pdJ,
                                                 const double* __restrict__ pdK,
@@ -111,7 +111,9 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
                                                 const double* __restrict__ ju0 = nullptr,
                                                 const double* __restrict__ ju1 = nullptr,
                                                 const double* __restrict__ ju2 = nullptr,
-                                                CompSet nlo = CompSet{}) {
+                                                CompSet nlo = CompSet{},
+                                                const double* __restrict__ jq33 = nullptr,
+                                                PlaneGeo geo = PlaneGeo{}) {
   const uint3 bb = xcd_block();
   __shared__ double sh[NC][3][SF_P];  // [component][plane slot][tile cell]
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
@@ -124,6 +126,11 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
   const long sj = d.sj;
   double j13[3] = {0.0, 0.0, 0.0}, j23[3] = {0.0, 0.0, 0.0}, pk[3] = {0.0, 0.0, 0.0};
   double z2[3] = {0.0, 0.0, 0.0};  // ju2 of the own column (NL's K faces)
+  // plane form: the coefficients are those of plane kz[k] (which the caches hold), J^-1 Q33 of the
+  // planes kp-2, kp-1, kp takes pdK's place (pdK is the mean of two), and only the lanes next to
+  // the I boundaries have J^-1 Q13, J^-1 Q23 terms
+  constexpr bool PL = G == kGeoPlane;
+  const bool ed = geo_edge(d, i), ed1 = geo_edge(d, i, 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
     const int slot = (kp - (k0 - 1)) % 3;
     __syncthreads();  // plane kp - 3, held in this slot, is no longer read
@@ -140,9 +147,13 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
     z2[0] = z2[1]; z2[1] = z2[2];
     if (act) {
       const long cp = cidx(d, i, j, kp);
-      j13[2] = jq13[cp];
-      j23[2] = jq23[cp];
-      pk[2] = pdK[cp];
+      if (PL) {
+        pk[2] = jq33[cidx(d, i, j, geo.plane(kp))];
+      } else {
+        j13[2] = jq13[cp];
+        j23[2] = jq23[cp];
+        pk[2] = pdK[cp];
+      }
       if (WNL) z2[2] = ju2[cp];
     }
     __syncthreads();
@@ -171,10 +182,22 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
         gpw(nlo.out[comp])[c] = 0.5 * t;
       }
     }
-    const double de = pdI[c], dw = pdI[c - 1], dn = pdJ[c], ds = pdJ[c - sj], dt = pk[1],
-                 db = pk[0];
-    const double e12 = jq12[c + 1], w12 = jq12[c - 1], e13 = jq13[c + 1], w13 = jq13[c - 1];
-    const double n12 = jq12[c + sj], s12 = jq12[c - sj], n23 = jq23[c + sj], s23 = jq23[c - sj];
+    double dt = pk[1], db = pk[0], e13 = 0.0, w13 = 0.0, n23 = 0.0, s23 = 0.0;
+    ColStencil cs6;
+    if (PL) {
+      cs6.load(pdI, pdJ, jq12, sj, cidx(d, i, j, geo.plane(k)));
+      dt = 0.5 * (pk[1] + pk[2]);
+      db = 0.5 * (pk[0] + pk[1]);
+      e13 = edge_load(gp(jq13), c + 1, ed1); w13 = edge_load(gp(jq13), c - 1, ed1);
+      n23 = edge_load(gp(jq23), c + sj, ed); s23 = edge_load(gp(jq23), c - sj, ed);
+      j13[0] = edge_load(gp(jq13), c - d.sk, ed); j13[2] = edge_load(gp(jq13), c + d.sk, ed);
+      j23[0] = edge_load(gp(jq23), c - d.sk, ed); j23[2] = edge_load(gp(jq23), c + d.sk, ed);
+    } else {
+      cs6.load(pdI, pdJ, jq12, sj, c);
+      e13 = jq13[c + 1]; w13 = jq13[c - 1]; n23 = jq23[c + sj]; s23 = jq23[c - sj];
+    }
+    const double de = cs6.de, dw = cs6.dw, dn = cs6.dn, ds = cs6.ds;
+    const double e12 = cs6.e12, w12 = cs6.w12, n12 = cs6.n12, s12 = cs6.s12;
 #pragma unroll
     for (int comp = 0; comp < NC; ++comp) {
 #define F(dk, dj, di) sh[comp][pl[(dk) + 1]][q0 + (dj) * SF_W + (di)]
@@ -187,16 +210,20 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
       t = t + db * (F(-1, 0, 0) - fc);
       double r = e12 * (F(0, 1, 1) - F(0, -1, 1));
       r = r - w12 * (F(0, 1, -1) - F(0, -1, -1));
-      r = r + e13 * (F(1, 0, 1) - F(-1, 0, 1));
-      r = r - w13 * (F(1, 0, -1) - F(-1, 0, -1));
+      if (!PL || ed1) {
+        r = r + e13 * (F(1, 0, 1) - F(-1, 0, 1));
+        r = r - w13 * (F(1, 0, -1) - F(-1, 0, -1));
+      }
       r = r + n12 * (F(0, 1, 1) - F(0, 1, -1));
       r = r - s12 * (F(0, -1, 1) - F(0, -1, -1));
-      r = r + n23 * (F(1, 1, 0) - F(-1, 1, 0));
-      r = r - s23 * (F(1, -1, 0) - F(-1, -1, 0));
-      r = r + j13[2] * (F(1, 0, 1) - F(1, 0, -1));
-      r = r - j13[0] * (F(-1, 0, 1) - F(-1, 0, -1));
-      r = r + j23[2] * (F(1, 1, 0) - F(1, -1, 0));
-      r = r - j23[0] * (F(-1, 1, 0) - F(-1, -1, 0));
+      if (!PL || ed) {
+        r = r + n23 * (F(1, 1, 0) - F(-1, 1, 0));
+        r = r - s23 * (F(1, -1, 0) - F(-1, -1, 0));
+        r = r + j13[2] * (F(1, 0, 1) - F(1, 0, -1));
+        r = r - j13[0] * (F(-1, 0, 1) - F(-1, 0, -1));
+        r = r + j23[2] * (F(1, 1, 0) - F(1, -1, 0));
+        r = r - j23[0] * (F(-1, 1, 0) - F(-1, -1, 0));
+      }
 #undef F
       t = t + 0.25 * r;
       gpw(cs.out[comp])[c] = 1.0 * t;
@@ -232,7 +259,7 @@ __device__ inline void pref_mean(const Dims& d, const double* __restrict__ p, do
   if (t == 0) out[0] = s / (double)(d.nk - 1);
 }
 
-template <int CORR, bool XZ0>
+template <int CORR, int G>
 __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
                                                     const double* const* __restrict__ m,
                                                     const double* __restrict__ djac,
@@ -240,7 +267,8 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
                                                     double* s0, double* s1, double* s2, double* u,
                                                     double* v, double* w,
                                                     const double* __restrict__ ufar,
-                                                    double* cflpart, double* pref) {
+                                                    double* cflpart, double* pref,
+                                                    PlaneGeo geo) {
   __shared__ double sh[256];
   if (CORR && blockIdx.x == tg.x * tg.y * tg.z) {  // one workgroup past the tiles
     pref_mean(d, p, pref, threadIdx.y * 64 + threadIdx.x, sh);
@@ -259,28 +287,81 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
   // (J zeta_s p) of the own column, planes kp-2, kp-1, kp, per component s
   double zp[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
   double cmax = 0.0;  // this thread's largest local CFL number
+  // plane form: J^-1 xi_x p, J^-1 xi_y p, J^-1 eta_x p, J^-1 eta_y p of the tile's cells at the
+  // plane of the cells formed
+  constexpr bool PL = G == kGeoPlane;
+  __shared__ double sp[4][PL ? SF_P : 1];
+  const int q0 = (ty + 1) * SF_W + tx + 1;
+  TileDer td;
+  ColDer cd{};
+  CellGeo ce;
+  if (PL) {
+    td.load(d, geo, bb, tid);
+    cd.load(d, geo, act ? i : 1, act ? j : 1);
+  }
+  double J = 0.0;
+  Met mv{};
+  const bool ed = geo_edge(d, i);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) { zp[q][0] = zp[q][1]; zp[q][1] = zp[q][2]; }
     if (act) {
       const long cp = cidx(d, i, j, kp);
-      const double jc = djac[cp], pc = p[cp];
+      const double pc = p[cp];
+      if (PL) {
+        ce.form(cd, geo.z(kp));
+        zp[0][2] = ce.j * edge_load(gp(m[2]), cp, ed) * pc;
+        zp[1][2] = ce.j * edge_load(gp(m[5]), cp, ed) * pc;
+        zp[2][2] = ce.j * ce.ztz * pc;
+      } else {
+        const double jc = djac[cp];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) zp[q][2] = jc * gp(m[3 * q + 2])[cp] * pc;
+        for (int q = 0; q < 3; ++q) zp[q][2] = jc * gp(m[3 * q + 2])[cp] * pc;
+      }
     }
     if (kp < k0 + 1) continue;  // uniform over the workgroup
     const int k = kp - 1;
+    if constexpr (PL) {
+      __syncthreads();  // the products of plane k - 1 are no longer read
+      td.each(d, geo, k, [&](int q, const CellGeo& e, long c) {
+        const double pc = p[c];
+        sp[0][q] = e.j * e.xix * pc; sp[1][q] = e.j * e.xiy * pc;
+        sp[2][q] = e.j * e.etx * pc; sp[3][q] = e.j * e.ety * pc;
+      });
+      __syncthreads();
+    }
     if (act) {
       const long c = cidx(d, i, j, k);
       double nv[3], sv[3], fv[3];
-      const double J = djac[c];
       // all loads of the cell precede its stores (which might alias them for the compiler)
+      if (PL) {
+        ce.form(cd, geo.z(k));
+        J = ce.j;
+        if (CORR) mv = plane_met(d, m, ce, i, j, k);
+      } else {
+        J = djac[c];
+        if (CORR) mv = load_met<G>(m, c);
+      }
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        double t = djac[c + 1] * mget<XZ0>(m, 3 * q, c + 1) * p[c + 1];
-        t = t - djac[c - 1] * mget<XZ0>(m, 3 * q, c - 1) * p[c - 1];
-        t = t + djac[c + sj] * mget<XZ0>(m, 3 * q + 1, c + sj) * p[c + sj];
-        t = t - djac[c - sj] * mget<XZ0>(m, 3 * q + 1, c - sj) * p[c - sj];
+        if constexpr (PL) {
+          double t = 0.0;
+          if (q < 2) {
+            t = sp[q][q0 + 1];
+            t = t - sp[q][q0 - 1];
+            t = t + sp[2 + q][q0 + SF_W];
+            t = t - sp[2 + q][q0 - SF_W];
+          }
+          t = t + zp[q][2];
+          t = t - zp[q][0];
+          sv[q] = -(0.5 * t);
+          fv[q] = CORR ? f[q][c] : 0.0;
+          continue;
+        }
+        double t = djac[c + 1] * mget<G>(m, 3 * q, c + 1) * p[c + 1];
+        t = t - djac[c - 1] * mget<G>(m, 3 * q, c - 1) * p[c - 1];
+        t = t + djac[c + sj] * mget<G>(m, 3 * q + 1, c + sj) * p[c + sj];
+        t = t - djac[c - sj] * mget<G>(m, 3 * q + 1, c - sj) * p[c - sj];
         t = t + zp[q][2];
         t = t - zp[q][0];
         sv[q] = -(0.5 * t);
@@ -301,9 +382,9 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
         bc_images(d, w, ufar + 2 * nf, 0.0, i, j, k, nv[2]);
 
         const double U = nv[0], V = nv[1], W = nv[2];
-        const double ca = fabs(gp(m[0])[c] * U + gp(m[3])[c] * V + mget<XZ0>(m, 6, c) * W);
-        const double cb = fabs(gp(m[1])[c] * U + gp(m[4])[c] * V + mget<XZ0>(m, 7, c) * W);
-        const double ce = fabs(gp(m[2])[c] * U + gp(m[5])[c] * V + gp(m[8])[c] * W);
+        const double ca = fabs(mv.v[0] * U + mv.v[3] * V + mv.v[6] * W);
+        const double cb = fabs(mv.v[1] * U + mv.v[4] * V + mv.v[7] * W);
+        const double ce = fabs(mv.v[2] * U + mv.v[5] * V + mv.v[8] * W);
         cmax = fmax(cmax, dtime * (ca + cb + ce));
       }
     }
@@ -318,13 +399,12 @@ __global__ void __launch_bounds__(256) k_psource_km(Dims d, int kc, uint3 tg,
   if (tid == 0) cflpart[blockIdx.x] = sh[0];
 }
 
-// J^-1 x contravariant velocity of cell c from the velocity (U, V, W) there (contra_vel.f90:13-23)
-template <bool XZ0>
-__device__ inline void contra_cell(const double* const* __restrict__ m, long c, double J, double U,
-                                   double V, double W, double (&ju)[3]) {
-  const double u1 = gp(m[0])[c] * U + gp(m[3])[c] * V + mget<XZ0>(m, 6, c) * W;
-  const double u2 = gp(m[1])[c] * U + gp(m[4])[c] * V + mget<XZ0>(m, 7, c) * W;
-  const double u3 = gp(m[2])[c] * U + gp(m[5])[c] * V + gp(m[8])[c] * W;
+// J^-1 x contravariant velocity of a cell with metrics m (contra_vel.f90:13-23)
+__device__ inline void contra_cell(const Met& m, double J, double U, double V, double W,
+                                   double (&ju)[3]) {
+  const double u1 = m.v[0] * U + m.v[3] * V + m.v[6] * W;
+  const double u2 = m.v[1] * U + m.v[4] * V + m.v[7] * W;
+  const double u3 = m.v[2] * U + m.v[5] * V + m.v[8] * W;
   ju[0] = J * u1;
   ju[1] = J * u2;
   ju[2] = J * u3;
@@ -341,39 +421,70 @@ struct Vec3P {
 // images.  As four launches (interior, BCU ghosts, JU on the I planes, JU's periodic copy) the
 // surface kernels took 6.7 + 13.7 + 5.5 us on 192 x 256 x 64 cells for strided columns of
 // 8 bytes per cache line.
-template <bool XZ0>
-__global__ void k_correct_contra(Dims d, const double* const* __restrict__ m,
-                                 const double* __restrict__ djac, double dtime, Vec3P s, Vec3P f,
-                                 Vec3P ju, const double* __restrict__ ufar) {
-  INTERIOR_IJK(d);
-  const double J = djac[c];
+// Plane form: a thread takes CC_KP planes of its column with the metrics in registers.
+constexpr int CC_KP = 4;
+template <int G>
+__global__ void __launch_bounds__(256) k_correct_contra(Dims d, const double* const* __restrict__ m,
+                                                        const double* __restrict__ djac,
+                                                        double dtime, Vec3P s, Vec3P f, Vec3P ju,
+                                                        const double* __restrict__ ufar,
+                                                        PlaneGeo geo) {
+  constexpr bool PL = G == kGeoPlane;
+  constexpr int KP = PL ? CC_KP : 1;
+  const uint3 bb = xcd_block();
+  const int i = 1 + bb.x * 64 + threadIdx.x;
+  const int j = 1 + bb.y * 4 + threadIdx.y;
+  const int k0 = 1 + (int)bb.z * KP;
+  if (i > d.ni - 1 || j > d.nj - 1) return;
+  ColDer cd{};
+  CellGeo ce;
+  if (PL) cd.load(d, geo, i, j);
   const long nf = (long)(d.nj + 1) * (d.nk + 1);
-  double n[3], a[3];
+  double fv[KP][3], sv[KP][3];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) n[q] = gp(f.p[q])[c] - dtime * gp(s.p[q])[c] / J;
-  contra_cell<XZ0>(m, c, J, n[0], n[1], n[2], a);
+  for (int r = 0; r < KP; ++r) {
+    const long c = cidx(d, i, j, min(k0 + r, d.nk - 1));
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    gpw(f.p[q])[c] = n[q];
-    bc_images(d, f.p[q], ufar + q * nf, 0.0, i, j, k, n[q]);
-    gpw(ju.p[q])[c] = a[q];
-    periodic_images(d, ju.p[q], i, j, k, a[q]);
+    for (int q = 0; q < 3; ++q) {
+      fv[r][q] = gp(f.p[q])[c];
+      sv[r][q] = gp(s.p[q])[c];
+    }
   }
-  if (i == 1 || i == d.ni - 1) {  // the row's ghosts, as bc_images forms them
-    for (int side = 0; side < 2; ++side) {
-      if (i != (side == 0 ? 1 : d.ni - 1)) continue;
-      const int ig = side == 0 ? 0 : d.ni;
-      const long cg = cidx(d, ig, j, k);
-      double g[3], b[3];
 #pragma unroll
-      for (int q = 0; q < 3; ++q)
-        g[q] = side == 0 ? -n[q] + 2.0 * 0.0
-                         : -n[q] + 2.0 * ufar[q * nf + j + (long)(d.nj + 1) * k];
-      contra_cell<XZ0>(m, cg, djac[cg], g[0], g[1], g[2], b);
+  for (int r = 0; r < KP; ++r) {
+    const int k = k0 + r;
+    if (k > d.nk - 1) break;
+    const long c = cidx(d, i, j, k);
+    if (PL) ce.form(cd, geo.z(k));
+    const double J = PL ? ce.j : djac[c];
+    const Met mc = PL ? plane_met(d, m, ce, i, j, k) : load_met<G>(m, c);
+    double n[3], a[3];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        gpw(ju.p[q])[cg] = b[q];
-        periodic_images(d, ju.p[q], ig, j, k, b[q]);
+    for (int q = 0; q < 3; ++q) n[q] = fv[r][q] - dtime * sv[r][q] / J;
+    contra_cell(mc, J, n[0], n[1], n[2], a);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      gpw(f.p[q])[c] = n[q];
+      bc_images(d, f.p[q], ufar + q * nf, 0.0, i, j, k, n[q]);
+      gpw(ju.p[q])[c] = a[q];
+      periodic_images(d, ju.p[q], i, j, k, a[q]);
+    }
+    if (i == 1 || i == d.ni - 1) {  // the row's ghosts, as bc_images forms them
+      for (int side = 0; side < 2; ++side) {
+        if (i != (side == 0 ? 1 : d.ni - 1)) continue;
+        const int ig = side == 0 ? 0 : d.ni;
+        const long ch = cidx(d, ig, j, k);
+        double g[3], b[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          g[q] = side == 0 ? -n[q] + 2.0 * 0.0
+                           : -n[q] + 2.0 * ufar[q * nf + j + (long)(d.nj + 1) * k];
+        contra_cell(load_met<PL ? kGeoXz0 : G>(m, ch), djac[ch], g[0], g[1], g[2], b);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          gpw(ju.p[q])[ch] = b[q];
+          periodic_images(d, ju.p[q], ig, j, k, b[q]);
+        }
       }
     }
   }
@@ -432,42 +543,57 @@ struct StepStart {
   double* tfar;        // of T, or nullptr without the passive temperature
 };
 
-template <bool XZ0>
+// Plane form: a thread takes SB_KP planes of its column with the metrics in registers.
+constexpr int SB_KP = 2;
+template <int G>
 __global__ void __launch_bounds__(256) k_step_begin(Dims d, const double* const* __restrict__ m,
                                                     const double* __restrict__ djac,
                                                     const double* __restrict__ theta, StepStart a,
-                                                    double dtime, double pi) {
+                                                    double dtime, double pi,
+                                                    PlaneGeo geo) {
+  constexpr bool PL = G == kGeoPlane;
+  constexpr int KP = PL ? SB_KP : 1;
   const uint3 bb = xcd_block();
   const int i = bb.x * 64 + threadIdx.x;
   const int j = bb.y * 4 + threadIdx.y;
-  const int k = bb.z;
+  const int k0 = (int)bb.z * KP;
   if (i > d.ni || j > d.nj) return;
-  const long c = cidx(d, i, j, k);
   const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
-  const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
-  const bool in = js == j && ks == k;
-  const long cs = cidx(d, i, js, ks);
-  double q[3], o[3];
+  ColDer cd{};
+  CellGeo ce;
+  if (PL) cd.load(d, geo, i, js);
 #pragma unroll
-  for (int f = 0; f < 3; ++f) {
-    q[f] = gp(a.f[f])[cs];
-    o[f] = in ? q[f] : gp(a.f[f])[c];
-  }
-  double b[3];
-  contra_cell<XZ0>(m, cs, djac[cs], q[0], q[1], q[2], b);
+  for (int r = 0; r < KP; ++r) {
+    const int k = k0 + r;
+    if (k > d.nk) break;
+    const long c = cidx(d, i, j, k);
+    const int ks = k == 0 ? d.nk - 1 : (k == d.nk ? 1 : k);
+    const bool in = js == j && ks == k;
+    const long cs = cidx(d, i, js, ks);
+    double q[3], o[3];
 #pragma unroll
-  for (int f = 0; f < 3; ++f) {
-    gpw(a.fn[f])[c] = o[f];
-    gpw(a.ju[f])[c] = b[f];
-  }
-  if (a.tfar) gpw(a.fn[3])[c] = gp(a.f[3])[c];
-  if (i == d.ni) {
-    const long nf = (long)(d.nj + 1) * (d.nk + 1), t = j + (long)(d.nj + 1) * k;
+    for (int f = 0; f < 3; ++f) {
+      q[f] = gp(a.f[f])[cs];
+      o[f] = in ? q[f] : gp(a.f[f])[c];
+    }
+    if (PL) ce.form(cd, col_zz(d, geo, i, ks));
+    const Met mc = PL ? plane_met(d, m, ce, i, js, ks) : load_met<G>(m, cs);
+    double b[3];
+    contra_cell(mc, PL ? ce.j : djac[cs], q[0], q[1], q[2], b);
 #pragma unroll
-    for (int f = 0; f < 3; ++f)
-      a.ufar[f * nf + t] =
-          in ? ufar_value(d, m, theta, a.f[f], f == 0 ? 1.0 : 0.0, dtime, pi, j, k) : 0.0;
-    if (a.tfar) a.tfar[t] = in ? ufar_value(d, m, theta, a.f[3], 0.0, dtime, pi, j, k) : 0.0;
+    for (int f = 0; f < 3; ++f) {
+      gpw(a.fn[f])[c] = o[f];
+      gpw(a.ju[f])[c] = b[f];
+    }
+    if (a.tfar) gpw(a.fn[3])[c] = gp(a.f[3])[c];
+    if (i == d.ni) {
+      const long nf = (long)(d.nj + 1) * (d.nk + 1), t = j + (long)(d.nj + 1) * k;
+#pragma unroll
+      for (int f = 0; f < 3; ++f)
+        a.ufar[f * nf + t] =
+            in ? ufar_value(d, m, theta, a.f[f], f == 0 ? 1.0 : 0.0, dtime, pi, j, k) : 0.0;
+      if (a.tfar) a.tfar[t] = in ? ufar_value(d, m, theta, a.f[3], 0.0, dtime, pi, j, k) : 0.0;
+    }
   }
 }
 
@@ -829,10 +955,10 @@ int fvm_k_contra_vel(FvmCtx* c) {
     ProfScope ps(c, "contra_vel");
     dim3 g((d.ni + 1 + 63) / 64, (d.nj - 1 + 3) / 4, d.nk - 1);
     if (c->xz_zero)
-      hipLaunchKernelGGL(k_contra<true>, g, kBlk, 0, c->stream, d, (const double* const*)m,
+      hipLaunchKernelGGL(k_contra<kGeoXz0>, g, kBlk, 0, c->stream, d, (const double* const*)m,
                          c->djac, c->u, c->v, c->w, c->ju[0], c->ju[1], c->ju[2]);
     else
-      hipLaunchKernelGGL(k_contra<false>, g, kBlk, 0, c->stream, d, (const double* const*)m,
+      hipLaunchKernelGGL(k_contra<kGeoAny>, g, kBlk, 0, c->stream, d, (const double* const*)m,
                          c->djac, c->u, c->v, c->w, c->ju[0], c->ju[1], c->ju[2]);
     HIP_CHECK(hipGetLastError());
   }
@@ -877,12 +1003,10 @@ int fvm_k_nl_dif(FvmCtx* c) {
   const dim3 g = march_grid(d, kc);
   const CompSet cs = {{c->un, c->vn, c->wn, c->tn}, {c->dif[0], c->dif[1], c->dif[2], c->dift}};
   const CompSet nlo = {{nullptr, nullptr, nullptr, nullptr}, {c->nl[0], c->nl[1], c->nl[2], c->adv}};
-  if (c->thermal)
-    hipLaunchKernelGGL((k_dif_km<4, true>), g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
-                       c->jq12, c->jq13, c->jq23, cs, c->ju[0], c->ju[1], c->ju[2], nlo);
-  else
-    hipLaunchKernelGGL((k_dif_km<3, true>), g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK,
-                       c->jq12, c->jq13, c->jq23, cs, c->ju[0], c->ju[1], c->ju[2], nlo);
+  auto kern = c->thermal ? (c->plane ? k_dif_km<4, true, kGeoPlane> : k_dif_km<4, true>)
+                         : (c->plane ? k_dif_km<3, true, kGeoPlane> : k_dif_km<3, true>);
+  hipLaunchKernelGGL(kern, g, kBlk, 0, c->stream, c->d, kc, c->pdI, c->pdJ, c->pdK, c->jq12,
+                     c->jq13, c->jq23, cs, c->ju[0], c->ju[1], c->ju[2], nlo, c->jq33, c->geo);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -893,11 +1017,13 @@ int fvm_k_p_source(FvmCtx* c) {
   const Dims d = c->d;
   const int kc = march_planes(d, PS_RES);
   const dim3 g = march_grid(d, kc);
-  auto kern = c->xz_zero ? k_psource_km<0, true> : k_psource_km<0, false>;
+  auto kern = c->plane
+                  ? k_psource_km<0, kGeoPlane>
+                  : (c->xz_zero ? k_psource_km<0, kGeoXz0> : k_psource_km<0, kGeoAny>);
   hipLaunchKernelGGL(kern, dim3(g.x * g.y * g.z), kBlk, 0, c->stream, c->d, kc,
                      make_uint3(g.x, g.y, g.z), (const double* const*)m, c->djac, c->p, 0.0,
                      c->s[0], c->s[1], c->s[2], nullptr, nullptr, nullptr, nullptr, nullptr,
-                     nullptr);
+                     nullptr, c->geo);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -1162,11 +1288,12 @@ int fvm_k_project(FvmCtx* c) {
   const long nb = (long)g.x * g.y * g.z;
   if (nb > c->ncflpart) return FVM_ERR_SIZE;
   c->ncflused = (int)nb;
-  auto kern = c->xz_zero ? k_psource_km<1, true> : k_psource_km<1, false>;
+  auto kern = c->plane ? k_psource_km<1, kGeoPlane>
+                       : (c->xz_zero ? k_psource_km<1, kGeoXz0> : k_psource_km<1, kGeoAny>);
   hipLaunchKernelGGL(kern, dim3((unsigned)nb + (c->two_d ? 0 : 1)), kBlk, 0, c->stream, c->d, kc,
                      make_uint3(g.x, g.y, g.z), (const double* const*)c->dm, c->djac, c->p,
                      c->prm.dtime, c->s[0], c->s[1], c->s[2], c->u, c->v, c->w, c->ufar,
-                     c->cflpart, c->scal + 2);
+                     c->cflpart, c->scal + 2, c->geo);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -1177,9 +1304,11 @@ int fvm_k_correct_bcu_contra(FvmCtx* c) {
   ProfScope ps(c, "correct_contra");
   const Vec3P s = {{c->s[0], c->s[1], c->s[2]}}, f = {{c->u, c->v, c->w}},
               ju = {{c->ju[0], c->ju[1], c->ju[2]}};
-  auto kern = c->xz_zero ? k_correct_contra<true> : k_correct_contra<false>;
-  hipLaunchKernelGGL(kern, interior_grid(d), kBlk, 0, c->stream, d, (const double* const*)c->dm,
-                     c->djac, c->prm.dtime, s, f, ju, c->ufar);
+  auto kern = c->plane ? k_correct_contra<kGeoPlane>
+                       : (c->xz_zero ? k_correct_contra<kGeoXz0> : k_correct_contra<kGeoAny>);
+  const dim3 g = march_grid(d, c->plane ? CC_KP : 1);
+  hipLaunchKernelGGL(kern, g, kBlk, 0, c->stream, d, (const double* const*)c->dm,
+                     c->djac, c->prm.dtime, s, f, ju, c->ufar, c->geo);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -1190,10 +1319,12 @@ int fvm_k_step_begin(FvmCtx* c) {
   ProfScope ps(c, "step_begin");
   const StepStart a = {{c->u, c->v, c->w, c->t}, {c->un, c->vn, c->wn, c->tn},
                        {c->ju[0], c->ju[1], c->ju[2]}, c->ufar, c->thermal ? c->tfar : nullptr};
-  const dim3 g((d.ni + 1 + 63) / 64, (d.nj + 1 + 3) / 4, d.nk + 1);
-  auto kern = c->xz_zero ? k_step_begin<true> : k_step_begin<false>;
+  const int kp = c->plane ? SB_KP : 1;
+  const dim3 g((d.ni + 1 + 63) / 64, (d.nj + 1 + 3) / 4, (d.nk + 1 + kp - 1) / kp);
+  auto kern = c->plane ? k_step_begin<kGeoPlane>
+                       : (c->xz_zero ? k_step_begin<kGeoXz0> : k_step_begin<kGeoAny>);
   hipLaunchKernelGGL(kern, g, kBlk, 0, c->stream, d, (const double* const*)c->dm, c->djac,
-                     c->theta, a, c->prm.dtime, c->pi);
+                     c->theta, a, c->prm.dtime, c->pi, c->geo);
   HIP_CHECK(hipGetLastError());
   c->u_is_un = true;
   c->ufar_stale = false;

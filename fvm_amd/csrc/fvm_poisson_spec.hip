@@ -37,7 +37,7 @@ const dim3 kBlk(64, 4, 1);
 // One pair of partial sums per workgroup.
 constexpr int RS_RES = 768;  // workgroups resident at a time (three per CU)
 
-template <typename T>
+template <typename T, int G>
 __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __restrict__ p,
                                                      const double* __restrict__ rhs,
                                                      const double* __restrict__ pdI,
@@ -46,7 +46,9 @@ __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __res
                                                      const double* __restrict__ jq12,
                                                      const double* __restrict__ jq13,
                                                      const double* __restrict__ jq23,
-                                                     T* __restrict__ R, double* part, int kc) {
+                                                     T* __restrict__ R, double* part, int kc,
+                                                     const double* __restrict__ jq33,
+                                                     PlaneGeo geo) {
   const uint3 bb = xcd_block();
   __shared__ double sh[3][SF_P];
   __shared__ double s0[256], s1[256];
@@ -61,6 +63,11 @@ __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __res
   // own-column values of planes kp-2, kp-1, kp
   double z13[3] = {0.0, 0.0, 0.0}, z23[3] = {0.0, 0.0, 0.0}, zk[3] = {0.0, 0.0, 0.0};
   double ra = 0.0, rb = 0.0;
+  // plane form: the coefficients are those of plane kz[k] (which the caches hold), J^-1 Q33 of the
+  // planes kp-2, kp-1, kp takes pdK's place (pdK is the mean of two), and only the lanes next to
+  // the I boundaries have J^-1 Q13, J^-1 Q23 terms
+  constexpr bool PL = G == kGeoPlane;
+  const bool ed = geo_edge(d, i), ed1 = geo_edge(d, i, 1);
   // the next plane's tile values and own-column values, loaded one plane ahead
   constexpr int NQ = (SF_P + 255) / 256;
   double pv[NQ], n13 = 0.0, n23 = 0.0, nk = 0.0;
@@ -73,9 +80,13 @@ __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __res
       pv[h] = p[cidx(d, gi, gj, kp)];
     }
     const long cp = cidx(d, act ? i : 1, act ? j : 1, kp);
-    n13 = jq13[cp];
-    n23 = jq23[cp];
-    nk = pdK[cp];
+    if (PL) {
+      nk = jq33[cidx(d, act ? i : 1, act ? j : 1, geo.plane(kp))];
+    } else {
+      n13 = jq13[cp];
+      n23 = jq23[cp];
+      nk = pdK[cp];
+    }
   };
   load(k0 - 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
@@ -96,25 +107,45 @@ __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __res
     const int pl[3] = {(slot + 1) % 3, (slot + 2) % 3, slot};
 #define P(dk, dj, di) sh[pl[(dk) + 1]][q0 + (dj) * SF_W + (di)]
     const long c = cidx(d, i, j, k);
-    const double de = pdI[c], dw = pdI[c - 1], dn = pdJ[c], ds = pdJ[c - sj], dt = zk[1],
-                 db = zk[0];
+    double dt = zk[1], db = zk[0], e13 = 0.0, w13 = 0.0, n23 = 0.0, s23 = 0.0;
+    ColStencil cs;
+    if (PL) {
+      cs.load(pdI, pdJ, jq12, sj, cidx(d, i, j, geo.plane(k)));
+      dt = 0.5 * (zk[1] + zk[2]);
+      db = 0.5 * (zk[0] + zk[1]);
+      if (ed1) { e13 = jq13[c + 1]; w13 = jq13[c - 1]; }
+      if (ed) {
+        n23 = jq23[c + sj]; s23 = jq23[c - sj];
+        z13[0] = jq13[c - d.sk]; z13[2] = jq13[c + d.sk];
+        z23[0] = jq23[c - d.sk]; z23[2] = jq23[c + d.sk];
+      }
+    } else {
+      cs.load(pdI, pdJ, jq12, sj, c);
+      e13 = jq13[c + 1]; w13 = jq13[c - 1]; n23 = jq23[c + sj]; s23 = jq23[c - sj];
+    }
+    const double de = cs.de, dw = cs.dw, dn = cs.dn, ds = cs.ds;
+    const double e12 = cs.e12, w12 = cs.w12, n12 = cs.n12, s12 = cs.s12;
     double ap = -de - dw - dn - ds - dt - db;
     double ae = -de, aw = -dw, an = -dn, as = -ds, at = -dt, ab = -db;
     if (i == 1) { ap = ap - aw; aw = 0.0; }
     if (i == d.ni - 1) ae = 0.0;
     // the cross terms DD
-    double x = jq12[c + 1] * (P(0, 1, 1) - P(0, -1, 1));
-    x = x - jq12[c - 1] * (P(0, 1, -1) - P(0, -1, -1));
-    x = x + jq13[c + 1] * (P(1, 0, 1) - P(-1, 0, 1));
-    x = x - jq13[c - 1] * (P(1, 0, -1) - P(-1, 0, -1));
-    x = x + jq12[c + sj] * (P(0, 1, 1) - P(0, 1, -1));
-    x = x - jq12[c - sj] * (P(0, -1, 1) - P(0, -1, -1));
-    x = x + jq23[c + sj] * (P(1, 1, 0) - P(-1, 1, 0));
-    x = x - jq23[c - sj] * (P(1, -1, 0) - P(-1, -1, 0));
-    x = x + z13[2] * (P(1, 0, 1) - P(1, 0, -1));
-    x = x - z13[0] * (P(-1, 0, 1) - P(-1, 0, -1));
-    x = x + z23[2] * (P(1, 1, 0) - P(1, -1, 0));
-    x = x - z23[0] * (P(-1, 1, 0) - P(-1, -1, 0));
+    double x = e12 * (P(0, 1, 1) - P(0, -1, 1));
+    x = x - w12 * (P(0, 1, -1) - P(0, -1, -1));
+    if (!PL || ed1) {
+      x = x + e13 * (P(1, 0, 1) - P(-1, 0, 1));
+      x = x - w13 * (P(1, 0, -1) - P(-1, 0, -1));
+    }
+    x = x + n12 * (P(0, 1, 1) - P(0, 1, -1));
+    x = x - s12 * (P(0, -1, 1) - P(0, -1, -1));
+    if (!PL || ed) {
+      x = x + n23 * (P(1, 1, 0) - P(-1, 1, 0));
+      x = x - s23 * (P(1, -1, 0) - P(-1, -1, 0));
+      x = x + z13[2] * (P(1, 0, 1) - P(1, 0, -1));
+      x = x - z13[0] * (P(-1, 0, 1) - P(-1, 0, -1));
+      x = x + z23[2] * (P(1, 1, 0) - P(1, -1, 0));
+      x = x - z23[0] * (P(-1, 1, 0) - P(-1, -1, 0));
+    }
     const double su = rhs[c] - 0.25 * x;
     const double pc = P(0, 0, 0);
     const double r = ae * P(0, 0, 1) + aw * P(0, 0, -1) + an * P(0, 1, 0) + as * P(0, -1, 0) +
@@ -615,6 +646,8 @@ int fvm_k_iter_p_sep(FvmCtx* c, bool mixed, double* resip, int* niter) {
   const Dims d = c->d;
   const int kc = march_planes(d, RS_RES);
   const dim3 g = march_grid(d, kc);
+  auto r32 = c->plane ? k_residual_km<float, kGeoPlane> : k_residual_km<float, kGeoAny>;
+  auto r64 = c->plane ? k_residual_km<double, kGeoPlane> : k_residual_km<double, kGeoAny>;
   long nb = (long)g.x * g.y * g.z;
   int outer = 0;
   double res = INFINITY, res_prev = INFINITY;
@@ -628,11 +661,11 @@ int fvm_k_iter_p_sep(FvmCtx* c, bool mixed, double* resip, int* niter) {
       ProfScope ps(c, "p_residual");
       ProfScope pk(c, "k_residual");
       if (use32)
-        hipLaunchKernelGGL(k_residual_km<float>, g, kBlk, 0, c->stream, d, c->p, c->rhs,
-                           c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d32.R, c->red, kc);
+        hipLaunchKernelGGL(r32, g, kBlk, 0, c->stream, d, c->p, c->rhs,
+                           c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d32.R, c->red, kc, c->jq33, c->geo);
       else
-        hipLaunchKernelGGL(k_residual_km<double>, g, kBlk, 0, c->stream, d, c->p, c->rhs,
-                           c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d64.R, c->red, kc);
+        hipLaunchKernelGGL(r64, g, kBlk, 0, c->stream, d, c->p, c->rhs,
+                           c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d64.R, c->red, kc, c->jq33, c->geo);
       mb = (outer > 0 || cap < 1) ? fvm_mail(c) : Mailbox{nullptr, nullptr, 0};
       hipLaunchKernelGGL(k_res_final, dim3(1), dim3(256), 0, c->stream, c->red, nb, c->scal + 4,
                          mb);
@@ -653,8 +686,8 @@ int fvm_k_iter_p_sep(FvmCtx* c, bool mixed, double* resip, int* niter) {
     if (use32 && outer > 0 && !(res < 0.5 * res_prev)) {
       // the FP32 approximate inverse stopped contracting: finish with the FP64 inverse
       use32 = false;
-      hipLaunchKernelGGL(k_residual_km<double>, g, kBlk, 0, c->stream, d, c->p, c->rhs,
-                         c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d64.R, c->red, kc);
+      hipLaunchKernelGGL(r64, g, kBlk, 0, c->stream, d, c->p, c->rhs,
+                         c->pdI, c->pdJ, c->pdK, c->jq12, c->jq13, c->jq23, S->d64.R, c->red, kc, c->jq33, c->geo);
       HIP_CHECK(hipGetLastError());
       ++c->sep_fallbacks;
     }

@@ -10,6 +10,7 @@
 #include "fvm_ctx.h"
 
 #include <algorithm>
+#include <vector>
 
 namespace {
 
@@ -275,6 +276,69 @@ __global__ void k_face(Dims d, const double* __restrict__ djac, const double* __
   }
 }
 
+// Grids from this size on take the plane form: an array of them exceeds the 4 MB L2 of an XCD.  On
+// smaller ones the arrays come from the caches and the operations of CellGeo only add latency: on
+// 96 x 128 x 16 cells the step's first kernel took 15.4 us in the plane form and 12.3 with the
+// arrays, convection and diffusion 14.3 and 14.8, whole steps the same; 40 steps on 149 x 208 x 40
+// took 43.7 ms in the plane form and 47.6.
+constexpr long kPlaneCells = 1L << 19;
+
+// The cross-section derivatives of every column, taken on plane 1, and z_zeta of every plane.
+__global__ void k_plane_geo(Dims d, const double* __restrict__ xxi, const double* __restrict__ yxi,
+                            const double* __restrict__ xet, const double* __restrict__ yet,
+                            const double* __restrict__ zzt, double* d2, double* zz) {
+  const int np = d.nk + 1;
+  for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < d.sk;
+       q += (long)gridDim.x * blockDim.x) {
+    d2[q] = xxi[q + d.sk]; d2[q + d.sk] = yxi[q + d.sk];
+    d2[q + 2 * d.sk] = xet[q + d.sk]; d2[q + 3 * d.sk] = yet[q + d.sk];
+    if (q < np) {
+      zz[q] = zzt[cidx(d, 1, 1, (int)q)];
+      zz[np + q] = zzt[cidx(d, 0, 1, (int)q)];
+      zz[2 * np + q] = zzt[cidx(d, d.ni, 1, (int)q)];
+    }
+  }
+}
+
+// *bad = 1 where what CellGeo forms differs from the stored geometry, or the squared filter width
+// from that of plane kz[k].  NaN (0/0 on a corner no kernel reads) counts as equal to NaN.
+__global__ void k_plane_check(Dims d, PlaneGeo g, const double* const* __restrict__ m,
+                              const double* __restrict__ djac, const double* __restrict__ jq11,
+                              const double* __restrict__ jq12, const double* __restrict__ jq22,
+                              const double* __restrict__ jq33, const double* __restrict__ filt2,
+                              int* bad) {
+  bool diff = false;
+  auto cmp = [&](double a, double b) { diff |= !(a == b) && !(a != a && b != b); };
+  for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < d.n;
+       q += (long)gridDim.x * blockDim.x) {
+    const long c2 = q % d.sk;
+    const int k = (int)(q / d.sk), j = (int)(c2 / d.sj), i = (int)(c2 % d.sj);
+    ColDer cd;
+    cd.load(d, g, i, j);
+    CellGeo e;
+    const int np = d.nk + 1;
+    e.form(cd, g.zz[i == 0 ? np + k : (i == d.ni ? 2 * np + k : k)]);
+    cmp(e.j, djac[q]);
+    cmp(e.xix, m[0][q]); cmp(e.etx, m[1][q]);
+    cmp(e.xiy, m[3][q]); cmp(e.ety, m[4][q]);
+    cmp(e.ztz, m[8][q]);
+    cmp(e.jq11(), jq11[q]); cmp(e.jq12(), jq12[q]);
+    cmp(e.jq22(), jq22[q]); cmp(e.jq33(), jq33[q]);
+    cmp(filt2[q], filt2[c2 + d.sk * g.kz[k]]);
+  }
+  if (diff) *bad = 1;
+}
+
+// *bad = 1 where one of the arrays is not zero, but for the columns of geo_edge if edge
+__global__ void k_zero_check(Dims d, PtrSet8 a, bool edge, int* bad) {
+  bool diff = false;
+  const double* __restrict__ p = a.p[blockIdx.y];
+  for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < d.n;
+       q += (long)gridDim.x * blockDim.x)
+    diff |= !(p[q] == 0.0) && !(edge && geo_edge(d, (int)(q % d.sj)));
+  if (diff) *bad = 1;
+}
+
 // wall triangles of every wall cell (init.f90:239-259, calccoef.f90:88-162): plane
 // coefficients A, B, C, D-offset distance d_n, |n| and area, two triangles per (j, k)
 __global__ void k_wall(Dims d, const double* __restrict__ xg, const double* __restrict__ yg,
@@ -418,19 +482,74 @@ int fvm_geom_setup(FvmCtx* c) {
   hipLaunchKernelGGL(k_wall, grid1(2L * (d.nj - 1) * (d.nk - 1), 256), B, 0, st, d, c->xg, c->yg,
                      c->zg, c->x, c->y, c->z, c->wall);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipStreamSynchronize(st));
+  if (d.n >= kPlaneCells) {  // tables of the plane form
+    const long np = d.nk + 1, nd = 4 * d.sk + 3 * np;
+    double* t = nullptr;
+    HIP_CHECK(hipMalloc((void**)&t, nd * sizeof(double) + np * sizeof(int)));
+    c->allocs.push_back(t);
+    c->geo.d2 = t;
+    c->geo.zz = t + 4 * d.sk;
+    c->geo.kz = reinterpret_cast<int*>(t + nd);
+    hipLaunchKernelGGL(k_plane_geo, grid1(d.sk, 256), B, 0, st, d, D[0], D[3], D[1], D[4], D[8], t,
+                       t + 4 * d.sk);
+  }
+  {  // xi_z and eta_z identically zero (z independent of xi and eta: an extruded grid)
+    int* bad = reinterpret_cast<int*>(c->red);
+    HIP_CHECK(hipMemsetAsync(bad, 0, sizeof(int), st));
+    PtrSet8 z{};
+    z.p[0] = c->m[6];
+    z.p[1] = c->m[7];
+    hipLaunchKernelGGL(k_zero_check, dim3(G.x, 2), B, 0, st, d, z, false, bad);
+    HIP_CHECK(hipGetLastError());
+    int h = 1;
+    HIP_CHECK(hipMemcpyAsync(&h, bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipStreamSynchronize(st));
+    c->xz_zero = h == 0;
+  }
   for (int a = 0; a < 9; ++a) HIP_CHECK(hipFree(D[a]));
   HIP_CHECK(hipFree(dD));
   HIP_CHECK(hipFree(dM));
-  {  // xi_z and eta_z identically zero (z independent of xi and eta: an extruded grid)
-    std::vector<double> h(d.n);
-    bool z = true;
-    for (int a = 6; a < 8 && z; ++a) {
-      HIP_CHECK(hipMemcpy(h.data(), c->m[a], d.n * sizeof(double), hipMemcpyDeviceToHost));
-      for (long q = 0; q < d.n && z; ++q) z = (h[q] == 0.0);
-    }
-    c->xz_zero = z;
+  return FVM_OK;
+}
+
+// Whether kGeoPlane's conditions hold, on the arrays themselves: nothing about the nodes is assumed.
+// Runs after the products of the AF stages' cross terms are formed.
+int fvm_plane_setup(FvmCtx* c) {
+  const Dims d = c->d;
+  hipStream_t st = c->stream;
+  if (!c->xz_zero || d.n < kPlaneCells) return FVM_OK;
+  const int np = d.nk + 1;
+  std::vector<double> zz(3 * np);
+  std::vector<int> kz(np);
+  HIP_CHECK(hipMemcpy(zz.data(), c->geo.zz, 3 * np * sizeof(double), hipMemcpyDeviceToHost));
+  for (int k = 0; k < np; ++k) {
+    int r = 0;
+    while (r < k && !(zz[r] == zz[k] && zz[np + r] == zz[np + k] &&
+                      zz[2 * np + r] == zz[2 * np + k]))
+      ++r;
+    kz[k] = r;
   }
+  HIP_CHECK(hipMemcpy(const_cast<int*>(c->geo.kz), kz.data(), np * sizeof(int),
+                      hipMemcpyHostToDevice));
+  int* bad = reinterpret_cast<int*>(c->red);
+  HIP_CHECK(hipMemsetAsync(bad, 0, sizeof(int), st));
+  hipLaunchKernelGGL(k_plane_check, grid1(d.n, 256), dim3(256), 0, st, d, c->geo,
+                     (const double* const*)c->dm, c->djac, c->jq11, c->jq12, c->jq22, c->jq33,
+                     c->filt2, bad);
+  PtrSet8 z{};
+  double* g[] = {c->m[2], c->m[5], c->jq13, c->jq23};
+  std::copy(g, g + 4, z.p);
+  hipLaunchKernelGGL(k_zero_check, dim3(grid1(d.n, 256).x, 4), dim3(256), 0, st, d, z, true, bad);
+  for (int s = 0; s < 2; ++s) {
+    double* p[] = {c->afp[s][1], c->afp[s][3], c->afp[s][4], c->afp[s][5], c->fa[s][2]};
+    std::copy(p, p + 5, z.p);
+    hipLaunchKernelGGL(k_zero_check, dim3(grid1(d.n, 256).x, 5), dim3(256), 0, st, d, z, true, bad);
+  }
+  HIP_CHECK(hipGetLastError());
+  int h = 1;
+  HIP_CHECK(hipMemcpyAsync(&h, bad, sizeof(int), hipMemcpyDeviceToHost, st));
+  HIP_CHECK(hipStreamSynchronize(st));
+  c->plane = h == 0;
   return FVM_OK;
 }
 

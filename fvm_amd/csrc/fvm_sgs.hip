@@ -23,13 +23,12 @@ struct Diff3 {
 };
 
 // The cell (i, j, k) = c writes its values' J and K ghost images as well.
-template <bool XZ0>
-__device__ inline void strain_store(const Dims& d, const double* const* __restrict__ m, int i,
-                                    int j, int k, long c, bool onesided, Diff3 u, Diff3 v,
-                                    Diff3 w, double* const* __restrict__ L, double* mag) {
-  const double xix = m[0][c], etx = m[1][c], ztx = m[2][c];
-  const double xiy = m[3][c], ety = m[4][c], zty = m[5][c];
-  const double xiz = XZ0 ? 0.0 : m[6][c], etz = XZ0 ? 0.0 : m[7][c], ztz = m[8][c];
+__device__ inline void strain_store(const Dims& d, const Met& m, int i, int j, int k, long c,
+                                    bool onesided, Diff3 u, Diff3 v, Diff3 w,
+                                    double* const* __restrict__ L, double* mag) {
+  const double xix = m.v[0], etx = m.v[1], ztx = m.v[2];
+  const double xiy = m.v[3], ety = m.v[4], zty = m.v[5];
+  const double xiz = m.v[6], etz = m.v[7], ztz = m.v[8];
   double l11, l12, l13, l22, l23, l33;
   if (!onesided) {
     double t;
@@ -95,8 +94,8 @@ __device__ inline void strain_iplane(const Dims& d, const double* const* __restr
     q.k = F[c + sk] - F[c - sk];
     return q;
   };
-  strain_store<false>(d, m, i, j, k, c, true, diff(io.in[0]), diff(io.in[1]), diff(io.in[2]), L,
-                      mag);
+  strain_store(d, load_met<kGeoAny>(m, c), i, j, k, c, true, diff(io.in[0]), diff(io.in[1]),
+               diff(io.in[2]), L, mag);
   if (NF == 4) {  // one-sided temperature gradient (stress_tensor_dy.f90:138-146, 188-196)
     const Diff3 g = diff(io.in[3]);
 #pragma unroll
@@ -123,11 +122,12 @@ __device__ inline void strain_iplane(const Dims& d, const double* const* __restr
 // launches it replaces took 20 + 9 + 7 us on 192 x 256 x 64 cells.
 constexpr int SF_RES = 768;  // workgroups resident at a time (three per CU)
 
-template <int NF, bool XZ0>
+template <int NF, int G>
 __global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc, uint3 tg,
                                                        const double* const* __restrict__ m,
                                                        SfOut io, double* const* __restrict__ L,
-                                                       double* mag) {
+                                                       double* mag,
+                                                       PlaneGeo geo) {
   const unsigned nb = tg.x * tg.y * tg.z;
   if (blockIdx.x >= nb) {
     const long t = (long)(blockIdx.x - nb) * 256 + threadIdx.y * 64 + threadIdx.x;
@@ -143,6 +143,10 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc, uint3 tg,
   const int k1 = min(k0 + kc - 1, d.nk - 1);
   const bool act = i <= d.ni - 1 && j <= d.nj - 1;
   const int q0 = (ty + 1) * SF_W + tx + 1;
+  Met mv{};
+  ColDer cd{};
+  CellGeo ce;
+  if (G == kGeoPlane) cd.load(d, geo, act ? i : 1, act ? j : 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
     const int slot = (kp - (k0 - 1)) % 3;
     __syncthreads();  // plane kp - 3, held in this slot, is no longer read
@@ -166,15 +170,20 @@ __global__ void __launch_bounds__(256) k_strain_filter(Dims d, int kc, uint3 tg,
       g[f].j = sh[f][s0][q0 + SF_W] - sh[f][s0][q0 - SF_W];
       g[f].k = sh[f][sp][q0] - sh[f][sm][q0];
     }
-    strain_store<XZ0>(d, m, i, j, k, c, false, g[0], g[1], g[2], L, mag);
-    if (NF == 4) {
+    if (G == kGeoPlane) {
+      ce.form(cd, geo.z(k));
+      mv = plane_met(d, m, ce, i, j, k);
+    } else {
+      mv = load_met<G>(m, c);
+    }
+    strain_store(d, mv, i, j, k, c, false, g[0], g[1], g[2], L, mag);
+    if constexpr (NF == 4) {
       const double ti = sh[3][s0][q0 + 1] - sh[3][s0][q0 - 1];
       const double tj = sh[3][s0][q0 + SF_W] - sh[3][s0][q0 - SF_W];
       const double tk = sh[3][sp][q0] - sh[3][sm][q0];
       const double t[3] = {
-          gp(m[0])[c] * ti + gp(m[1])[c] * tj + gp(m[2])[c] * tk,
-          gp(m[3])[c] * ti + gp(m[4])[c] * tj + gp(m[5])[c] * tk,
-          mget<XZ0>(m, 6, c) * ti + mget<XZ0>(m, 7, c) * tj + gp(m[8])[c] * tk};
+          mv.v[0] * ti + mv.v[1] * tj + mv.v[2] * tk, mv.v[3] * ti + mv.v[4] * tj + mv.v[5] * tk,
+          mv.v[6] * ti + mv.v[7] * tj + mv.v[8] * tk};
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         gpw(io.dt[q])[c] = 0.5 * t[q];
@@ -225,7 +234,7 @@ constexpr int SD_RES = 768;  // the same for the K-marching SGS divergences (thr
 constexpr int LM_W = 66, LM_H = 6;  // tile with halo
 constexpr int LM_NQ = (LM_W * LM_H + 255) / 256;  // tile cells staged per thread
 
-template <bool XZ0>
+template <int G>
 __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __restrict__ m,
                                             const double* __restrict__ U,
                                             const double* __restrict__ V,
@@ -235,7 +244,8 @@ __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __re
                                             const double* __restrict__ WH,
                                             const double* const* __restrict__ L,
                                             const double* __restrict__ filt2, double* part,
-                                            double* magh_out, int kc) {
+                                            double* magh_out, int kc,
+                                            PlaneGeo geo) {
   const uint3 bb = xcd_block();
   __shared__ double sh[10][LM_W * LM_H];
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
@@ -266,6 +276,11 @@ __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __re
   double X[12], Y[12];
 #pragma unroll
   for (int q = 0; q < 12; ++q) X[q] = Y[q] = 0.0;
+  Met mv{};
+  double fw2 = 0.0;
+  ColDer cd{};
+  CellGeo ce;
+  if (G == kGeoPlane) cd.load(d, geo, act ? i : 1, act ? j : 1);
   // this thread's sums of LM, MM and the cell count over the cells with 0.5 LM/MM >= 0
   double sa = 0.0, sb = 0.0, sn = 0.0;
   load_tile(k0 - 1);
@@ -291,9 +306,18 @@ __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __re
     // operands of the cell finished in this iteration, (i, j, kp - 1)
     const bool fin = kp >= k0 + 1 && act;
     const long c = fin ? cidx(d, i, j, kp - 1) : cidx(d, 1, 1, 1);
-    const double xix = gp(m[0])[c], etx = gp(m[1])[c], ztx = gp(m[2])[c];
-    const double xiy = gp(m[3])[c], ety = gp(m[4])[c], zty = gp(m[5])[c];
-    const double xiz = mget<XZ0>(m, 6, c), etz = mget<XZ0>(m, 7, c), ztz = gp(m[8])[c];
+    if (G == kGeoPlane) {
+      const int im = act ? i : 1, jm = act ? j : 1, km = kp >= k0 + 1 ? kp - 1 : k0;
+      ce.form(cd, geo.z(km));
+      mv = plane_met(d, m, ce, im, jm, km);
+      fw2 = gp(filt2)[cidx(d, im, jm, geo.plane(km))];
+    } else {
+      mv = load_met<G>(m, c);
+      fw2 = gp(filt2)[c];
+    }
+    const double xix = mv.v[0], etx = mv.v[1], ztx = mv.v[2];
+    const double xiy = mv.v[3], ety = mv.v[4], zty = mv.v[5];
+    const double xiz = mv.v[6], etz = mv.v[7], ztz = mv.v[8];
     double hs[3][6];  // u^, v^, w^ at i+1, i-1, j+1, j-1, k+1, k-1
     const double* hf[3] = {UH, VH, WH};
 #pragma unroll
@@ -304,7 +328,6 @@ __global__ void __launch_bounds__(256, 2) k_lm(Dims d, const double* const* __re
       hs[f][4] = h[c + sk]; hs[f][5] = h[c - sk];
     }
     const double uh = gp(UH)[c], vh = gp(VH)[c], wh = gp(WH)[c];
-    const double fw2 = gp(filt2)[c];
     double Pn[12];
 #pragma unroll
     for (int q = 0; q < 12; ++q) Pn[q] = 0.0;
@@ -622,14 +645,15 @@ __global__ void k_nut(Dims d, const double* __restrict__ cavg, const double* __r
 // slots (the I and J differences of plane k and the own-column value of plane k+1), and the
 // own-column products of plane k-1 are kept in registers.  Differences, products and sums are
 // the reference's, in its order.
-template <bool XZ0>
+template <int G>
 __global__ void __launch_bounds__(256) k_sgs_div(Dims d, int kc, const double* const* __restrict__ m,
                                                  const double* __restrict__ filt2,
                                                  const double* __restrict__ cavg,
                                                  const double* const* __restrict__ L,
                                                  const double* __restrict__ djac, double* nlx,
                                                  double* nly, double* nlz, double* sx, double* sy,
-                                                 double* sz, int mode) {
+                                                 double* sz, int mode,
+                                                 PlaneGeo geo) {
   const uint3 bb = xcd_block();
   __shared__ double sh[2][6][SF_P];  // [plane slot][product][tile cell]
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
@@ -649,19 +673,30 @@ __global__ void __launch_bounds__(256) k_sgs_div(Dims d, int kc, const double* c
   double Pm[6];  // own-column products of plane k-1
 #pragma unroll
   for (int q = 0; q < 6; ++q) Pm[q] = 0.0;
+  constexpr int NQ = (SF_P + 255) / 256;
+  Met mv{};
+  double J = 0.0;
+  ColDer cd{};
+  CellGeo ce;
+  if (G == kGeoPlane) cd.load(d, geo, act ? i : 1, act ? j : 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
     const int slot = (kp - (k0 - 1)) & 1;
+    const long dk2 = G == kGeoPlane ? d.sk * (geo.plane(kp) - kp) : 0;  // filt2 of plane kz[kp]
     __syncthreads();  // plane kp - 2, held in this slot, is no longer read
-    for (int e = tid; e < SF_P; e += 256) {
+#pragma unroll
+    for (int h = 0; h < NQ; ++h) {
+      const int e = tid + 256 * h;
+      if (e >= SF_P) continue;
       const int gi = min(bb.x * 64 + e % SF_W, d.ni);
       const int gj = min(bb.y * 4 + e / SF_W, d.nj);
       const long c = cidx(d, gi, gj, kp);
       const double l11 = S0[c], l12 = S1[c], l13 = S2[c], l22 = S3[c], l23 = S4[c], l33 = S5[c];
+      const double fw2 = filt2[c + dk2];
       // nu_t = C Delta^2 |S| as k_nut forms it, with |S| from the strain rates in
       // strain_store's order (the value it stored)
       const double s2 = l11 * l11 + l12 * l12 + l13 * l13 + l12 * l12 + l22 * l22 + l23 * l23 +
                         l13 * l13 + l23 * l23 + l33 * l33;
-      const double tn = 2.0 * (C * filt2[c] * sqrt(2.0 * s2));
+      const double tn = 2.0 * (C * fw2 * sqrt(2.0 * s2));
       sh[slot][0][e] = tn * l11;
       sh[slot][1][e] = tn * l12;
       sh[slot][2][e] = tn * l13;
@@ -680,11 +715,16 @@ __global__ void __launch_bounds__(256) k_sgs_div(Dims d, int kc, const double* c
     const int sc = slot ^ 1;
     const int k = kp - 1;
     const long c = cidx(d, i, j, k);
-    const double J = (mode & 1) ? djac[c] : 0.0;
     // the metrics and NL of the cell are loaded before its stores (which might alias them)
-    double mv[9], nv[3];
-#pragma unroll
-    for (int a = 0; a < 9; ++a) mv[a] = mget<XZ0>(m, a, c);
+    double nv[3];
+    if (G == kGeoPlane) {
+      ce.form(cd, geo.z(k));
+      mv = plane_met(d, m, ce, i, j, k);
+      J = ce.j;
+    } else {
+      J = (mode & 1) ? djac[c] : 0.0;
+      mv = load_met<G>(m, c);
+    }
 #pragma unroll
     for (int row = 0; row < 3; ++row) nv[row] = (mode & 1) ? nl[row][c] : 0.0;
 #pragma unroll
@@ -700,7 +740,7 @@ __global__ void __launch_bounds__(256) k_sgs_div(Dims d, int kc, const double* c
           else if (dir == 1) { pp = sh[sc][q][e0 + SF_W]; pn = sh[sc][q][e0 - SF_W]; }
           else { pp = sh[slot][q][e0]; pn = Pm[q]; }
           const double inner = -pp + pn;
-          const double term = mv[3 * col + dir] * inner;
+          const double term = mv.v[3 * col + dir] * inner;
           t = (col == 0 && dir == 0) ? term : t + term;
         }
       }
@@ -731,10 +771,11 @@ int fvm_k_sgs_out(FvmCtx* c) {
   const Dims d = c->d;
   const int kc = march_planes(d, SD_RES);
   const dim3 gs = march_grid(d, kc);
-  auto kern = c->xz_zero ? k_sgs_div<true> : k_sgs_div<false>;
+  auto kern = c->plane ? k_sgs_div<kGeoPlane>
+                        : (c->xz_zero ? k_sgs_div<kGeoXz0> : k_sgs_div<kGeoAny>);
   hipLaunchKernelGGL(kern, gs, kBlk, 0, c->stream, d, kc, (const double* const*)c->dm, c->filt2,
                      c->scal + 0, (const double* const*)c->dlss, c->djac, c->nl[0], c->nl[1],
-                     c->nl[2], c->sgs[0], c->sgs[1], c->sgs[2], 2);
+                     c->nl[2], c->sgs[0], c->sgs[1], c->sgs[2], 2, c->geo);
   HIP_CHECK(hipGetLastError());
   c->sgs_stale = false;
   return FVM_OK;
@@ -752,23 +793,25 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
     const dim3 g = march_grid(d, kc);
     const SfOut io = {{c->u, c->v, c->w, c->t}, {c->uh[0], c->uh[1], c->uh[2], c->that},
                       {c->dtd[0], c->dtd[1], c->dtd[2]}, c->ufar, c->tfar};
-    auto kern = th ? k_strain_filter<4, false>
-                   : (c->xz_zero ? k_strain_filter<3, true> : k_strain_filter<3, false>);
+    auto kern = th ? (c->plane ? k_strain_filter<4, kGeoPlane> : k_strain_filter<4, kGeoAny>)
+                   : (c->plane ? k_strain_filter<3, kGeoPlane>
+                               : (c->xz_zero ? k_strain_filter<3, kGeoXz0>
+                                             : k_strain_filter<3, kGeoAny>));
     const unsigned nb = g.x * g.y * g.z;
     const long ni = 2L * (d.nj - 1) * (d.nk - 1);  // cells of the two I ghost planes
     hipLaunchKernelGGL(kern, dim3(nb + (unsigned)((ni + 255) / 256)), kBlk, 0, st, d, kc,
                        make_uint3(g.x, g.y, g.z), (const double* const*)m, io,
-                       (double* const*)c->dlss, c->mag);
+                       (double* const*)c->dlss, c->mag, c->geo);
     HIP_CHECK(hipGetLastError());
   }
   {
     ProfScope pk(c, "k_lm");
     const int kc = march_planes(d, LM_RES);
     const dim3 gl = march_grid(d, kc);
-    auto kern = c->xz_zero ? k_lm<true> : k_lm<false>;
+    auto kern = c->plane ? k_lm<kGeoPlane> : (c->xz_zero ? k_lm<kGeoXz0> : k_lm<kGeoAny>);
     hipLaunchKernelGGL(kern, gl, kBlk, 0, st, d, (const double* const*)m, c->u, c->v, c->w,
                        c->uh[0], c->uh[1], c->uh[2], (const double* const*)c->dlss, c->filt2,
-                       c->red, th ? c->magh : nullptr, kc);
+                       c->red, th ? c->magh : nullptr, kc, c->geo);
     HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_lm_final, dim3(1), dim3(256), 0, st, c->red, (int)(gl.x * gl.y * gl.z),
                        c->scal + 0);
@@ -784,11 +827,12 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
     ProfScope pk(c, "k_sgs_div");
     const int kc = march_planes(d, SD_RES);
   const dim3 gs = march_grid(d, kc);
-    auto kern = c->xz_zero ? k_sgs_div<true> : k_sgs_div<false>;
+    auto kern = c->plane ? k_sgs_div<kGeoPlane>
+                        : (c->xz_zero ? k_sgs_div<kGeoXz0> : k_sgs_div<kGeoAny>);
     hipLaunchKernelGGL(kern, gs, kBlk, 0, st, d, kc, (const double* const*)m, c->filt2, c->scal + 0,
                        (const double* const*)c->dlss, c->djac, c->nl[0], c->nl[1], c->nl[2],
                        c->sgs[0], c->sgs[1], c->sgs[2],
-                       (nl_update ? 1 : 0) | (sgs_out ? 2 : 0));
+                       (nl_update ? 1 : 0) | (sgs_out ? 2 : 0), c->geo);
     HIP_CHECK(hipGetLastError());
     c->sgs_stale = !sgs_out;
   }
