@@ -94,11 +94,16 @@ struct Case2D {
   float* h[NH2];       // FP32 change form planes
   double* a[NA2];      // adjoint planes (null until the adjoint is initialised)
   double* ab[NAB2];
+  int* as0[2];         // line at which the transposed sweep of a chunk starts, per stage
 };
 
 // lines per chunk of the batched AF sweeps, and chunks of a sweep over nl lines
 constexpr int SW_C = 16;
 __host__ __device__ inline int sw_nchunk(int nl) { return (nl + SW_C - 1) / SW_C; }
+
+// lines per chunk of the transposed sweeps (the adjoint)
+constexpr int AS_C = 8;
+__host__ __device__ inline int as_nchunk(int nl) { return (nl + AS_C - 1) / AS_C; }
 
 // per-case device scalars
 enum ST {

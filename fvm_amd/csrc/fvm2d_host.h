@@ -20,6 +20,10 @@ struct AF2D {
   std::vector<double> nat[2], bt[2], ga2, gc2;
   std::vector<double> awwall[2], aefar[2];  // pre-fold AW(1, J), AE(NI-1, J) per stage
   std::vector<double> ae1;                  // stage-1 AE after the far-field fold
+  // per stage and line L the factor by which a change of the transposed sweep's line L + 1 reaches
+  // line L at most, in the norms sum_r s(r) |e(r)| with s(r) the row sums of T: the largest
+  // Cdn(r) / s(r) of line L + 1 (s^T T^-T = 1 for the M-matrix T)
+  std::vector<double> rho[2];
 };
 
 int geo2d_build(int ni, int nj, const double* xg, const double* yg, Geo2D& g);

@@ -11,6 +11,8 @@
 #include "fvm2d.h"
 #include "fvm2d_host.h"
 
+#include <algorithm>
+
 namespace {
 inline long ix(int sj, int i, int j) { return (long)i + (long)sj * j; }
 }
@@ -262,6 +264,14 @@ void geo2d_af(const Geo2D& g, double re, double dt, AF2D& a) {
     // transposed factors along the sweep lines (a = -AW or -AS, c = -AE or -AN)
     {
       const int nl = s == 0 ? nj - 1 : ni - 1, nr = s == 0 ? ni - 1 : nj - 1;
+      a.rho[s].assign(nl + 2, 0.0);
+      for (int L = 2; L <= nl; ++L)
+        for (int r = 1; r <= nr; ++r) {
+          const long c = s == 0 ? ix(sj, r, L) : ix(sj, L, r);
+          const double cdn = s == 0 ? AS[c] : AW[c];
+          const double sum = AP[c] - (s == 0 ? AW[c] + AE[c] : AS[c] + AN[c]);
+          a.rho[s][L - 1] = std::max(a.rho[s][L - 1], cdn / sum);
+        }
       for (int L = 1; L <= nl; ++L) {
         std::vector<double> av(nr + 2, 0.0), cv(nr + 2, 0.0), dv(nr + 2, 0.0);
         for (int r = 1; r <= nr; ++r) {
