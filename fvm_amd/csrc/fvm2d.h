@@ -35,6 +35,7 @@ enum F2 {
   F_U, F_V, F_P, F_NLX, F_NLY,
   // step work arrays
   F_UN, F_VN, F_DIFX, F_DIFY, F_SU, F_SV, F_SU1, F_SV1, F_RHS,
+  F_X1U, F_X1V,                // I-line sweep (FP64): its result and BCU's ghosts of its input
   F_TQU, F_TQV, F_TXU, F_TXV,  // J-line sweep: right-hand sides and iterates, J-line-major
   NF2
 };
@@ -94,7 +95,8 @@ struct Case2D {
   float* h[NH2];       // FP32 change form planes
   double* a[NA2];      // adjoint planes (null until the adjoint is initialised)
   double* ab[NAB2];
-  int* as0[2];         // line at which the transposed sweep of a chunk starts, per stage
+  int* lead[2];        // per stage and line: the line at which a sweep of it and those after it
+  int* as0[2];         // starts, and (transposed sweep) of it and those before it
 };
 
 // lines per chunk of the batched AF sweeps, and chunks of a sweep over nl lines

@@ -201,23 +201,33 @@ __device__ inline void bcu_ghosts_wave(P F, int ni, int nj, int sj, B uwall, B u
 // runs as two affine-map scans over the 64 lanes (lane l holds rows l R .. l R + R - 1,
 // R = ceil(rows / 64) of the case).
 //
-// Chunked form: the lines of a case are cut into chunks of SW_C consecutive lines and each
-// (case, component, chunk) is one wavefront; a chunk takes the line before it from the
-// preceding chunk's last line of the previous pass (block Jacobi across chunks, the stage input
-// in the first pass).  The passes are nilpotent (exact after as many passes as chunks) and each
-// contracts the chunk-boundary error by rho^SW_C, rho < 1 the ratio of the lagged coupling to
-// the diagonal dominance of the line operator; a pass after the first re-solves a chunk's lines
-// only until a line stops changing (max change <= tol max |x|), the rest keep their values.
-// The last pass books the largest relative change of a chunk's last line in the case's
-// ST_AFCH.  The operands of line L + 1 are loaded while line L is solved.
+// The lines of a case are cut into chunks and each (case, component, chunk) is one wavefront.  A line
+// passes a change of the line before it on by at most rho, the largest ratio of the lagged coupling
+// to the row sum of the line operator (T^-1 s = 1 for the M-matrix T with row sums s).
+//
+// FP64 (k2_sweep): a chunk starts its lead lines earlier, with nothing from the line before them:
+// by the product of their rho that is worth less than 1e-20 in the chunk (b2_af; up to line 1 where
+// the dominance is weak), so one pass gives every line the full sweep's result.  As block Jacobi
+// passes (below) with a launch before for the boundary lines, twelve FP64 cases of 0.5 M cells took
+// 13 + 22 + 2 x 12 us for the I lines and 35 + 2 x 22 for the J lines of a step; they take 30 and 37.
+// A line is bound by the latency of its loads and of the two scans: with one line loaded ahead and
+// rows loaded one by one it took 34 and 61.
+//
+// FP32 change form (k2_sweep_pass), resolved to FP32 rounding only: a chunk of SW_C lines takes the
+// line before it from the preceding chunk's last line of the previous pass (block Jacobi across
+// chunks, no change in the first pass).  Each pass contracts the chunk-boundary error by rho^SW_C;
+// a pass after the first re-solves a chunk's lines only until a line stops changing (max change
+// <= tol max |x|), the rest keep their values.  The last pass books the largest relative change of
+// a chunk's last line in the case's ST_AFCH.
+//
+// The operands of the next line are loaded while a line is solved.
 // DIR 0: I lines (rows along I, lines J = 1..NJ-1, lagged coupling AS = AN(J-1));
 // DIR 1: J lines (rows along J, lines I = 1..NI-1, lagged coupling AW); the line ends take the
 // ghost values (BCU of the stage input) as Dirichlet data.
 // ---------------------------------------------------------------------------------------------
-template <int R, typename T>
+template <int R>
 struct LineOps {
-  T cdn[R], q[R], iv[R], na[R], bf[R], xo[R];
-  T g0, g1;                                        // ghosts before / after the line
+  float cdn[R], q[R], iv[R], na[R], bf[R], xo[R];
 };
 
 // R consecutive floats from a 16-byte (R % 4 == 0) or 8-byte (R % 2 == 0) aligned address
@@ -241,13 +251,12 @@ __device__ __forceinline__ void load_rows(float (&d)[R], gptr<const float> p) {
 }
 
 // roff: the offset of row 0 in a line (the padded FP32 J-line-major layout)
-template <int R, int DIR, bool EARLY, typename T>
-__device__ inline void sweep_load(LineOps<R, T>& o, gptr<const T> F, gptr<const T> Q,
-                                  gptr<const T> invd, gptr<const T> na, gptr<const T> bf,
-                                  gptr<const T> cdn, long base, long rs, long roff, long dnoff,
-                                  int n, int r0, int l) {
-  constexpr bool DELTA = std::is_same<T, float>::value;
-  if constexpr (DELTA && DIR == 1 && R % 2 == 0) {
+template <int R, int DIR, bool EARLY>
+__device__ inline void sweep_load(LineOps<R>& o, gptr<const float> F, gptr<const float> Q,
+                                  gptr<const float> invd, gptr<const float> na,
+                                  gptr<const float> bf, gptr<const float> cdn, long base, long rs,
+                                  long roff, long dnoff, int n, int r0) {
+  if constexpr (DIR == 1 && R % 2 == 0) {
     // a lane's rows as vectors (row r at base + roff + 1 + r; dnoff = 0 in this direction).
     // The last lane's rows past n lie inside the padded plane and are never used.
     const long c0 = base + roff + 1 + r0;
@@ -259,7 +268,7 @@ __device__ inline void sweep_load(LineOps<R, T>& o, gptr<const T> F, gptr<const 
     if (EARLY) load_rows<R>(o.xo, F + c0);
     else {
 #pragma unroll
-      for (int q = 0; q < R; ++q) o.xo[q] = (T)0;
+      for (int q = 0; q < R; ++q) o.xo[q] = 0.0f;
     }
   } else {
 #pragma unroll
@@ -272,57 +281,40 @@ __device__ inline void sweep_load(LineOps<R, T>& o, gptr<const T> F, gptr<const 
         o.iv[q] = invd[c];
         o.na[q] = na[c];
         o.bf[q] = bf[c];
-        o.xo[q] = EARLY ? F[c] : (T)0;  // the previous pass's value of the row
+        o.xo[q] = EARLY ? F[c] : 0.0f;  // the previous pass's value of the row
       }
     }
   }
-  // the change form's ghosts do not change
-  o.g0 = !DELTA && l == 0 ? F[base] : (T)0;
-  o.g1 = !DELTA && l == 63 ? F[base + rs * (n + 1)] : (T)0;
 }
 
-// T = double: the sweep of the stage on the field itself (DIR 1 on the J-line-major copies: the
-// iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_rhs2 and returned by
-// k2_correct).  T = float: the change form.  The sweep solves T_L d_L = r_L + AS d_(L-1) for the
-// change d = x - x0 of the stage input x0, with r the FP64 residual of x0 (k2_explicit,
-// k2_rhs2), zero ghosts and a zero ghost line; the iterate is H_DU / H_DV (J-line-major for
-// DIR 1).  The I-line stage's last pass adds the change to the FP64 field, the J-line stage's
-// k2_correct does.  First pass: the line before a chunk is the stage input's (no change in the
-// change form; the field in the FP64 J stage, whose iterate is a copy; k2_sweep_seed's boundary
-// lines in the FP64 I stage, which overwrites the field).
-template <int R, int DIR, bool EARLY, typename T>
+// The change form: the sweep solves T_L d_L = r_L + AS d_(L-1) for the change d = x - x0 of the
+// stage input x0, with r the FP64 residual of x0 (k2_explicit, k2_rhs2), zero ghosts and a zero
+// ghost line; the iterate is H_DU / H_DV (J-line-major for DIR 1).  The I-line stage's last pass
+// adds the change to the FP64 field, the J-line stage's k2_correct does.  The line before a chunk
+// has no change in the first pass.
+template <int R, int DIR, bool EARLY>
 __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double tol, int final) {
-  constexpr bool DELTA = std::is_same<T, float>::value;
+  using T = float;
   const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  T *F0, *Q0, *iv0, *na0, *bf0, *cd0;
-  if constexpr (DELTA) {
-    F0 = cs.h[comp ? H_DV : H_DU];
-    Q0 = cs.h[DIR == 0 ? (comp ? H_RV : H_RU) : (comp ? H_TRV : H_TRU)];
-    iv0 = cs.h[DIR == 0 ? H_INVD1 : H_TINVD2];
-    na0 = cs.h[DIR == 0 ? H_NA1 : H_TNA2];
-    bf0 = cs.h[DIR == 0 ? H_B1 : H_TB2];
-    cd0 = cs.h[DIR == 0 ? H_AN1 : H_TAW2];
-  } else {
-    F0 = DIR == 0 ? cs.f[comp ? F_V : F_U] : cs.f[comp ? F_TXV : F_TXU];
-    Q0 = DIR == 0 ? cs.f[comp ? F_SV1 : F_SU1] : cs.f[comp ? F_TQV : F_TQU];
-    iv0 = cs.f[DIR == 0 ? G_INVD1 : G_TINVD2];
-    na0 = cs.f[DIR == 0 ? G_NA1 : G_TNA2];
-    bf0 = cs.f[DIR == 0 ? G_B1 : G_TB2];
-    cd0 = cs.f[DIR == 0 ? G_AN1 : G_TAW2];
-  }
+  T* const F0 = cs.h[comp ? H_DV : H_DU];
+  T* const Q0 = cs.h[DIR == 0 ? (comp ? H_RV : H_RU) : (comp ? H_TRV : H_TRU)];
+  T* const iv0 = cs.h[DIR == 0 ? H_INVD1 : H_TINVD2];
+  T* const na0 = cs.h[DIR == 0 ? H_NA1 : H_TNA2];
+  T* const bf0 = cs.h[DIR == 0 ? H_B1 : H_TB2];
+  T* const cd0 = cs.h[DIR == 0 ? H_AN1 : H_TAW2];
   // global-address-space views: global (not flat) loads, which do not wait on LDS and scalar
   // traffic, so the next line's loads stay in flight while this line is solved
   const gptr<T> F = glb(F0);
   const gptr<const T> Q = glb((const T*)Q0), invd = glb((const T*)iv0), na = glb((const T*)na0);
   const gptr<const T> bf = glb((const T*)bf0), cdn = glb((const T*)cd0);
   // the change form's I-line stage adds its last pass's change to the field
-  const bool add = DELTA && DIR == 0 && final;
+  const bool add = DIR == 0 && final;
   const gptr<double> F64 = glb(add ? cs.f[comp ? F_V : F_U] : nullptr);
   const int n = DIR == 0 ? ni - 1 : nj - 1;       // rows per line
   const int nl = DIR == 0 ? nj - 1 : ni - 1;      // lines
   const long rs = 1;                              // row stride
-  const long ls = DIR == 0 ? sj : (DELTA ? tls32(nj) : nj + 1);  // line stride
-  const long roff = DIR == 1 && DELTA ? J32_OFF : 0;  // row 0's offset in a line
+  const long ls = DIR == 0 ? sj : tls32(nj);  // line stride
+  const long roff = DIR == 1 ? J32_OFF : 0;  // row 0's offset in a line
   const long dnoff = DIR == 0 ? -(long)sj : 0;    // lower coupling of row c at cdn[c + dnoff]
   const int nch = sw_nchunk(nl);
   const int a0 = 1 + ca * SW_C, a1 = min(a0 + SW_C - 1, nl);
@@ -334,30 +326,20 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = r0 + q;
-    // the line before the chunk: the ghost line 0 (no change in the change form), or the
-    // preceding chunk's last line
+    // the line before the chunk: the ghost line 0 (no change), or the preceding chunk's last line
     T v = (T)0;
-    if (r < n && (EARLY || !DELTA)) {
-      if (ca == 0) {
-        if (!DELTA) v = F[rs * (r + 1)];
-      } else if (!EARLY && DIR == 1) {
-        v = (T)glb(cs.f[comp ? F_V : F_U])[(a0 - 1) + (long)sj * (r + 1)];
-      } else {
-        v = (T)bnd[bin + (long)(ca - 1) * n + r];
-      }
-    }
+    if (EARLY && r < n && ca > 0) v = (T)bnd[bin + (long)(ca - 1) * n + r];
     prev[q] = v;
   }
-  LineOps<R, T> cur, nxt;
-  sweep_load<R, DIR, EARLY>(cur, F, Q, invd, na, bf, cdn, ls * a0, rs, roff, dnoff, n, r0, l);
+  LineOps<R> cur, nxt;
+  sweep_load<R, DIR, EARLY>(cur, F, Q, invd, na, bf, cdn, ls * a0, rs, roff, dnoff, n, r0);
   bool stopped = false;
   T xrun = (T)0;
   int L = a0;
   for (; L <= a1; ++L) {
     const long base = ls * L;
     if (L < a1)
-      sweep_load<R, DIR, EARLY>(nxt, F, Q, invd, na, bf, cdn, base + ls, rs, roff, dnoff, n, r0,
-                                l);
+      sweep_load<R, DIR, EARLY>(nxt, F, Q, invd, na, bf, cdn, base + ls, rs, roff, dnoff, n, r0);
     T al[R], be[R], bb[R];
     T At = (T)0, Bt = (T)1;
 #pragma unroll
@@ -374,7 +356,7 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
       Bt = be[q] * Bt;
     }
     // lane l starts from the exclusive prefix applied to the ghost before the first row
-    T yin = wave::prefix_apply(At, Bt, wave::lane_value(cur.g0, 0));
+    T yin = wave::prefix_apply(At, Bt, (T)0);
     T y[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
@@ -390,7 +372,7 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
       }
     }
     // and from the exclusive suffix applied to the ghost after the last row
-    T xin = wave::suffix_apply(Dt, Ct, wave::lane_value(cur.g1, 63));
+    T xin = wave::suffix_apply(Dt, Ct, (T)0);
     T dl = (T)0;
 #pragma unroll
     for (int q = R - 1; q >= 0; --q) {
@@ -462,37 +444,180 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
   }
 }
 
-// The FP64 I stage's first chunk boundary lines (the stage input's last line of every chunk) and
-// BCU's ghosts of the stage input (by each (case, component)'s chunk-0 wavefront; the ghosts and
-// the interior lines copied here do not overlap); block table as the passes'.
-__global__ void __launch_bounds__(64) k2_sweep_seed(const Case2D* __restrict__ tab,
-                                                    const int* __restrict__ bcase,
-                                                    const int* __restrict__ btile) {
+// R consecutive doubles, the pairs among them by 16-byte loads (aligned to 8 bytes as the rows are):
+// a wavefront's lanes are R rows apart, so every load instruction touches 8 R bytes times 64 lanes of
+// cache lines and their number is what a line costs
+typedef double sw_d2 __attribute__((ext_vector_type(2), aligned(8)));
+template <int R>
+__device__ __forceinline__ void row_pairs(double (&d)[R], gptr<const double> p) {
+#pragma unroll
+  for (int k = 0; k < R / 2; ++k) {
+    const sw_d2 v = *(gptr<const sw_d2>)(p + 2 * k);
+    d[2 * k] = v.x; d[2 * k + 1] = v.y;
+  }
+  if constexpr (R % 2 == 1) d[R - 1] = p[R - 1];
+}
+
+// The FP64 sweep of chunk ca of nlc lines.  DIR 0: from the field (the stage input, left as it is)
+// and F_SU1 / F_SV1 to F_X1U / F_X1V, whose ghosts are BCU's of the stage input.  DIR 1: on the
+// J-line-major copies (iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_rhs2
+// and returned by k2_correct), whose line ends and line 0 hold BCU's ghosts.
+template <int R, int DIR>
+__device__ void sweep_lead(const Case2D& cs, int comp, int ca, int nlc) {
+  const int ni = cs.ni, nj = cs.nj;
+  const auto F = glb((const double*)cs.f[DIR == 0 ? (comp ? F_V : F_U) : (comp ? F_TXV : F_TXU)]);
+  const auto X = glb(cs.f[DIR == 0 ? (comp ? F_X1V : F_X1U) : (comp ? F_TXV : F_TXU)]);
+  const auto Q = glb((const double*)cs.f[DIR == 0 ? (comp ? F_SV1 : F_SU1) : (comp ? F_TQV : F_TQU)]);
+  const auto invd = glb((const double*)cs.f[DIR == 0 ? G_INVD1 : G_TINVD2]);
+  const auto na = glb((const double*)cs.f[DIR == 0 ? G_NA1 : G_TNA2]);
+  const auto bf = glb((const double*)cs.f[DIR == 0 ? G_B1 : G_TB2]);
+  const auto cdn = glb((const double*)cs.f[DIR == 0 ? G_AN1 : G_TAW2]);
+  const auto uwall = glb((const double*)cs.b[comp ? B_VWALL : B_UWALL]);
+  const auto ufar = glb((const double*)cs.b[comp ? B_VFAR : B_UFAR]);
+  const int n = DIR == 0 ? ni - 1 : nj - 1, nl = DIR == 0 ? nj - 1 : ni - 1;
+  const long ls = DIR == 0 ? cs.sj : nj + 1;
+  const long dnoff = DIR == 0 ? -ls : 0;  // lower coupling of row c at cdn[c + dnoff]
+  const int a0 = 1 + ca * nlc, a1 = min(a0 + nlc - 1, nl);
+  const int l = threadIdx.x, r0 = l * R;
+  if (DIR == 0 && ca == 0) {  // the ghost lines 0, NJ: periodic images of lines NJ-1, 1
+    for (int q = l; q < 2 * (ni + 1); q += 64) {
+      const int i = q >> 1, js = q & 1 ? 1 : nj - 1;
+      const long c = ls * js;
+      X[i + (q & 1 ? ls * nj : 0)] = i == 0 ? -F[c + 1] + 2.0 * uwall[js]
+                                            : (i == ni ? -F[c + n] + 2.0 * ufar[js] : F[c + i]);
+    }
+  }
+  struct Ops {
+    double cdn[R], q[R], iv[R], na[R], bf[R];
+    double g0, g1;  // DIR 0: the stage input's first and last row; DIR 1: the line ends' ghosts
+  };
+  auto load = [&](Ops& o, int L) {
+    const long base = ls * L;
+    // a lane's rows, as pairs; rows past n (up to R - 1 of them: the ghost and the next line) and
+    // the lanes past n are not used
+    const long c = base + (r0 < n ? r0 : 0) + 1;
+    row_pairs<R>(o.cdn, cdn + c + dnoff);
+    row_pairs<R>(o.q, Q + c);
+    row_pairs<R>(o.iv, invd + c);
+    row_pairs<R>(o.na, na + c);
+    row_pairs<R>(o.bf, bf + c);
+    o.g0 = F[base + (DIR == 0 ? 1 : 0)];
+    o.g1 = F[base + (DIR == 0 ? n : n + 1)];
+  };
+  const int Ls = cs.lead[DIR][a0];
+  double prev[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    prev[q] = Ls == 1 && r0 + q < n ? F[(DIR == 0 ? ls * (nj - 1) : 0) + r0 + q + 1] : 0.0;
+  auto solve = [&](const Ops& cur, int L) {
+    double al[R], be[R], bb[R];
+    double At = 0.0, Bt = 1.0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      if (r0 + q < n) {
+        al[q] = (cur.cdn[q] * prev[q] + cur.q[q]) * cur.iv[q];
+        be[q] = cur.na[q];
+        bb[q] = cur.bf[q];
+      } else {
+        al[q] = 0.0; be[q] = 1.0; bb[q] = 0.0;
+      }
+      At = al[q] + be[q] * At;
+      Bt = be[q] * Bt;
+    }
+    // lane l starts from the exclusive prefix applied to the ghost before the first row (an I
+    // line's is folded into its operator)
+    double yin = wave::prefix_apply(At, Bt, DIR == 0 ? 0.0 : cur.g0);
+    double y[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      y[q] = al[q] + be[q] * yin;
+      yin = y[q];
+    }
+    double Ct = 1.0, Dt = 0.0;
+#pragma unroll
+    for (int q = R - 1; q >= 0; --q) {
+      if (r0 + q < n) {
+        Dt = y[q] - bb[q] * Dt;
+        Ct = -bb[q] * Ct;
+      }
+    }
+    // and from the exclusive suffix applied to the ghost after the last row
+    double xin = wave::suffix_apply(Dt, Ct, DIR == 0 ? 0.0 : cur.g1);
+    const long base = ls * L;
+#pragma unroll
+    for (int q = R - 1; q >= 0; --q) {
+      if (r0 + q < n) {
+        const double x = y[q] - bb[q] * xin;
+        xin = x;
+        prev[q] = x;
+      }
+    }
+    if (L >= a0) {
+      const long c = base + r0 + 1;
+      if (r0 + R <= n) {
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k)
+          *(gptr<sw_d2>)(X + c + 2 * k) = sw_d2{prev[2 * k], prev[2 * k + 1]};
+        if (R % 2 == 1) X[c + R - 1] = prev[R - 1];
+      } else {
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+          if (r0 + q < n) X[c + q] = prev[q];
+      }
+    }
+    if (DIR == 0 && L >= a0) {  // BCU's wall and far-field ghosts of the stage input
+      if (l == 0) X[base] = -cur.g0 + 2.0 * uwall[L];
+      if (l == 63) X[base + ni] = -cur.g1 + 2.0 * ufar[L];
+    }
+  };
+  // lines loaded ahead, as the registers allow
+  constexpr int SW_AHEAD = R <= 3 ? 3 : (R <= 5 ? 2 : 1);
+  Ops ring[SW_AHEAD];
+#pragma unroll
+  for (int d = 0; d < SW_AHEAD; ++d) load(ring[d], min(Ls + d, a1));
+  for (int L = Ls; L <= a1; L += SW_AHEAD) {
+#pragma unroll
+    for (int d = 0; d < SW_AHEAD; ++d) {
+      if (L + d > a1) break;
+      const Ops cur = ring[d];
+      load(ring[d], min(L + d + SW_AHEAD, a1));  // past the chunk: its last line again
+      __builtin_amdgcn_sched_barrier(0);
+      solve(cur, L + d);
+    }
+  }
+}
+
+template <int DIR>
+__global__ void __launch_bounds__(64) k2_sweep(const Case2D* __restrict__ tab,
+                                               const int* __restrict__ bcase,
+                                               const int* __restrict__ btile, int nlc) {
   const int cc = bcase[blockIdx.x];
   if (cc < 0) return;
   const Case2D& cs = tab[cc];
-  const int t = btile[blockIdx.x];
-  const int comp = t & 1, ca = t >> 1;
-  const auto F = glb(cs.f[comp ? F_V : F_U]);
-  if (ca == 0)
-    bcu_ghosts_wave(F, cs.ni, cs.nj, cs.sj, glb(cs.b[comp ? B_VWALL : B_UWALL]),
-                    glb(cs.b[comp ? B_VFAR : B_UFAR]));
-  const int n = cs.ni - 1, nl = cs.nj - 1, nch = sw_nchunk(nl);
-  const int a1 = min((ca + 1) * SW_C, nl);
-  const auto dst = glb(cs.swb) + ((long)comp * nch + ca) * n;  // slot 0
-  for (int r = threadIdx.x; r < n; r += 64) dst[r] = F[(long)cs.sj * a1 + r + 1];
+  const int comp = btile[blockIdx.x] & 1, ca = btile[blockIdx.x] >> 1;
+  const int n = DIR == 0 ? cs.ni - 1 : cs.nj - 1;
+  switch ((n + 63) >> 6) {  // the case's own rows per lane
+    case 1: sweep_lead<1, DIR>(cs, comp, ca, nlc); break;
+    case 2: sweep_lead<2, DIR>(cs, comp, ca, nlc); break;
+    case 3: sweep_lead<3, DIR>(cs, comp, ca, nlc); break;
+    case 4: sweep_lead<4, DIR>(cs, comp, ca, nlc); break;
+    case 5: sweep_lead<5, DIR>(cs, comp, ca, nlc); break;
+    case 6: sweep_lead<6, DIR>(cs, comp, ca, nlc); break;
+    case 7: sweep_lead<7, DIR>(cs, comp, ca, nlc); break;
+    default: sweep_lead<8, DIR>(cs, comp, ca, nlc); break;
+  }
 }
 
 // One pass over the chunks of every case (block table: case, 2 chunk + component; entries with
 // case -1 pad the table to whole XCD rounds).  The change form's I-line stage leaves the field
 // alone in its first pass: 2 ncase workgroups past the table's nblk then set BCU's ghosts of the
 // stage input, which the stage-2 right-hand side reads.
-template <int DIR, bool EARLY, typename T>
+template <int DIR, bool EARLY>
 __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ tab,
                                                     const int* __restrict__ bcase,
                                                     const int* __restrict__ btile, int slot,
                                                     double tol, int final, int nblk) {
-  if (std::is_same<T, float>::value && DIR == 0 && !EARLY && (int)blockIdx.x >= nblk) {
+  if (DIR == 0 && !EARLY && (int)blockIdx.x >= nblk) {
     const int w = (int)blockIdx.x - nblk, comp = w & 1;
     const Case2D& cg = tab[w >> 1];
     bcu_ghosts_wave(glb(cg.f[comp ? F_V : F_U]), cg.ni, cg.nj, cg.sj,
@@ -506,14 +631,14 @@ __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ t
   const int comp = t & 1, ca = t >> 1;
   const int n = DIR == 0 ? cs.ni - 1 : cs.nj - 1;
   switch ((n + 63) >> 6) {  // the case's own rows per lane
-    case 1: sweep_chunk<1, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 2: sweep_chunk<2, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 3: sweep_chunk<3, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 4: sweep_chunk<4, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 5: sweep_chunk<5, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 6: sweep_chunk<6, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    case 7: sweep_chunk<7, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
-    default: sweep_chunk<8, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 1: sweep_chunk<1, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 2: sweep_chunk<2, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 3: sweep_chunk<3, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 4: sweep_chunk<4, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 5: sweep_chunk<5, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 6: sweep_chunk<6, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 7: sweep_chunk<7, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    default: sweep_chunk<8, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
   }
 }
 
@@ -539,8 +664,8 @@ __global__ void __launch_bounds__(256) k2_rhs2(const Case2D* __restrict__ tab,
   const int tx = (ni - 1 + 31) / 32, t = btile[blockIdx.x];
   const int i0 = 1 + (t % tx) * 32, j0 = 1 + (t / tx) * 32;
   const int l = threadIdx.x;
-  const auto U = glb(cs.f[F_U]);
-  const auto V = glb(cs.f[F_V]);
+  const auto U = glb(cs.f[AF32 ? F_U : F_X1U]);
+  const auto V = glb(cs.f[AF32 ? F_V : F_X1V]);
 #pragma unroll 1
   for (int r = 0; r < 4; ++r) {
     const int li = l % 32, lj = l / 32 + 8 * r;
