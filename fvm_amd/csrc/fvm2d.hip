@@ -444,20 +444,6 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
   }
 }
 
-// R consecutive doubles, the pairs among them by 16-byte loads (aligned to 8 bytes as the rows are):
-// a wavefront's lanes are R rows apart, so every load instruction touches 8 R bytes times 64 lanes of
-// cache lines and their number is what a line costs
-typedef double sw_d2 __attribute__((ext_vector_type(2), aligned(8)));
-template <int R>
-__device__ __forceinline__ void row_pairs(double (&d)[R], gptr<const double> p) {
-#pragma unroll
-  for (int k = 0; k < R / 2; ++k) {
-    const sw_d2 v = *(gptr<const sw_d2>)(p + 2 * k);
-    d[2 * k] = v.x; d[2 * k + 1] = v.y;
-  }
-  if constexpr (R % 2 == 1) d[R - 1] = p[R - 1];
-}
-
 // The FP64 sweep of chunk ca of nlc lines.  DIR 0: from the field (the stage input, left as it is)
 // and F_SU1 / F_SV1 to F_X1U / F_X1V, whose ghosts are BCU's of the stage input.  DIR 1: on the
 // J-line-major copies (iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_rhs2

@@ -45,7 +45,7 @@ int fvm_mail_wait(FvmCtx* c, const Mailbox& mb, int n, double* dst) {
     }
   }
   std::atomic_thread_fence(std::memory_order_acquire);
-  const volatile double* m = c->hmail;
+  const volatile double* m = mb.dst;
   for (int q = 0; q < n; ++q) dst[q] = m[q];
   return FVM_OK;
 }
@@ -396,6 +396,7 @@ static int create_impl(const fvm_params* prm, const double* xg, const double* yg
   r = fvm_af_setup(c);
   if (r) { fvm_destroy(c); return r; }
   r = fvm_sep_setup(c);
+  if (!r && c->prm.poisson_mode == 0) r = fvm_zebra_setup(c);
   if (r) { fvm_destroy(c); return r; }
   *out = c;
   return FVM_OK;

@@ -348,6 +348,20 @@ __device__ inline void publish(const Mailbox& mb, const double* v, int n) {
   *mb.seq = mb.s;
 }
 
+// R consecutive doubles of a lane of a 64-lane line scan, the pairs among them by 16-byte loads
+// (aligned to 8 bytes as the rows are): the lanes are R rows apart, so every load instruction
+// touches 8 R bytes times 64 lanes of cache lines, and their number is what a line costs
+typedef double sw_d2 __attribute__((ext_vector_type(2), aligned(8)));
+template <int R>
+__device__ __forceinline__ void row_pairs(double (&d)[R], gptr<const double> p) {
+#pragma unroll
+  for (int k = 0; k < R / 2; ++k) {
+    const sw_d2 v = *(gptr<const sw_d2>)(p + 2 * k);
+    d[2 * k] = v.x; d[2 * k + 1] = v.y;
+  }
+  if constexpr (R % 2 == 1) d[R - 1] = p[R - 1];
+}
+
 // up to eight arrays passed by value (no device pointer table needed)
 struct PtrSet8 {
   double* p[8];

@@ -103,6 +103,8 @@ struct FvmCtx {
   unsigned long long* hseq = nullptr;
   unsigned long long seq = 0;
 
+  double* pl[3] = {};  // Thomas factors of the radial lines of the FP64 zebra sweeps
+
   int nred = 0;
   // separable approximate inverse of the pressure operator (fvm_poisson_spec.hip)
   void* sep = nullptr;
@@ -204,6 +206,8 @@ int fvm_mail_wait(FvmCtx* c, const Mailbox& mb, int n, double* dst);
 int fvm_geom_setup(FvmCtx* c);
 int fvm_af_products(FvmCtx* c);
 int fvm_plane_setup(FvmCtx* c);
+int fvm_zebra_setup(FvmCtx* c);
+long fvm_k_p_su(FvmCtx* c);
 int fvm_k_set_dtime(FvmCtx* c, double dtime);
 int fvm_af_setup(FvmCtx* c);
 int fvm_af_scan_setup(FvmCtx* c);

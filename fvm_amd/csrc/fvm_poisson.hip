@@ -15,6 +15,7 @@
 // FP64 and runs the line sweeps in FP32 on the correction e of a defect-correction loop:
 // r = b - A p (FP64), e ~ A^-1 r by FP32 zebra sweeps, p += e (FP64).
 #include "fvm_ctx.h"
+#include "fvm_wave.h"
 
 namespace {
 
@@ -22,8 +23,9 @@ const dim3 kBlk(64, 4, 1);
 
 // div / dt from the face volume fluxes (iter_p.f90:31-34)
 __global__ void k_p_rhs(Dims d, const double* __restrict__ ju0, const double* __restrict__ ju1,
-                        const double* __restrict__ ju2, double dtime, double* rhs) {
+                        const double* __restrict__ ju2, double dtime, double* rhs, double* stop) {
   const uint3 bb = xcd_block();
+  if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x + threadIdx.y == 0) *stop = 0.0;
   const int i = 1 + bb.x * 64 + threadIdx.x;
   const int j = 1 + bb.y * 4 + threadIdx.y;
   const int k = 1 + bb.z;
@@ -142,65 +144,39 @@ __device__ inline PCoef pcoef(const Dims& d, int i, long c, const double* __rest
   return q;
 }
 
-// SU = rhs - DD(p) and, when asked, the per-block sums of |r| and |AP p| of the current
-// iterate: r = sum A_nb p_nb + SU - AP p (iter_p.f90:45-58)
-__global__ void k_p_su(Dims d, const double* __restrict__ p, const double* __restrict__ rhs,
-                       const double* __restrict__ pdI, const double* __restrict__ pdJ,
-                       const double* __restrict__ pdK, const double* __restrict__ jq12,
-                       const double* __restrict__ jq13, const double* __restrict__ jq23,
-                       double* psu, int want_res, double* part) {
-  const uint3 bb = xcd_block();
-  __shared__ double s0[256], s1[256];
-  const int i = 1 + bb.x * 64 + threadIdx.x;
-  const int j = 1 + bb.y * 4 + threadIdx.y;
-  const int k = 1 + bb.z;
-  const int t = threadIdx.x + 64 * threadIdx.y;
-  double ra = 0.0, rb = 0.0;
-  if (i <= d.ni - 1 && j <= d.nj - 1) {
-    const long c = cidx(d, i, j, k);
-    double su = rhs[c] - cross_p(d, c, p, jq12, jq13, jq23);
-    psu[c] = su;
-    if (want_res) {
-      PCoef q = pcoef(d, i, c, pdI, pdJ, pdK);
-      double r = q.ae * p[c + 1] + q.aw * p[c - 1] + q.an * p[c + d.sj] + q.as * p[c - d.sj] +
-                 q.at * p[c + d.sk] + q.ab * p[c - d.sk] + su - q.ap * p[c];
-      ra = fabs(r);
-      rb = fabs(q.ap * p[c]);
-    }
-  }
-  if (!want_res) return;
-  s0[t] = ra; s1[t] = rb;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) { s0[t] += s0[t + s]; s1[t] += s1[t + s]; }
-    __syncthreads();
-  }
-  if (t == 0) {
-    long bid = bb.x + (long)gridDim.x * (bb.y + (long)gridDim.y * bb.z);
-    part[2 * bid] = s0[0];
-    part[2 * bid + 1] = s1[0];
-  }
-}
-
-__global__ void k_p_res_final(const double* __restrict__ part, long nb, double* out) {
+// Sums of the parts, the scaled residual, and stop = 1 once it is at most tol or no number (tol < 0:
+// never); the kernels of sweeps enqueued past that end at once and leave out[0..2] as they are.
+__global__ void k_p_res_final(const double* __restrict__ part, long nb, double* out, double tol,
+                              double* stop, Mailbox mb) {
   __shared__ double s0[256], s1[256];
   const int t = threadIdx.x;
-  double a = 0.0, b = 0.0;
-  for (long q = t; q < nb; q += blockDim.x) { a += part[2 * q]; b += part[2 * q + 1]; }
-  s0[t] = a; s1[t] = b;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) { s0[t] += s0[t + s]; s1[t] += s1[t + s]; }
+  const bool ended = *stop != 0.0;  // uniform
+  if (!ended) {
+    double a = 0.0, b = 0.0;
+    for (long q = t; q < nb; q += blockDim.x) { a += part[2 * q]; b += part[2 * q + 1]; }
+    s0[t] = a; s1[t] = b;
     __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+      if (t < s) { s0[t] += s0[t + s]; s1[t] += s1[t + s]; }
+      __syncthreads();
+    }
+    if (t == 0) {
+      out[0] = s0[0]; out[1] = s1[0]; out[2] = scaled_residual(s0[0], s1[0]);
+      if (tol >= 0.0 && !(out[2] > tol)) *stop = 1.0;
+    }
   }
-  if (t == 0) { out[0] = s0[0]; out[1] = s1[0]; out[2] = scaled_residual(s0[0], s1[0]); }
+  if (t == 0) {
+    const double v[3] = {out[0], out[1], out[2]};
+    publish(mb, v, 3);
+  }
 }
 
 // BCP ghosts, wall p(0) = p(1) and outflow cubic extrapolation (bcp.f90:22-32), and the periodic
 // copy of MPI_X in one pass over the ghost surface: every ghost is a function of the interior
 // cells of one radial line, that of its periodic partner (js, ks)
 template <typename T>
-__global__ void k_bcp(Dims d, T* p) {
+__global__ void k_bcp(Dims d, T* p, const double* __restrict__ stop) {
+  if (stop && *stop != 0.0) return;
   const long cnt = bc_ghost_count(d);
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < cnt;
        t += (long)gridDim.x * blockDim.x) {
@@ -248,7 +224,92 @@ __global__ void __launch_bounds__(64) k_p_sweep(Dims d, T* p, const T* __restric
   for (int r = threadIdx.x; r < n; r += 64) p[base + r + 1] = ld[r];
 }
 
-// Mixed precision: FP32 defect r32 = (b - A p) with b = SU from k_p_su; the correction
+// Thomas factors of the radial lines of the FP64 sweeps (setup only): 1/D, -A/D, B with A = -AW,
+// D = AP - A B(i-1), B = -AE/D; one thread per line.
+__global__ void k_p_line_factor(Dims d, const double* __restrict__ pdI,
+                                const double* __restrict__ pdJ, const double* __restrict__ pdK,
+                                double* invd, double* na, double* bf) {
+  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (t >= (long)(d.nj - 1) * (d.nk - 1)) return;
+  const int j = 1 + (int)(t % (d.nj - 1)), k = 1 + (int)(t / (d.nj - 1));
+  double b = 0.0;
+  for (int i = 1; i <= d.ni - 1; ++i) {
+    const long c = cidx(d, i, j, k);
+    const PCoef q = pcoef(d, i, c, pdI, pdJ, pdK);
+    const double D = q.ap + q.aw * b;
+    invd[c] = 1.0 / D;
+    na[c] = q.aw / D;
+    b = -q.ae / D;
+    bf[c] = b;
+  }
+}
+
+// One zebra half-sweep in FP64: every radial line (j,k) with (j+k) % 2 == colour by one wavefront,
+// R rows per lane, as two affine-map scans over its precomputed factors (lisolv.f90:15-30).  By
+// cyclic reduction through LDS, with the coefficients formed anew, a half-sweep of 96 x 128 x 32
+// cells took 9.8 us, so 5.1.
+template <int R>
+__global__ void __launch_bounds__(64) k_p_line(Dims d, double* p, const double* __restrict__ su,
+                                               const double* __restrict__ pdJ,
+                                               const double* __restrict__ pdK,
+                                               const double* __restrict__ invd,
+                                               const double* __restrict__ na,
+                                               const double* __restrict__ bf, int colour,
+                                               const double* __restrict__ stop) {
+  if (*stop != 0.0) return;
+  const int k = 1 + blockIdx.y;
+  const int j = 1 + ((colour + 1 + k) & 1) + 2 * blockIdx.x;  // (j + k) % 2 == colour
+  if (j > d.nj - 1) return;
+  const int n = d.ni - 1, r0 = threadIdx.x * R;
+  // rows past n (up to R - 1 of them: the ghost and the next line) and the lanes past n are not used
+  const long c = cidx(d, 1, j, k) + (r0 < n ? r0 : 0);
+  double pn[R], ps[R], pt[R], pb[R], s[R], dn[R], ds[R], dt[R], db[R], iv[R], nv[R], bv[R];
+  row_pairs<R>(pn, gp(p) + c + d.sj);
+  row_pairs<R>(ps, gp(p) + c - d.sj);
+  row_pairs<R>(pt, gp(p) + c + d.sk);
+  row_pairs<R>(pb, gp(p) + c - d.sk);
+  row_pairs<R>(s, gp(su) + c);
+  row_pairs<R>(dn, gp(pdJ) + c);
+  row_pairs<R>(ds, gp(pdJ) + c - d.sj);
+  row_pairs<R>(dt, gp(pdK) + c);
+  row_pairs<R>(db, gp(pdK) + c - d.sk);
+  row_pairs<R>(iv, gp(invd) + c);
+  row_pairs<R>(nv, gp(na) + c);
+  row_pairs<R>(bv, gp(bf) + c);
+  double al[R], At = 0.0, Bt = 1.0;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const bool in = r0 + q < n;
+    const double rhs = -dn[q] * pn[q] + -ds[q] * ps[q] + -dt[q] * pt[q] + -db[q] * pb[q] + s[q];
+    al[q] = rhs * iv[q];
+    At = in ? al[q] + nv[q] * At : At;
+    Bt = in ? nv[q] * Bt : Bt;
+  }
+  double yin = wave::prefix_apply(At, Bt, 0.0);
+  double y[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    y[q] = al[q] + nv[q] * yin;
+    yin = y[q];
+  }
+  double Ct = 1.0, Dt = 0.0;
+#pragma unroll
+  for (int q = R - 1; q >= 0; --q) {
+    const bool in = r0 + q < n;
+    Dt = in ? y[q] - bv[q] * Dt : Dt;
+    Ct = in ? -bv[q] * Ct : Ct;
+  }
+  double xin = wave::suffix_apply(Dt, Ct, 0.0);
+#pragma unroll
+  for (int q = R - 1; q >= 0; --q) {
+    if (r0 + q < n) {
+      xin = y[q] - bv[q] * xin;
+      p[c + q] = xin;
+    }
+  }
+}
+
+// Mixed precision: FP32 defect r32 = (b - A p) with b = SU; the correction
 // equation A e = r keeps the operator's cross terms on e as well.
 __global__ void k_p_defect32(Dims d, const double* __restrict__ p, const double* __restrict__ psu,
                              const double* __restrict__ pdI, const double* __restrict__ pdJ,
@@ -294,47 +355,80 @@ __global__ void k_p_add(Dims d, double* p, const float* __restrict__ e) {
 
 int fvm_k_bcp(FvmCtx* c) {
   hipLaunchKernelGGL(k_bcp<double>, grid1(bc_ghost_count(c->d), 256), dim3(256), 0, c->stream,
-                     c->d, c->p);
+                     c->d, c->p, nullptr);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
 
 static int bcp32(FvmCtx* c, float* e) {
   hipLaunchKernelGGL(k_bcp<float>, grid1(bc_ghost_count(c->d), 256), dim3(256), 0, c->stream,
-                     c->d, e);
+                     c->d, e, nullptr);
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
 
-// residual sums of the current iterate (after fresh BCP ghosts), SU for the next sweep
-static int su_and_residual(FvmCtx* c, bool want, double* res) {
-  const Dims d = c->d;
-  dim3 g((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, d.nk - 1);
-  long nb = (long)g.x * g.y * g.z;
+// residual sums of the current iterate (after fresh BCP ghosts), SU for the next sweep; with want,
+// published to mb (tol: k_p_res_final)
+static int su_and_residual(FvmCtx* c, bool want, double tol, const Mailbox& mb) {
+  long nb;
   {
     ProfScope ps(c, "p_su");
-    hipLaunchKernelGGL(k_p_su, g, kBlk, 0, c->stream, d, c->p, c->rhs, c->pdI, c->pdJ, c->pdK,
-                       c->jq12, c->jq13, c->jq23, c->psu, want ? 1 : 0, c->red);
+    nb = fvm_k_p_su(c);
     HIP_CHECK(hipGetLastError());
   }
   if (want) {
-    hipLaunchKernelGGL(k_p_res_final, dim3(1), dim3(256), 0, c->stream, c->red, nb, c->scal + 4);
+    hipLaunchKernelGGL(k_p_res_final, dim3(1), dim3(256), 0, c->stream, c->red, nb, c->scal + 4,
+                       tol, c->scal + 7, mb);
     HIP_CHECK(hipGetLastError());
-    const int rf = fvm_fetch(c, c->scal + 4, 3, c->hscal + 4);
-    if (rf) return rf;
-    *res = c->hscal[6];
   }
   return FVM_OK;
 }
 
-template <typename T>
-static int zebra(FvmCtx* c, T* p, const T* su) {
-  const Dims d = c->d;
-  dim3 g((d.nj - 1 + 1) / 2, d.nk - 1);
-  ProfScope ps(c, sizeof(T) == 8 ? "p_sweep64" : "p_sweep32");
+static dim3 zebra_grid(const Dims& d) { return dim3((d.nj - 1 + 1) / 2, d.nk - 1); }
+
+static int zebra32(FvmCtx* c, float* p, const float* su) {
+  ProfScope ps(c, "p_sweep32");
   for (int colour = 0; colour < 2; ++colour)
-    hipLaunchKernelGGL(k_p_sweep<T>, g, dim3(64), 0, c->stream, d, p, su, c->pdI, c->pdJ,
-                       c->pdK, colour);
+    hipLaunchKernelGGL(k_p_sweep<float>, zebra_grid(c->d), dim3(64), 0, c->stream, c->d, p, su,
+                       c->pdI, c->pdJ, c->pdK, colour);
+  HIP_CHECK(hipGetLastError());
+  return FVM_OK;
+}
+
+template <int R>
+static void zebra64_r(FvmCtx* c) {
+  for (int colour = 0; colour < 2; ++colour)
+    hipLaunchKernelGGL(k_p_line<R>, zebra_grid(c->d), dim3(64), 0, c->stream, c->d, c->p, c->psu,
+                       c->pdJ, c->pdK, c->pl[0], c->pl[1], c->pl[2], colour, c->scal + 7);
+}
+
+// The line factors of the FP64 zebra sweeps (geometry only), with the set-up of a context that runs
+// them.
+int fvm_zebra_setup(FvmCtx* c) {
+  const Dims d = c->d;
+  double* t = nullptr;
+  HIP_CHECK(hipMalloc((void**)&t, 3 * d.n * sizeof(double)));
+  c->allocs.push_back(t);
+  for (int q = 0; q < 3; ++q) c->pl[q] = t + q * d.n;
+  hipLaunchKernelGGL(k_p_line_factor, grid1((long)(d.nj - 1) * (d.nk - 1), 64), dim3(64), 0,
+                     c->stream, d, c->pdI, c->pdJ, c->pdK, c->pl[0], c->pl[1], c->pl[2]);
+  HIP_CHECK(hipGetLastError());
+  return FVM_OK;
+}
+
+static int zebra64(FvmCtx* c) {
+  const Dims d = c->d;
+  ProfScope ps(c, "p_sweep64");
+  switch ((d.ni - 1 + 63) / 64) {
+    case 1: zebra64_r<1>(c); break;
+    case 2: zebra64_r<2>(c); break;
+    case 3: zebra64_r<3>(c); break;
+    case 4: zebra64_r<4>(c); break;
+    case 5: zebra64_r<5>(c); break;
+    case 6: zebra64_r<6>(c); break;
+    case 7: zebra64_r<7>(c); break;
+    default: zebra64_r<8>(c); break;
+  }
   HIP_CHECK(hipGetLastError());
   return FVM_OK;
 }
@@ -369,7 +463,7 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
   {
     ProfScope ps(c, "p_rhs");
     hipLaunchKernelGGL(k_p_rhs, gi, kBlk, 0, c->stream, d, c->ju[0], c->ju[1], c->ju[2],
-                       c->prm.dtime, c->rhs);
+                       c->prm.dtime, c->rhs, c->scal + 7);
     HIP_CHECK(hipGetLastError());
   }
   if (c->prm.poisson_mode >= 2) {
@@ -384,21 +478,42 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
   double res = INFINITY;
   int r;
   if (c->prm.poisson_mode == 0) {
-    // FP64 zebra line Gauss-Seidel
-    for (;;) {
-      r = fvm_k_bcp(c);
-      if (r) return r;
-      bool want = (sweeps % every == 0) || sweeps >= cap;
-      r = su_and_residual(c, want, &res);
-      if (r) return r;
-      if (want) {
-        ++outer;
-        if (!(res == res)) return FVM_ERR_NAN;
-        if (res <= tol || sweeps >= cap) break;
+    // FP64 zebra line Gauss-Seidel.  The host enqueues up to kAhead residual tests ahead of the one
+    // it waits for; the device ends the sweeps itself (k_p_res_final's flag), so those enqueued past
+    // the end change nothing.  A wait for every test left the device idle for the host's reaction
+    // and the next launches, and its own launch to publish, a third of a sweep on 96 x 128 x 32 cells.
+    constexpr int kAhead = 3;
+    Mailbox mb[kAhead + 1];
+    int at[kAhead + 1];  // sweeps done at the test
+    int put = 0, got = 0, sent = 0;
+    for (bool end = false; !end;) {
+      for (; sent <= cap && put - got <= kAhead; ++sent) {  // enqueue: test (and a sweep before it)
+        if (sent > 0) {
+          r = zebra64(c);
+          if (r) return r;
+        }
+        hipLaunchKernelGGL(k_bcp<double>, grid1(bc_ghost_count(d), 256), dim3(256), 0, c->stream, d,
+                           c->p, c->scal + 7);
+        const bool want = sent % every == 0 || sent >= cap;
+        Mailbox m{nullptr, nullptr, 0};
+        if (want) {
+          m = fvm_mail(c);
+          m.dst = c->hmail + 8 + 4 * (put % (kAhead + 1));
+          mb[put % (kAhead + 1)] = m;
+          at[put % (kAhead + 1)] = sent;
+          ++put;
+        }
+        r = su_and_residual(c, want, tol, m);
+        if (r) return r;
       }
-      r = zebra<double>(c, c->p, c->psu);
+      const int q = got++ % (kAhead + 1);
+      r = fvm_mail_wait(c, mb[q], 3, c->hscal + 4);
       if (r) return r;
-      ++sweeps;
+      res = c->hscal[6];
+      sweeps = at[q];
+      ++outer;
+      if (!(res == res)) return FVM_ERR_NAN;
+      end = res <= tol || sweeps >= cap;
     }
   } else {
     // FP32 zebra sweeps on the correction inside FP64 defect correction
@@ -409,8 +524,11 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
     for (;;) {
       r = fvm_k_bcp(c);
       if (r) return r;
-      r = su_and_residual(c, true, &res);
+      const Mailbox m = fvm_mail(c);
+      r = su_and_residual(c, true, -1.0, m);
+      if (!r) r = fvm_mail_wait(c, m, 3, c->hscal + 4);
       if (r) return r;
+      res = c->hscal[6];
       ++outer;
       if (!(res == res)) return FVM_ERR_NAN;
       if (res <= tol || sweeps >= cap) break;
@@ -429,7 +547,7 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
                              c->jq23, esu);
           HIP_CHECK(hipGetLastError());
         }
-        r = zebra<float>(c, e, esu);
+        r = zebra32(c, e, esu);
         if (r) return r;
         ++sweeps;
       }
