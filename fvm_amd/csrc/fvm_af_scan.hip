@@ -184,24 +184,34 @@ __global__ void k_to_float(long n, const double* __restrict__ a, float* b) {
     b[t] = (float)a[t];
 }
 
-// boundary lines of the FP64 I stage's first pass: the stage input at the last line of every
-// chunk (bnd[((comp nb + b-1) nchunk + ca) n + p-1]).  That stage writes its iterate over the
-// field, so a chunk cannot read its neighbour's line there; the J stage, whose iterate is a work
-// array, and the change form, whose stage input is the zero change, take it in the first pass.
-__global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, double* bnd) {
-  const ScanGeo g = scan_geo(d, 0);
-  const long tot = (long)A.nc * g.nb * nchunk * g.n;
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot;
-       t += (long)gridDim.x * blockDim.x) {
-    const int p = 1 + (int)(t % g.n);
-    long r = t / g.n;
-    const int ca = (int)(r % nchunk);
-    r /= nchunk;
-    const int b = 1 + (int)(r % g.nb);
-    const int comp = (int)(r / g.nb);
-    const int a = min((ca + 1) * SC_C, g.na);
-    bnd[t] = A.f[comp][g.ns_p * p + g.ns_a * a + g.ns_b * b];
+// The largest ratio of the coupling to line a - 1 to the row sum of the line operator, per line a: the
+// factor by which a change of line a - 1 reaches line a at most (T^-1 s = 1 for the M-matrix T with
+// row sums s).  One workgroup per line (setup only).
+template <int S>
+__global__ void __launch_bounds__(256) k_scan_rho(Dims d, const double* const* __restrict__ fa,
+                                                  const double* __restrict__ ap0, double* rho) {
+  __shared__ double sh[256];
+  const ScanGeo g = scan_geo(d, S);
+  const int a = 1 + blockIdx.x, t = threadIdx.x;
+  double m = 0.0;
+  for (long q = t; q < (long)g.n * g.nb; q += 256) {
+    const int p = 1 + (int)(q % g.n), b = 1 + (int)(q / g.n);
+    const long c = g.ns_p * p + g.ns_a * a + g.ns_b * b;
+    const int i = S == 0 ? p : a;
+    double ae = fa[0][c], aw = fa[0][c - 1], an = fa[1][c], as = fa[1][c - d.sj],
+           at = fa[2][c], ab = fa[2][c - d.sk];
+    double ap = ap0[c] + ae + aw + an + as + at + ab;
+    if (i == 1) { ap = ap + aw; aw = 0.0; }
+    if (i == d.ni - 1) { ap = ap + ae; ae = 0.0; }
+    m = fmax(m, (S == 0 ? as : aw) / (ap - (S == 0 ? aw + ae : as + an)));
   }
+  sh[t] = m;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (t < w) sh[t] = fmax(sh[t], sh[t + w]);
+    __syncthreads();
+  }
+  if (t == 0) rho[a] = sh[0];
 }
 
 // R consecutive elements from an address aligned to 4 (R % 4 == 0) or 2 (R % 2 == 0) elements
@@ -236,6 +246,121 @@ __device__ __forceinline__ void load_rows(double (&d)[R], gptr<const double> p) 
 __device__ inline double shfl_up_d(double v, int o) { return __shfl_up(v, o, 64); }
 __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o, 64); }
 
+// The FP64 sweep of a stage in one pass: wavefront w owns chunk ca (nlc lines) of plane b for one
+// component and starts lead[a0] lines early, with nothing from the line before them, where that is
+// worth less than 1e-20 in the chunk (products of k_scan_rho's ratios; up to line 1 where the
+// dominance is weak).  Up to three lines are loaded ahead, rows in pairs.  The iterate is the field
+// itself for the I lines (whose line ends BCU's folds leave without coupling) and the line-major work
+// array for the J lines.  A value that is not finite sets *bad.  As passes over chunks of 16 lines
+// until the chunks' last lines settled, with a launch before for the I lines' first boundary lines
+// and a host wait after each stage's second pass, the two stages of a slab of 128 x 256 cells took 62
+// us of kernels and two waits a step; they take 39.
+template <int S, int R>
+__global__ void __launch_bounds__(64) k_scan_lead(Dims d, AFArgs A, const double* __restrict__ beta,
+                                                  const double* __restrict__ invd,
+                                                  const double* __restrict__ bb,
+                                                  const double* __restrict__ cam,
+                                                  const double* const* qt, double* const* xot,
+                                                  const int* __restrict__ lead, int nlc, int nchunk,
+                                                  volatile double* bad, long G) {
+  const ScanGeo g = scan_geo(d, S);
+  const long lin = blockIdx.x;
+  const long w = (lin % 8) * (G / 8) + lin / 8;  // XCD-aware: neighbouring items share an XCD
+  if (w >= (long)A.nc * nchunk * g.nb) return;
+  const int comp = (int)(w % A.nc);
+  const long wr = w / A.nc;
+  const int ca = (int)(wr % nchunk), b = 1 + (int)(wr / nchunk);
+  const int a0 = 1 + ca * nlc, a1 = min(a0 + nlc - 1, g.na);
+  const int l = threadIdx.x, p0 = l * R + 1;
+  const GP qc = gp(qt[comp]), fc = gp(A.f[comp]);
+  const gptr<double> xc = glb(xot[comp]);
+  struct Ops {
+    double be[R], iv[R], bv[R], cm[R], qv[R], y0, xn;
+  };
+  auto load = [&](Ops& o, int a) {
+    // rows past n (up to R - 1 of them: the ghost and the next line) and the lanes past n are not used
+    const long c = g.ls_a * a + g.ls_b * b + g.off + (p0 <= g.n ? p0 : 1);
+    row_pairs<R>(o.be, gp(beta) + c);
+    row_pairs<R>(o.iv, gp(invd) + c);
+    row_pairs<R>(o.bv, gp(bb) + c);
+    row_pairs<R>(o.cm, gp(cam) + c);
+    row_pairs<R>(o.qv, qc + c);
+    const long nb0 = g.ns_a * a + g.ns_b * b;  // the ghosts before and after the line
+    o.y0 = S == 1 ? fc[nb0] : 0.0;
+    o.xn = S == 1 ? fc[nb0 + g.ns_p * (g.n + 1)] : 0.0;
+  };
+  const int Ls = lead[a0];
+  double xp[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    xp[r] = Ls == 1 && p0 + r <= g.n ? fc[g.ns_p * (p0 + r) + g.ns_b * b] : 0.0;
+  bool fin = true;
+  auto solve = [&](const Ops& o, int a) {
+    double al[R], y[R];
+    double Bt = 1.0, At = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      al[r] = (o.qv[r] + o.cm[r] * xp[r]) * o.iv[r];
+      const bool in = p0 + r <= g.n;
+      At = in ? al[r] + o.be[r] * At : At;
+      Bt = in ? o.be[r] * Bt : Bt;
+    }
+    double yin = wave::prefix_apply(At, Bt, o.y0);  // y0, xn: the same on every lane
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      y[r] = al[r] + o.be[r] * yin;
+      yin = p0 + r <= g.n ? y[r] : yin;
+    }
+    double Ct = 1.0, Dt = 0.0;
+#pragma unroll
+    for (int r = R - 1; r >= 0; --r) {
+      const bool in = p0 + r <= g.n;
+      Dt = in ? y[r] - o.bv[r] * Dt : Dt;
+      Ct = in ? -o.bv[r] * Ct : Ct;
+    }
+    double xin = wave::suffix_apply(Dt, Ct, o.xn);
+#pragma unroll
+    for (int r = R - 1; r >= 0; --r) {
+      const bool in = p0 + r <= g.n;
+      const double x = y[r] - o.bv[r] * xin;
+      xin = in ? x : xin;
+      xp[r] = in ? x : 0.0;
+    }
+    if (a < a0) return;
+    const long c = g.ls_a * a + g.ls_b * b + g.off + p0;
+    if (p0 + R - 1 <= g.n) {
+#pragma unroll
+      for (int k = 0; k < R / 2; ++k)
+        *(gptr<sw_d2>)(xc + c + 2 * k) = sw_d2{xp[2 * k], xp[2 * k + 1]};
+      if (R % 2 == 1) xc[c + R - 1] = xp[R - 1];
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (p0 + r <= g.n) xc[c + r] = xp[r];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) fin = fin && fabs(xp[r]) < INFINITY;
+  };
+  constexpr int AHEAD = R <= 3 ? 3 : (R <= 4 ? 2 : 1);
+  Ops ring[AHEAD];
+#pragma unroll
+  for (int q = 0; q < AHEAD; ++q) load(ring[q], min(Ls + q, a1));
+  for (int a = Ls; a <= a1; a += AHEAD) {
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) {
+      if (a + q > a1) break;
+      const Ops o = ring[q];
+      load(ring[q], min(a + q + AHEAD, a1));  // past the chunk: its last line again
+      __builtin_amdgcn_sched_barrier(0);
+      solve(o, a + q);
+    }
+  }
+  if (!fin) {
+    *bad = 1.0;
+    __threadfence_system();
+  }
+}
+
 // One pass: wavefront w owns chunk ca of plane b for one component and sweeps its lines in
 // order (the component is the fastest index of w, so the three wavefronts sharing the line
 // factors run side by side on one XCD).  Lane l owns rows l*R+1 .. l*R+R.  The loads of line
@@ -258,19 +383,19 @@ __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o,
 // is FP32; the FP64 field is updated with the converged change afterwards.  The stage's field is
 // then neither read nor written, so the workgroups past the first G of the first pass set its
 // BCU ghosts (bc_ghost), which the right-hand sides of the next stage read: one launch less.
-template <int S, int R, bool EARLY, typename T>
-__global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __restrict__ beta,
-                                                  const T* __restrict__ invd,
-                                                  const T* __restrict__ bb,
-                                                  const T* __restrict__ cam,
+template <int S, int R, bool EARLY>
+__global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float* __restrict__ beta,
+                                                  const float* __restrict__ invd,
+                                                  const float* __restrict__ bb,
+                                                  const float* __restrict__ cam,
                                                   const double* const* qt, double* const* xot,
-                                                  const T* __restrict__ bnd_in,
-                                                  T* bnd_out, int nchunk, double* part,
+                                                  const float* __restrict__ bnd_in,
+                                                  float* bnd_out, int nchunk, double* part,
                                                   double tol, double* sinkd, long G) {
-  constexpr bool DELTA = std::is_same<T, float>::value;
+  using T = float;
   const ScanGeo g = scan_geo(d, S);
   const long lin = blockIdx.x;
-  if (DELTA && !EARLY && lin >= G) {  // uniform over the workgroup
+  if (!EARLY && lin >= G) {  // uniform over the workgroup
     const long cnt = bc_ghost_count(d), step = ((long)gridDim.x - G) * 64;
     for (long t = (lin - G) * 64 + threadIdx.x; t < A.nc * cnt; t += step)
       bc_ghost(d, A.f[t / cnt], A.ufar + (t / cnt) * (long)(d.nj + 1) * (d.nk + 1), 0.0, t % cnt);
@@ -289,30 +414,23 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
     const int a1 = min(a0 + SC_C - 1, g.na);
     const int p0 = l * R + 1;
     const gptr<const T> qc = glb(reinterpret_cast<const T*>(qt[comp]));
-    const GP fc = gp(A.f[comp]);
     const gptr<T> xc = glb(reinterpret_cast<T*>(xot[comp]));
     T xp[R];
-    // line a0-1: the stage input's ghost line for the first chunk, else the preceding
+    // line a0-1: no change in the first pass and before the first chunk, else the preceding
     // chunk's last line of the previous pass
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int p = p0 + r;
       T v = (T)0;
-      if (p <= g.n) {
-        if (DELTA && (ca == 0 || !EARLY))
-          v = (T)0;
-        else if (ca == 0 || (S == 1 && !EARLY))
-          v = (T)fc[g.ns_p * p + g.ns_a * (a0 - 1) + g.ns_b * b];
-        else
-          v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
-      }
+      if (EARLY && p <= g.n && ca > 0)
+        v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
       xp[r] = v;
     }
     // Operands of one line.  Rows past n (the last lane's tail) read row n and are never kept,
     // and the next line is always fetched (the last line again at the end of the chunk): with
     // no load or store behind a branch the compiler counts the loads in flight exactly and
     // waits only for the ones it needs, so the next line's loads overlap this line's scans.
-    T be[R], iv[R], bv[R], cm[R], qv[R], xv[R], y0n, xnn;
+    T be[R], iv[R], bv[R], cm[R], qv[R], xv[R];
     auto load = [&](int a) {
       const long lb = g.ls_a * a + g.ls_b * b + g.off;
       if constexpr (S == 1 && R % 2 == 0) {
@@ -338,14 +456,6 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
           xv[r] = EARLY ? xc[o] : (T)0;  // the previous pass's value of the line
         }
       }
-      if (DELTA) {
-        y0n = (T)0;
-        xnn = (T)0;
-      } else {
-        const long nb0 = g.ns_a * a + g.ns_b * b;  // natural base of the line
-        y0n = (T)fc[nb0];                          // row 0 ghost
-        xnn = (T)fc[nb0 + g.ns_p * (g.n + 1)];     // row n+1 ghost
-      }
     };
     load(a0);
     bool stopped = false;
@@ -353,7 +463,6 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
     const T ttol = (T)tol;
     for (int a = a0; a <= a1; ++a) {
       const long lb = g.ls_a * a + g.ls_b * b + g.off;
-      const T y0 = y0n, xn = xnn;
       // forward: y(p) = al(p) + be(p) y(p-1)
       T al[R], bt[R], bw[R], xo[R];
       T Bt = (T)1, At = (T)0;
@@ -369,7 +478,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
       }
       load(min(a + 1, a1));  // next line's operands in flight during the scans
       __builtin_amdgcn_sched_barrier(0);  // keep those loads ahead of the scans
-      T yin = wave::prefix_apply(At, Bt, y0);  // y0, xn: the same on every lane
+      T yin = wave::prefix_apply(At, Bt, (T)0);
       T y[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -384,7 +493,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __r
         Dt = in ? y[r] - bw[r] * Dt : Dt;
         Ct = in ? -bw[r] * Ct : Ct;
       }
-      T xin = wave::suffix_apply(Dt, Ct, xn);
+      T xin = wave::suffix_apply(Dt, Ct, (T)0);
       T dl = (T)0;
 #pragma unroll
       for (int r = R - 1; r >= 0; --r) {
@@ -458,9 +567,88 @@ __global__ void k_scan_max(const double* __restrict__ part, long nb, double* out
   }
 }
 
-template <int S, int R, typename T>
-int scan_stage(FvmCtx* c, const AFArgs& A, int* iters, bool temp) {
+// Q (or the FP32 residual): the right-hand-side kernel left it in A.su (natural layout); the J stage
+// uses a line-major copy.  The iterate is the field itself for the FP64 I stage, else a work array
+// (line-major for J).
+template <typename T>
+struct ScanBufs {
+  double *q[3] = {}, *xo[3] = {}, *fo[3] = {};
+  double** tab = nullptr;  // device: q at [0..2], iterate at [3..5], field at [6..8]
+};
+
+template <int S, typename T>
+int scan_prepare(FvmCtx* c, const AFArgs& A, bool temp, ScanBufs<T>& B) {
   constexpr bool DELTA = std::is_same<T, float>::value;
+  const Dims d = c->d;
+  const int nc = A.nc;
+  for (int k = 0; k < nc; ++k) {
+    B.q[k] = S == 0 ? A.su[k] : c->afb[k][1];
+    B.xo[k] = (S == 0 && !DELTA) ? A.f[k] : c->afb[k][0];
+    B.fo[k] = A.f[k];
+  }
+  // the buffers are the context's own, so the table is uploaded once and again only if they change
+  // (the temperature has a table of its own)
+  double* tab[9] = {B.q[0], B.q[1], B.q[2], B.xo[0], B.xo[1], B.xo[2], B.fo[0], B.fo[1], B.fo[2]};
+  B.tab = temp ? c->scantab_t[S] : c->scantab[S];
+  double** htab = temp ? c->scantab_th[S] : c->scantab_h[S];
+  if (memcmp(tab, htab, sizeof(tab)) != 0) {
+    HIP_CHECK(hipMemcpyAsync(B.tab, tab, sizeof(tab), hipMemcpyHostToDevice, c->stream));
+    memcpy(htab, tab, sizeof(tab));
+  }
+  if (S == 1) {
+    ProfScope pk(c, "af_scan_q");
+    PtrSet8 qn{};
+    for (int k = 0; k < nc; ++k) qn.p[k] = A.su[k];
+    hipLaunchKernelGGL(k_scan_q1v<T>, dim3((d.ni - 1 + 31) / 32, (d.nj - 1 + 31) / 32, nc * (d.nk - 1)),
+                       dim3(256), 0, c->stream, d, qn, (double* const*)B.tab);
+    HIP_CHECK(hipGetLastError());
+  }
+  return FVM_OK;
+}
+
+// the J stage's line-major iterate back into the field
+template <typename T>
+int scan_unpack(FvmCtx* c, int nc, const ScanBufs<T>& B) {
+  const Dims d = c->d;
+  ProfScope pk(c, "af_scan_unpack");
+  hipLaunchKernelGGL(k_scan_unpack1<T>, dim3((d.ni - 1 + 63) / 64, (d.nj - 1 + 31) / 32, nc * (d.nk - 1)),
+                     dim3(256), 0, c->stream, d, (const double* const*)(B.tab + 3), B.tab + 6);
+  HIP_CHECK(hipGetLastError());
+  return FVM_OK;
+}
+
+// Lines per chunk of the FP64 sweeps: a chunk's lead-in (7 to 15 lines) is solved twice, so short
+// chunks are for grids whose wavefronts do not fill the chip.  I and J stage with chunks of 8, 16 and
+// 32 lines, us: 128 x 256 cells (768 lines of u, v, w in the I stage) 16 + 26, 20 + 28, 29 + 40;
+// 96 x 128 x 32 (12288) 20 + 20, 21 + 21, 29 + 29; 149 x 208 x 40 (24960) 43 + 48, 38 + 46, 50 + 54;
+// 240 x 320 x 96 (92160) 191 + 227, 175 + 207, 165 + 196.
+int scan_lines(long lines) {
+  return lines <= 8 * 2048L ? 8 : (lines <= 16 * 4096L ? 16 : 32);
+}
+
+template <int S, int R>
+int scan_stage64(FvmCtx* c, const AFArgs& A, bool temp) {
+  const Dims d = c->d;
+  const ScanGeo g = scan_geo(d, S);
+  ScanBufs<double> B;
+  int r = scan_prepare<S, double>(c, A, temp, B);
+  if (r) return r;
+  const int nlc = scan_lines((long)A.nc * g.nb * g.na), nchunk = (g.na + nlc - 1) / nlc;
+  const long G = ((long)A.nc * nchunk * g.nb + 7) / 8 * 8;
+  const double* const* lf = temp ? c->lft[S] : c->lf[S];
+  {
+    ProfScope pk(c, S == 0 ? "k_scan_pass_i" : "k_scan_pass_j");
+    hipLaunchKernelGGL((k_scan_lead<S, R>), dim3((unsigned)G), dim3(64), 0, c->stream, d, A, lf[0],
+                       lf[1], lf[2], lf[3], (const double* const*)B.tab, B.tab + 3,
+                       (const int*)c->lead[temp][S], nlc, nchunk, c->hmail + kMailBad, G);
+    HIP_CHECK(hipGetLastError());
+  }
+  return S == 1 ? scan_unpack<double>(c, A.nc, B) : FVM_OK;
+}
+
+template <int S, int R>
+int scan_stage32(FvmCtx* c, const AFArgs& A, int* iters) {
+  using T = float;
   const Dims d = c->d;
   hipStream_t st = c->stream;
   const ScanGeo g = scan_geo(d, S);
@@ -469,57 +657,23 @@ int scan_stage(FvmCtx* c, const AFArgs& A, int* iters, bool temp) {
   const long nwork = (long)nc * nchunk * g.nb;
   const long G = (nwork + 7) / 8 * 8;
   if (2 * G > c->nred) return FVM_ERR_SIZE;
-  // Q (or the FP32 residual): the right-hand-side kernel left it in A.su (natural layout); the
-  // J stage uses a line-major copy.  The iterate is the field itself for the FP64 I stage, else
-  // a work array (line-major for J).
-  double* q[3] = {};
-  for (int k = 0; k < nc; ++k) q[k] = S == 0 ? A.su[k] : c->afb[k][1];
-  double* xo[3] = {};
-  for (int k = 0; k < nc; ++k) xo[k] = (S == 0 && !DELTA) ? A.f[k] : c->afb[k][0];
-  double* fo[3] = {};
-  for (int k = 0; k < nc; ++k) fo[k] = A.f[k];
-  // device pointer table of this stage: q at [0..2], iterate at [3..5], field at [6..8]; the
-  // buffers are the context's own, so it is uploaded once and again only if they change
-  // (the temperature has a table of its own)
-  double* tab[9] = {q[0], q[1], q[2], xo[0], xo[1], xo[2], fo[0], fo[1], fo[2]};
-  double** dtab = temp ? c->scantab_t[S] : c->scantab[S];
-  double** htab = temp ? c->scantab_th[S] : c->scantab_h[S];
-  if (memcmp(tab, htab, sizeof(tab)) != 0) {
-    HIP_CHECK(hipMemcpyAsync(dtab, tab, sizeof(tab), hipMemcpyHostToDevice, st));
-    memcpy(htab, tab, sizeof(tab));
-  }
-  double* const* dq = dtab;
-  double* const* dxo = dtab + 3;
+  ScanBufs<T> B;
+  const int rp = scan_prepare<S, T>(c, A, false, B);
+  if (rp) return rp;
+  double* const* dq = B.tab;
+  double* const* dxo = B.tab + 3;
   T* bnd[2] = {reinterpret_cast<T*>(c->bnd[0]), reinterpret_cast<T*>(c->bnd[1])};
-  {
-    ProfScope pk(c, "af_scan_q");
-    if (S == 1) {
-      PtrSet8 qn{};
-      for (int k = 0; k < nc; ++k) qn.p[k] = A.su[k];
-      hipLaunchKernelGGL(k_scan_q1v<T>, dim3((d.ni - 1 + 31) / 32, (d.nj - 1 + 31) / 32, nc * (d.nk - 1)),
-                         dim3(256), 0, st, d, qn, dq);
-    } else if (!DELTA) {
-      hipLaunchKernelGGL(k_scan_seed, grid1((long)nc * g.nb * nchunk * g.n, 256), dim3(256), 0,
-                         st, d, A, nchunk, c->bnd[0]);
-    }
-    HIP_CHECK(hipGetLastError());
-  }
   // the FP32 change is resolved to its own precision
-  double tol = c->prm.af_tol > 0 ? c->prm.af_tol : 1e-14;
-  if (DELTA) tol = std::max(tol, 6e-8);
+  const double tol = std::max(c->prm.af_tol > 0 ? c->prm.af_tol : 1e-14, 6e-8);
   const int cap = nchunk + 1;
   int slot = 0, it = 0;
-  const T* const* lf;
-  if (DELTA)
-    lf = reinterpret_cast<const T* const*>(c->lf32[S]);
-  else
-    lf = reinterpret_cast<const T* const*>(temp ? c->lft[S] : c->lf[S]);
+  const T* const* lf = reinterpret_cast<const T* const*>(c->lf32[S]);
   for (;;) {
     {
       ProfScope pk(c, S == 0 ? "k_scan_pass_i" : "k_scan_pass_j");
-      auto kern = it > 0 ? k_scan_pass<S, R, true, T> : k_scan_pass<S, R, false, T>;
+      auto kern = it > 0 ? k_scan_pass<S, R, true> : k_scan_pass<S, R, false>;
       // the change form's first pass also sets the field's BCU ghosts: four per lane
-      const long ng = DELTA && it == 0 ? (nc * bc_ghost_count(d) + 255) / 256 : 0;
+      const long ng = it == 0 ? (nc * bc_ghost_count(d) + 255) / 256 : 0;
       hipLaunchKernelGGL(kern, dim3((unsigned)(G + ng)), dim3(64), 0, st, d, A, lf[0], lf[1],
                          lf[2], lf[3], (const double* const*)dq, dxo, bnd[slot], bnd[slot ^ 1],
                          nchunk, c->red, tol, c->sink, G);
@@ -541,14 +695,12 @@ int scan_stage(FvmCtx* c, const AFArgs& A, int* iters, bool temp) {
     if (dm <= tol * xm || it >= cap) break;
   }
   if (S == 1) {
-    ProfScope pk(c, "af_scan_unpack");
-    hipLaunchKernelGGL(k_scan_unpack1<T>, dim3((d.ni - 1 + 63) / 64, (d.nj - 1 + 31) / 32, nc * (d.nk - 1)),
-                       dim3(256), 0, st, d, (const double* const*)dxo, dtab + 6);
-    HIP_CHECK(hipGetLastError());
-  } else if (DELTA) {
+    const int r = scan_unpack<T>(c, nc, B);
+    if (r) return r;
+  } else {
     ProfScope pk(c, "af_scan_add");
     PtrSet8 dl{}, f{};
-    for (int k = 0; k < nc; ++k) { dl.p[k] = xo[k]; f.p[k] = A.f[k]; }
+    for (int k = 0; k < nc; ++k) { dl.p[k] = B.xo[k]; f.p[k] = A.f[k]; }
     const int nkb = (d.nk - 1 + ADD0_KP - 1) / ADD0_KP;
     hipLaunchKernelGGL(k_scan_add0, dim3((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, nc * nkb),
                        dim3(64, 4, 1), 0, st, d, dl, f);
@@ -590,7 +742,32 @@ int fvm_af_scan_setup(FvmCtx* c) {
       else
         hipLaunchKernelGGL(k_scan_factor<1>, grid1(nl, 64), dim3(64), 0, st, d,
                            (const double* const*)c->dfa[1], a0, L[0], L[1], L[2], L[3]);
+      if (s == 0)
+        hipLaunchKernelGGL(k_scan_rho<0>, dim3(g.na), dim3(256), 0, st, d,
+                           (const double* const*)c->dfa[0], a0, c->red);
+      else
+        hipLaunchKernelGGL(k_scan_rho<1>, dim3(g.na), dim3(256), 0, st, d,
+                           (const double* const*)c->dfa[1], a0, c->red);
       HIP_CHECK(hipGetLastError());
+      std::vector<double> rho(g.na + 1);
+      HIP_CHECK(hipMemcpyAsync(rho.data(), c->red, rho.size() * sizeof(double),
+                               hipMemcpyDeviceToHost, st));
+      HIP_CHECK(hipStreamSynchronize(st));
+      // the line at which a sweep of line a0 and those after it starts: what it leaves out, the line
+      // before, reaches line a0 by less than 1e-20
+      std::vector<int> lead(g.na + 1, 1);
+      for (int a0l = 1; a0l <= g.na; ++a0l) {
+        int a = a0l;
+        for (double q = rho[a]; a > 1 && !(q <= 1e-20); q *= rho[a]) --a;
+        lead[a0l] = a;
+      }
+      if (!c->lead[set][s]) {
+        HIP_CHECK(hipMalloc((void**)&c->lead[set][s], lead.size() * sizeof(int)));
+        c->allocs.push_back(c->lead[set][s]);
+      }
+      HIP_CHECK(hipMemcpyAsync(c->lead[set][s], lead.data(), lead.size() * sizeof(int),
+                               hipMemcpyHostToDevice, st));
+      HIP_CHECK(hipStreamSynchronize(st));
     }
     if (c->prm.af_mode == 2) {  // FP32 copies of the momentum factors (correction form)
       for (int q = 0; q < 4; ++q) {
@@ -615,27 +792,35 @@ int fvm_af_scan_setup(FvmCtx* c) {
   return FVM_OK;
 }
 
-template <typename T>
-static int scan_stage_r(FvmCtx* c, int s, const AFArgs& A, int* iters, bool temp) {
-  const ScanGeo g = scan_geo(c->d, s);
-  const int R = (g.n + 63) / 64;
-  if (s == 0) {
-    if (R <= 3) return scan_stage<0, 3, T>(c, A, iters, temp);
-    if (R <= 4) return scan_stage<0, 4, T>(c, A, iters, temp);
-    if (R <= 6) return scan_stage<0, 6, T>(c, A, iters, temp);
-    return scan_stage<0, SC_R, T>(c, A, iters, temp);
-  }
-  if (R <= 3) return scan_stage<1, 3, T>(c, A, iters, temp);
-  if (R <= 4) return scan_stage<1, 4, T>(c, A, iters, temp);
-  if (R <= 6) return scan_stage<1, 6, T>(c, A, iters, temp);
-  return scan_stage<1, SC_R, T>(c, A, iters, temp);
-}
-
 int fvm_af_scan_stage(FvmCtx* c, int s, const AFArgs& A, int* iters, bool temp, bool delta) {
   if (A.nc < 1 || A.nc > 3 || (temp && !c->lft[s][0])) return FVM_ERR_ARG;
+  const int R = (scan_geo(c->d, s).n + 63) / 64;
   if (delta) {
     if (temp || !c->lf32[s][0]) return FVM_ERR_ARG;
-    return scan_stage_r<float>(c, s, A, iters, false);
+    if (s == 0) {
+      if (R <= 3) return scan_stage32<0, 3>(c, A, iters);
+      if (R <= 4) return scan_stage32<0, 4>(c, A, iters);
+      if (R <= 6) return scan_stage32<0, 6>(c, A, iters);
+      return scan_stage32<0, SC_R>(c, A, iters);
+    }
+    if (R <= 3) return scan_stage32<1, 3>(c, A, iters);
+    if (R <= 4) return scan_stage32<1, 4>(c, A, iters);
+    if (R <= 6) return scan_stage32<1, 6>(c, A, iters);
+    return scan_stage32<1, SC_R>(c, A, iters);
   }
-  return scan_stage_r<double>(c, s, A, iters, temp);
+  *iters = 1;
+  if (s == 0) {
+    if (R <= 1) return scan_stage64<0, 1>(c, A, temp);
+    if (R <= 2) return scan_stage64<0, 2>(c, A, temp);
+    if (R <= 3) return scan_stage64<0, 3>(c, A, temp);
+    if (R <= 4) return scan_stage64<0, 4>(c, A, temp);
+    if (R <= 6) return scan_stage64<0, 6>(c, A, temp);
+    return scan_stage64<0, SC_R>(c, A, temp);
+  }
+  if (R <= 1) return scan_stage64<1, 1>(c, A, temp);
+  if (R <= 2) return scan_stage64<1, 2>(c, A, temp);
+  if (R <= 3) return scan_stage64<1, 3>(c, A, temp);
+  if (R <= 4) return scan_stage64<1, 4>(c, A, temp);
+  if (R <= 6) return scan_stage64<1, 6>(c, A, temp);
+  return scan_stage64<1, SC_R>(c, A, temp);
 }

@@ -505,7 +505,27 @@ int fvm_set_thermal(fvm_ctx* c, double pe) {
   return fvm_thermal_setup(c);
 }
 
-int fvm_iter_t(fvm_ctx* c) { return c ? fvm_k_iter_t(c) : FVM_ERR_ARG; }
+// Whether the FP64 line sweeps since sweeps_begin gave finite values; their kernels have ended.
+static void sweeps_begin(FvmCtx* c) { c->hmail[kMailBad] = 0.0; }
+static int sweeps_finite(FvmCtx* c) {
+  const volatile double* m = c->hmail;
+  if (m[kMailBad] == 0.0) return FVM_OK;
+  fprintf(stderr, "fvm_amd: non-finite AF stage iterate\n");
+  return FVM_ERR_NAN;
+}
+// the same at an entry point that runs the sweeps alone
+static int sweeps_check(FvmCtx* c, int r) {
+  if (r) return r;
+  double v;
+  r = fvm_fetch(c, c->scal, 1, &v);
+  return r ? r : sweeps_finite(c);
+}
+
+int fvm_iter_t(fvm_ctx* c) {
+  if (!c) return FVM_ERR_ARG;
+  sweeps_begin(c);
+  return sweeps_check(c, fvm_k_iter_t(c));
+}
 
 int fvm_writedata_fields(fvm_ctx* c) { return c ? fvm_k_writedata_fields(c) : FVM_ERR_ARG; }
 
@@ -630,7 +650,8 @@ int fvm_iter_u_c(fvm_ctx* c, int in, int inm, int ina, int inb, int inc, int ind
   if (comp < 0 || !f || !fn || !nl || !nl1 || !dif || !s || fn == f) return FVM_ERR_ARG;
   int r = ufar_fresh(c);
   if (r) return r;
-  return fvm_k_iter_u_one(c, comp, f, fn, nl, nl1, dif, s);
+  sweeps_begin(c);
+  return sweeps_check(c, fvm_k_iter_u_one(c, comp, f, fn, nl, nl1, dif, s));
 }
 
 int fvm_correct_c(fvm_ctx* c, int f, int s, double sign) {
@@ -657,7 +678,11 @@ int fvm_contra_vel(fvm_ctx* c) { return c ? fvm_k_contra_vel(c) : FVM_ERR_ARG; }
 int fvm_nl(fvm_ctx* c) { return c ? fvm_k_nl(c) : FVM_ERR_ARG; }
 int fvm_dif(fvm_ctx* c) { return c ? fvm_k_dif(c) : FVM_ERR_ARG; }
 int fvm_p_source(fvm_ctx* c) { return c ? fvm_k_p_source(c) : FVM_ERR_ARG; }
-int fvm_iter_u(fvm_ctx* c) { return c ? fvm_k_iter_u(c) : FVM_ERR_ARG; }
+int fvm_iter_u(fvm_ctx* c) {
+  if (!c) return FVM_ERR_ARG;
+  sweeps_begin(c);
+  return sweeps_check(c, fvm_k_iter_u(c));
+}
 
 int fvm_stress_tensor_dy(fvm_ctx* c, double* c_avg) {
   if (!c) return FVM_ERR_ARG;
@@ -710,6 +735,7 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
   if (!c) return FVM_ERR_ARG;
   fvm_step_info st{};
   int r;
+  sweeps_begin(c);
 #define CK(x) do { r = (x); if (r && r != FVM_ERR_NOCONV) return r; } while (0)
   CK(fvm_k_step_begin(c));                        // main.f90:42-48
   CK(fvm_k_nl_dif(c));                            // :51-57 and DIF :72-75 in one pass
@@ -738,6 +764,7 @@ int fvm_step(fvm_ctx* c, fvm_step_info* info) {
     r = fvm_mail_wait(c, mb, 17, c->hscal);
   }
 #undef CK
+  if (!r) r = sweeps_finite(c);
   if (r) return r;
   st.c_avg = c->prm.use_les ? c->hscal[0] : 0.0;
   st.c_t = (c->thermal && c->prm.use_les) ? c->hscal[1] : 0.0;

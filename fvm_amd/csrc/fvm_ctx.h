@@ -82,6 +82,8 @@ struct FvmCtx {
   bool af_scan[2] = {};
   double* lf[2][4] = {};
   float* lf32[2][4] = {};   // FP32 copies of lf (af_mode 2: FP32 change form)
+  int* lead[2][2] = {};  // FP64 line sweeps of u, v, w (0) and T (1), stages I and J: per line the
+                         // line at which a chunk that begins with it starts
   double* bnd[2] = {};
   long nbnd = 0;
   // reductions
@@ -201,6 +203,7 @@ struct ProfScope {
 
 // stage launchers (return FVM_OK or an error code)
 int fvm_fetch(FvmCtx* c, const double* src, int n, double* dst);
+constexpr int kMailBad = 50;  // mailbox slot an FP64 line sweep sets when a value is not finite
 Mailbox fvm_mail(FvmCtx* c);  // a fresh sequence number for a kernel that publishes itself
 int fvm_mail_wait(FvmCtx* c, const Mailbox& mb, int n, double* dst);
 int fvm_geom_setup(FvmCtx* c);
