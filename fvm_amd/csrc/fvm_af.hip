@@ -623,24 +623,25 @@ __global__ void k_copy_ghosts(Dims d, const double* __restrict__ src, double* ds
 // read of SU and the factors, one write of the result.  The components of a line sit in the
 // wavefronts of one workgroup (threadIdx.y), which load the shared factors together: one HBM
 // read of them serves all three.
-template <int NMAX>
+template <int NMAX, bool FOLD>
 __global__ void __launch_bounds__(192) k_af_thomas_k_reg(Dims d, AFArgs A,
                                                          const double* __restrict__ ta,
                                                          const double* __restrict__ td,
-                                                         const double* __restrict__ tb) {
+                                                         const double* __restrict__ tb,
+                                                         const double* __restrict__ ap0) {
   const int i = 1 + blockIdx.x * 64 + threadIdx.x;
   const int j = 1 + blockIdx.y;
   const int comp = threadIdx.y;
   if (i > d.ni - 1 || j > d.nj - 1) return;
   const GPW f = gpw(A.f[comp]);
-  const GP su = gp(A.su[comp]);
+  const GP su = FOLD ? (GP)f : gp(A.su[comp]);
   const int n = d.nk - 1;
   const long c0 = cidx(d, i, j, 0);
   // Rows are handled in blocks of KB: the operands of block b+1 are loaded before block b is
   // solved (the scheduling barrier keeps them there), so one memory latency covers KB rows
   // instead of each row waiting for its own loads.  Rows past n repeat row n and are never kept,
   // so no load sits behind a branch on n.
-  constexpr int KB = 8, NB = NMAX / KB;
+  constexpr int KB = NMAX > 32 ? 4 : 8, NB = NMAX / KB;
   static_assert(NMAX % KB == 0, "row blocks");
   double xs[NMAX];
   // the K ghosts of the stage input are the periodic partners, rows n and 1
@@ -649,16 +650,17 @@ __global__ void __launch_bounds__(192) k_af_thomas_k_reg(Dims d, AFArgs A,
 #pragma unroll
   for (int r = 0; r < KB; ++r) {
     const long c = c0 + (long)min(r + 1, n) * d.sk;
-    bs[r] = su[c]; ba[r] = ta[c]; bd[r] = td[c];
+    bs[r] = FOLD ? ap0[c] * su[c] : su[c]; ba[r] = ta[c]; bd[r] = td[c];
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    double ns[KB], na[KB], nd[KB];
+    double ns[KB], na[KB], nd[KB], np[KB];
     if (b + 1 < NB) {
 #pragma unroll
       for (int r = 0; r < KB; ++r) {
         const long c = c0 + (long)min((b + 1) * KB + r + 1, n) * d.sk;
         ns[r] = su[c]; na[r] = ta[c]; nd[r] = td[c];
+        if (FOLD) np[r] = ap0[c];
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -671,7 +673,10 @@ __global__ void __launch_bounds__(192) k_af_thomas_k_reg(Dims d, AFArgs A,
     }
     if (b + 1 < NB) {
 #pragma unroll
-      for (int r = 0; r < KB; ++r) { bs[r] = ns[r]; ba[r] = na[r]; bd[r] = nd[r]; }
+      for (int r = 0; r < KB; ++r) {
+        bs[r] = FOLD ? np[r] * ns[r] : ns[r];
+        ba[r] = na[r]; bd[r] = nd[r];
+      }
     }
   }
   double bt[KB];
@@ -794,11 +799,13 @@ __global__ void k_af_factor_k(Dims d, const double* const* __restrict__ fa,
 // The K-line sweep when its lines are independent: one thread per line and component, lanes
 // along I (coalesced), the reference's forward elimination and back substitution in its
 // operation order, in place.  With the I and J couplings identically zero the lagged-neighbour
-// sum C of the reference is exactly SU (the BCU additions to SU multiply the same zeros).
+// sum C of the reference is exactly SU (the BCU additions to SU multiply the same zeros).  With
+// ap0, where the stage's cross terms vanish too (xi_z = eta_z = 0), SU = AP0 x_in is formed here.
 __global__ void __launch_bounds__(192) k_af_thomas_k(Dims d, AFArgs A,
                                                      const double* __restrict__ ta,
                                                      const double* __restrict__ td,
-                                                     const double* __restrict__ tb) {
+                                                     const double* __restrict__ tb,
+                                                     const double* __restrict__ ap0) {
   const int i = 1 + blockIdx.x * 64 + threadIdx.x;
   const int j = 1 + blockIdx.y;
   const int comp = threadIdx.y;
@@ -811,7 +818,7 @@ __global__ void __launch_bounds__(192) k_af_thomas_k(Dims d, AFArgs A,
   double x = f[c0 + (long)n * d.sk], xn = f[c0 + d.sk];
   for (int k = 1; k <= n; ++k) {
     const long c = c0 + (long)k * d.sk;
-    x = (su[c] - ta[c] * x) / td[c];
+    x = ((ap0 ? ap0[c] * f[c] : su[c]) - ta[c] * x) / td[c];
     f[c] = x;
   }
   for (int k = n; k >= 1; --k) {
@@ -882,6 +889,25 @@ static int chunk_stage(FvmCtx* c, AFArgs& A, int* iters) {
   return FVM_OK;
 }
 
+// The K-line sweep with the factors ta, td, tb; ap0 as in k_af_thomas_k.  Lines of up to 64 rows keep
+// their forward results in registers, as many as the line asks for.  With a launch for SU before it
+// and 64 rows always, 32 x 64 x 16 cells took 3.3 + 12.3 us, now 6.0; 192 x 256 x 64 cells 31 + 63,
+// now 72; 384 x 512 x 128 cells (through memory) 284 + 788, now 836.  128 rows in registers spill:
+// 2136 us.
+static int thomas_k(FvmCtx* c, const AFArgs& A, const double* ta, const double* td,
+                    const double* tb, const double* ap0) {
+  const Dims d = c->d;
+  const int n = d.nk - 1;
+  auto kern = n <= 16   ? (ap0 ? k_af_thomas_k_reg<16, true> : k_af_thomas_k_reg<16, false>)
+              : n <= 32 ? (ap0 ? k_af_thomas_k_reg<32, true> : k_af_thomas_k_reg<32, false>)
+              : n <= 64 ? (ap0 ? k_af_thomas_k_reg<64, true> : k_af_thomas_k_reg<64, false>)
+                        : k_af_thomas_k;
+  hipLaunchKernelGGL(kern, dim3((d.ni - 1 + 63) / 64, d.nj - 1, 1), dim3(64, A.nc, 1), 0, c->stream,
+                     d, A, ta, td, tb, ap0);
+  HIP_CHECK(hipGetLastError());
+  return FVM_OK;
+}
+
 // With last_ghosts unset the ghosts of the third stage's input are not set where nothing reads
 // them (the K-line solve takes its end values from the periodic partners): the caller sets every
 // ghost of u, v, w next.
@@ -909,7 +935,9 @@ int fvm_k_iter_u(FvmCtx* c, bool last_ghosts) {
       A.dif[q] = c->dif[q]; A.s[q] = c->s[q]; A.su[q] = c->su[q];
     }
     A.ufar = c->ufar;
-    {
+    const bool klines = s == 2 && chunked && c->tk_a && c->af_zero_a[2] && c->af_zero_b[2];
+    const bool fold = klines && c->dd2_zero;  // the K-line sweep forms SU itself
+    if (!fold) {
       ProfScope ps(c, "af_rhs");
       const int qf = (s < 2 && chunked && c->af_scan[s]) ? 1 : 0;
       const double* const* fas = (const double* const*)c->dfa[s];
@@ -937,7 +965,6 @@ int fvm_k_iter_u(FvmCtx* c, bool last_ghosts) {
     }
     // boundary ghosts of the stage input (BCU, iter_u.f90:83,160,237); the change form's first
     // pass sets them itself
-    const bool klines = s == 2 && chunked && c->tk_a && c->af_zero_a[2] && c->af_zero_b[2];
     const bool scan = s < 2 && chunked && c->af_scan[s];
     int r = (scan && f32) || (klines && !last_ghosts) ? FVM_OK : fvm_k_bcu_ghosts(c, fld, 3);
     if (r) return r;
@@ -945,14 +972,8 @@ int fvm_k_iter_u(FvmCtx* c, bool last_ghosts) {
     if (klines) {
       // independent K-lines: the exact sweep in one pass
       ProfScope pk(c, "k_af_thomas_k");
-      const dim3 g((d.ni - 1 + 63) / 64, d.nj - 1, 1);
-      if (d.nk - 1 <= 64)
-        hipLaunchKernelGGL(k_af_thomas_k_reg<64>, g, dim3(64, A.nc, 1), 0, st, d, A, c->tk_a,
-                           c->tk_d, c->tk_b);
-      else
-        hipLaunchKernelGGL(k_af_thomas_k, g, dim3(64, A.nc, 1), 0, st, d, A, c->tk_a, c->tk_d,
-                           c->tk_b);
-      HIP_CHECK(hipGetLastError());
+      r = thomas_k(c, A, c->tk_a, c->tk_d, c->tk_b, fold ? c->ap0 : nullptr);
+      if (r) return r;
       c->af_iters[s] = 1;
     } else if (scan) {
       int it = 0;
@@ -1005,6 +1026,7 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
   for (int s = 0; s < nstage; ++s) {
     const bool chunked = c->prm.af_mode == 0 || c->prm.af_mode == 2;  // FP64 scans here
     const bool exact_k = s == 2 && chunked && c->tk_a && c->af_zero_a[2] && c->af_zero_b[2];
+    const bool fold = exact_k && c->dd2_zero;  // the K-line sweep forms SU itself
     const bool scan = s < 2 && chunked && c->af_scan[s];
     if (!exact_k && !scan && c->prm.af_mode != 1) {
       fprintf(stderr, "fvm_amd: ITER_U of one component needs line-separable stage couplings "
@@ -1031,7 +1053,7 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
       if (s == 1)
         hipLaunchKernelGGL((k_af_rhs_km<1, false, 1>), gk, kBlk, 0, st, d, kc, A,
                            (const double* const*)c->dafp[1], c->ap0, c->prm.re, fas, qf, 0, c->prm.dtime, c->geo);
-      if (s == 2)
+      if (s == 2 && !fold)
         hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm,
                            c->djac, c->ap0, c->prm.re, fas, qf, dz);
       HIP_CHECK(hipGetLastError());
@@ -1040,14 +1062,8 @@ int fvm_k_iter_u_one(FvmCtx* c, int comp, double* f, const double* fn, const dou
     if (r) return r;
     ProfScope ps(c, s == 0 ? "af_sweep_i" : (s == 1 ? "af_sweep_j" : "af_sweep_k"));
     if (exact_k) {
-      const dim3 g((d.ni - 1 + 63) / 64, d.nj - 1, 1);
-      if (d.nk - 1 <= 64)
-        hipLaunchKernelGGL(k_af_thomas_k_reg<64>, g, dim3(64, 1, 1), 0, st, d, A, c->tk_a,
-                           c->tk_d, c->tk_b);
-      else
-        hipLaunchKernelGGL(k_af_thomas_k, g, dim3(64, 1, 1), 0, st, d, A, c->tk_a, c->tk_d,
-                           c->tk_b);
-      HIP_CHECK(hipGetLastError());
+      r = thomas_k(c, A, c->tk_a, c->tk_d, c->tk_b, fold ? c->ap0 : nullptr);
+      if (r) return r;
     } else if (scan) {
       int it = 0;
       r = fvm_af_scan_stage(c, s, A, &it);
@@ -1180,7 +1196,7 @@ int fvm_k_iter_t(FvmCtx* c) {
         auto kern = c->plane ? k_af_rhs_km<1, true, 3, false, kGeoPlane> : k_af_rhs_km<1, true>;
         hipLaunchKernelGGL(kern, gk, kBlk, 0, st, d, kc, A, (const double* const*)c->dafp[1], c->ap0t, c->pe, fas, 1, 0, c->prm.dtime, c->geo);
       }
-      if (s == 2) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0t, c->pe, fas, 0, c->dd2_zero ? 1 : 0);
+      if (s == 2 && !c->dd2_zero) hipLaunchKernelGGL(k_af_rhs<2>, gi, kBlk, 0, st, d, A, (const double* const*)c->dm, c->djac, c->ap0t, c->pe, fas, 0, 0);
       HIP_CHECK(hipGetLastError());
     }
     // iter_t.f90:84,150,226; nothing reads the third stage's ghosts before the final BCT
@@ -1192,14 +1208,8 @@ int fvm_k_iter_t(FvmCtx* c) {
       r = fvm_af_scan_stage(c, s, A, &it, true);
       if (r) return r;
     } else {
-      const dim3 g((d.ni - 1 + 63) / 64, d.nj - 1, 1);
-      if (d.nk - 1 <= 64)
-        hipLaunchKernelGGL(k_af_thomas_k_reg<64>, g, dim3(64, 1, 1), 0, st, d, A, c->tk_at,
-                           c->tk_dt, c->tk_bt);
-      else
-        hipLaunchKernelGGL(k_af_thomas_k, g, dim3(64, 1, 1), 0, st, d, A, c->tk_at, c->tk_dt,
-                           c->tk_bt);
-      HIP_CHECK(hipGetLastError());
+      r = thomas_k(c, A, c->tk_at, c->tk_dt, c->tk_bt, c->dd2_zero ? c->ap0t : nullptr);
+      if (r) return r;
     }
   }
   return fvm_k_bct_ghosts(c, c->t);  // BCT(T, T_N), main.f90:147
