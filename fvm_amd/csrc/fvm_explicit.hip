@@ -901,16 +901,21 @@ __global__ void __launch_bounds__(256) k_calccoef2d(Dims d, const double* __rest
       const double dudn = (u[c] * s2 - v[c] * c2 - vel_rot) / dn1;
       tm[0][t] = 2.0 * p[c] * area * ct;
       tm[1][t] = 2.0 * p[c] * area * st;
-      tm[2][t] = (2.0 / re) * dudn * area * st;
+      tm[2][t] = -((2.0 / re) * dudn * area * st);  // added: the others are subtracted
       tm[3][t] = (2.0 / re) * dudn * area * ct;
     }
     __syncthreads();
-    if (t < 4) {
+    if (t < 4) {  // 16 LDS reads in flight ahead of the serial chain of sums
       const int m = min(256, d.nj - j0);
-      if (t == 2)
-        for (int q = 0; q < m; ++q) acc = acc + tm[2][q];
-      else
-        for (int q = 0; q < m; ++q) acc = acc - tm[t][q];
+      int q = 0;
+      for (; q + 16 <= m; q += 16) {
+        double x[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] = tm[t][q + e];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc = acc - x[e];
+      }
+      for (; q < m; ++q) acc = acc - tm[t][q];
     }
     __syncthreads();
   }

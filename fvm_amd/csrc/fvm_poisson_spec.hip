@@ -488,10 +488,14 @@ __global__ void k_avg_faces(Dims d, const double* __restrict__ pdI, const double
 }
 
 // Largest power-of-two column count whose two LDS buffers and twiddle table fit in lds_max
-// bytes (at least 1).
-inline int fft_cols(int n, size_t elem, size_t lds_max, int cap) {
+// bytes (at least 1), less while the transforms of cols columns in rows planes are fewer than two
+// workgroups per CU, down to low.  On 32 x 64 x 16 cells with all columns that fit, 16 workgroups of
+// 32 pairs, a J transform took 11 us and its inverse 12, a K transform 6.4;
+// so 5.4, 6.5 and 4.6.
+inline int fft_cols(int n, size_t elem, size_t lds_max, int cap, long cols, long rows, int low) {
   int c = 1;
   while (2 * c <= cap && (size_t)(2 * (2 * c) * n + n) * elem <= lds_max) c *= 2;
+  while (c > low && (cols + c - 1) / c * rows < 512) c /= 2;
   return c;
 }
 
@@ -543,8 +547,8 @@ int sep_init(FvmCtx* c, SepState& st, SepData<T>& S, const std::vector<double>& 
                         hipMemcpyHostToDevice));
   }
   // columns per workgroup: two buffers and the twiddles in at most 64 KB of LDS
-  S.colsJ = fft_cols(nj1, sizeof(Cx<T>), 64 * 1024, 32);
-  S.colsK = fft_cols(nk1, sizeof(Cx<T>), 64 * 1024, 64);
+  S.colsJ = fft_cols(nj1, sizeof(Cx<T>), 64 * 1024, 32, (n1 + 1) / 2, nk1, 2);
+  S.colsK = fft_cols(nk1, sizeof(Cx<T>), 64 * 1024, 64, n1, st.MJ, 4);
   hipLaunchKernelGGL(k_mode_factor, dim3((st.MJ + 63) / 64, nk1), dim3(64), 0, c->stream, n1,
                      st.MJ, nj1, nk1, dE_dev, dW_dev, dN_dev, dT_dev, S.invd, S.bf);
   HIP_CHECK(hipGetLastError());
