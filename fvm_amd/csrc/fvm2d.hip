@@ -230,60 +230,24 @@ struct LineOps {
   float cdn[R], q[R], iv[R], na[R], bf[R], xo[R];
 };
 
-// R consecutive floats from a 16-byte (R % 4 == 0) or 8-byte (R % 2 == 0) aligned address
-typedef float sw_f4 __attribute__((ext_vector_type(4)));
-typedef float sw_f2 __attribute__((ext_vector_type(2)));
-template <int R>
-__device__ __forceinline__ void load_rows(float (&d)[R], gptr<const float> p) {
-  if constexpr (R % 4 == 0) {
-#pragma unroll
-    for (int k = 0; k < R / 4; ++k) {
-      const sw_f4 v = ((gptr<const sw_f4>)p)[k];
-      d[4 * k] = v.x; d[4 * k + 1] = v.y; d[4 * k + 2] = v.z; d[4 * k + 3] = v.w;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < R / 2; ++k) {
-      const sw_f2 v = ((gptr<const sw_f2>)p)[k];
-      d[2 * k] = v.x; d[2 * k + 1] = v.y;
-    }
-  }
-}
-
 // roff: the offset of row 0 in a line (the padded FP32 J-line-major layout)
-template <int R, int DIR, bool EARLY>
+template <int R, bool EARLY>
 __device__ inline void sweep_load(LineOps<R>& o, gptr<const float> F, gptr<const float> Q,
                                   gptr<const float> invd, gptr<const float> na,
-                                  gptr<const float> bf, gptr<const float> cdn, long base, long rs,
-                                  long roff, long dnoff, int n, int r0) {
-  if constexpr (DIR == 1 && R % 2 == 0) {
-    // a lane's rows as vectors (row r at base + roff + 1 + r; dnoff = 0 in this direction).
-    // The last lane's rows past n lie inside the padded plane and are never used.
-    const long c0 = base + roff + 1 + r0;
-    load_rows<R>(o.cdn, cdn + c0);
-    load_rows<R>(o.q, Q + c0);
-    load_rows<R>(o.iv, invd + c0);
-    load_rows<R>(o.na, na + c0);
-    load_rows<R>(o.bf, bf + c0);
-    if (EARLY) load_rows<R>(o.xo, F + c0);
-    else {
+                                  gptr<const float> bf, gptr<const float> cdn, long base, long roff,
+                                  long dnoff, int n, int r0) {
+  // a lane's rows as vectors; rows past n (up to R - 1 of them: the ghost and the next line) and the
+  // lanes past n are not used
+  const long c0 = base + roff + 1 + (r0 < n ? r0 : 0);
+  row_vec<R>(o.cdn, cdn + c0 + dnoff);
+  row_vec<R>(o.q, Q + c0);
+  row_vec<R>(o.iv, invd + c0);
+  row_vec<R>(o.na, na + c0);
+  row_vec<R>(o.bf, bf + c0);
+  if (EARLY) row_vec<R>(o.xo, F + c0);  // the previous pass's values
+  else {
 #pragma unroll
-      for (int q = 0; q < R; ++q) o.xo[q] = 0.0f;
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = r0 + q;
-      if (r < n) {
-        const long c = base + roff + rs * (r + 1);
-        o.cdn[q] = cdn[c + dnoff];
-        o.q[q] = Q[c];
-        o.iv[q] = invd[c];
-        o.na[q] = na[c];
-        o.bf[q] = bf[c];
-        o.xo[q] = EARLY ? F[c] : 0.0f;  // the previous pass's value of the row
-      }
-    }
+    for (int q = 0; q < R; ++q) o.xo[q] = 0.0f;
   }
 }
 
@@ -332,14 +296,14 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
     prev[q] = v;
   }
   LineOps<R> cur, nxt;
-  sweep_load<R, DIR, EARLY>(cur, F, Q, invd, na, bf, cdn, ls * a0, rs, roff, dnoff, n, r0);
+  sweep_load<R, EARLY>(cur, F, Q, invd, na, bf, cdn, ls * a0, roff, dnoff, n, r0);
   bool stopped = false;
   T xrun = (T)0;
   int L = a0;
   for (; L <= a1; ++L) {
     const long base = ls * L;
     if (L < a1)
-      sweep_load<R, DIR, EARLY>(nxt, F, Q, invd, na, bf, cdn, base + ls, rs, roff, dnoff, n, r0);
+      sweep_load<R, EARLY>(nxt, F, Q, invd, na, bf, cdn, base + ls, roff, dnoff, n, r0);
     T al[R], be[R], bb[R];
     T At = (T)0, Bt = (T)1;
 #pragma unroll

@@ -214,35 +214,6 @@ __global__ void __launch_bounds__(256) k_scan_rho(Dims d, const double* const* _
   if (t == 0) rho[a] = sh[0];
 }
 
-// R consecutive elements from an address aligned to 4 (R % 4 == 0) or 2 (R % 2 == 0) elements
-typedef float sc_f4 __attribute__((ext_vector_type(4)));
-typedef float sc_f2 __attribute__((ext_vector_type(2)));
-typedef double sc_d2 __attribute__((ext_vector_type(2)));
-template <int R>
-__device__ __forceinline__ void load_rows(float (&d)[R], gptr<const float> p) {
-  if constexpr (R % 4 == 0) {
-#pragma unroll
-    for (int k = 0; k < R / 4; ++k) {
-      const sc_f4 v = ((gptr<const sc_f4>)p)[k];
-      d[4 * k] = v.x; d[4 * k + 1] = v.y; d[4 * k + 2] = v.z; d[4 * k + 3] = v.w;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < R / 2; ++k) {
-      const sc_f2 v = ((gptr<const sc_f2>)p)[k];
-      d[2 * k] = v.x; d[2 * k + 1] = v.y;
-    }
-  }
-}
-template <int R>
-__device__ __forceinline__ void load_rows(double (&d)[R], gptr<const double> p) {
-#pragma unroll
-  for (int k = 0; k < R / 2; ++k) {
-    const sc_d2 v = ((gptr<const sc_d2>)p)[k];
-    d[2 * k] = v.x; d[2 * k + 1] = v.y;
-  }
-}
-
 __device__ inline double shfl_up_d(double v, int o) { return __shfl_up(v, o, 64); }
 __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o, 64); }
 
@@ -383,6 +354,9 @@ __global__ void __launch_bounds__(64) k_scan_lead(Dims d, AFArgs A, const double
 // is FP32; the FP64 field is updated with the converged change afterwards.  The stage's field is
 // then neither read nor written, so the workgroups past the first G of the first pass set its
 // BCU ghosts (bc_ghost), which the right-hand sides of the next stage read: one launch less.
+// Loads of rows one by one (I lines: the J lines' were vectors) took the first I pass 55 us on
+// 192 x 256 x 64 cells and 473 on 384 x 512 x 128, row vectors 42 and 319; loading further lines ahead
+// gains nothing (44).
 template <int S, int R, bool EARLY>
 __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float* __restrict__ beta,
                                                   const float* __restrict__ invd,
@@ -426,35 +400,24 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
         v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
       xp[r] = v;
     }
-    // Operands of one line.  Rows past n (the last lane's tail) read row n and are never kept,
-    // and the next line is always fetched (the last line again at the end of the chunk): with
-    // no load or store behind a branch the compiler counts the loads in flight exactly and
-    // waits only for the ones it needs, so the next line's loads overlap this line's scans.
+    // Operands of one line.  Rows past n (up to R - 1 of them: the ghost and the next line) and the
+    // lanes past n are never kept, and the next line is always fetched (the last line again at the
+    // end of the chunk): with no load or store behind a branch the compiler counts the loads in
+    // flight exactly and waits only for the ones it needs, so the next line's loads overlap this
+    // line's scans.
     T be[R], iv[R], bv[R], cm[R], qv[R], xv[R];
+    const int pc = p0 <= g.n ? p0 : 1;
     auto load = [&](int a) {
-      const long lb = g.ls_a * a + g.ls_b * b + g.off;
-      if constexpr (S == 1 && R % 2 == 0) {
-        // J lines: a lane's rows p0 .. p0+R-1 as vectors (lb + p0 is a multiple of 4 for R = 4,
-        // 8 and of 2 for R = 6); rows past n lie in the padded line (or the next one, or the
-        // slack after the last) and are never kept
-        const long o = lb + p0;
-        load_rows<R>(be, glb(beta) + o);
-        load_rows<R>(iv, glb(invd) + o);
-        load_rows<R>(bv, glb(bb) + o);
-        load_rows<R>(cm, glb(cam) + o);
-        load_rows<R>(qv, qc + o);
-        if (EARLY) load_rows<R>(xv, (gptr<const T>)xc + o);
-        else {
+      const long o = g.ls_a * a + g.ls_b * b + g.off + pc;
+      row_vec<R>(be, glb(beta) + o);
+      row_vec<R>(iv, glb(invd) + o);
+      row_vec<R>(bv, glb(bb) + o);
+      row_vec<R>(cm, glb(cam) + o);
+      row_vec<R>(qv, qc + o);
+      if (EARLY) row_vec<R>(xv, (gptr<const T>)xc + o);  // the previous pass's values
+      else {
 #pragma unroll
-          for (int r = 0; r < R; ++r) xv[r] = (T)0;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const long o = lb + min(p0 + r, g.n);
-          be[r] = beta[o]; iv[r] = invd[o]; bv[r] = bb[o]; cm[r] = cam[o]; qv[r] = qc[o];
-          xv[r] = EARLY ? xc[o] : (T)0;  // the previous pass's value of the line
-        }
+        for (int r = 0; r < R; ++r) xv[r] = (T)0;
       }
     };
     load(a0);

@@ -362,6 +362,29 @@ __device__ __forceinline__ void row_pairs(double (&d)[R], gptr<const double> p) 
   if constexpr (R % 2 == 1) d[R - 1] = p[R - 1];
 }
 
+// the same for floats, by loads of up to 16 bytes (aligned to 4 as the rows are)
+typedef float sw_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float sw_f3 __attribute__((ext_vector_type(3), aligned(4)));
+typedef float sw_f2 __attribute__((ext_vector_type(2), aligned(4)));
+template <int R>
+__device__ __forceinline__ void row_vec(float (&d)[R], gptr<const float> p) {
+#pragma unroll
+  for (int k = 0; k < R / 4; ++k) {
+    const sw_f4 v = *(gptr<const sw_f4>)(p + 4 * k);
+    d[4 * k] = v.x; d[4 * k + 1] = v.y; d[4 * k + 2] = v.z; d[4 * k + 3] = v.w;
+  }
+  constexpr int B = R / 4 * 4;
+  if constexpr (R % 4 == 3) {
+    const sw_f3 v = *(gptr<const sw_f3>)(p + B);
+    d[B] = v.x; d[B + 1] = v.y; d[B + 2] = v.z;
+  } else if constexpr (R % 4 == 2) {
+    const sw_f2 v = *(gptr<const sw_f2>)(p + B);
+    d[B] = v.x; d[B + 1] = v.y;
+  } else if constexpr (R % 4 == 1) {
+    d[B] = p[B];
+  }
+}
+
 // up to eight arrays passed by value (no device pointer table needed)
 struct PtrSet8 {
   double* p[8];
