@@ -79,11 +79,11 @@ __device__ __forceinline__ gptr<T> glb(T* p) { return (gptr<T>)p; }
 //   strain and test filter  149 -> 138  1153 -> 1028    predictor's p gradient   76 -> 43  614 -> 283
 //   SGS model coefficient   181 -> 157  1232 -> 1088    corrector with CFL      135 -> 88  989 -> 687
 //   SGS stress divergence   111 -> 75    979 -> 612     Poisson residual         52 -> 48  438 -> 304
-//   convection, diffusion   131 -> 129   981 -> 892     predictor correction    100 -> 86  880 -> 619
+//   convection, diffusion   131 -> 119   981 -> 871     predictor correction    100 -> 86  880 -> 619
 //   AF right-hand side, I   167 -> 125  1298 -> 936     the same, J             100 -> 78  796 -> 526
 // The convection/diffusion pass and the Poisson residual, which need J^-1 Q_ij of four neighbours
 // for few arrays of their own, read the stored arrays on plane kz[k], of which the
-// caches hold the few that differ; forming them anew took 150 and 46 us, 897 and 298 us.
+// caches hold the few that differ; forming them anew took 150 (129) and 46 us, 897 (892) and 298 us.
 constexpr int kGeoAny = 0, kGeoXz0 = 1, kGeoPlane = 2;
 // metric a of the table (grouped per Cartesian component: xi_s, eta_s, zeta_s for s = x, y, z) at
 // cell c; a is a compile-time constant at every call, so the choice folds away.  The products and

@@ -96,13 +96,16 @@ __global__ void k_nl(Dims d, const double* __restrict__ ju0, const double* __res
 // stencils are read from HBM once per column; J^-1 Q13, J^-1 Q23 and D_T of the planes K+-1
 // ride along in registers.
 constexpr int DF_RES = 1024;  // workgroups of k_dif_km resident at a time (four per CU)
+constexpr int DF_RES_PLANE = 768;  // in the plane form, whose loads ahead take more registers
 
 // With WNL set the same pass also forms NL(IN, NLOUT) of k_nl (RLES/nl.f90:23-31, its operation
 // order) from the staged planes and the face fluxes of ju (ju2 of the planes K+-1 in registers):
 // the whole step runs NL and DIF in one pass over u_n, v_n, w_n (DIF does not depend on NL or on
-// the SGS term added to NL in between).
+// the SGS term added to NL in between).  Bound by the latency of a plane's loads: ahead by a plane
+// (plane form; the occupancy falls from four waves to three), 192 x 256 x 64 cells took 119 us for
+// 129, 384 x 512 x 128 871 for 892; before the barrier instead of after it, 32 x 64 x 16 7.1 for 8.8.
 template <int NC, bool WNL = false, int G = kGeoAny>
-__global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
+__global__ void __launch_bounds__(256, G == kGeoPlane ? 3 : (NC < 4 ? 4 : 1)) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
                                                 const double* __restrict__ pdJ,
                                                 const double* __restrict__ pdK,
                                                 const double* __restrict__ jq12,
@@ -131,32 +134,60 @@ __global__ void __launch_bounds__(256) k_dif_km(Dims d, int kc, const double* __
   // the I boundaries have J^-1 Q13, J^-1 Q23 terms
   constexpr bool PL = G == kGeoPlane;
   const bool ed = geo_edge(d, i), ed1 = geo_edge(d, i, 1);
+  // the tile values and own-column values of a plane, in the plane form loaded one plane ahead (in
+  // flight while the cells of the plane before are formed)
+  constexpr bool PF = PL;
+  constexpr bool ST = PF || NC < 4;  // else straight to LDS: four components would spill
+  double tv[SF_NQ][NC], n13 = 0.0, n23 = 0.0, nk = 0.0, nz = 0.0;
+  auto load = [&](int kp) {
+#pragma unroll
+    for (int h = 0; h < (ST ? SF_NQ : 0); ++h) {
+      const int q = min(tid + 256 * h, SF_P - 1);
+      const long c = cidx(d, min((int)bb.x * 64 + q % SF_W, d.ni),
+                          min((int)bb.y * 4 + q / SF_W, d.nj), kp);
+#pragma unroll
+      for (int comp = 0; comp < NC; ++comp) tv[h][comp] = gp(cs.in[comp])[c];
+    }
+    const int im = act ? i : 1, jm = act ? j : 1;
+    const long cp = cidx(d, im, jm, kp);
+    if (PL) {
+      nk = jq33[cidx(d, im, jm, geo.plane(kp))];
+    } else {
+      n13 = jq13[cp];
+      n23 = jq23[cp];
+      nk = pdK[cp];
+    }
+    if (WNL) nz = ju2[cp];
+  };
+  if (PF) load(k0 - 1);
   for (int kp = k0 - 1; kp <= k1 + 1; ++kp) {
     const int slot = (kp - (k0 - 1)) % 3;
+    if (!PF) load(kp);
     __syncthreads();  // plane kp - 3, held in this slot, is no longer read
-    for (int q = tid; q < SF_P; q += 256) {
-      const int gi = min(bb.x * 64 + q % SF_W, d.ni);
-      const int gj = min(bb.y * 4 + q / SF_W, d.nj);
-      const long c = cidx(d, gi, gj, kp);
+    if constexpr (ST) {
 #pragma unroll
-      for (int comp = 0; comp < NC; ++comp) sh[comp][slot][q] = gp(cs.in[comp])[c];
-    }
-    j13[0] = j13[1]; j13[1] = j13[2];
-    j23[0] = j23[1]; j23[1] = j23[2];
-    pk[0] = pk[1]; pk[1] = pk[2];
-    z2[0] = z2[1]; z2[1] = z2[2];
-    if (act) {
-      const long cp = cidx(d, i, j, kp);
-      if (PL) {
-        pk[2] = jq33[cidx(d, i, j, geo.plane(kp))];
-      } else {
-        j13[2] = jq13[cp];
-        j23[2] = jq23[cp];
-        pk[2] = pdK[cp];
+      for (int h = 0; h < SF_NQ; ++h) {
+        const int q = tid + 256 * h;
+        if (q < SF_P) {
+#pragma unroll
+          for (int comp = 0; comp < NC; ++comp) sh[comp][slot][q] = tv[h][comp];
+        }
       }
-      if (WNL) z2[2] = ju2[cp];
+    } else {
+      for (int q = tid; q < SF_P; q += 256) {
+        const int gi = min(bb.x * 64 + q % SF_W, d.ni);
+        const int gj = min(bb.y * 4 + q / SF_W, d.nj);
+        const long c = cidx(d, gi, gj, kp);
+#pragma unroll
+        for (int comp = 0; comp < NC; ++comp) sh[comp][slot][q] = gp(cs.in[comp])[c];
+      }
     }
+    j13[0] = j13[1]; j13[1] = j13[2]; j13[2] = n13;
+    j23[0] = j23[1]; j23[1] = j23[2]; j23[2] = n23;
+    pk[0] = pk[1]; pk[1] = pk[2]; pk[2] = nk;
+    z2[0] = z2[1]; z2[1] = z2[2]; z2[2] = nz;
     __syncthreads();
+    if (PF && kp + 1 <= k1 + 1) load(kp + 1);
     if (kp < k0 + 1 || !act) continue;
     const int k = kp - 1;
     const int pl[3] = {(slot + 1) % 3, (slot + 2) % 3, slot};
@@ -1004,7 +1035,7 @@ int fvm_k_nl_dif(FvmCtx* c) {
   if (c->thermal) std::swap(c->adv, c->adv1);
   ProfScope ps(c, "nl_dif");
   const Dims d = c->d;
-  const int kc = march_planes(d, DF_RES);
+  const int kc = march_planes(c->d, c->plane ? DF_RES_PLANE : DF_RES);
   const dim3 g = march_grid(d, kc);
   const CompSet cs = {{c->un, c->vn, c->wn, c->tn}, {c->dif[0], c->dif[1], c->dif[2], c->dift}};
   const CompSet nlo = {{nullptr, nullptr, nullptr, nullptr}, {c->nl[0], c->nl[1], c->nl[2], c->adv}};
