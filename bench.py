@@ -41,34 +41,33 @@ KERNEL_BYTES = {
     # the same pass in the FP32 change form: FP32 factors 16 bytes shared, {r} -> {delta}
     # 3 x 8 bytes
     "k_scan_pass_i/f32": (40, 1), "k_scan_pass_j/f32": (40, 1),
-    # exact K-line sweep: Thomas factors {A, D, B} shared, {SU} -> {x} per component
-    "k_af_thomas_k": (72, 1),
+    # exact K-line sweep: Thomas factors {A, D, B} and 2 Re J/dt shared, {x_in} -> {x} per
+    # component
+    "k_af_thomas_k": (80, 1),
     # chunked fallback pass over the 3 components: {phi_in, SU, J, 3 stage metric products}
     # -> phi_out = 7 doubles per cell and component
     "k_af_chunk_i": (56, 3), "k_af_chunk_j": (56, 3), "k_af_chunk_k": (56, 3),
-    # The metric sets below count 7 of the 9 metrics: xi_z and eta_z vanish identically on the
-    # extruded grid and are not read.
-    # strain rates fused with the 27-point test filter: {u,v,w, xi 7} -> {S 6, |S|, u^ 3}
-    "k_strain_filter": (8 * 20, 1),
-    # AF right-hand side, stage 1: {phi 3 (= U_N at the first stage of a step), 6 metric
-    # products, 2 Re J/dt, NL 3, NL_NM1 3, DIF 3, S 3, 3 face coefficients} -> SU 3; stage 2:
-    # {phi 3, products 6, 2 Re J/dt, faces 3} -> SU 3
-    "k_af_rhs_i": (8 * 28, 1), "k_af_rhs_j": (8 * 16, 1),
-    # Poisson residual (mixed form): {p, rhs, D_E, D_N, D_T, J^-1 Q12, Q13, Q23} -> r (FP32)
-    "k_residual": (8 * 8 + 4, 1),
-    # DIF: {u_n, v_n, w_n, D_E, D_N, D_T, J^-1 Q12, Q13, Q23} -> DIF 3
-    "dif": (8 * 12, 1),
-    # NL and DIF in one pass (the step): {u_n, v_n, w_n, JU 3, D_E, D_N, D_T, J^-1 Q12, Q13,
-    # Q23} -> {NL 3, DIF 3}
-    "nl_dif": (8 * 18, 1),
-    # P_SOURCE + projection: {p, J, xi 7, u, v, w} -> {S 3, u, v, w}
-    "psource_correct": (8 * 18, 1),
-    # Germano identity terms: {u,v,w, u^ 3, xi 7, S 6, Delta^2} -> workgroup sums of LM, MM
-    # (|S| is formed from S as it is staged)
-    "k_lm": (8 * 20, 1),
-    # SGS divergence in the step: {xi 7, nu_t, S 6, J, NL 3} -> {NL 3} (SGS_x,y,z are formed
-    # when they are read)
-    "k_sgs_div": (8 * 21, 1),
+    # The sets below are those of the plane form (extruded grids from 2^19 cells): the metrics are
+    # formed from a plane of cross-section derivatives, the other geometry is read on the few K
+    # planes that differ, and neither counts per cell.
+    # strain rates fused with the 27-point test filter: {u,v,w} -> {S 6, |S|, u^ 3}
+    "k_strain_filter": (8 * 13, 1),
+    # AF right-hand side, stage 1: {phi 3 (= U_N at the first stage of a step), NL 3, NL_NM1 3,
+    # DIF 3, S 3} -> r 3 (FP32); stage 2: {phi 3} -> r 3 (FP32)
+    "k_af_rhs_i": (8 * 15 + 4 * 3, 1), "k_af_rhs_j": (8 * 3 + 4 * 3, 1),
+    # Poisson residual (mixed form): {p, rhs} -> r (FP32)
+    "k_residual": (8 * 2 + 4, 1),
+    # DIF: {u_n, v_n, w_n} -> DIF 3
+    "dif": (8 * 6, 1),
+    # NL and DIF in one pass (the step): {u_n, v_n, w_n, JU 3} -> {NL 3, DIF 3}
+    "nl_dif": (8 * 12, 1),
+    # P_SOURCE + projection: {p, u, v, w} -> {S 3, u, v, w}
+    "psource_correct": (8 * 10, 1),
+    # Germano identity terms: {u,v,w, u^ 3, S 6} -> workgroup sums of LM, MM (|S| is formed from
+    # S as it is staged)
+    "k_lm": (8 * 12, 1),
+    # SGS divergence in the step: {S 6, NL 3} -> {NL 3} (SGS_x,y,z are formed when they are read)
+    "k_sgs_div": (8 * 12, 1),
 }
 
 
@@ -265,16 +264,12 @@ KERNEL_BYTES_2D = {
     # phase A: {u, v, p, J, xi_x, xi_y, eta_x, eta_y, D_E, D_N, J Q12, 2 Re J/dt, stage-1 cross
     # weights, AN, NLX, NLY} -> {U_N, V_N, NL 2, DIF 2, S 2, SU 2}
     "k2_explicit": 8 * 26,
-    # I-line sweep: factors {1/D, beta, B, AN} + per component {SU, x_old, x}
-    "k2_sweep_i": 8 * 10,
-    # J-line sweep: factors {1/D, beta, B, AE, AW} + per component {SU, x_old, x}
-    "k2_sweep_j": 8 * 11,
-    # stage-2 right-hand side: {u, v, 2 Re J/dt, cross weights, AE} -> SU 2
-    "k2_rhs2": 8 * 7,
-    # predictor correction: {u, v, S 2, J} -> {u, v}
+    # I- and J-line sweep: factors {1/D, beta, B, AN or AW} + per component {SU, x}
+    "k2_sweep_i": 8 * 8, "k2_sweep_j": 8 * 8,
+    # stage-2 right-hand side: {u, v, 2 Re J/dt, cross weights, AE} -> {SU 2, x_in 2}, J-line-major
+    "k2_rhs2": 8 * 9,
+    # predictor correction: {u, v (J-line-major), S 2, J} -> {u, v}
     "k2_correct": 8 * 7,
-    # Poisson source: {u, v, J, 4 metrics} -> RHS
-    "k2_prhs": 8 * 8,
     # residual: {p, RHS, D_E, D_N, J Q12} -> r (FP32 in the mixed form)
     "k2_residual": 8 * 5 + 4,
     # projection: {p, J, 4 metrics, u, v} -> {u, v, S 2}
@@ -282,9 +277,9 @@ KERNEL_BYTES_2D = {
 }
 # the FP32 change form of the AF sweeps (--ens-form mixed): phase A and the stage-2
 # right-hand side read AE / AN instead of 2 Re J/dt and store the residual in FP32; the sweeps
-# move the same operands in FP32
+# move the same operands in FP32, with the previous pass's x; the correction adds the FP32 change
 KERNEL_BYTES_2D_AF32 = dict(KERNEL_BYTES_2D, k2_explicit=8 * 24 + 4 * 2, k2_sweep_i=4 * 10,
-                            k2_sweep_j=4 * 11, k2_rhs2=8 * 5 + 4 * 2)
+                            k2_sweep_j=4 * 10, k2_rhs2=8 * 5 + 4 * 2, k2_correct=8 * 7 + 4 * 2)
 
 
 def cpu_baseline_ensemble(cases, log, budget_s=20.0):
