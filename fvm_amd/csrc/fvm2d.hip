@@ -871,14 +871,6 @@ __device__ inline bool res_done(const Case2D& cs, int q, int last, bool record, 
   return done;
 }
 
-__global__ void k2_begin_p(const Case2D* __restrict__ tab) {
-  const Case2D& cs = tab[blockIdx.x];
-  if (threadIdx.x == 0) {
-    cs.stat[ST_DONE] = 0.0;
-    cs.stat[ST_NAN] = 0.0;
-  }
-}
-
 // Forward real J transform of the residual (two radial rows per complex sequence) into the
 // half spectrum S[i + n1 m], one workgroup per (case, tile of 2 ncol rows); see
 // fvm_poisson_spec.hip for the 3D form.  q >= 0: the pass after the residual of pass q, which every

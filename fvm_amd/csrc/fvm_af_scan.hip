@@ -18,11 +18,13 @@
 //   first-order affine recurrences, evaluated by one 64-lane wavefront as an affine-map scan
 //   (each lane composes its block of rows, then a six-step scan of DPP lane moves, no LDS).
 //   Q = SU' + (coupling to line a+1) x_in(a+1) is formed once per stage.
-// * A wavefront owns SC_C consecutive lines of one plane and sweeps them in order; chunks are
-//   coupled through the last line of the preceding chunk from the previous pass (block Jacobi
-//   across chunks).  The passes are nilpotent (exact after nchunk passes) and contractive by the
-//   diagonal dominance of AP; the host stops once the chunk boundary lines no longer change
-//   (max change <= af_tol max |x|).  The result equals the reference's sweep up to rounding.
+// * FP64 sweeps (k_scan_lead): one pass, each wavefront starting some lines before its own.
+// * FP32 change form (k_scan_pass): a wavefront owns SC_C consecutive lines of one plane and
+//   sweeps them in order; chunks are coupled through the last line of the preceding chunk from
+//   the previous pass (block Jacobi across chunks).  The passes are nilpotent (exact after
+//   nchunk passes) and contractive by the diagonal dominance of AP; the host stops once the
+//   chunk boundary lines no longer change (max change <= af_tol max |x|).
+// * The result equals the reference's sweep up to rounding.
 // * Rows are contiguous for every load: I-lines are contiguous in the natural layout; for
 //   J-lines the line factors, Q and the iterate live in a line-major copy (J fastest), and the
 //   converged iterate is transposed back into the field.
