@@ -574,7 +574,10 @@ struct StepStart {
   double* tfar;        // of T, or nullptr without the passive temperature
 };
 
-// Plane form: a thread takes SB_KP planes of its column with the metrics in registers.
+// Bound by HBM (three fields in, six out).  The threads run over the plane's cells as they lie in
+// memory: rows of NI + 1 cells in tiles of 64 left a tile of two lanes at NI = 193, 93 us at
+// 192 x 256 x 64 cells against 74.  Plane form: a thread takes SB_KP planes of its column with the
+// metrics in registers (1, 2 and 4 planes: 74, 74 and 77 us).
 constexpr int SB_KP = 2;
 template <int G>
 __global__ void __launch_bounds__(256) k_step_begin(Dims d, const double* const* __restrict__ m,
@@ -585,10 +588,10 @@ __global__ void __launch_bounds__(256) k_step_begin(Dims d, const double* const*
   constexpr bool PL = G == kGeoPlane;
   constexpr int KP = PL ? SB_KP : 1;
   const uint3 bb = xcd_block();
-  const int i = bb.x * 64 + threadIdx.x;
-  const int j = bb.y * 4 + threadIdx.y;
+  const int t = (int)bb.x * 256 + (int)threadIdx.y * 64 + (int)threadIdx.x;  // cell of the plane
+  const int j = t / (d.ni + 1), i = t - j * (d.ni + 1);
   const int k0 = (int)bb.z * KP;
-  if (i > d.ni || j > d.nj) return;
+  if (j > d.nj) return;
   const int js = j == 0 ? d.nj - 1 : (j == d.nj ? 1 : j);
   ColDer cd{};
   CellGeo ce;
@@ -618,12 +621,12 @@ __global__ void __launch_bounds__(256) k_step_begin(Dims d, const double* const*
     }
     if (a.tfar) gpw(a.fn[3])[c] = gp(a.f[3])[c];
     if (i == d.ni) {
-      const long nf = (long)(d.nj + 1) * (d.nk + 1), t = j + (long)(d.nj + 1) * k;
+      const long nf = (long)(d.nj + 1) * (d.nk + 1), tf = j + (long)(d.nj + 1) * k;
 #pragma unroll
       for (int f = 0; f < 3; ++f)
-        a.ufar[f * nf + t] =
+        a.ufar[f * nf + tf] =
             in ? ufar_value(d, m, theta, a.f[f], f == 0 ? 1.0 : 0.0, dtime, pi, j, k) : 0.0;
-      if (a.tfar) a.tfar[t] = in ? ufar_value(d, m, theta, a.f[3], 0.0, dtime, pi, j, k) : 0.0;
+      if (a.tfar) a.tfar[tf] = in ? ufar_value(d, m, theta, a.f[3], 0.0, dtime, pi, j, k) : 0.0;
     }
   }
 }
@@ -1356,7 +1359,7 @@ int fvm_k_step_begin(FvmCtx* c) {
   const StepStart a = {{c->u, c->v, c->w, c->t}, {c->un, c->vn, c->wn, c->tn},
                        {c->ju[0], c->ju[1], c->ju[2]}, c->ufar, c->thermal ? c->tfar : nullptr};
   const int kp = c->plane ? SB_KP : 1;
-  const dim3 g((d.ni + 1 + 63) / 64, (d.nj + 1 + 3) / 4, (d.nk + 1 + kp - 1) / kp);
+  const dim3 g(((d.ni + 1) * (d.nj + 1) + 255) / 256, 1, (d.nk + 1 + kp - 1) / kp);
   auto kern = c->plane ? k_step_begin<kGeoPlane>
                        : (c->xz_zero ? k_step_begin<kGeoXz0> : k_step_begin<kGeoAny>);
   hipLaunchKernelGGL(kern, g, kBlk, 0, c->stream, d, (const double* const*)c->dm, c->djac,
