@@ -348,6 +348,17 @@ __device__ inline void publish(const Mailbox& mb, const double* v, int n) {
   *mb.seq = mb.s;
 }
 
+// the same by every thread of a workgroup (which passes it whole) from LDS: the values cross in one
+// store instruction; as one store after another by one lane, each waits for the host link
+__device__ inline void publish_wide(const Mailbox& mb, const double* sv, int n) {
+  if (!mb.dst) return;
+  __syncthreads();
+  if ((int)threadIdx.x < n) mb.dst[threadIdx.x] = sv[threadIdx.x];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) *mb.seq = mb.s;
+}
+
 // R consecutive doubles of a lane of a 64-lane line scan, the pairs among them by 16-byte loads
 // (aligned to 8 bytes as the rows are): the lanes are R rows apart, so every load instruction
 // touches 8 R bytes times 64 lanes of cache lines, and their number is what a line costs
