@@ -11,13 +11,13 @@
 #include "fvm_ctx.h"
 
 // Copies n <= 48 device scalars into the host mailbox, then (after a system-scope fence) the
-// sequence number s: a host that sees s also sees the scalars.  One thread; vector stores.
+// sequence number s: a host that sees s also sees the scalars.  One store of n lanes (publish_wide).
 __global__ void k_publish(const double* __restrict__ src, int n, volatile double* dst,
                           volatile unsigned long long* seq, unsigned long long s) {
-  if (threadIdx.x != 0) return;
-  for (int q = 0; q < n; ++q) dst[q] = src[q];
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
   __threadfence_system();
-  *seq = s;
+  __syncthreads();
+  if (threadIdx.x == 0) *seq = s;
 }
 
 Mailbox fvm_mail(FvmCtx* c) {
