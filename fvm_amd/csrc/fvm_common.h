@@ -359,6 +359,24 @@ __device__ inline void publish_wide(const Mailbox& mb, const double* sv, int n) 
   if (threadIdx.x == 0) *mb.seq = mb.s;
 }
 
+// A thread's share of nb > 0 pairs of partial sums of absolute values (every blockDim.x-th pair from its
+// own), eight pairs in flight and added in their order; those past the end add zero.
+__device__ inline void part_sums(const double* __restrict__ part, long nb, double& a, double& b) {
+  a = 0.0; b = 0.0;
+  for (long q = threadIdx.x; q < nb; q += 8L * blockDim.x) {
+    double x[8], y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const long p = q + (long)u * blockDim.x, pc = p < nb ? p : nb - 1;
+      const double px = part[2 * pc], py = part[2 * pc + 1];
+      x[u] = p < nb ? px : 0.0;
+      y[u] = p < nb ? py : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) { a += x[u]; b += y[u]; }
+  }
+}
+
 // R consecutive doubles of a lane of a 64-lane line scan, the pairs among them by 16-byte loads
 // (aligned to 8 bytes as the rows are): the lanes are R rows apart, so every load instruction
 // touches 8 R bytes times 64 lanes of cache lines, and their number is what a line costs

@@ -178,22 +178,10 @@ __global__ void __launch_bounds__(256) k_residual_km(Dims d, const double* __res
 }
 
 __global__ void k_res_final(const double* __restrict__ part, long nb, double* out, Mailbox mb) {
-  __shared__ double s0[256], s1[256];
+  __shared__ double s0[256], s1[256], v[3];
   const int t = threadIdx.x;
-  double a = 0.0, b = 0.0;
-  long q = t;
-  // eight partial pairs in flight per lane, added in the same order as one at a time
-  for (; q + 7L * blockDim.x < nb; q += 8L * blockDim.x) {
-    double x[8], y[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      x[u] = part[2 * (q + (long)u * blockDim.x)];
-      y[u] = part[2 * (q + (long)u * blockDim.x) + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) { a += x[u]; b += y[u]; }
-  }
-  for (; q < nb; q += blockDim.x) { a += part[2 * q]; b += part[2 * q + 1]; }
+  double a, b;
+  part_sums(part, nb, a, b);
   s0[t] = a; s1[t] = b;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
@@ -203,9 +191,9 @@ __global__ void k_res_final(const double* __restrict__ part, long nb, double* ou
   if (t == 0) {
     const double q = scaled_residual(s0[0], s1[0]);
     out[0] = s0[0]; out[1] = s1[0]; out[2] = q;
-    const double v[3] = {s0[0], s1[0], q};
-    publish(mb, v, 3);
+    v[0] = s0[0]; v[1] = s1[0]; v[2] = q;
   }
+  publish_wide(mb, v, 3);
 }
 
 // Radial line operator of Fourier mode (mJ, mK): lo x(r-1) + dg x(r) + up x(r+1) with
