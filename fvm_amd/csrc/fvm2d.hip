@@ -213,9 +213,13 @@ __device__ inline void bcu_ghosts_wave(P F, int ni, int nj, int sj, B uwall, B u
 // A line is bound by the latency of its loads and of the two scans: with one line loaded ahead and
 // rows loaded one by one it took 34 and 61.
 //
-// FP32 change form (k2_sweep_pass), resolved to FP32 rounding only: a chunk of SW_C lines takes the
+// Chunk passes (k2_sweep_pass): the FP32 change form, resolved to FP32 rounding only, and the FP64
+// sweeps of batches with FP32 pressure corrections.  Those round the residual to FP32, so that a
+// velocity that differs in its last bit moves the pressure by 1e-9 to 1e-7 of its norm (RESIMAX 1e-8),
+// and the one-pass sweeps give other last bits: the pressure of a run would no longer be that of an
+// earlier build.  A chunk of SW_C lines takes the
 // line before it from the preceding chunk's last line of the previous pass (block Jacobi across
-// chunks, no change in the first pass).  Each pass contracts the chunk-boundary error by rho^SW_C;
+// chunks; the stage input's, which has no change, in the first pass).  Each pass contracts the chunk-boundary error by rho^SW_C;
 // a pass after the first re-solves a chunk's lines only until a line stops changing (max change
 // <= tol max |x|), the rest keep their values.  The last pass books the largest relative change of
 // a chunk's last line in the case's ST_AFCH.
@@ -225,17 +229,18 @@ __device__ inline void bcu_ghosts_wave(P F, int ni, int nj, int sj, B uwall, B u
 // DIR 1: J lines (rows along J, lines I = 1..NI-1, lagged coupling AW); the line ends take the
 // ghost values (BCU of the stage input) as Dirichlet data.
 // ---------------------------------------------------------------------------------------------
-template <int R>
+template <int R, typename T>
 struct LineOps {
-  float cdn[R], q[R], iv[R], na[R], bf[R], xo[R];
+  T cdn[R], q[R], iv[R], na[R], bf[R], xo[R];
+  T g0, g1;  // ghosts before / after the line
 };
 
 // roff: the offset of row 0 in a line (the padded FP32 J-line-major layout)
-template <int R, bool EARLY>
-__device__ inline void sweep_load(LineOps<R>& o, gptr<const float> F, gptr<const float> Q,
-                                  gptr<const float> invd, gptr<const float> na,
-                                  gptr<const float> bf, gptr<const float> cdn, long base, long roff,
-                                  long dnoff, int n, int r0) {
+template <int R, int DIR, bool EARLY, typename T>
+__device__ inline void sweep_load(LineOps<R, T>& o, gptr<const T> F, gptr<const T> Q,
+                                  gptr<const T> invd, gptr<const T> na, gptr<const T> bf,
+                                  gptr<const T> cdn, long base, long roff, long dnoff, int n,
+                                  int r0) {
   // a lane's rows as vectors; rows past n (up to R - 1 of them: the ghost and the next line) and the
   // lanes past n are not used
   const long c0 = base + roff + 1 + (r0 < n ? r0 : 0);
@@ -247,38 +252,52 @@ __device__ inline void sweep_load(LineOps<R>& o, gptr<const float> F, gptr<const
   if (EARLY) row_vec<R>(o.xo, F + c0);  // the previous pass's values
   else {
 #pragma unroll
-    for (int q = 0; q < R; ++q) o.xo[q] = 0.0f;
+    for (int q = 0; q < R; ++q) o.xo[q] = (T)0;
   }
+  // an I line's ghosts are folded into its operator, and those of a change are zero
+  constexpr bool GHOSTS = DIR == 1 && std::is_same<T, double>::value;
+  o.g0 = GHOSTS ? F[base] : (T)0;
+  o.g1 = GHOSTS ? F[base + n + 1] : (T)0;
 }
 
 // The change form: the sweep solves T_L d_L = r_L + AS d_(L-1) for the change d = x - x0 of the
 // stage input x0, with r the FP64 residual of x0 (k2_explicit, k2_rhs2), zero ghosts and a zero
 // ghost line; the iterate is H_DU / H_DV (J-line-major for DIR 1).  The I-line stage's last pass
 // adds the change to the FP64 field, the J-line stage's k2_correct does.  The line before a chunk
-// has no change in the first pass.
-template <int R, int DIR, bool EARLY>
+// has no change in the first pass.  T = double: operands and iterates as sweep_lead's.
+template <int R, int DIR, bool EARLY, typename T>
 __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double tol, int final) {
-  using T = float;
+  constexpr bool DELTA = std::is_same<T, float>::value;
   const int ni = cs.ni, nj = cs.nj, sj = cs.sj;
-  T* const F0 = cs.h[comp ? H_DV : H_DU];
-  T* const Q0 = cs.h[DIR == 0 ? (comp ? H_RV : H_RU) : (comp ? H_TRV : H_TRU)];
-  T* const iv0 = cs.h[DIR == 0 ? H_INVD1 : H_TINVD2];
-  T* const na0 = cs.h[DIR == 0 ? H_NA1 : H_TNA2];
-  T* const bf0 = cs.h[DIR == 0 ? H_B1 : H_TB2];
-  T* const cd0 = cs.h[DIR == 0 ? H_AN1 : H_TAW2];
+  T *F0, *Q0, *iv0, *na0, *bf0, *cd0;
+  if constexpr (DELTA) {
+    F0 = cs.h[comp ? H_DV : H_DU];
+    Q0 = cs.h[DIR == 0 ? (comp ? H_RV : H_RU) : (comp ? H_TRV : H_TRU)];
+    iv0 = cs.h[DIR == 0 ? H_INVD1 : H_TINVD2];
+    na0 = cs.h[DIR == 0 ? H_NA1 : H_TNA2];
+    bf0 = cs.h[DIR == 0 ? H_B1 : H_TB2];
+    cd0 = cs.h[DIR == 0 ? H_AN1 : H_TAW2];
+  } else {
+    F0 = cs.f[DIR == 0 ? (comp ? F_X1V : F_X1U) : (comp ? F_TXV : F_TXU)];
+    Q0 = cs.f[DIR == 0 ? (comp ? F_SV1 : F_SU1) : (comp ? F_TQV : F_TQU)];
+    iv0 = cs.f[DIR == 0 ? G_INVD1 : G_TINVD2];
+    na0 = cs.f[DIR == 0 ? G_NA1 : G_TNA2];
+    bf0 = cs.f[DIR == 0 ? G_B1 : G_TB2];
+    cd0 = cs.f[DIR == 0 ? G_AN1 : G_TAW2];
+  }
   // global-address-space views: global (not flat) loads, which do not wait on LDS and scalar
   // traffic, so the next line's loads stay in flight while this line is solved
   const gptr<T> F = glb(F0);
   const gptr<const T> Q = glb((const T*)Q0), invd = glb((const T*)iv0), na = glb((const T*)na0);
   const gptr<const T> bf = glb((const T*)bf0), cdn = glb((const T*)cd0);
   // the change form's I-line stage adds its last pass's change to the field
-  const bool add = DIR == 0 && final;
+  const bool add = DELTA && DIR == 0 && final;
   const gptr<double> F64 = glb(add ? cs.f[comp ? F_V : F_U] : nullptr);
   const int n = DIR == 0 ? ni - 1 : nj - 1;       // rows per line
   const int nl = DIR == 0 ? nj - 1 : ni - 1;      // lines
   const long rs = 1;                              // row stride
-  const long ls = DIR == 0 ? sj : tls32(nj);  // line stride
-  const long roff = DIR == 1 ? J32_OFF : 0;  // row 0's offset in a line
+  const long ls = DIR == 0 ? sj : (DELTA ? tls32(nj) : nj + 1);  // line stride
+  const long roff = DIR == 1 && DELTA ? J32_OFF : 0;  // row 0's offset in a line
   const long dnoff = DIR == 0 ? -(long)sj : 0;    // lower coupling of row c at cdn[c + dnoff]
   const int nch = sw_nchunk(nl);
   const int a0 = 1 + ca * SW_C, a1 = min(a0 + SW_C - 1, nl);
@@ -290,20 +309,29 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = r0 + q;
-    // the line before the chunk: the ghost line 0 (no change), or the preceding chunk's last line
+    // the line before the chunk: the preceding chunk's last line, in the first pass that of the
+    // stage input (no change); before the first chunk the ghost line 0
     T v = (T)0;
-    if (EARLY && r < n && ca > 0) v = (T)bnd[bin + (long)(ca - 1) * n + r];
+    if (r < n && ca > 0 && EARLY) v = (T)bnd[bin + (long)(ca - 1) * n + r];
+    if (!DELTA && r < n && (ca == 0 || !EARLY)) {
+      if (DIR == 0)  // (line 0: the periodic image of line NJ-1)
+        v = (T)glb(cs.f[comp ? F_V : F_U])[ls * (ca == 0 ? nj - 1 : a0 - 1) + r + 1];
+      else if (ca == 0)
+        v = F[r + 1];
+      else
+        v = (T)glb(cs.f[comp ? F_X1V : F_X1U])[(a0 - 1) + (long)sj * (r + 1)];
+    }
     prev[q] = v;
   }
-  LineOps<R> cur, nxt;
-  sweep_load<R, EARLY>(cur, F, Q, invd, na, bf, cdn, ls * a0, roff, dnoff, n, r0);
+  LineOps<R, T> cur, nxt;
+  sweep_load<R, DIR, EARLY, T>(cur, F, Q, invd, na, bf, cdn, ls * a0, roff, dnoff, n, r0);
   bool stopped = false;
   T xrun = (T)0;
   int L = a0;
   for (; L <= a1; ++L) {
     const long base = ls * L;
     if (L < a1)
-      sweep_load<R, EARLY>(nxt, F, Q, invd, na, bf, cdn, base + ls, roff, dnoff, n, r0);
+      sweep_load<R, DIR, EARLY, T>(nxt, F, Q, invd, na, bf, cdn, base + ls, roff, dnoff, n, r0);
     T al[R], be[R], bb[R];
     T At = (T)0, Bt = (T)1;
 #pragma unroll
@@ -320,7 +348,7 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
       Bt = be[q] * Bt;
     }
     // lane l starts from the exclusive prefix applied to the ghost before the first row
-    T yin = wave::prefix_apply(At, Bt, (T)0);
+    T yin = wave::prefix_apply(At, Bt, cur.g0);
     T y[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
@@ -336,7 +364,7 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
       }
     }
     // and from the exclusive suffix applied to the ghost after the last row
-    T xin = wave::suffix_apply(Dt, Ct, (T)0);
+    T xin = wave::suffix_apply(Dt, Ct, cur.g1);
     T dl = (T)0;
 #pragma unroll
     for (int q = R - 1; q >= 0; --q) {
@@ -408,6 +436,21 @@ __device__ void sweep_chunk(const Case2D& cs, int comp, int ca, int slot, double
   }
 }
 
+// BCU's ghost lines J = 0, NJ of the stage input F into X: the periodic images of lines NJ-1, 1
+__device__ inline void ghost_lines(const Case2D& cs, int comp, gptr<const double> F,
+                                   gptr<double> X) {
+  const auto uwall = glb((const double*)cs.b[comp ? B_VWALL : B_UWALL]);
+  const auto ufar = glb((const double*)cs.b[comp ? B_VFAR : B_UFAR]);
+  const int ni = cs.ni, nj = cs.nj;
+  const long ls = cs.sj;
+  for (int q = threadIdx.x; q < 2 * (ni + 1); q += 64) {
+    const int i = q >> 1, js = q & 1 ? 1 : nj - 1;
+    const long c = ls * js;
+    X[i + (q & 1 ? ls * nj : 0)] = i == 0 ? -F[c + 1] + 2.0 * uwall[js]
+                                          : (i == ni ? -F[c + ni - 1] + 2.0 * ufar[js] : F[c + i]);
+  }
+}
+
 // The FP64 sweep of chunk ca of nlc lines.  DIR 0: from the field (the stage input, left as it is)
 // and F_SU1 / F_SV1 to F_X1U / F_X1V, whose ghosts are BCU's of the stage input.  DIR 1: on the
 // J-line-major copies (iterate F_TX*, right-hand side F_TQ*, factors and AW G_T*, made by k2_rhs2
@@ -429,14 +472,7 @@ __device__ void sweep_lead(const Case2D& cs, int comp, int ca, int nlc) {
   const long dnoff = DIR == 0 ? -ls : 0;  // lower coupling of row c at cdn[c + dnoff]
   const int a0 = 1 + ca * nlc, a1 = min(a0 + nlc - 1, nl);
   const int l = threadIdx.x, r0 = l * R;
-  if (DIR == 0 && ca == 0) {  // the ghost lines 0, NJ: periodic images of lines NJ-1, 1
-    for (int q = l; q < 2 * (ni + 1); q += 64) {
-      const int i = q >> 1, js = q & 1 ? 1 : nj - 1;
-      const long c = ls * js;
-      X[i + (q & 1 ? ls * nj : 0)] = i == 0 ? -F[c + 1] + 2.0 * uwall[js]
-                                            : (i == ni ? -F[c + n] + 2.0 * ufar[js] : F[c + i]);
-    }
-  }
+  if (DIR == 0 && ca == 0) ghost_lines(cs, comp, F, X);
   struct Ops {
     double cdn[R], q[R], iv[R], na[R], bf[R];
     double g0, g1;  // DIR 0: the stage input's first and last row; DIR 1: the line ends' ghosts
@@ -559,10 +595,10 @@ __global__ void __launch_bounds__(64) k2_sweep(const Case2D* __restrict__ tab,
 }
 
 // One pass over the chunks of every case (block table: case, 2 chunk + component; entries with
-// case -1 pad the table to whole XCD rounds).  The change form's I-line stage leaves the field
-// alone in its first pass: 2 ncase workgroups past the table's nblk then set BCU's ghosts of the
-// stage input, which the stage-2 right-hand side reads.
-template <int DIR, bool EARLY>
+// case -1 pad the table to whole XCD rounds).  The I-line stage leaves the field alone in its first
+// pass: 2 ncase workgroups past the table's nblk then set BCU's ghosts of the stage input, which the
+// stage-2 right-hand side reads, in the field or (T = double) in the stage's result.
+template <int DIR, bool EARLY, typename T>
 __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ tab,
                                                     const int* __restrict__ bcase,
                                                     const int* __restrict__ btile, int slot,
@@ -570,8 +606,19 @@ __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ t
   if (DIR == 0 && !EARLY && (int)blockIdx.x >= nblk) {
     const int w = (int)blockIdx.x - nblk, comp = w & 1;
     const Case2D& cg = tab[w >> 1];
-    bcu_ghosts_wave(glb(cg.f[comp ? F_V : F_U]), cg.ni, cg.nj, cg.sj,
-                    glb(cg.b[comp ? B_VWALL : B_UWALL]), glb(cg.b[comp ? B_VFAR : B_UFAR]));
+    const auto F = glb(cg.f[comp ? F_V : F_U]);
+    const auto uwall = glb(cg.b[comp ? B_VWALL : B_UWALL]), ufar = glb(cg.b[comp ? B_VFAR : B_UFAR]);
+    if (std::is_same<T, float>::value) {
+      bcu_ghosts_wave(F, cg.ni, cg.nj, cg.sj, uwall, ufar);
+    } else {
+      const auto X = glb(cg.f[comp ? F_X1V : F_X1U]);
+      ghost_lines(cg, comp, F, X);
+      for (int j = 1 + threadIdx.x; j <= cg.nj - 1; j += 64) {
+        const long c = (long)cg.sj * j;
+        X[c] = -F[c + 1] + 2.0 * uwall[j];
+        X[c + cg.ni] = -F[c + cg.ni - 1] + 2.0 * ufar[j];
+      }
+    }
     return;
   }
   const int cc = bcase[blockIdx.x];
@@ -581,14 +628,14 @@ __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ t
   const int comp = t & 1, ca = t >> 1;
   const int n = DIR == 0 ? cs.ni - 1 : cs.nj - 1;
   switch ((n + 63) >> 6) {  // the case's own rows per lane
-    case 1: sweep_chunk<1, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 2: sweep_chunk<2, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 3: sweep_chunk<3, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 4: sweep_chunk<4, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 5: sweep_chunk<5, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 6: sweep_chunk<6, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    case 7: sweep_chunk<7, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
-    default: sweep_chunk<8, DIR, EARLY>(cs, comp, ca, slot, tol, final); break;
+    case 1: sweep_chunk<1, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 2: sweep_chunk<2, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 3: sweep_chunk<3, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 4: sweep_chunk<4, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 5: sweep_chunk<5, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 6: sweep_chunk<6, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    case 7: sweep_chunk<7, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
+    default: sweep_chunk<8, DIR, EARLY, T>(cs, comp, ca, slot, tol, final); break;
   }
 }
 

@@ -18,8 +18,10 @@
 //   first-order affine recurrences, evaluated by one 64-lane wavefront as an affine-map scan
 //   (each lane composes its block of rows, then a six-step scan of DPP lane moves, no LDS).
 //   Q = SU' + (coupling to line a+1) x_in(a+1) is formed once per stage.
-// * FP64 sweeps (k_scan_lead): one pass, each wavefront starting some lines before its own.
-// * FP32 change form (k_scan_pass): a wavefront owns SC_C consecutive lines of one plane and
+// * FP64 sweeps before an FP64 pressure, and of T (k_scan_lead): one pass, each wavefront starting
+//   some lines before its own.
+// * FP32 change form, and FP64 sweeps before FP32 pressure corrections (k_scan_pass): a wavefront
+//   owns SC_C consecutive lines of one plane and
 //   sweeps them in order; chunks are coupled through the last line of the preceding chunk from
 //   the previous pass (block Jacobi across chunks).  The passes are nilpotent (exact after
 //   nchunk passes) and contractive by the diagonal dominance of AP; the host stops once the
@@ -186,6 +188,24 @@ __global__ void k_to_float(long n, const double* __restrict__ a, float* b) {
     b[t] = (float)a[t];
 }
 
+// boundary lines of the FP64 I stage's first chunk pass: the stage input at the last line of every
+// chunk (bnd[((comp nb + b-1) nchunk + ca) n + p-1])
+__global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, double* bnd) {
+  const ScanGeo g = scan_geo(d, 0);
+  const long tot = (long)A.nc * g.nb * nchunk * g.n;
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot;
+       t += (long)gridDim.x * blockDim.x) {
+    const int p = 1 + (int)(t % g.n);
+    long r = t / g.n;
+    const int ca = (int)(r % nchunk);
+    r /= nchunk;
+    const int b = 1 + (int)(r % g.nb);
+    const int comp = (int)(r / g.nb);
+    const int a = min((ca + 1) * SC_C, g.na);
+    bnd[t] = A.f[comp][g.ns_p * p + g.ns_a * a + g.ns_b * b];
+  }
+}
+
 // The largest ratio of the coupling to line a - 1 to the row sum of the line operator, per line a: the
 // factor by which a change of line a - 1 reaches line a at most (T^-1 s = 1 for the M-matrix T with
 // row sums s).  One workgroup per line (setup only).
@@ -216,7 +236,6 @@ __global__ void __launch_bounds__(256) k_scan_rho(Dims d, const double* const* _
   if (t == 0) rho[a] = sh[0];
 }
 
-__device__ inline double shfl_up_d(double v, int o) { return __shfl_up(v, o, 64); }
 __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o, 64); }
 
 // The FP64 sweep of a stage in one pass: wavefront w owns chunk ca (nlc lines) of plane b for one
@@ -359,19 +378,23 @@ __global__ void __launch_bounds__(64) k_scan_lead(Dims d, AFArgs A, const double
 // Loads of rows one by one (I lines: the J lines' were vectors) took the first I pass 55 us on
 // 192 x 256 x 64 cells and 473 on 384 x 512 x 128, row vectors 42 and 319; loading further lines ahead
 // gains nothing (44).
-template <int S, int R, bool EARLY>
-__global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float* __restrict__ beta,
-                                                  const float* __restrict__ invd,
-                                                  const float* __restrict__ bb,
-                                                  const float* __restrict__ cam,
+//
+// T = double: the FP64 sweep whose velocity FP32 pressure corrections follow (chunked64).  The line
+// before a chunk is the stage input's in the first pass: the field's in the J stage, whose iterate is
+// a work array, k_scan_seed's in the I stage, which writes its iterate over the field.
+template <int S, int R, bool EARLY, typename T>
+__global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const T* __restrict__ beta,
+                                                  const T* __restrict__ invd,
+                                                  const T* __restrict__ bb,
+                                                  const T* __restrict__ cam,
                                                   const double* const* qt, double* const* xot,
-                                                  const float* __restrict__ bnd_in,
-                                                  float* bnd_out, int nchunk, double* part,
+                                                  const T* __restrict__ bnd_in,
+                                                  T* bnd_out, int nchunk, double* part,
                                                   double tol, double* sinkd, long G) {
-  using T = float;
+  constexpr bool DELTA = std::is_same<T, float>::value;
   const ScanGeo g = scan_geo(d, S);
   const long lin = blockIdx.x;
-  if (!EARLY && lin >= G) {  // uniform over the workgroup
+  if (DELTA && !EARLY && lin >= G) {  // uniform over the workgroup
     const long cnt = bc_ghost_count(d), step = ((long)gridDim.x - G) * 64;
     for (long t = (lin - G) * 64 + threadIdx.x; t < A.nc * cnt; t += step)
       bc_ghost(d, A.f[t / cnt], A.ufar + (t / cnt) * (long)(d.nj + 1) * (d.nk + 1), 0.0, t % cnt);
@@ -390,16 +413,21 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
     const int a1 = min(a0 + SC_C - 1, g.na);
     const int p0 = l * R + 1;
     const gptr<const T> qc = glb(reinterpret_cast<const T*>(qt[comp]));
+    const GP fc = gp(A.f[comp]);
     const gptr<T> xc = glb(reinterpret_cast<T*>(xot[comp]));
     T xp[R];
-    // line a0-1: no change in the first pass and before the first chunk, else the preceding
-    // chunk's last line of the previous pass
+    // line a0-1: the preceding chunk's last line of the previous pass; in the first pass and before
+    // the first chunk the stage input's, which has no change
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int p = p0 + r;
       T v = (T)0;
-      if (EARLY && p <= g.n && ca > 0)
-        v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
+      if (p <= g.n && !(DELTA && (ca == 0 || !EARLY))) {
+        if (ca == 0 || (S == 1 && !EARLY))
+          v = (T)fc[g.ns_p * p + g.ns_a * (a0 - 1) + g.ns_b * b];
+        else
+          v = bnd_in[(((long)comp * g.nb + (b - 1)) * nchunk + (ca - 1)) * g.n + (p - 1)];
+      }
       xp[r] = v;
     }
     // Operands of one line.  Rows past n (up to R - 1 of them: the ghost and the next line) and the
@@ -407,7 +435,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
     // end of the chunk): with no load or store behind a branch the compiler counts the loads in
     // flight exactly and waits only for the ones it needs, so the next line's loads overlap this
     // line's scans.
-    T be[R], iv[R], bv[R], cm[R], qv[R], xv[R];
+    T be[R], iv[R], bv[R], cm[R], qv[R], xv[R], y0n = (T)0, xnn = (T)0;
     const int pc = p0 <= g.n ? p0 : 1;
     auto load = [&](int a) {
       const long o = g.ls_a * a + g.ls_b * b + g.off + pc;
@@ -421,6 +449,11 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
 #pragma unroll
         for (int r = 0; r < R; ++r) xv[r] = (T)0;
       }
+      if (!DELTA) {  // the ghosts before and after the line, which have no change
+        const long nb0 = g.ns_a * a + g.ns_b * b;
+        y0n = (T)fc[nb0];
+        xnn = (T)fc[nb0 + g.ns_p * (g.n + 1)];
+      }
     };
     load(a0);
     bool stopped = false;
@@ -428,6 +461,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
     const T ttol = (T)tol;
     for (int a = a0; a <= a1; ++a) {
       const long lb = g.ls_a * a + g.ls_b * b + g.off;
+      const T y0 = y0n, xn = xnn;
       // forward: y(p) = al(p) + be(p) y(p-1)
       T al[R], bt[R], bw[R], xo[R];
       T Bt = (T)1, At = (T)0;
@@ -443,7 +477,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
       }
       load(min(a + 1, a1));  // next line's operands in flight during the scans
       __builtin_amdgcn_sched_barrier(0);  // keep those loads ahead of the scans
-      T yin = wave::prefix_apply(At, Bt, (T)0);
+      T yin = wave::prefix_apply(At, Bt, y0);  // y0, xn: the same on every lane
       T y[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -458,7 +492,7 @@ __global__ void __launch_bounds__(64) k_scan_pass(Dims d, AFArgs A, const float*
         Dt = in ? y[r] - bw[r] * Dt : Dt;
         Ct = in ? -bw[r] * Ct : Ct;
       }
-      T xin = wave::suffix_apply(Dt, Ct, (T)0);
+      T xin = wave::suffix_apply(Dt, Ct, xn);
       T dl = (T)0;
 #pragma unroll
       for (int r = R - 1; r >= 0; --r) {
@@ -611,9 +645,9 @@ int scan_stage64(FvmCtx* c, const AFArgs& A, bool temp) {
   return S == 1 ? scan_unpack<double>(c, A.nc, B) : FVM_OK;
 }
 
-template <int S, int R>
-int scan_stage32(FvmCtx* c, const AFArgs& A, int* iters) {
-  using T = float;
+template <int S, int R, typename T>
+int scan_stage_chunks(FvmCtx* c, const AFArgs& A, int* iters) {
+  constexpr bool DELTA = std::is_same<T, float>::value;
   const Dims d = c->d;
   hipStream_t st = c->stream;
   const ScanGeo g = scan_geo(d, S);
@@ -628,17 +662,24 @@ int scan_stage32(FvmCtx* c, const AFArgs& A, int* iters) {
   double* const* dq = B.tab;
   double* const* dxo = B.tab + 3;
   T* bnd[2] = {reinterpret_cast<T*>(c->bnd[0]), reinterpret_cast<T*>(c->bnd[1])};
-  // the FP32 change is resolved to its own precision
-  const double tol = std::max(c->prm.af_tol > 0 ? c->prm.af_tol : 1e-14, 6e-8);
+  if (S == 0 && !DELTA) {
+    hipLaunchKernelGGL(k_scan_seed, grid1((long)nc * g.nb * nchunk * g.n, 256), dim3(256), 0, st, d,
+                       A, nchunk, c->bnd[0]);
+    HIP_CHECK(hipGetLastError());
+  }
+  double tol = c->prm.af_tol > 0 ? c->prm.af_tol : 1e-14;
+  if (DELTA) tol = std::max(tol, 6e-8);  // the FP32 change is resolved to its own precision
   const int cap = nchunk + 1;
   int slot = 0, it = 0;
-  const T* const* lf = reinterpret_cast<const T* const*>(c->lf32[S]);
+  const T* const* lf;
+  if constexpr (DELTA) lf = c->lf32[S];
+  else lf = c->lf[S];
   for (;;) {
     {
       ProfScope pk(c, S == 0 ? "k_scan_pass_i" : "k_scan_pass_j");
-      auto kern = it > 0 ? k_scan_pass<S, R, true> : k_scan_pass<S, R, false>;
+      auto kern = it > 0 ? k_scan_pass<S, R, true, T> : k_scan_pass<S, R, false, T>;
       // the change form's first pass also sets the field's BCU ghosts: four per lane
-      const long ng = it == 0 ? (nc * bc_ghost_count(d) + 255) / 256 : 0;
+      const long ng = DELTA && it == 0 ? (nc * bc_ghost_count(d) + 255) / 256 : 0;
       hipLaunchKernelGGL(kern, dim3((unsigned)(G + ng)), dim3(64), 0, st, d, A, lf[0], lf[1],
                          lf[2], lf[3], (const double* const*)dq, dxo, bnd[slot], bnd[slot ^ 1],
                          nchunk, c->red, tol, c->sink, G);
@@ -662,7 +703,7 @@ int scan_stage32(FvmCtx* c, const AFArgs& A, int* iters) {
   if (S == 1) {
     const int r = scan_unpack<T>(c, nc, B);
     if (r) return r;
-  } else {
+  } else if (DELTA) {
     ProfScope pk(c, "af_scan_add");
     PtrSet8 dl{}, f{};
     for (int k = 0; k < nc; ++k) { dl.p[k] = B.xo[k]; f.p[k] = A.f[k]; }
@@ -757,35 +798,43 @@ int fvm_af_scan_setup(FvmCtx* c) {
   return FVM_OK;
 }
 
+// Whether the FP64 sweeps of u, v, w go by chunk passes: where FP32 pressure corrections follow.  Those
+// round the residual to FP32, so that a velocity that differs in its last bit moves the pressure by
+// 1e-9 to 1e-7 of its norm (RESIMAX 1e-8), and one-pass sweeps give other last bits than chunk
+// passes: the pressure of a run would no longer be that of an earlier build.  A slab of 128 x 256
+// cells takes 62 us for the two stages by passes and 39 by one pass.  T feeds no pressure.
+static bool chunked64(const FvmCtx* c) {
+  return c->prm.poisson_mode == 1 || c->prm.poisson_mode == 3;
+}
+
+template <int S, typename T>
+static int chunks_by_rows(FvmCtx* c, const AFArgs& A, int* iters) {
+  const int R = (scan_geo(c->d, S).n + 63) / 64;
+  if (R <= 3) return scan_stage_chunks<S, 3, T>(c, A, iters);
+  if (R <= 4) return scan_stage_chunks<S, 4, T>(c, A, iters);
+  if (R <= 6) return scan_stage_chunks<S, 6, T>(c, A, iters);
+  return scan_stage_chunks<S, SC_R, T>(c, A, iters);
+}
+
+template <int S>
+static int lead_by_rows(FvmCtx* c, const AFArgs& A, bool temp) {
+  const int R = (scan_geo(c->d, S).n + 63) / 64;
+  if (R <= 1) return scan_stage64<S, 1>(c, A, temp);
+  if (R <= 2) return scan_stage64<S, 2>(c, A, temp);
+  if (R <= 3) return scan_stage64<S, 3>(c, A, temp);
+  if (R <= 4) return scan_stage64<S, 4>(c, A, temp);
+  if (R <= 6) return scan_stage64<S, 6>(c, A, temp);
+  return scan_stage64<S, SC_R>(c, A, temp);
+}
+
 int fvm_af_scan_stage(FvmCtx* c, int s, const AFArgs& A, int* iters, bool temp, bool delta) {
   if (A.nc < 1 || A.nc > 3 || (temp && !c->lft[s][0])) return FVM_ERR_ARG;
-  const int R = (scan_geo(c->d, s).n + 63) / 64;
   if (delta) {
     if (temp || !c->lf32[s][0]) return FVM_ERR_ARG;
-    if (s == 0) {
-      if (R <= 3) return scan_stage32<0, 3>(c, A, iters);
-      if (R <= 4) return scan_stage32<0, 4>(c, A, iters);
-      if (R <= 6) return scan_stage32<0, 6>(c, A, iters);
-      return scan_stage32<0, SC_R>(c, A, iters);
-    }
-    if (R <= 3) return scan_stage32<1, 3>(c, A, iters);
-    if (R <= 4) return scan_stage32<1, 4>(c, A, iters);
-    if (R <= 6) return scan_stage32<1, 6>(c, A, iters);
-    return scan_stage32<1, SC_R>(c, A, iters);
+    return s == 0 ? chunks_by_rows<0, float>(c, A, iters) : chunks_by_rows<1, float>(c, A, iters);
   }
+  if (!temp && chunked64(c))
+    return s == 0 ? chunks_by_rows<0, double>(c, A, iters) : chunks_by_rows<1, double>(c, A, iters);
   *iters = 1;
-  if (s == 0) {
-    if (R <= 1) return scan_stage64<0, 1>(c, A, temp);
-    if (R <= 2) return scan_stage64<0, 2>(c, A, temp);
-    if (R <= 3) return scan_stage64<0, 3>(c, A, temp);
-    if (R <= 4) return scan_stage64<0, 4>(c, A, temp);
-    if (R <= 6) return scan_stage64<0, 6>(c, A, temp);
-    return scan_stage64<0, SC_R>(c, A, temp);
-  }
-  if (R <= 1) return scan_stage64<1, 1>(c, A, temp);
-  if (R <= 2) return scan_stage64<1, 2>(c, A, temp);
-  if (R <= 3) return scan_stage64<1, 3>(c, A, temp);
-  if (R <= 4) return scan_stage64<1, 4>(c, A, temp);
-  if (R <= 6) return scan_stage64<1, 6>(c, A, temp);
-  return scan_stage64<1, SC_R>(c, A, temp);
+  return s == 0 ? lead_by_rows<0>(c, A, temp) : lead_by_rows<1>(c, A, temp);
 }

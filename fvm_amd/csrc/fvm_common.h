@@ -414,6 +414,11 @@ __device__ __forceinline__ void row_vec(float (&d)[R], gptr<const float> p) {
   }
 }
 
+template <int R>
+__device__ __forceinline__ void row_vec(double (&d)[R], gptr<const double> p) {
+  row_pairs<R>(d, p);
+}
+
 // up to eight arrays passed by value (no device pointer table needed)
 struct PtrSet8 {
   double* p[8];

@@ -50,8 +50,9 @@ typedef struct fvm_params {
                               field (mixed form; the K stage, ITER_T and the one-component
                               entries stay FP64)                                            */
   double af_tol;        /* chunked iteration: stop when max change <= af_tol * max |u|
-                           (<= 0: 1e-14).  The FP64 I/J line scans need no iteration: one
-                           pass with lead-in lines, worth less than 1e-20 at their start   */
+                           (<= 0: 1e-14).  The FP64 I/J line scans before an FP64 pressure
+                           (poisson_mode 0, 2) and of T need no iteration: one pass with
+                           lead-in lines, worth less than 1e-20 at their start            */
 } fvm_params;
 
 /* Per-step diagnostics (RLES/calccoef.f90:11-201 scalars and the ITER_P counters). */
@@ -62,7 +63,7 @@ typedef struct fvm_step_info {
   double pref;          /* span-mean far-field pressure subtracted from p                */
   double c_avg;         /* dynamic Smagorinsky coefficient C = <LM>/<2MM>                */
   double cfl, cpb, cd, cl, cd_p, cd_v, cl_p, cl_v;
-  int af_iters[3];      /* passes of the three AF stage sweeps (1: FP64 line scans)     */
+  int af_iters[3];      /* passes of the three AF stage sweeps (1: one-pass line scans) */
   double nu;            /* Nusselt number NU (calccoef.f90:117-184); 0 without the
                            passive temperature                                           */
   double c_t;           /* dynamic coefficient of the subgrid heat flux
