@@ -396,7 +396,7 @@ static int create_impl(const fvm_params* prm, const double* xg, const double* yg
   r = fvm_af_setup(c);
   if (r) { fvm_destroy(c); return r; }
   r = fvm_sep_setup(c);
-  if (!r && c->prm.poisson_mode == 0) r = fvm_zebra_setup(c);
+  if (!r && c->prm.poisson_mode == 0 && c->prm.af_mode != 2) r = fvm_zebra_setup(c);
   if (r) { fvm_destroy(c); return r; }
   *out = c;
   return FVM_OK;

@@ -61,6 +61,10 @@ FORMS = {
     "batch_sep32": lambda: _batch([(50, 65, 100.0, 1e-3), (18, 289, 200.0, 1e-3),
                                    (82, 97, 40.0, 1e-2)], 8),
     "box_sep32": lambda: _les(35, 49, 5, 6, False, poisson_mode=3, resimax=1e-8),
+    # FP32 line sweeps (change form), FP64 pressure by line relaxation
+    "slab_af32_zebra": lambda: _slab(50, 65, 100.0, 1e-3, 12, poisson_mode=0, af_mode=2,
+                                     resimax=1e-4),
+    "box_af32_zebra": lambda: _les(26, 33, 5, 6, False, poisson_mode=0, af_mode=2, resimax=1e-4),
 }
 
 
