@@ -379,7 +379,7 @@ __global__ void __launch_bounds__(64) k_scan_lead(Dims d, AFArgs A, const double
 // 192 x 256 x 64 cells and 473 on 384 x 512 x 128, row vectors 42 and 319; loading further lines ahead
 // gains nothing (44).
 //
-// T = double: the FP64 sweep whose velocity FP32 pressure corrections follow (chunked64).  The line
+// T = double: the FP64 sweep whose velocity FP32 pressure corrections follow.  The line
 // before a chunk is the stage input's in the first pass: the field's in the J stage, whose iterate is
 // a work array, k_scan_seed's in the I stage, which writes its iterate over the field.
 template <int S, int R, bool EARLY, typename T>
@@ -798,15 +798,6 @@ int fvm_af_scan_setup(FvmCtx* c) {
   return FVM_OK;
 }
 
-// Whether the FP64 sweeps of u, v, w go by chunk passes: where FP32 pressure corrections follow.  Those
-// round the residual to FP32, so that a velocity that differs in its last bit moves the pressure by
-// 1e-9 to 1e-7 of its norm (RESIMAX 1e-8), and one-pass sweeps give other last bits than chunk
-// passes: the pressure of a run would no longer be that of an earlier build.  A slab of 128 x 256
-// cells takes 62 us for the two stages by passes and 39 by one pass.  T feeds no pressure.
-static bool chunked64(const FvmCtx* c) {
-  return c->prm.poisson_mode == 1 || c->prm.poisson_mode == 3;
-}
-
 template <int S, typename T>
 static int chunks_by_rows(FvmCtx* c, const AFArgs& A, int* iters) {
   const int R = (scan_geo(c->d, S).n + 63) / 64;
@@ -833,7 +824,10 @@ int fvm_af_scan_stage(FvmCtx* c, int s, const AFArgs& A, int* iters, bool temp, 
     if (temp || !c->lf32[s][0]) return FVM_ERR_ARG;
     return s == 0 ? chunks_by_rows<0, float>(c, A, iters) : chunks_by_rows<1, float>(c, A, iters);
   }
-  if (!temp && chunked64(c))
+  // One-pass sweeps give other last bits than chunk passes, with which a run before FP32 pressure
+  // corrections would no longer have the pressure of an earlier build.  A slab of 128 x 256 cells
+  // takes 62 us for the two stages by passes and 39 by one pass.  T feeds no pressure.
+  if (!temp && fp32_pressure(c))
     return s == 0 ? chunks_by_rows<0, double>(c, A, iters) : chunks_by_rows<1, double>(c, A, iters);
   *iters = 1;
   return s == 0 ? lead_by_rows<0>(c, A, temp) : lead_by_rows<1>(c, A, temp);

@@ -154,6 +154,12 @@ struct FvmCtx {
   HostIo io;                 // pinned slots of fvm_set_field / fvm_get_field
 };
 
+// Whether the pressure corrections are FP32.  They round a residual of the velocity: one that differs
+// in its last bit moves the pressure by 1e-12 to 1e-7 of its norm.
+inline bool fp32_pressure(const FvmCtx* c) {
+  return c->prm.poisson_mode == 1 || c->prm.poisson_mode == 3;
+}
+
 // K planes per workgroup of a K-marching stencil kernel, and its launch grid (64 x 4 (I x J) tiles
 // by groups of kc planes).  A workgroup's time is the latency of its kc + 2 planes (two halo
 // planes), one after the other, and `resident` workgroups run at a time (256 CUs times what

@@ -65,6 +65,9 @@ FORMS = {
     "slab_af32_zebra": lambda: _slab(50, 65, 100.0, 1e-3, 12, poisson_mode=0, af_mode=2,
                                      resimax=1e-4),
     "box_af32_zebra": lambda: _les(26, 33, 5, 6, False, poisson_mode=0, af_mode=2, resimax=1e-4),
+    # the model's sums, FP64 line sweeps (chunk passes, and the exact order), FP32 pressure corrections
+    "les_sep32": lambda: _les(22, 49, 17, 12, True, poisson_mode=3, resimax=1e-8),
+    "les_exact_sep32": lambda: _les(18, 33, 17, 8, True, poisson_mode=3, af_mode=1, resimax=1e-8),
 }
 
 
