@@ -493,16 +493,19 @@ int fvm_k_iter_p(FvmCtx* c, double* resip, int* niter) {
   double res = INFINITY;
   int r;
   if (c->prm.poisson_mode == 0) {
-    // FP64 zebra line Gauss-Seidel.  The host enqueues up to kAhead residual tests ahead of the one
-    // it waits for; the device ends the sweeps itself (k_p_res_final's flag), so those enqueued past
-    // the end change nothing.  A wait for every test left the device idle for the host's reaction
-    // and the next launches, and its own launch to publish, a third of a sweep on 96 x 128 x 32 cells.
+    // FP64 zebra line Gauss-Seidel.  The host enqueues up to kAhead sweeps, and their residual tests,
+    // past the test it waits for; the device ends the sweeps itself (k_p_res_final's flag), so those
+    // enqueued past the end change nothing.  A wait for every test left the device idle for the host's
+    // reaction and the next launches, and its own launch to publish, a third of a sweep on
+    // 96 x 128 x 32 cells.  Counting tests instead of sweeps, a step on that grid whose first test ends
+    // the sweeps took 2.35 ms with a test every 50 sweeps; so 0.35.
     constexpr int kAhead = 3;
     Mailbox mb[kAhead + 1];
     int at[kAhead + 1];  // sweeps done at the test
     int put = 0, got = 0, sent = 0;
     for (bool end = false; !end;) {
-      for (; sent <= cap && put - got <= kAhead; ++sent) {  // enqueue: test (and a sweep before it)
+      for (; sent <= cap && (put == got || sent - at[got % (kAhead + 1)] <= kAhead); ++sent) {
+        // a sweep, but for the first, and a test
         if (sent > 0) {
           r = zebra64(c);
           if (r) return r;
