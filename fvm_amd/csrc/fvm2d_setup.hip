@@ -265,13 +265,6 @@ void geo2d_af(const Geo2D& g, double re, double dt, AF2D& a) {
     {
       const int nl = s == 0 ? nj - 1 : ni - 1, nr = s == 0 ? ni - 1 : nj - 1;
       a.rho[s].assign(nl + 2, 0.0);
-      for (int L = 2; L <= nl; ++L)
-        for (int r = 1; r <= nr; ++r) {
-          const long c = s == 0 ? ix(sj, r, L) : ix(sj, L, r);
-          const double cdn = s == 0 ? AS[c] : AW[c];
-          const double sum = AP[c] - (s == 0 ? AW[c] + AE[c] : AS[c] + AN[c]);
-          a.rho[s][L - 1] = std::max(a.rho[s][L - 1], cdn / sum);
-        }
       for (int L = 1; L <= nl; ++L) {
         std::vector<double> av(nr + 2, 0.0), cv(nr + 2, 0.0), dv(nr + 2, 0.0);
         for (int r = 1; r <= nr; ++r) {
@@ -280,11 +273,21 @@ void geo2d_af(const Geo2D& g, double re, double dt, AF2D& a) {
           cv[r] = s == 0 ? -AE[c] : -AN[c];
         }
         double bprev = 0.0;
+        double rc = 0.0, rs = 1.0;  // the largest Cdn / s so far, compared without divisions
         for (int r = 1; r <= nr; ++r) {
           const long c = s == 0 ? ix(sj, r, L) : ix(sj, L, r);
           dv[r] = AP[c] - av[r] * bprev;
           bprev = cv[r] / dv[r];
+          const double cdn = s == 0 ? AS[c] : AW[c], sum = AP[c] + (av[r] + cv[r]);
+          if (!(cdn * sum >= 0.0 && sum != 0.0)) {  // no M-matrix
+            rc = 1.0;
+            rs = 0.0;
+          } else if (fabs(cdn) * rs > rc * fabs(sum)) {
+            rc = fabs(cdn);
+            rs = fabs(sum);
+          }
         }
+        if (L > 1) a.rho[s][L - 1] = rc / rs;
         for (int r = 1; r <= nr; ++r) {
           const long c = s == 0 ? ix(sj, r, L) : ix(sj, L, r);
           a.nat[s][c] = r == 1 ? 0.0 : -cv[r - 1] / dv[r];
