@@ -104,8 +104,12 @@ constexpr int DF_RES_PLANE = 768;  // in the plane form, whose loads ahead take 
 // the SGS term added to NL in between).  Bound by the latency of a plane's loads: ahead by a plane
 // (plane form; the occupancy falls from four waves to three), 192 x 256 x 64 cells took 119 us for
 // 129, 384 x 512 x 128 871 for 892; before the barrier instead of after it, 32 x 64 x 16 7.1 for 8.8.
+// With stored arrays the compiler's own choice of registers (four waves all the same) is the better one:
+// held to four waves by the launch bounds, 192 x 256 x 64 cells took 156 us for 129, 240 x 320 x 96
+// 360 for 298.  Planes per workgroup at the first size, events around the launches: 4 134 us, 8 141,
+// 13 (march_planes) 129, 16 136.
 template <int NC, bool WNL = false, int G = kGeoAny>
-__global__ void __launch_bounds__(256, G == kGeoPlane ? 3 : (NC < 4 ? 4 : 1)) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
+__global__ void __launch_bounds__(256, G == kGeoPlane ? 3 : 1) k_dif_km(Dims d, int kc, const double* __restrict__ pdI,
                                                 const double* __restrict__ pdJ,
                                                 const double* __restrict__ pdK,
                                                 const double* __restrict__ jq12,
