@@ -817,6 +817,12 @@ int fvm_profile_get(fvm_ctx* c, char* names, double* ms, long* calls, int cap) {
   return q;
 }
 
+int fvm_geometry_form(fvm_ctx* c, int* form) {
+  if (!c || !form) return FVM_ERR_ARG;
+  *form = c->plane ? kGeoPlane : (c->xz_zero ? kGeoXz0 : kGeoAny);
+  return FVM_OK;
+}
+
 int fvm_divergence(fvm_ctx* c, double* out) {
   if (!c || !out) return FVM_ERR_ARG;
   return fvm_k_div_norm(c, out);

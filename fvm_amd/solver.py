@@ -144,6 +144,14 @@ class Solver3D:
         capi.check(self.L.fvm_divergence(self.h, capi._dptr(out)), "divergence")
         return {"max": float(out[0]), "mean": float(out[1]), "rel": float(out[2])}
 
+    @property
+    def geometry_form(self):
+        """What the kernels take the metrics from: "stored", "stored, xi_z = eta_z = 0" or "plane"
+        (formed anew from one plane's derivatives); results do not depend on it."""
+        f = ctypes.c_int()
+        capi.check(self.L.fvm_geometry_form(self.h, ctypes.byref(f)), "geometry_form")
+        return ("stored", "stored, xi_z = eta_z = 0", "plane")[f.value]
+
     # kernel timing ----------------------------------------------------------------------
     def profile(self, on=True):
         capi.check(self.L.fvm_profile_enable(self.h, 1 if on else 0), "profile_enable")

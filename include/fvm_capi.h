@@ -290,6 +290,12 @@ int fvm_calccoef(fvm_ctx* ctx, fvm_step_info* info);    /* CALCCOEF (calccoef.f9
  * fluxes, which the next step recomputes anyway. */
 int fvm_divergence(fvm_ctx* ctx, double* out);
 
+/* The geometry the kernels of a context work with: 0 the stored metrics, 1 the same with
+ * xi_z = eta_z = 0 left out (a grid extruded along z), 2 metrics formed anew per cell from one
+ * plane's derivatives (extruded grids from 2^19 cells, ghosts included).  Results do not depend on
+ * it.  Setting FVM_DJAC or a metric ends form 2. */
+int fvm_geometry_form(fvm_ctx* ctx, int* form);
+
 /* fvm_calccoef without any device allocation: the same kernels and results, with the CFL and
  * force partial sums in a static device array of 1 MiB (131072 doubles) per GPU instead of the
  * context's reduction buffer.  No counterpart in the reference; it is for callers that cannot
