@@ -711,6 +711,9 @@ int scan_stage_chunks(FvmCtx* c, const AFArgs& A, int* iters) {
 int fvm_af_scan_setup(FvmCtx* c) {
   const Dims d = c->d;
   hipStream_t st = c->stream;
+  // bytes of a number of the chunk passes: FP64 sweeps before FP32 pressure corrections, the FP32
+  // change form, or none
+  const size_t eb = fp32_pressure(c) ? sizeof(double) : (c->prm.af_mode == 2 ? sizeof(float) : 0);
   long nbnd = 0;
   // the factor arrays hold the natural (I) and the padded J-line-major (J) layouts
   const long ne = std::max((long)d.n, scan_jline_elems(d.ni, d.nj, d.nk));
@@ -754,9 +757,9 @@ int fvm_af_scan_setup(FvmCtx* c) {
       HIP_CHECK(hipGetLastError());
     }
   }
-  if (nbnd > c->nbnd) {
+  if (eb && nbnd > c->nbnd) {
     for (int q = 0; q < 2; ++q) {
-      HIP_CHECK(hipMalloc((void**)&c->bnd[q], nbnd * sizeof(double)));
+      HIP_CHECK(hipMalloc((void**)&c->bnd[q], nbnd * eb));
       c->allocs.push_back(c->bnd[q]);
     }
     c->nbnd = nbnd;
