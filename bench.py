@@ -266,8 +266,8 @@ KERNEL_BYTES_2D = {
     "k2_explicit": 8 * 26,
     # I- and J-line sweep: factors {1/D, beta, B, AN or AW} + per component {SU, x}
     "k2_sweep_i": 8 * 8, "k2_sweep_j": 8 * 8,
-    # stage-2 right-hand side: {u, v, 2 Re J/dt, cross weights, AE} -> {SU 2, x_in 2}, J-line-major
-    "k2_rhs2": 8 * 9,
+    # stage-2 right-hand side: {u, v, 2 Re J/dt, cross weights, AE} -> SU 2, J-line-major
+    "k2_rhs2": 8 * 7,
     # predictor correction: {u, v (J-line-major), S 2, J} -> {u, v}
     "k2_correct": 8 * 7,
     # residual: {p, RHS, D_E, D_N, J Q12} -> r (FP32 in the mixed form)

@@ -642,7 +642,7 @@ __global__ void __launch_bounds__(64) k2_sweep_pass(const Case2D* __restrict__ t
 // Stage-2 right-hand side SU = 2 Re DJAC / dt U + DD(U) with the stage-2 cross weights
 // (iter_u.f90:84-98) and BCU's folds with the stage-2 AW(1), AE(NI-1) (bcu.f90:15, 34), written
 // J-line-major for the J-line sweep: a workgroup forms a 32 x 32 (I x J) tile of interior cells
-// and transposes it through LDS.  FP64: the stage input goes along, with the BCU ghosts that the
+// and transposes it through LDS.  FP64: the stage input goes along for its BCU ghosts that the
 // sweep reads (line 0, the line ends J = 0, NJ).  AF32: instead of SU, the FP64 residual of the
 // stage input against the stage-2 line operator, in FP32.  As a stencil pass into a natural plane
 // and a transposition of it (and a pass of BCU and boundary lines before) the three launches took
@@ -720,10 +720,9 @@ __global__ void __launch_bounds__(256) k2_rhs2(const Case2D* __restrict__ tab,
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
       dst[a][o] = tile[a][lj][li];
-      if (!AF32) {  // the stage input and its BCU ghosts
+      if (!AF32) {  // the stage input's BCU ghosts
         const auto X = glb(cs.f[a ? F_TXV : F_TXU]);
         const double x = tile[NT - 2 + a][lj][li];
-        X[o] = x;
         if (i == 1) X[j] = -x + 2.0 * glb(cs.b[a ? B_VWALL : B_UWALL])[j];
         if (j == nj - 1) X[o - (nj - 1)] = x;  // J = 0
         if (j == 1) X[o + (nj - 1)] = x;       // J = NJ
