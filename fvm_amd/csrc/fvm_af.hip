@@ -1183,7 +1183,7 @@ int fvm_k_iter_t(FvmCtx* c) {
   A.ufar = c->tfar;
   const dim3 gi((d.ni - 1 + 63) / 64, (d.nj - 1 + 3) / 4, d.nk - 1);
   const int kc = march_planes(d, RK_RES);
-      const dim3 gk = march_grid(d, kc);
+  const dim3 gk = march_grid(d, kc);
   for (int s = 0; s < 3; ++s) {
     {
       ProfScope ps(c, "t_rhs");

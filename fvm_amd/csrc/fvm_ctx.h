@@ -70,11 +70,11 @@ struct FvmCtx {
   int af_iters[3] = {};
   // stage couplings that vanish identically on this grid (a: along the sweep, b: across it)
   bool af_zero_a[3] = {}, af_zero_b[3] = {};
-  double af_b_ratio[3] = {};
+  double af_b_ratio[3] = {};  // max over cells of (|b couplings|) / (2 Re J^-1/dt)
   bool xz_zero = false;       // xi_z = eta_z = 0 on every cell (metric kernels skip them)
   bool plane = false;         // and kGeoPlane's conditions hold
   PlaneGeo geo{};
-  bool dd2_zero = false;      // xi_z = eta_z = 0 around every cell: stage-3 cross terms vanish  // max over cells of (|b couplings|) / (2 Re J^-1/dt)
+  bool dd2_zero = false;      // xi_z = eta_z = 0 around every cell: stage-3 cross terms vanish
   // Thomas factors A, D, B of the K-line stage when its lines are independent
   double *tk_a = nullptr, *tk_d = nullptr, *tk_b = nullptr;
   // line-scan form of the I and J stages when the K couplings vanish: per stage the line

@@ -829,7 +829,7 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
   {
     ProfScope pk(c, "k_sgs_div");
     const int kc = march_planes(d, SD_RES);
-  const dim3 gs = march_grid(d, kc);
+    const dim3 gs = march_grid(d, kc);
     auto kern = c->plane ? k_sgs_div<kGeoPlane>
                         : (c->xz_zero ? k_sgs_div<kGeoXz0> : k_sgs_div<kGeoAny>);
     hipLaunchKernelGGL(kern, gs, kBlk, 0, st, d, kc, (const double* const*)m, c->filt2, c->scal + 0,
@@ -851,7 +851,7 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
     hipLaunchKernelGGL(k_nut, grid1(d.n, 256), dim3(256), 0, st, d, c->scal + 1, c->filt2,
                        c->mag, c->kappa);
     const int kc = march_planes(d, SD_RES);
-  const dim3 gs = march_grid(d, kc);
+    const dim3 gs = march_grid(d, kc);
     hipLaunchKernelGGL(k_sgs_t_div, gs, kBlk, 0, st, d, kc, (const double* const*)m, c->kappa,
                        c->dtd[0], c->dtd[1], c->dtd[2], c->djac, c->adv, c->sgst);
     HIP_CHECK(hipGetLastError());
