@@ -275,6 +275,9 @@ KERNEL_BYTES_2D = {
     # projection: {p, J, 4 metrics, u, v} -> {u, v, S 2}
     "k2_project": 8 * 12,
 }
+# FP32 Poisson corrections alone (--ens-form mixed-poisson): the FP64 sweeps go by chunk passes, with
+# the previous pass's x
+KERNEL_BYTES_2D_P32 = dict(KERNEL_BYTES_2D, k2_sweep_i=8 * 10, k2_sweep_j=8 * 10)
 # the FP32 change form of the AF sweeps (--ens-form mixed): phase A and the stage-2
 # right-hand side read AE / AN instead of 2 Re J/dt and store the residual in FP32; the sweeps
 # move the same operands in FP32, with the previous pass's x; the correction adds the FP32 change
@@ -371,7 +374,8 @@ def run_ensemble(a, log):
         log(f"  {k:16s} {ms:9.3f} ms {calls:6d} launches {ms / calls * 1e3:9.1f} us/launch "
             f"({100 * ms / tot:.1f}%)")
     rows = []
-    for k, nb in (KERNEL_BYTES_2D_AF32 if a.ens_form == "mixed" else KERNEL_BYTES_2D).items():
+    for k, nb in {"mixed": KERNEL_BYTES_2D_AF32,
+                  "mixed-poisson": KERNEL_BYTES_2D_P32}.get(a.ens_form, KERNEL_BYTES_2D).items():
         if k in prof:
             ms, calls = prof[k]
             avg = ms / calls * 1e-3

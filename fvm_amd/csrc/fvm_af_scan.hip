@@ -608,7 +608,10 @@ int scan_unpack(FvmCtx* c, int nc, const ScanBufs<T>& B) {
 // chunks are for grids whose wavefronts do not fill the chip.  I and J stage with chunks of 8, 16 and
 // 32 lines, us: 128 x 256 cells (768 lines of u, v, w in the I stage) 16 + 26, 20 + 28, 29 + 40;
 // 96 x 128 x 32 (12288) 20 + 20, 21 + 21, 29 + 29; 149 x 208 x 40 (24960) 43 + 48, 38 + 46, 50 + 54;
-// 240 x 320 x 96 (92160) 191 + 227, 175 + 207, 165 + 196.
+// 240 x 320 x 96 (92160) 191 + 227, 175 + 207, 165 + 196.  Where the dominance is weak the lead-ins
+// are most of the plane, and a sweep takes longer, but not as long as by passes (both stages, us):
+// 192 x 256 x 64 cells 336 by passes and 293 at Re 5, dt 0.05, 361 and 328 at Re 1, dt 0.1;
+// 240 x 320 x 96 974 and 515 at Re 20, dt 0.05, 1024 and 571 at Re 1, dt 0.02.
 int scan_lines(long lines) {
   return lines <= 8 * 2048L ? 8 : (lines <= 16 * 4096L ? 16 : 32);
 }
