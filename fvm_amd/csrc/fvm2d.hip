@@ -217,7 +217,7 @@ __device__ inline void bcu_ghosts_wave(P F, int ni, int nj, int sj, B uwall, B u
 // sweeps of batches with FP32 pressure corrections.  Those round the residual to FP32, so that a
 // velocity that differs in its last bit moves the pressure by 1e-9 to 1e-7 of its norm (RESIMAX 1e-8),
 // and the one-pass sweeps give other last bits: the pressure of a run would no longer be that of an
-// earlier build.  A chunk of SW_C lines takes the
+// earlier version.  A chunk of SW_C lines takes the
 // line before it from the preceding chunk's last line of the previous pass (block Jacobi across
 // chunks; the stage input's, which has no change, in the first pass).  Each pass contracts the chunk-boundary error by rho^SW_C;
 // a pass after the first re-solves a chunk's lines only until a line stops changing (max change

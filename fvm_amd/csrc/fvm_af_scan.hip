@@ -798,7 +798,7 @@ int fvm_af_scan_stage(FvmCtx* c, int s, const AFArgs& A, int* iters, bool temp, 
     return s == 0 ? chunks_by_rows<0, float>(c, A, iters) : chunks_by_rows<1, float>(c, A, iters);
   }
   // One-pass sweeps give other last bits than chunk passes, with which a run before FP32 pressure
-  // corrections would no longer have the pressure of an earlier build.  A slab of 128 x 256 cells
+  // corrections would no longer have the pressure of an earlier version.  A slab of 128 x 256 cells
   // takes 62 us for the two stages by passes and 39 by one pass.  T feeds no pressure.
   if (!temp && fp32_pressure(c))
     return s == 0 ? chunks_by_rows<0, double>(c, A, iters) : chunks_by_rows<1, double>(c, A, iters);

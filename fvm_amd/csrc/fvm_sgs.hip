@@ -808,7 +808,7 @@ int fvm_k_sgs(FvmCtx* c, bool sgs_out, bool nl_update) {
     ProfScope pk(c, "k_lm");
     // The planes of a workgroup group the sums of LM and MM.  Between FP64 line sweeps and FP32
     // pressure corrections the last bit of C reaches the pressure (fp32_pressure): 16 planes on every
-    // grid, as in earlier builds (32 x 64 x 16 cells: 68 us against 17).
+    // grid, as in earlier versions (32 x 64 x 16 cells: 68 us against 17).
     const int kc = fp32_pressure(c) && c->prm.af_mode != 2 ? 16 : march_planes(d, LM_RES);
     const dim3 gl = march_grid(d, kc);
     auto kern = c->plane ? k_lm<kGeoPlane> : (c->xz_zero ? k_lm<kGeoXz0> : k_lm<kGeoAny>);

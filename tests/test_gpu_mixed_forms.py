@@ -1,9 +1,9 @@
-"""Runs whose FP64 part feeds an FP32 one keep the results of earlier builds: the FP32 part rounds a
+"""Runs whose FP64 part feeds an FP32 one keep the results of earlier versions: the FP32 part rounds a
 residual of the FP64 fields, so operands that differ in their last bit come out 1e-12 to 1e-7 apart.
-The fields of a few steps against those recorded on an MI355X with the build in which every form took
+The fields of a few steps against those recorded on an MI355X with the version in which every form took
 its lines by chunk passes, the pressure lines by reduction and the model's sums by 16 planes (python
-tests/test_gpu_mixed_forms.py writes the records of the build at hand).  Equality is exact: runs of
-one build repeat to the bit, and so must the same operations in the same order."""
+tests/test_gpu_mixed_forms.py writes the records of the version at hand).  Equality is exact: runs of
+one version repeat to the bit, and so must the same operations in the same order."""
 import os
 
 import numpy as np
@@ -76,7 +76,7 @@ def _path(form):
 
 
 @pytest.mark.parametrize("form", FORMS)
-def test_fields_of_earlier_builds(form):
+def test_fields_of_earlier_versions(form):
     got = FORMS[form]()
     with np.load(_path(form), allow_pickle=False) as z:
         assert sorted(z.files) == sorted(got)
